@@ -1,0 +1,446 @@
+"""The work this library is used for, as measurable cases.
+
+listed() names the cases, draw() gives more of the same ranges, prepare() makes what a
+caller holds before the call (context, circuit, target, inputs on the GPU), run() is one
+pass through the public entry points, work() the bytes and operations a pass cannot do
+without, exact() the same outputs from plain torch in 64 bits.
+
+Kinds (the field "kind"):
+  single   cost and gradient of one parameter vector through the decomposition class,
+           host arrays in and out: one step of a caller's own optimiser
+  cost     costs of a batch of parameter vectors resident on the GPU: line-search probes,
+           agent populations, multi-start screening
+  grad     costs and gradients of such a batch
+  apply    the circuit applied in place to a batch of matrices on the GPU
+  deriv    all derivative matrices of the circuit at one point, on the GPU
+  descend  the first evaluations of many decompositions of one circuit, each on its own
+           target from its own random start, host arrays in and out: the screening
+           stage that keeps the most promising starts
+  train    a stretch of the warm-start network's training ended by a checkpoint
+"""
+import math
+import os
+import sys
+
+import numpy as np
+import torch
+
+_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+_PKG = os.path.join(_ROOT, "sequential-quantum-gate-decomposer_amd")
+if _PKG not in sys.path:
+    sys.path.insert(0, _PKG)
+
+U3, RX, RY, RZ, CNOT, CZ, CRY = 7, 9, 8, 10, 5, 4, 14
+_PARAMS = {U3: 3, RX: 1, RY: 1, RZ: 1, CRY: 1, CNOT: 0, CZ: 0}
+
+
+# ---- cases -------------------------------------------------------------------
+
+
+def listed():
+    return [
+        # one optimiser step of the smallest circuits users decompose (4 qubits, 84 angles)
+        {"name": "single_4q", "kind": "single", "n": 4, "layers": 12, "circuit": "ansatz"},
+        # one optimiser step at 8 qubits and 264 angles: the latency a scipy-style caller sees
+        {"name": "single_8q", "kind": "single", "n": 8, "layers": 40, "circuit": "ansatz"},
+        # the headline: 512 probes of the 8-qubit 40-layer circuit against a 256 x 256 target
+        {"name": "cost_8q_b512", "kind": "cost", "n": 8, "layers": 40, "circuit": "ansatz", "cols": 256,
+         "offset": 0, "batch": 512, "f32": False},
+        # complex64 screening at the largest register the batched path takes
+        {"name": "cost_10q_b64_f32", "kind": "cost", "n": 10, "layers": 60, "circuit": "ansatz", "cols": 1024,
+         "offset": 0, "batch": 64, "f32": True},
+        # gradients of the headline batch: many-start gradient descent
+        {"name": "grad_8q_b512", "kind": "grad", "n": 8, "layers": 40, "circuit": "ansatz", "cols": 256,
+         "offset": 0, "batch": 512, "f32": False},
+        # a rectangular target with a trace offset, every gate kind, an odd batch, complex64
+        {"name": "grad_8q_rect_b37_f32", "kind": "grad", "n": 8, "layers": 32, "circuit": "mixed", "cols": 160,
+         "offset": 80, "batch": 37, "f32": True},
+        # gradients at the largest register, a small batch
+        {"name": "grad_10q_b16", "kind": "grad", "n": 10, "layers": 60, "circuit": "ansatz", "cols": 1024,
+         "offset": 0, "batch": 16, "f32": False},
+        # a batch of unitaries built or advanced on the GPU, its own angles per matrix
+        {"name": "apply_8q_b512", "kind": "apply", "n": 8, "layers": 40, "circuit": "ansatz", "cols": 256,
+         "batch": 512, "f32": False},
+        # registers above the tile limit: a few columns of a 12-qubit register, many at once
+        {"name": "apply_12q_c48_b24", "kind": "apply", "n": 12, "layers": 60, "circuit": "ansatz", "cols": 48,
+         "batch": 24, "f32": False},
+        # the derivative matrices of the 8-qubit circuit (264 of 256 x 256)
+        {"name": "deriv_8q", "kind": "deriv", "n": 8, "layers": 40, "circuit": "ansatz"},
+        # many 4-qubit decompositions from random starts, the screening evaluations
+        {"name": "descend_4q_2048", "kind": "descend", "n": 4, "layers": 12, "circuit": "ansatz", "runs": 2048,
+         "evals": 24},
+        # the warm-start network at its configured size and batch
+        {"name": "train_4q_b1024", "kind": "train", "n": 4, "layers": 12, "batch": 1024, "steps": 32,
+         "hidden": 1024},
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+# matrix elements times gate layers of the largest drawn batch of its kind
+_MOST = {"cost": 512 * 65536 * 40, "grad": 256 * 65536 * 40, "apply": 512 * 65536 * 40, "deriv": 264 * 65536 * 40}
+
+
+def draw(rng):
+    kind = rng.choice(["single", "cost", "cost", "grad", "grad", "apply", "deriv", "descend", "train"])
+    circuit = rng.choice(["ansatz", "ansatz", "mixed"])
+    if kind == "single":
+        n = rng.randint(2, 8)
+        return {"kind": kind, "n": n, "layers": _log_int(rng, max(2, n), 5 * n), "circuit": circuit}
+    if kind in ("cost", "grad"):
+        n = rng.randint(3, 10)
+        layers = _log_int(rng, 2 * n, 6 * n)
+        d = 1 << n
+        cols = d if rng.random() < 0.6 else rng.randint(d // 2, d)
+        offset = rng.randint(0, d - cols)
+        most = max(1, min(4096, _MOST[kind] // (d * cols * layers)))
+        return {"kind": kind, "n": n, "layers": layers, "circuit": circuit, "cols": cols, "offset": offset,
+                "batch": _log_int(rng, 1, most), "f32": rng.random() < 0.4}
+    if kind == "apply":
+        n = rng.randint(3, 13)
+        layers = _log_int(rng, 2 * n, 5 * n)
+        cols = _log_int(rng, 1, min(1 << n, 512))
+        most = max(1, min(4096, _MOST[kind] // ((1 << n) * cols * layers)))
+        return {"kind": kind, "n": n, "layers": layers, "circuit": circuit, "cols": cols,
+                "batch": _log_int(rng, 1, most), "f32": rng.random() < 0.4}
+    if kind == "deriv":
+        n = rng.randint(3, 8)
+        return {"kind": kind, "n": n, "layers": _log_int(rng, 2 * n, 5 * n), "circuit": circuit}
+    if kind == "descend":
+        n = rng.randint(3, 5)
+        return {"kind": kind, "n": n, "layers": rng.randint(2 * n, 3 * n), "circuit": "ansatz",
+                "runs": _log_int(rng, 64, {3: 4096, 4: 2048, 5: 512}[n]), "evals": rng.randint(8, 24)}
+    n = rng.randint(3, 4)
+    return {"kind": "train", "n": n, "layers": rng.randint(2 * n, 3 * n), "batch": _log_int(rng, 64, 1024),
+            "steps": _log_int(rng, 4, 32), "hidden": rng.choice([256, 512, 1024])}
+
+
+# ---- inputs (plain numpy / torch) ---------------------------------------------
+
+
+def _gates(case):
+    """(gates, parameter count): rows of (type, target, control, first parameter)."""
+    n, layers = case["n"], case["layers"]
+    rng = np.random.default_rng(1000 * n + layers)
+    rows, P = [], 0
+
+    def add(t, target, control=-1):
+        nonlocal P
+        rows.append((t, target, control, P if _PARAMS[t] else 0))
+        P += _PARAMS[t]
+
+    for q in range(n):
+        add(U3, q)
+    for k in range(layers):
+        a = int(rng.integers(0, n - 1))
+        if case.get("circuit", "ansatz") == "ansatz":
+            add(CNOT, a, a + 1)
+            add(U3, a)
+            add(U3, a + 1)
+        else:
+            b = int(rng.integers(0, n - 1))
+            b = b if b < a else b + 1
+            add((CNOT, CZ, CRY)[k % 3], a, b)
+            add((RX, RY, RZ, U3)[k % 4], a)
+            add((U3, RZ, RY)[k % 3], b)
+    return rows, P
+
+
+def _haar(d, rng):
+    z = rng.standard_normal((d, d)) + 1j * rng.standard_normal((d, d))
+    q, r = np.linalg.qr(z)
+    ph = np.diag(r) / np.abs(np.diag(r))
+    return np.ascontiguousarray(q * ph)
+
+
+def _angles(rng, *shape):
+    return rng.uniform(0.0, 2.0 * np.pi, size=shape)
+
+
+def _kernel(t, p):
+    """Entries k00, k01, k10, k11 of a gate's 2 x 2 kernel from raw angles p (B, ...)."""
+    e = lambda re, im: torch.complex(re, im)[:, None, None, None]  # noqa: E731
+    z = torch.zeros_like(p[:, 0])
+    s, c = torch.sin(p[:, 0]), torch.cos(p[:, 0])
+    if t == U3:
+        ph, la = p[:, 1], p[:, 2]
+        return (e(c, z), e(-s * torch.cos(la), -s * torch.sin(la)), e(s * torch.cos(ph), s * torch.sin(ph)),
+                e(c * torch.cos(ph + la), c * torch.sin(ph + la)))
+    if t == RX:
+        return e(c, z), e(z, -s), e(z, -s), e(c, z)
+    if t == RZ:
+        return e(c, -s), e(z, z), e(z, z), e(c, s)
+    return e(c, z), e(-s, z), e(s, z), e(c, z)  # RY, CRY
+
+
+def _one(M, n, gate, kern, zero_control0=False):
+    """A gate (or, with kern, its 2 x 2 kernel replaced) applied to M (B, 2^n, m)."""
+    t, q, ctl, _ = gate
+    d = 1 << n
+    rows = torch.arange(d, device=M.device)
+    if t == CNOT:
+        return M[:, torch.where((rows >> ctl) & 1 == 1, rows ^ (1 << q), rows)]
+    if t == CZ:
+        both = ((rows >> ctl) & 1) * ((rows >> q) & 1)
+        return M * (1 - 2 * both).to(M.dtype)[None, :, None]
+    V = M.reshape(M.shape[0], d >> (q + 1), 2, 1 << q, M.shape[2])
+    x0, x1 = V[:, :, 0], V[:, :, 1]
+    k00, k01, k10, k11 = kern
+    Y = torch.stack((k00 * x0 + k01 * x1, k10 * x0 + k11 * x1), dim=2).reshape(-1, d, M.shape[2])
+    if t == CRY:
+        on = ((rows >> ctl) & 1 == 1)[None, :, None]
+        Y = torch.where(on, Y, torch.zeros_like(Y) if zero_control0 else M)
+    return Y
+
+
+def _apply(gates, n, p, M):
+    """The circuit at raw angles p (B, P) applied to M (B or 1, 2^n, m)."""
+    for g in gates:
+        k = _kernel(g[0], p[:, g[3]:g[3] + _PARAMS[g[0]]]) if _PARAMS[g[0]] else None
+        M = _one(M, n, g, k)
+    return M
+
+
+def _device():
+    return "cuda" if torch.cuda.is_available() else "cpu"
+
+
+def _inputs(case, seed):
+    """Host inputs of a case, from the seed alone."""
+    rng = np.random.default_rng([seed, 77])
+    gates, P = _gates(case)
+    kind, d = case["kind"], 1 << case["n"]
+    if kind == "single":
+        return {"gates": gates, "P": P, "U": _haar(d, rng), "p": _angles(rng, P)}
+    if kind in ("cost", "grad"):
+        U = np.ascontiguousarray(_haar(d, rng)[:, :case["cols"]])
+        return {"gates": gates, "P": P, "U": U, "p": _angles(rng, case["batch"], P)}
+    if kind == "apply":
+        return {"gates": gates, "P": P, "p": _angles(rng, case["batch"], P)}
+    if kind == "deriv":
+        return {"gates": gates, "P": P, "U": _haar(d, rng), "p": _angles(rng, P)}
+    if kind == "descend":
+        # reachable targets: the adjoints of the circuit at hidden angles
+        hidden = torch.from_numpy(_angles(rng, case["runs"], P)).to(_device())
+        eye = torch.eye(d, dtype=torch.complex128, device=hidden.device)[None]
+        V = _apply(gates, case["n"], hidden, eye)
+        T = V.conj().transpose(1, 2).contiguous().cpu().numpy()
+        return {"gates": gates, "P": P, "targets": T, "p": _angles(rng, case["runs"], P)}
+    # train: unitaries of the circuit as features, sin / cos of their angles as labels
+    count = case["batch"] * case["steps"]
+    th = torch.from_numpy(_angles(rng, count, P)).to(_device())
+    eye = torch.eye(d, dtype=torch.complex128, device=th.device)[None]
+    V = torch.cat([_apply(gates, case["n"], th[s:s + 4096], eye) for s in range(0, count, 4096)]).reshape(count, -1)
+    X = (torch.cat([V.real, V.imag], dim=1) * math.sqrt(d)).float().contiguous()
+    Y = torch.cat([torch.sin(th), torch.cos(th)], dim=1).float().contiguous()
+    dims = [2 * d * d] + 3 * [case["hidden"]] + [2 * P]
+    w = [np.concatenate([rng.standard_normal((dims[i + 1], dims[i])).ravel() * math.sqrt(2.0 / dims[i]),
+                         np.zeros(dims[i + 1])]) for i in range(4)]
+    return {"P": P, "X": X, "Y": Y, "dims": dims, "w": np.concatenate(w).astype(np.float32)}
+
+
+def _matrices(case, seed):
+    """The matrices an apply case starts from: a batch of random columns of unit norm."""
+    gen = torch.Generator(device=_device()).manual_seed(seed * 2 + 1)
+    shape = (case["batch"], 1 << case["n"], case["cols"])
+    M = torch.randn(shape, dtype=torch.complex128, device=_device(), generator=gen)
+    M /= math.sqrt(1 << case["n"])
+    return M.to(torch.complex64) if case["f32"] else M
+
+
+# ---- the framework's side ----------------------------------------------------
+
+
+def prepare(case, seed):
+    from squander_hip import _native as nat
+    from squander_hip.circuit import Circuit
+    from squander_hip.decomposition import N_Qubit_Decomposition_custom
+    from squander_hip.mlp import WarmStartMLP
+    from squander_hip.optimizer import default_options
+
+    kind, n = case["kind"], case["n"]
+    x = _inputs(case, seed)
+    s = {"kind": kind, "case": case}
+    if kind == "single":
+        s["dec"] = N_Qubit_Decomposition_custom(x["U"])
+        s["dec"].set_Gate_Structure(Circuit.from_gate_array(n, x["gates"]))
+        s["p"] = x["p"]
+        return s
+    s["ctx"] = ctx = nat.Context(0)
+    s["prec"] = nat.PREC_F32 if case.get("f32") else nat.PREC_F64
+    if kind != "train":
+        ctx.set_circuit(n, np.asarray(x["gates"], dtype=np.int32))
+    if kind in ("cost", "grad"):
+        ctx.set_target(x["U"])
+        ctx.set_trace_offset(case["offset"])
+        s["p"] = torch.from_numpy(x["p"]).cuda()
+        s["f"] = torch.empty(case["batch"], dtype=torch.float64, device="cuda")
+        if kind == "grad":
+            s["g"] = torch.empty((case["batch"], x["P"]), dtype=torch.float64, device="cuda")
+    elif kind == "apply":
+        s["p"] = torch.from_numpy(x["p"]).cuda()
+        s["M"] = _matrices(case, seed)
+    elif kind == "deriv":
+        s["p"] = torch.from_numpy(x["p"]).cuda()
+        s["U"] = torch.from_numpy(x["U"]).cuda()
+        s["D"] = torch.empty((x["P"],) + x["U"].shape, dtype=torch.complex128, device="cuda")
+    elif kind == "descend":
+        s["targets"], s["x0"] = x["targets"], x["p"]
+        s["index"] = np.arange(case["runs"], dtype=np.int32)
+        s["options"] = default_options(n, max_inner_iterations=case["evals"], max_outer_iterations=1)
+    else:
+        s["net"] = WarmStartMLP(ctx, x["dims"][0], case["hidden"], 3, x["dims"][-1], seed=seed)
+        s["net"].set_params(x["w"])
+        s["X"], s["Y"] = x["X"].cuda(), x["Y"].cuda()
+    torch.cuda.synchronize()
+    return s
+
+
+def run(s):
+    kind, case = s["kind"], s["case"]
+    if kind == "single":
+        return s["dec"].Optimization_Problem_Combined(s["p"])
+    ctx = s["ctx"]
+    L, h = ctx._L, ctx.h
+    if kind == "cost":
+        ctx.check(L.sqh_optimization_problem_batch_dev(h, s["p"].data_ptr(), case["batch"], s["prec"],
+                                                       s["f"].data_ptr()))
+        return s["f"]
+    if kind == "grad":
+        ctx.check(L.sqh_optimization_problem_combined_batch_dev(h, s["p"].data_ptr(), case["batch"], s["prec"],
+                                                                s["f"].data_ptr(), s["g"].data_ptr()))
+        return s["f"], s["g"]
+    if kind == "apply":
+        d, m = 1 << case["n"], case["cols"]
+        ctx.check(L.sqh_apply_to_dev(h, s["p"].data_ptr(), s["p"].shape[1], s["M"].data_ptr(), d, m, m, d * m,
+                                     case["batch"], int(case["f32"])))
+        return s["M"]
+    if kind == "deriv":
+        d = 1 << case["n"]
+        ctx.check(L.sqh_apply_derivate_to_dev(h, s["p"].data_ptr(), s["U"].data_ptr(), d, d, d, s["D"].data_ptr()))
+        return s["D"]
+    if kind == "descend":
+        from squander_hip.optimizer import decompose_batch
+        r = decompose_batch(ctx, s["targets"], s["index"], s["x0"], s["options"])
+        return r["x"], r["f"]
+    B = case["batch"]
+    for k in range(case["steps"]):
+        s["net"].train_step_dev(s["X"][k * B:].data_ptr(), s["Y"][k * B:].data_ptr(), B, 1e-3, want_loss=False)
+    return s["net"].get_params()
+
+
+# ---- work and exact values ---------------------------------------------------
+
+
+def work(case):
+    """Arithmetic: a parametric gate's real rotation, 6 flop per matrix element (3 where
+    it is controlled), its phases merged into neighbours; a gradient is a forward pass,
+    an adjoint pass and the correlations; the network 2 flop per weight and pass."""
+    gates, P = _gates(case)
+    kind, d = case["kind"], 1 << case["n"]
+    per = sum({U3: 6.0, RX: 6.0, RY: 6.0, RZ: 0.0, CRY: 3.0}.get(g[0], 0.0) for g in gates)
+    z = 8 if case.get("f32") else 16
+    if kind == "single":
+        return {"bytes": 16.0 * d * d + 16.0 * P, "flops": 3 * per * d * d}
+    if kind in ("cost", "grad"):
+        B, m = case["batch"], case["cols"]
+        g = 1 if kind == "grad" else 0
+        return {"bytes": z * d * m + 8.0 * B * (P * (1 + g) + 1), "flops": (1 + 2 * g) * per * d * m * B}
+    if kind == "apply":
+        B, m = case["batch"], case["cols"]
+        return {"bytes": 2.0 * z * d * m * B + 8.0 * B * P, "flops": per * d * m * B}
+    if kind == "deriv":
+        # a derivative shares the circuit up to its gate with the others
+        return {"bytes": 16.0 * d * d * (P + 1), "flops": 0.5 * per * d * d * P}
+    if kind == "descend":
+        R = case["runs"]
+        return {"bytes": 16.0 * R * d * d + 16.0 * R * P, "flops": 3 * per * d * d * R * case["evals"]}
+    dims = [2 * d * d] + 3 * [case["hidden"]] + [2 * P]
+    w = sum(dims[i] * dims[i + 1] for i in range(4))
+    B, K = case["batch"], case["steps"]
+    first = dims[0] * dims[1]  # its input takes no gradient
+    return {"bytes": K * (4.0 * B * (dims[0] + dims[-1]) + 24.0 * w) + 4.0 * w,
+            "flops": K * 2.0 * B * (3 * w - first)}
+
+
+def _exact_costs(case, x, grad):
+    U = torch.from_numpy(x["U"]).to(_device())[None]
+    p = torch.from_numpy(x["p"]).to(_device()).reshape(-1, x["P"])
+    n, m, off = case["n"], U.shape[2], case.get("offset", 0)
+    step = max(1, (1 << 22) // (U.shape[1] * m)) if grad else max(1, (1 << 26) // (U.shape[1] * m))
+    cs = torch.arange(m, device=U.device)
+    fs, gs = [], []
+    for s in range(0, p.shape[0], step):
+        q = p[s:s + step].clone().requires_grad_(grad)
+        with torch.set_grad_enabled(grad):
+            f = 1.0 - _apply(x["gates"], n, q, U)[:, cs + off, cs].real.sum(dim=1) / m
+            if grad:
+                gs.append(torch.autograd.grad(f.sum(), q)[0])
+        fs.append(f.detach())
+    f = torch.cat(fs)
+    return (f, torch.cat(gs)) if grad else f
+
+
+def _exact_derivs(case, x):
+    n = case["n"]
+    M = torch.from_numpy(x["U"]).to(_device())[None]
+    p = torch.from_numpy(x["p"]).to(_device())[None]
+    D = M[:0]
+    for g in x["gates"]:
+        q = p[:, g[3]:g[3] + _PARAMS[g[0]]]
+        k = _kernel(g[0], q) if _PARAMS[g[0]] else None
+        D = _one(D, n, g, k)
+        new = []
+        for j in range(_PARAMS[g[0]]):
+            one = torch.zeros_like(q)
+            one[:, j] = 1.0
+            dk = torch.autograd.functional.jvp(lambda a: _kernel(g[0], a), q, one)[1]
+            new.append(_one(M, n, g, dk, zero_control0=True))
+        M = _one(M, n, g, k)
+        D = torch.cat([D] + new)
+    return D
+
+
+def _exact_training(case, x):
+    dev = _device()
+    B, dims = case["batch"], x["dims"]
+    w = torch.from_numpy(x["w"]).to(dev).double()
+    X, Y = x["X"].to(dev).double(), x["Y"].to(dev).double()
+    m, v = torch.zeros_like(w), torch.zeros_like(w)
+    for k in range(case["steps"]):
+        w.requires_grad_(True)
+        h, o = X[k * B:(k + 1) * B], 0
+        for i in range(4):
+            a, b = dims[i], dims[i + 1]
+            h = h @ w[o:o + a * b].reshape(b, a).t() + w[o + a * b:o + a * b + b]
+            o += a * b + b
+            if i < 3:
+                h = torch.nn.functional.gelu(h)
+        g, = torch.autograd.grad(((h - Y[k * B:(k + 1) * B]) ** 2).mean(), w)
+        w = w.detach()
+        m = 0.9 * m + 0.1 * g
+        v = 0.999 * v + 0.001 * g * g
+        w = w - 1e-3 * (m / (1 - 0.9 ** (k + 1))) / ((v / (1 - 0.999 ** (k + 1))).sqrt() + 1e-8)
+    return w
+
+
+def exact(case, seed):
+    """None for descend: line searches branch on their values, so a plain restatement
+    of the optimiser in other arithmetic is another run."""
+    kind = case["kind"]
+    if kind == "descend":
+        return None
+    x = _inputs(case, seed)
+    if kind == "single":
+        f, g = _exact_costs(case, x, True)
+        return float(f[0]), g[0]
+    if kind in ("cost", "grad"):
+        return _exact_costs(case, x, kind == "grad")
+    if kind == "apply":
+        M = _matrices(case, seed).to(torch.complex128)
+        return _apply(x["gates"], case["n"], torch.from_numpy(x["p"]).to(M.device), M)
+    if kind == "deriv":
+        return _exact_derivs(case, x)
+    return _exact_training(case, x)
