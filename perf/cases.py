@@ -15,7 +15,8 @@ Kinds (the field "kind"):
   deriv    all derivative matrices of the circuit at one point, on the GPU
   descend  the first evaluations of many decompositions of one circuit, each on its own
            target from its own random start, host arrays in and out: the screening
-           stage that keeps the most promising starts
+           stage that keeps the most promising starts.  Few evaluations, so that a
+           change of rounding does not yet move the line searches onto other paths
   train    a stretch of the warm-start network's training ended by a checkpoint
 """
 import math
@@ -68,7 +69,7 @@ def listed():
         {"name": "deriv_8q", "kind": "deriv", "n": 8, "layers": 40, "circuit": "ansatz"},
         # many 4-qubit decompositions from random starts, the screening evaluations
         {"name": "descend_4q_2048", "kind": "descend", "n": 4, "layers": 12, "circuit": "ansatz", "runs": 2048,
-         "evals": 24},
+         "evals": 6},
         # the warm-start network at its configured size and batch
         {"name": "train_4q_b1024", "kind": "train", "n": 4, "layers": 12, "batch": 1024, "steps": 32,
          "hidden": 1024},
@@ -111,7 +112,7 @@ def draw(rng):
     if kind == "descend":
         n = rng.randint(3, 5)
         return {"kind": kind, "n": n, "layers": rng.randint(2 * n, 3 * n), "circuit": "ansatz",
-                "runs": _log_int(rng, 64, {3: 4096, 4: 2048, 5: 512}[n]), "evals": rng.randint(8, 24)}
+                "runs": _log_int(rng, 64, {3: 4096, 4: 2048, 5: 512}[n]), "evals": rng.randint(4, 6)}
     n = rng.randint(3, 4)
     return {"kind": "train", "n": n, "layers": rng.randint(2 * n, 3 * n), "batch": _log_int(rng, 64, 1024),
             "steps": _log_int(rng, 4, 32), "hidden": rng.choice([256, 512, 1024])}
