@@ -248,6 +248,20 @@ __global__ void k_f32_to_bf16(const float* __restrict__ a, bf16* __restrict__ b,
     if (i < n) b[i] = (bf16)a[i];
 }
 
+// One layer's parameters between the padded device layout (W [np][kp], b [np]) and the
+// caller's flat one (W [no][ni], then b [no]).  The copy to or from the host is then one
+// contiguous transfer: copied row by row (hipMemcpy2D, a transfer per weight row) the
+// 2.8 M parameters of the 512-3x1024-168 network took 23 ms, packed they take 0.7 ms.
+__global__ __launch_bounds__(256) void k_pack_layer(float* __restrict__ W, float* __restrict__ b, int no, int ni,
+                                                    int kp, float* __restrict__ flat, bool to_flat) {
+    const long long nw = (long long)no * ni;
+    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nw + no) return;
+    float* p = i < nw ? &W[(i / ni) * kp + i % ni] : &b[i - nw];
+    if (to_flat) flat[i] = *p;
+    else *p = flat[i];
+}
+
 // Host launchers ------------------------------------------------------------------
 
 template <bool AT, bool BT, int EPI>
@@ -324,6 +338,13 @@ hipError_t mlp_adam(float* w, void* wb, const float* g, float* m, float* v, size
     const float c1 = 1.0f - powf(b1, (float)step), c2 = 1.0f - powf(b2, (float)step);
     hipLaunchKernelGGL(k_adam, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, w, (bf16*)wb, g, m, v, n, lr, b1,
                        b2, eps, c1, c2);
+    return hipGetLastError();
+}
+
+hipError_t mlp_pack_layer(float* W, float* b, int no, int ni, int kp, float* flat, bool to_flat, hipStream_t s) {
+    const long long n = (long long)no * ni + no;
+    hipLaunchKernelGGL(k_pack_layer, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, W, b, no, ni, kp, flat,
+                       to_flat);
     return hipGetLastError();
 }
 

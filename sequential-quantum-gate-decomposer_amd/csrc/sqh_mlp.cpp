@@ -25,6 +25,7 @@ hipError_t mlp_bias_grad(const float* dz, int ld, int B, int N, float* db, hipSt
 hipError_t mlp_out_grad(const float* dy, int B, int out, int ldy, int Bp, float* dyf, void* dyb, hipStream_t s);
 hipError_t mlp_adam(float* w, void* wb, const float* g, float* m, float* v, size_t n, float lr, float b1, float b2,
                     float eps, int step, hipStream_t s);
+hipError_t mlp_pack_layer(float* W, float* b, int no, int ni, int kp, float* flat, bool to_flat, hipStream_t s);
 hipError_t mlp_f32_to_bf16(const float* a, void* b, size_t n, hipStream_t s);
 }  // namespace sqh
 
@@ -41,6 +42,7 @@ struct sqh_mlp {
     std::vector<DevBuf> W, Wb, b, mW, vW, mb, vb, gW, gb;
     std::vector<DevBuf> H, Z, dZf, dZb;  // activations per layer (H[0] = input)
     DevBuf part;
+    DevBuf flat;                     // the parameters in the caller's flat layout
     int cap = 0;                     // padded batch the activation buffers hold
     int step = 0;
 
@@ -48,6 +50,7 @@ struct sqh_mlp {
         for (auto* v : {&W, &Wb, &b, &mW, &vW, &mb, &vb, &gW, &gb, &H, &Z, &dZf, &dZb})
             for (auto& x : *v) x.release();
         part.release();
+        flat.release();
     }
     hipStream_t st() const { return ctx->stream; }
 };
@@ -143,23 +146,23 @@ int for_each_layer(sqh_mlp* m, F&& f) {
 
 int copy_params(sqh_mlp* m, float* host, bool to_host, bool grads) {
     sqh_ctx* c = m->ctx;
-    return for_each_layer(m, [&](int l, long long off) -> int {
+    const size_t bytes = (size_t)sqh_mlp_param_count(m) * sizeof(float);
+    HIPTRY(c, m->flat.ensure(bytes));
+    if (!to_host) HIPTRY(c, hipMemcpyAsync(m->flat.p, host, bytes, hipMemcpyHostToDevice, m->st()));
+    int rc = for_each_layer(m, [&](int l, long long off) -> int {
         const int no = m->dim[l + 1], ni = m->dim[l], kp = m->dpad[l];
         DevBuf& Wd = grads ? m->gW[l] : m->W[l];
         DevBuf& bd = grads ? m->gb[l] : m->b[l];
-        if (to_host) {
-            HIPTRY(c, hipMemcpy2D(host + off, (size_t)ni * 4, Wd.p, (size_t)kp * 4, (size_t)ni * 4, no,
-                                  hipMemcpyDeviceToHost));
-            HIPTRY(c, hipMemcpy(host + off + (long long)no * ni, bd.p, (size_t)no * 4, hipMemcpyDeviceToHost));
-        } else {
-            HIPTRY(c, hipMemcpy2D(Wd.p, (size_t)kp * 4, host + off, (size_t)ni * 4, (size_t)ni * 4, no,
-                                  hipMemcpyHostToDevice));
-            HIPTRY(c, hipMemcpy(bd.p, host + off + (long long)no * ni, (size_t)no * 4, hipMemcpyHostToDevice));
+        HIPTRY(c, mlp_pack_layer(Wd.as<float>(), bd.as<float>(), no, ni, kp, m->flat.as<float>() + off, to_host,
+                                 m->st()));
+        if (!to_host)
             HIPTRY(c, mlp_f32_to_bf16(m->W[l].as<float>(), m->Wb[l].p, (size_t)m->dpad[l + 1] * kp, m->st()));
-            HIPTRY(c, hipStreamSynchronize(m->st()));
-        }
         return SQH_OK;
     });
+    if (rc) return rc;
+    if (to_host) HIPTRY(c, hipMemcpyAsync(host, m->flat.p, bytes, hipMemcpyDeviceToHost, m->st()));
+    HIPTRY(c, hipStreamSynchronize(m->st()));
+    return SQH_OK;
 }
 
 }  // namespace
@@ -235,6 +238,7 @@ long long sqh_mlp_param_count(const sqh_mlp* m) {
 int sqh_mlp_get_params(sqh_mlp* m, float* out) {
     if (!m || !out) return SQH_ERR_ARG;
     std::lock_guard<std::mutex> lk(m->ctx->mu);
+    HIPTRY(m->ctx, hipSetDevice(m->ctx->device));
     HIPTRY(m->ctx, hipStreamSynchronize(m->st()));
     return copy_params(m, out, true, false);
 }
@@ -242,6 +246,7 @@ int sqh_mlp_get_params(sqh_mlp* m, float* out) {
 int sqh_mlp_set_params(sqh_mlp* m, const float* in) {
     if (!m || !in) return SQH_ERR_ARG;
     std::lock_guard<std::mutex> lk(m->ctx->mu);
+    HIPTRY(m->ctx, hipSetDevice(m->ctx->device));
     HIPTRY(m->ctx, hipStreamSynchronize(m->st()));
     return copy_params(m, const_cast<float*>(in), false, false);
 }
