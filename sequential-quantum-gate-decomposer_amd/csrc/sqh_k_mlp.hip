@@ -2,34 +2,32 @@
 // BF16 weights/activations and FP32 accumulation on the gfx950 matrix cores
 // (v_mfma_f32_16x16x32_bf16), GELU hidden layers, mean-squared-error loss and Adam.
 //
-// GEMM convention: C[M][N] = sum_k A(m,k) B(k,n) with A(m,k) = A[m*lda+k] (or
-// A[k*lda+m] when AT) and B(k,n) = B[k*ldb+n] (or B[n*ldb+k] when BT).  A workgroup
-// of 4 wavefronts computes a 64x64 tile, each wavefront a 32x32 quarter as 2x2
-// MFMA 16x16 blocks, K advancing 32 per step through LDS.  M, N are multiples of
-// 64 and K of 32 (the host pads every dimension).
+// Every product is C[M][N] = sum_k A[m][k] B[n][k] with both operands K-contiguous:
+// the layer outputs H and gradients dZ are written in both orders by the epilogue that
+// produces them, and Adam keeps the transposed BF16 weights beside the plain ones, so
+//   forward          H[l+1] = gelu(H[l] W^T + b):  A = H[l]  (rows = samples), B = W
+//   data gradient    dZ[l-1] = (dZ[l] W) gelu'(Z): A = dZ[l],                  B = W^T
+//   weight gradient  dW = dZ^T H:                  A = dZ[l]^T,                B = H[l]^T
+// M, N and K are multiples of 64 (the host pads every dimension with zeros).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 
+#include "sqh_mlp.h"
+
 namespace sqh {
 
 typedef __bf16 bf16;
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 enum MlpEpi : int {
-    EPI_HIDDEN = 0,   // z = acc + bias -> Z (fp32), H = bf16(gelu(z))
-    EPI_OUTPUT = 1,   // y = acc + bias -> Y (fp32)
-    EPI_BWD_DATA = 2, // dz = acc * gelu'(Zin) -> dZf (fp32), dZb (bf16)
-    EPI_STORE = 3,    // C (fp32) = acc
-};
-
-struct EpiArgs {
-    const float* bias;
-    float* zf;        // fp32 output (Z, Y, dZ or C)
-    bf16* hb;         // bf16 output (H or dZ)
-    const float* zin; // pre-activation for gelu' (EPI_BWD_DATA)
-    int ld;           // leading dimension of the outputs / zin
+    EPI_HIDDEN = 0,    // z = acc + bias -> Z, H = bf16(gelu(z)) -> H, H^T
+    EPI_HIDDEN_ONLY,   // the same, H alone (no backward pass follows)
+    EPI_OUTPUT,        // y = acc + bias -> the caller's B x out array
+    EPI_MSE,           // y = acc + bias, dY = 2 (y - t) / (B out) -> dZ, dZ^T, bias partials, loss
+    EPI_BWD_DATA,      // dz = acc gelu'(Z) -> dZ, dZ^T, bias partials
 };
 
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
@@ -40,212 +38,279 @@ __device__ __forceinline__ float gelu_grad(float z) {
     return cdf + z * pdf;
 }
 
-// One operand tile (64 rows of M or N x KS values of K) between global memory, the
-// thread's registers and LDS ([row][k], k contiguous, rows padded by 8 values).  KMAJ:
-// the operand is stored K-major (row k holds the 64 rows' values contiguously), so its
-// 8-value vectors run along the rows and are transposed on the way into LDS.
-template <bool KMAJ, int KS>
-struct GemmTile {
-    static constexpr int V = 64 * KS / 8 / 256;  // 8-value vectors per thread
-    bf16x8 r[V];
-    __device__ __forceinline__ void load(const bf16* __restrict__ X, int ld, int row0, int k0, int tid) {
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-            const int v = tid + 256 * i;
-            if constexpr (!KMAJ) {
-                const int row = v / (KS / 8), kk = (v % (KS / 8)) * 8;
-                r[i] = *reinterpret_cast<const bf16x8*>(&X[(size_t)(row0 + row) * ld + k0 + kk]);
-            } else {
-                const int k = v / 8, rr = (v % 8) * 8;
-                r[i] = *reinterpret_cast<const bf16x8*>(&X[(size_t)(k0 + k) * ld + row0 + rr]);
-            }
-        }
-    }
-    __device__ __forceinline__ void store(bf16 (*S)[KS + 8], int tid) const {
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-            const int v = tid + 256 * i;
-            if constexpr (!KMAJ) {
-                const int row = v / (KS / 8), kk = (v % (KS / 8)) * 8;
-                *reinterpret_cast<bf16x8*>(&S[row][kk]) = r[i];
-            } else {
-                const int k = v / 8, rr = (v % 8) * 8;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) S[rr + j][k] = r[i][j];
-            }
-        }
-    }
-};
+// The product of one TM x TN tile by a workgroup of 4 wavefronts, left as four partial
+// tiles in LDS.  Wavefront w takes the 32-wide K steps w, w + 4, ... of the whole tile, so
+// each operand value is loaded once per workgroup, straight from global memory into the
+// MFMA operand registers (mlp_frag order): no LDS and no barrier in the loop, and D steps
+// of loads in flight per wavefront.  What bounds it is the operands' way from the L2 (a
+// CU takes 64 bytes a cycle: 1.7 us for K = 1024 at 64 x 64).  Tiles shared through LDS between 32 x 32 quarters, K in stages of 256 behind
+// barriers, took 12 us (both operands K-contiguous) and 20 us (transposed on the way into
+// LDS) for 1024 x 1024 x 1024; this form 7.5 us with its epilogue, 5 of them launch, first
+// loads, the partials' sum and the epilogue.  Eight wavefronts of an eighth of K each: 7.9.
+// A lane's result item r of tile (i, j) is C[16 i + 4 (lane / 16) + r][16 j + lane % 16].
+constexpr int kPitch = 4;  // floats of padding per partial-tile row
 
-// C[64 x 64 tile] = A B on the matrix cores: 4 wavefronts of 32 x 32 (2 x 2
-// v_mfma_f32_16x16x32_bf16 tiles), K in stages of KS through double-buffered LDS with
-// one barrier per stage; the next stage's global loads are in flight while the current
-// stage's MFMAs run.  AT: A stored K-major (A^T given); BT: B stored N-major (B^T
-// given).  Fused epilogues (EPI) write FP32 and BF16 results.
-template <bool AT, bool BT, int EPI, int KS>
-__global__ __launch_bounds__(256) void k_gemm_bf16(const bf16* __restrict__ A, int lda, const bf16* __restrict__ B,
-                                                   int ldb, int K, EpiArgs e) {
-    // [2 buffers][A, B][64][KS + 8] in dynamic LDS (up to 135 KiB at KS = 256)
-    extern __shared__ __align__(16) unsigned char gemm_smem[];
-    typedef bf16 Row[KS + 8];
-    Row* const rows = reinterpret_cast<Row*>(gemm_smem);  // A0, B0, A1, B1: 64 rows each
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    f32x4 acc[2][2];
+template <int TM, int TN>
+__device__ __forceinline__ void mlp_product(const bf16* __restrict__ A, const bf16* __restrict__ B, int K, int m0, int n0, float* __restrict__ red) {
+    constexpr int I = TM / 16, J = TN / 16, D = TM < 64 ? 8 : 3;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nl = lane & 15, g = lane >> 4;
+    const int ks = K >> 5;                                     // 32-wide K steps
+    const int S = ks > wave ? (ks - wave + 3) / 4 : 0;  // this wavefront's
+    const bf16* pa = A + ((size_t)(m0 >> 4) * ks + wave) * 512 + lane * 8;
+    const bf16* pb = B + ((size_t)(n0 >> 4) * ks + wave) * 512 + lane * 8;
+    f32x4 acc[I][J];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < I; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    GemmTile<AT, KS> ta;
-    GemmTile<!BT, KS> tb;
-    ta.load(A, lda, m0, 0, tid);
-    tb.load(B, ldb, n0, 0, tid);
-    ta.store(rows, tid);
-    tb.store(rows + 64, tid);
-    __syncthreads();
-    const int S = K / KS;
-    for (int st = 0; st < S; ++st) {
-        const int cur = st & 1;
-        Row* const As = rows + 128 * cur;
-        Row* const Bs = rows + 128 * cur + 64;
-        if (st + 1 < S) {
-            ta.load(A, lda, m0, (st + 1) * KS, tid);
-            tb.load(B, ldb, n0, (st + 1) * KS, tid);
+        for (int j = 0; j < J; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 a[D][I], b[D][J];
+    auto load = [&](int d, int s) {
+#pragma unroll
+        for (int i = 0; i < I; ++i) a[d][i] = *reinterpret_cast<const bf16x8*>(pa + ((size_t)i * ks + 4 * s) * 512);
+#pragma unroll
+        for (int j = 0; j < J; ++j) b[d][j] = *reinterpret_cast<const bf16x8*>(pb + ((size_t)j * ks + 4 * s) * 512);
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d < S) load(d, d);
+    for (int s = 0; s < S; s += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (s + d < S) {
+#pragma unroll
+                for (int i = 0; i < I; ++i)
+#pragma unroll
+                    for (int j = 0; j < J; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][i], b[d][j], acc[i][j], 0, 0, 0);
+                if (s + d + D < S) load(d, s + d + D);
+            }
         }
-#pragma unroll
-        for (int ks = 0; ks < KS; ks += 32) {
-            bf16x8 a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                a[i] = *reinterpret_cast<const bf16x8*>(&As[wm + i * 16 + (lane & 15)][ks + 8 * (lane >> 4)]);
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                b[j] = *reinterpret_cast<const bf16x8*>(&Bs[wn + j * 16 + (lane & 15)][ks + 8 * (lane >> 4)]);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (st + 1 < S) {
-            ta.store(rows + 128 * (cur ^ 1), tid);
-            tb.store(rows + 128 * (cur ^ 1) + 64, tid);
-        }
-        __syncthreads();
     }
+    float* part = red + wave * TM * (TN + kPitch);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < I; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) part[(16 * i + 4 * g + r) * (TN + kPitch) + 16 * j + nl] = acc[i][j][r];
+    __syncthreads();
+}
+
+// Threads of the epilogue and the 4 x 4 block of the tile each holds: rows 4 rg .. + 3,
+// columns 4 cg .. + 3, the four wavefronts' partials summed in wavefront order.
+template <int TM, int TN>
+__device__ __forceinline__ bool mlp_block(const float* __restrict__ red, int& rg, int& cg, f32x4 (&v)[4]) {
+    if (threadIdx.x >= TM * TN / 16) return false;
+    rg = threadIdx.x / (TN / 4);
+    cg = threadIdx.x % (TN / 4);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float* p = red + (4 * rg + r) * (TN + kPitch) + 4 * cg;
+        f32x4 s = *reinterpret_cast<const f32x4*>(p);
+#pragma unroll
+        for (int w = 1; w < 4; ++w) s += *reinterpret_cast<const f32x4*>(p + w * TM * (TN + kPitch));
+        v[r] = s;
+    }
+    return true;
+}
+
+// A 4 x 4 block as BF16 into X (rows x cols) and, when XT is given, into its transpose.
+__device__ __forceinline__ void mlp_store_bf16(const f32x4 (&v)[4], int row, int col, bf16* X, int cols, bf16* XT,
+                                               int rows) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const bf16x4 h = {(bf16)v[r][0], (bf16)v[r][1], (bf16)v[r][2], (bf16)v[r][3]};
+        *reinterpret_cast<bf16x4*>(&X[mlp_frag(row + r, col, cols)]) = h;
+    }
+    if (XT) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const bf16x4 h = {(bf16)v[0][c], (bf16)v[1][c], (bf16)v[2][c], (bf16)v[3][c]};
+            *reinterpret_cast<bf16x4*>(&XT[mlp_frag(col + c, row, rows)]) = h;
+        }
+    }
+}
+
+// Column sums of a tile's dZ (each thread holds the sums of its four rows) into the
+// tile row's slice of the bias partials; sums in a fixed order.
+template <int TM, int TN>
+__device__ __forceinline__ void mlp_bias_partials(bool active, int rg, int cg, const f32x4 (&v)[4],
+                                                  float* __restrict__ red, float* __restrict__ bpart, int n0) {
+    __syncthreads();  // the partial tiles are consumed
+    if (active) *reinterpret_cast<f32x4*>(red + rg * TN + 4 * cg) = (v[0] + v[1]) + (v[2] + v[3]);
+    __syncthreads();
+    if (threadIdx.x < TN) {
+        float s = 0.f;
+#pragma unroll
+        for (int k = 0; k < TM / 4; ++k) s += red[k * TN + threadIdx.x];
+        bpart[n0 + threadIdx.x] = s;
+    }
+}
+
+template <int TM, int TN, int EPI>
+__global__ __launch_bounds__(256, 2) void k_mlp_layer(MlpLayerArgs a) {
+    __shared__ __align__(16) float red[4 * TM * (TN + kPitch)];
+    const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
+    mlp_product<TM, TN>((const bf16*)a.A, (const bf16*)a.B, a.K, m0, n0, red);
+    int rg = 0, cg = 0;
+    f32x4 v[4];
+    const bool active = mlp_block<TM, TN>(red, rg, cg, v);
+    const int row = m0 + 4 * rg, col = n0 + 4 * cg;
+    if constexpr (EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_ONLY) {
+        if (active) {
+            const f32x4 bias = *reinterpret_cast<const f32x4*>(&a.bias[col]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = m0 + wm + i * 16 + 4 * (lane >> 4) + r;
-                const int col = n0 + wn + j * 16 + (lane & 15);
-                const size_t o = (size_t)row * e.ld + col;
-                const float v = acc[i][j][r];
-                if constexpr (EPI == EPI_HIDDEN) {
-                    const float z = v + e.bias[col];
-                    e.zf[o] = z;
-                    e.hb[o] = (bf16)gelu(z);
-                } else if constexpr (EPI == EPI_OUTPUT) {
-                    e.zf[o] = v + e.bias[col];
-                } else if constexpr (EPI == EPI_BWD_DATA) {
-                    const float dz = v * gelu_grad(e.zin[o]);
-                    e.zf[o] = dz;
-                    e.hb[o] = (bf16)dz;
-                } else {
-                    e.zf[o] = v;
+                v[r] += bias;
+                if constexpr (EPI == EPI_HIDDEN)
+                    *reinterpret_cast<f32x4*>(&a.Z[(size_t)(row + r) * a.N + col]) = v[r];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[r][c] = gelu(v[r][c]);
+            }
+            mlp_store_bf16(v, row, col, (bf16*)a.X, a.N, EPI == EPI_HIDDEN ? (bf16*)a.XT : nullptr,
+                           a.M);
+        }
+    } else if constexpr (EPI == EPI_OUTPUT) {
+        if (active) {
+            const f32x4 bias = *reinterpret_cast<const f32x4*>(&a.bias[col]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                v[r] += bias;
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (row + r < a.batch && col + c < a.out) a.y[(size_t)(row + r) * a.out + col + c] = v[r][c];
+            }
+        }
+    } else if constexpr (EPI == EPI_MSE) {
+        double l = 0.0;
+        if (active) {
+            const f32x4 bias = *reinterpret_cast<const f32x4*>(&a.bias[col]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                v[r] += bias;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    float gr = 0.f;
+                    if (row + r < a.batch && col + c < a.out) {
+                        const float d = v[r][c] - a.t[(size_t)(row + r) * a.out + col + c];
+                        l += (double)d * d;
+                        gr = 2.0f * d / ((float)a.batch * (float)a.out);
+                    }
+                    v[r][c] = gr;
                 }
             }
-}
-
-// x (B x in, fp32, row stride in) -> padded bf16 (Bp x in_pad); rows >= B are zero.
-__global__ void k_to_bf16_padded(const float* __restrict__ x, int B, int in, bf16* __restrict__ out, int Bp,
-                                 int in_pad) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)Bp * in_pad) return;
-    const int r = (int)(i / in_pad), c = (int)(i % in_pad);
-    out[i] = (bf16)((r < B && c < in) ? x[(size_t)r * in + c] : 0.0f);
-}
-
-// Mean squared error over the B x out real entries; dY = 2 (y - t) / (B * out) (bf16 and
-// fp32), padded entries get 0.  Per-block partial losses go to part[blockIdx].
-__global__ __launch_bounds__(256) void k_mse(const float* __restrict__ y, int ldy, const float* __restrict__ t, int B,
-                                             int out, int Bp, float* __restrict__ dyf, bf16* __restrict__ dyb,
-                                             double* __restrict__ part) {
-    __shared__ double sh[4];
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    double l = 0.0;
-    if (i < (size_t)Bp * ldy) {
-        const int r = (int)(i / ldy), c = (int)(i % ldy);
-        float g = 0.0f;
-        if (r < B && c < out) {
-            const float d = y[i] - t[(size_t)r * out + c];
-            l = (double)d * d;
-            g = 2.0f * d / ((float)B * (float)out);
+            mlp_store_bf16(v, row, col, (bf16*)a.X, a.N, (bf16*)a.XT, a.M);
         }
-        dyf[i] = g;
-        dyb[i] = (bf16)g;
-    }
-    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = l;
-    __syncthreads();
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
-}
-
-// Output gradient supplied by the caller (dy: B x out, FP32) into the padded FP32 and
-// BF16 buffers of the last layer; padding rows and columns are zero.
-__global__ __launch_bounds__(256) void k_out_grad(const float* __restrict__ dy, int B, int out, int ldy, int Bp,
-                                                  float* __restrict__ dyf, bf16* __restrict__ dyb) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)Bp * ldy) return;
-    const int r = (int)(i / ldy), c = (int)(i % ldy);
-    const float g = (r < B && c < out) ? dy[(size_t)r * out + c] : 0.0f;
-    dyf[i] = g;
-    dyb[i] = (bf16)g;
-}
-
-// db[n] = sum over the first B rows of dz[:, n]: a workgroup per 16 columns, its 64
-// row slices each summing every 64th row, then combined in LDS in a fixed order (the
-// sum is the same on every run).  64 row slices keep 64 workgroups of 16 wavefronts
-// busy for a 1024-wide layer, where 4 slices per 64 columns kept 16 workgroups.
-__global__ __launch_bounds__(1024) void k_bias_grad(const float* __restrict__ dz, int ld, int B, int N,
-                                                    float* __restrict__ db) {
-    __shared__ float part[64][17];
-    const int cx = threadIdx.x & 15, ry = threadIdx.x >> 4;
-    const int n = blockIdx.x * 16 + cx;
-    float s = 0.0f;
-    if (n < N)
-        for (int r = ry; r < B; r += 64) s += dz[(size_t)r * ld + n];
-    part[ry][cx] = s;
-    __syncthreads();
-    if (ry == 0 && n < N) {
-        float t = 0.0f;
-        for (int k = 0; k < 64; ++k) t += part[k][cx];
-        db[n] = t;
+        mlp_bias_partials<TM, TN>(active, rg, cg, v, red, a.bpart + (size_t)blockIdx.y * a.N, n0);
+        __shared__ double sh[4];
+        for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o, 64);
+        if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = l;
+        __syncthreads();
+        if (threadIdx.x == 0) a.loss[blockIdx.y * gridDim.x + blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
+    } else {
+        if (active) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const f32x4 z = *reinterpret_cast<const f32x4*>(&a.Z[(size_t)(row + r) * a.N + col]);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[r][c] *= gelu_grad(z[c]);
+            }
+            mlp_store_bf16(v, row, col, (bf16*)a.X, a.N, (bf16*)a.XT, a.M);
+        }
+        mlp_bias_partials<TM, TN>(active, rg, cg, v, red, a.bpart + (size_t)blockIdx.y * a.N, n0);
     }
 }
 
-// Adam on fp32 master weights; refreshes the bf16 copy when wb is given.
-__global__ void k_adam(float* __restrict__ w, bf16* __restrict__ wb, const float* __restrict__ g,
-                       float* __restrict__ m, float* __restrict__ v, size_t n, float lr, float b1, float b2, float eps,
-                       float c1, float c2) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-    w[i] = wi;
-    if (wb) wb[i] = (bf16)wi;
+// Adam on an FP32 master weight.
+__device__ __forceinline__ float mlp_adam(float w, float g, float& m, float& v, const MlpAdam& p) {
+    m = p.b1 * m + (1.0f - p.b1) * g;
+    v = p.b2 * v + (1.0f - p.b2) * g * g;
+    return w - p.lr * (m / p.c1) / (sqrtf(v / p.c2) + p.eps);
 }
 
-__global__ void k_f32_to_bf16(const float* __restrict__ a, bf16* __restrict__ b, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) b[i] = (bf16)a[i];
+// Weight and bias gradients of up to kMlpGroup layers in one launch, each either applied
+// by Adam where it is formed (the gradient never travels through memory) or stored.  The
+// weights' and moments' 28 bytes a parameter bound it: 28 us for 2.8 M parameters at a batch
+// of 1024, where the products, the column sums and the updates of the four layers, a launch
+// each, took 148.
+// Workgroups: the layers' weight tiles, then 64 bias entries per workgroup.
+template <int TM, int TN, bool ADAM>
+__global__ __launch_bounds__(256, 2) void k_mlp_weights(MlpWeightsArgs a) {
+    __shared__ __align__(16) float red[4 * TM * (TN + kPitch)];
+    int t = blockIdx.x, l = 0;
+    while (l + 1 < a.layers && t >= a.first[l + 1]) ++l;
+    const MlpWeights& w = a.w[l];
+    t -= a.first[l];
+    const int tn = w.in / TN, tiles = (w.out / TM) * tn;
+    if (t < tiles) {
+        const int m0 = t / tn * TM, n0 = t % tn * TN;
+        mlp_product<TM, TN>((const bf16*)w.dZT, (const bf16*)w.HT, a.batch, m0, n0, red);
+        int rg = 0, cg = 0;
+        f32x4 v[4];
+        if (!mlp_block<TM, TN>(red, rg, cg, v)) return;
+        const int row = m0 + 4 * rg, col = n0 + 4 * cg;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const size_t o = (size_t)(row + r) * w.in + col;
+            if constexpr (ADAM) {
+                f32x4 x = *reinterpret_cast<f32x4*>(&w.W[o]);
+                f32x4 m = *reinterpret_cast<f32x4*>(&w.mW[o]);
+                f32x4 s = *reinterpret_cast<f32x4*>(&w.vW[o]);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    float mc = m[c], sc = s[c];
+                    x[c] = mlp_adam(x[c], v[r][c], mc, sc, a.adam);
+                    m[c] = mc;
+                    s[c] = sc;
+                }
+                *reinterpret_cast<f32x4*>(&w.W[o]) = x;
+                *reinterpret_cast<f32x4*>(&w.mW[o]) = m;
+                *reinterpret_cast<f32x4*>(&w.vW[o]) = s;
+                v[r] = x;
+            } else {
+                *reinterpret_cast<f32x4*>(&w.gW[o]) = v[r];
+            }
+        }
+        if constexpr (ADAM) mlp_store_bf16(v, row, col, (bf16*)w.Wb, w.in, (bf16*)w.WbT, w.out);
+        return;
+    }
+    // bias entries: the partials of every tile row, four interleaved slices per entry
+    const int n = (t - tiles) * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;
+    float s = 0.f;
+    for (int k = q; k < w.parts; k += 4) s += w.bpart[(size_t)k * w.out + n];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    if (q == 0) {
+        const float g = (red[n & 63] + red[64 + (n & 63)]) + (red[128 + (n & 63)] + red[192 + (n & 63)]);
+        if constexpr (ADAM) w.b[n] = mlp_adam(w.b[n], g, w.mb[n], w.vb[n], a.adam);
+        else w.gb[n] = g;
+    }
+}
+
+// An FP32 array (rows x cols real entries, row stride ldx) as zero-padded BF16 in both
+// orders: X[row][col] (Rp x Cp) and, when given, XT[col][row]; bpart (when given)
+// receives the column sums of each 64-row slice.  64 x 64 per workgroup: the network's
+// input batch, the caller's output gradient and the weights.
+__global__ __launch_bounds__(256) void k_mlp_convert(const float* __restrict__ x, int rows, int cols, int ldx,
+                                                     bf16* __restrict__ X, bf16* __restrict__ XT, int Rp, int Cp,
+                                                     float* __restrict__ bpart) {
+    __shared__ __align__(16) float tile[64 * 65];
+    const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
+    for (int i = threadIdx.x; i < 64 * 64; i += 256) {
+        const int r = i >> 6, c = i & 63;
+        tile[r * 65 + c] =
+            (r0 + r < rows && c0 + c < cols) ? x[(size_t)(r0 + r) * ldx + c0 + c] : 0.0f;
+    }
+    __syncthreads();
+    const int rg = threadIdx.x >> 4, cg = threadIdx.x & 15;
+    f32x4 v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[r][c] = tile[(4 * rg + r) * 65 + 4 * cg + c];
+    mlp_store_bf16(v, r0 + 4 * rg, c0 + 4 * cg, X, Cp, XT, Rp);
+    if (bpart) mlp_bias_partials<64, 64>(true, rg, cg, v, tile, bpart + (size_t)blockIdx.y * Cp, c0);
 }
 
 // One layer's parameters between the padded device layout (W [np][kp], b [np]) and the
@@ -264,80 +329,57 @@ __global__ __launch_bounds__(256) void k_pack_layer(float* __restrict__ W, float
 
 // Host launchers ------------------------------------------------------------------
 
-template <bool AT, bool BT, int EPI>
-static hipError_t gemm(const void* A, int lda, const void* B, int ldb, int M, int N, int K, const EpiArgs& e,
-                       hipStream_t s) {
-    if (M % 64 || N % 64 || K % 32 || K <= 0) return hipErrorInvalidValue;
-    // the widest K stage dividing K: fewer stages, each with more MFMAs per load wait
-#define SQH_GEMM_KS(ks)                                                                                     \
-    if (K % ks == 0) {                                                                                      \
-        const size_t shm = 4 * 64 * (ks + 8) * sizeof(bf16);                                                \
-        hipLaunchKernelGGL((k_gemm_bf16<AT, BT, EPI, ks>), dim3(N / 64, M / 64), dim3(256), shm, s,         \
-                           (const bf16*)A, lda, (const bf16*)B, ldb, K, e);                                 \
-        return hipGetLastError();                                                                           \
+// 64 x 64 tiles load half the operand bytes per flop of 32 x 32 ones (7.5 against 8.6 us
+// for a 1024 x 1024 x 1024 product); below 256 of them, one per CU, the smaller tiles put
+// four times the CUs to work.
+static bool small_tiles(long long tiles64) { return tiles64 < 256; }
+
+int mlp_tile_rows(int M, int N) { return small_tiles((long long)(M / 64) * (N / 64)) ? 32 : 64; }
+
+static bool bad_dims(int M, int N, int K) { return M % 64 || N % 64 || K % 64 || M <= 0 || N <= 0 || K <= 0; }
+
+template <int EPI>
+static hipError_t layer(const MlpLayerArgs& a, hipStream_t s) {
+    if (bad_dims(a.M, a.N, a.K)) return hipErrorInvalidValue;
+    if (mlp_tile_rows(a.M, a.N) == 32)
+        hipLaunchKernelGGL((k_mlp_layer<32, 32, EPI>), dim3(a.N / 32, a.M / 32), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_mlp_layer<64, 64, EPI>), dim3(a.N / 64, a.M / 64), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t mlp_hidden(const MlpLayerArgs& a, bool train, hipStream_t s) {
+    return train ? layer<EPI_HIDDEN>(a, s) : layer<EPI_HIDDEN_ONLY>(a, s);
+}
+hipError_t mlp_output(const MlpLayerArgs& a, hipStream_t s) { return layer<EPI_OUTPUT>(a, s); }
+hipError_t mlp_output_mse(const MlpLayerArgs& a, hipStream_t s) { return layer<EPI_MSE>(a, s); }
+hipError_t mlp_backward_data(const MlpLayerArgs& a, hipStream_t s) { return layer<EPI_BWD_DATA>(a, s); }
+
+hipError_t mlp_weights(MlpWeightsArgs a, bool adam, hipStream_t s) {
+    if (a.layers < 1 || a.layers > kMlpGroup) return hipErrorInvalidValue;
+    long long tiles64 = 0;
+    for (int l = 0; l < a.layers; ++l) {
+        if (bad_dims(a.w[l].out, a.w[l].in, a.batch)) return hipErrorInvalidValue;
+        tiles64 += (long long)(a.w[l].out / 64) * (a.w[l].in / 64);
     }
-    SQH_GEMM_KS(256)
-    SQH_GEMM_KS(128)
-    SQH_GEMM_KS(64)
-    SQH_GEMM_KS(32)
-#undef SQH_GEMM_KS
-    return hipErrorInvalidValue;
-}
-
-// Z[M x N] = H[M x K] W[N x K]^T + b  (hidden: also H' = gelu(Z); output: Y)
-hipError_t mlp_gemm_forward(bool hidden, const void* H, int K, const void* W, const float* bias, int M, int N,
-                            float* Z, void* Hout, hipStream_t s) {
-    EpiArgs e{bias, Z, (bf16*)Hout, nullptr, N};
-    return hidden ? gemm<false, true, EPI_HIDDEN>(H, K, W, K, M, N, K, e, s)
-                  : gemm<false, true, EPI_OUTPUT>(H, K, W, K, M, N, K, e, s);
-}
-
-// dH[M x K] = dZ[M x N] W[N x K], then dZprev = dH * gelu'(Zprev)
-hipError_t mlp_gemm_backward_data(const void* dZ, int N, const void* W, int K, int M, const float* Zprev,
-                                  float* dZprev_f, void* dZprev_b, hipStream_t s) {
-    EpiArgs e{nullptr, dZprev_f, (bf16*)dZprev_b, Zprev, K};
-    return gemm<false, false, EPI_BWD_DATA>(dZ, N, W, K, M, K, N, e, s);
-}
-
-// dW[N x K] = dZ[B x N]^T H[B x K]
-hipError_t mlp_gemm_backward_weights(const void* dZ, int N, const void* H, int K, int B, float* dW, hipStream_t s) {
-    EpiArgs e{nullptr, dW, nullptr, nullptr, K};
-    return gemm<true, false, EPI_STORE>(dZ, N, H, K, N, K, B, e, s);
-}
-
-hipError_t mlp_to_bf16_padded(const float* x, int B, int in, void* out, int Bp, int in_pad, hipStream_t s) {
-    const size_t n = (size_t)Bp * in_pad;
-    hipLaunchKernelGGL(k_to_bf16_padded, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, B, in, (bf16*)out, Bp,
-                       in_pad);
+    const int T = small_tiles(tiles64) ? 32 : 64;
+    int first = 0;
+    for (int l = 0; l < a.layers; ++l) {
+        a.first[l] = first;
+        first += (a.w[l].out / T) * (a.w[l].in / T) + a.w[l].out / 64;
+    }
+    if (T == 32 && adam) hipLaunchKernelGGL((k_mlp_weights<32, 32, true>), dim3(first), dim3(256), 0, s, a);
+    else if (T == 32) hipLaunchKernelGGL((k_mlp_weights<32, 32, false>), dim3(first), dim3(256), 0, s, a);
+    else if (adam) hipLaunchKernelGGL((k_mlp_weights<64, 64, true>), dim3(first), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_mlp_weights<64, 64, false>), dim3(first), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-hipError_t mlp_mse(const float* y, int ldy, const float* t, int B, int out, int Bp, float* dyf, void* dyb,
-                   double* part, int* nblocks, hipStream_t s) {
-    const size_t n = (size_t)Bp * ldy;
-    const unsigned g = (unsigned)((n + 255) / 256);
-    *nblocks = (int)g;
-    hipLaunchKernelGGL(k_mse, dim3(g), dim3(256), 0, s, y, ldy, t, B, out, Bp, dyf, (bf16*)dyb, part);
-    return hipGetLastError();
-}
-
-hipError_t mlp_out_grad(const float* dy, int B, int out, int ldy, int Bp, float* dyf, void* dyb, hipStream_t s) {
-    const size_t n = (size_t)Bp * ldy;
-    hipLaunchKernelGGL(k_out_grad, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, dy, B, out, ldy, Bp, dyf,
-                       (bf16*)dyb);
-    return hipGetLastError();
-}
-
-hipError_t mlp_bias_grad(const float* dz, int ld, int B, int N, float* db, hipStream_t s) {
-    hipLaunchKernelGGL(k_bias_grad, dim3((N + 15) / 16), dim3(1024), 0, s, dz, ld, B, N, db);
-    return hipGetLastError();
-}
-
-hipError_t mlp_adam(float* w, void* wb, const float* g, float* m, float* v, size_t n, float lr, float b1, float b2,
-                    float eps, int step, hipStream_t s) {
-    const float c1 = 1.0f - powf(b1, (float)step), c2 = 1.0f - powf(b2, (float)step);
-    hipLaunchKernelGGL(k_adam, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, w, (bf16*)wb, g, m, v, n, lr, b1,
-                       b2, eps, c1, c2);
+hipError_t mlp_convert(const float* x, int rows, int cols, int ldx, void* X, void* XT, int Rp, int Cp, float* bpart,
+                       hipStream_t s) {
+    if (Rp % 64 || Cp % 64 || Rp <= 0 || Cp <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_mlp_convert, dim3(Cp / 64, Rp / 64), dim3(256), 0, s, x, rows, cols, ldx, (bf16*)X, (bf16*)XT,
+                       Rp, Cp, bpart);
     return hipGetLastError();
 }
 
@@ -345,11 +387,6 @@ hipError_t mlp_pack_layer(float* W, float* b, int no, int ni, int kp, float* fla
     const long long n = (long long)no * ni + no;
     hipLaunchKernelGGL(k_pack_layer, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, W, b, no, ni, kp, flat,
                        to_flat);
-    return hipGetLastError();
-}
-
-hipError_t mlp_f32_to_bf16(const float* a, void* b, size_t n, hipStream_t s) {
-    hipLaunchKernelGGL(k_f32_to_bf16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, (bf16*)b, n);
     return hipGetLastError();
 }
 

@@ -11,23 +11,7 @@
 #include <vector>
 
 #include "sqh_context.h"
-
-namespace sqh {
-hipError_t mlp_gemm_forward(bool hidden, const void* H, int K, const void* W, const float* bias, int M, int N,
-                            float* Z, void* Hout, hipStream_t s);
-hipError_t mlp_gemm_backward_data(const void* dZ, int N, const void* W, int K, int M, const float* Zprev,
-                                  float* dZprev_f, void* dZprev_b, hipStream_t s);
-hipError_t mlp_gemm_backward_weights(const void* dZ, int N, const void* H, int K, int B, float* dW, hipStream_t s);
-hipError_t mlp_to_bf16_padded(const float* x, int B, int in, void* out, int Bp, int in_pad, hipStream_t s);
-hipError_t mlp_mse(const float* y, int ldy, const float* t, int B, int out, int Bp, float* dyf, void* dyb,
-                   double* part, int* nblocks, hipStream_t s);
-hipError_t mlp_bias_grad(const float* dz, int ld, int B, int N, float* db, hipStream_t s);
-hipError_t mlp_out_grad(const float* dy, int B, int out, int ldy, int Bp, float* dyf, void* dyb, hipStream_t s);
-hipError_t mlp_adam(float* w, void* wb, const float* g, float* m, float* v, size_t n, float lr, float b1, float b2,
-                    float eps, int step, hipStream_t s);
-hipError_t mlp_pack_layer(float* W, float* b, int no, int ni, int kp, float* flat, bool to_flat, hipStream_t s);
-hipError_t mlp_f32_to_bf16(const float* a, void* b, size_t n, hipStream_t s);
-}  // namespace sqh
+#include "sqh_mlp.h"
 
 using namespace sqh;
 
@@ -39,17 +23,22 @@ struct sqh_mlp {
     sqh_ctx* ctx = nullptr;
     int L = 0;                       // weight layers
     std::vector<int> dim, dpad;      // real and padded widths, L + 1 entries
-    std::vector<DevBuf> W, Wb, b, mW, vW, mb, vb, gW, gb;
-    std::vector<DevBuf> H, Z, dZf, dZb;  // activations per layer (H[0] = input)
-    DevBuf part;
+    // FP32 master weights, their BF16 copies in both orders, Adam's moments, gradients
+    // (kept only by sqh_mlp_gradients)
+    std::vector<DevBuf> W, Wb, WbT, b, mW, vW, mb, vb, gW, gb;
+    // per layer for a batch: input activations and their transposes, pre-activations,
+    // output gradients and their transposes, bias gradient partials
+    std::vector<DevBuf> H, HT, Z, dZ, dZT, bpart;
+    std::vector<int> parts;          // slices of bpart the last backward pass wrote
+    DevBuf loss;                     // loss partials
     DevBuf flat;                     // the parameters in the caller's flat layout
-    int cap = 0;                     // padded batch the activation buffers hold
+    int loss_parts = 0;              // loss partials the last forward pass wrote
     int step = 0;
 
     ~sqh_mlp() {
-        for (auto* v : {&W, &Wb, &b, &mW, &vW, &mb, &vb, &gW, &gb, &H, &Z, &dZf, &dZb})
+        for (auto* v : {&W, &Wb, &WbT, &b, &mW, &vW, &mb, &vb, &gW, &gb, &H, &HT, &Z, &dZ, &dZT, &bpart})
             for (auto& x : *v) x.release();
-        part.release();
+        loss.release();
         flat.release();
     }
     hipStream_t st() const { return ctx->stream; }
@@ -57,79 +46,145 @@ struct sqh_mlp {
 
 namespace {
 
-int ensure_batch(sqh_mlp* m, int Bp) {
+// Activation buffers for a padded batch of Bp (train: those of the backward pass too).
+int ensure_batch(sqh_mlp* m, int Bp, bool train) {
     sqh_ctx* c = m->ctx;
-    if (Bp <= m->cap) return SQH_OK;
-    for (int l = 0; l <= m->L; ++l) HIPTRY(c, m->H[l].ensure((size_t)Bp * m->dpad[l] * 2));
     for (int l = 0; l < m->L; ++l) {
-        HIPTRY(c, m->Z[l].ensure((size_t)Bp * m->dpad[l + 1] * 4));
-        HIPTRY(c, m->dZf[l].ensure((size_t)Bp * m->dpad[l + 1] * 4));
-        HIPTRY(c, m->dZb[l].ensure((size_t)Bp * m->dpad[l + 1] * 2));
+        const size_t in = m->dpad[l], outd = m->dpad[l + 1], out = (size_t)Bp * outd;
+        HIPTRY(c, m->H[l].ensure((size_t)Bp * in * 2));
+        if (!train) continue;
+        HIPTRY(c, m->HT[l].ensure(in * Bp * 2));
+        if (l + 1 < m->L) HIPTRY(c, m->Z[l].ensure(out * 4));
+        HIPTRY(c, m->dZ[l].ensure((size_t)Bp * outd * 2));
+        HIPTRY(c, m->dZT[l].ensure(outd * Bp * 2));
+        HIPTRY(c, m->bpart[l].ensure(out / 32 * 4));
     }
-    HIPTRY(c, m->part.ensure((size_t)Bp * m->dpad[m->L] / 256 * 8 + 64));
-    m->cap = Bp;
+    if (train) HIPTRY(c, m->loss.ensure((size_t)Bp * m->dpad[m->L] / 1024 * sizeof(double)));
     return SQH_OK;
 }
 
-int forward(sqh_mlp* m, const float* d_x, int B, int Bp) {
+// Layer l's product over the padded batch, forward (A = its input, B = W).
+MlpLayerArgs layer_args(sqh_mlp* m, int l, int Bp) {
+    MlpLayerArgs a;
+    a.A = m->H[l].p;
+    a.B = m->Wb[l].p;
+    a.M = Bp;
+    a.N = m->dpad[l + 1];
+    a.K = m->dpad[l];
+    a.bias = m->b[l].as<float>();
+    return a;
+}
+
+// The input and the hidden layers (train: with what the backward pass reads).
+int forward_hidden(sqh_mlp* m, const float* d_x, int B, int Bp, bool train) {
     sqh_ctx* c = m->ctx;
-    HIPTRY(c, mlp_to_bf16_padded(d_x, B, m->dim[0], m->H[0].p, Bp, m->dpad[0], m->st()));
-    for (int l = 0; l < m->L; ++l) {
-        const bool hidden = l + 1 < m->L;
-        HIPTRY(c, mlp_gemm_forward(hidden, m->H[l].p, m->dpad[l], m->Wb[l].p, m->b[l].as<float>(), Bp, m->dpad[l + 1],
-                                   m->Z[l].as<float>(), hidden ? m->H[l + 1].p : nullptr, m->st()));
+    HIPTRY(c, mlp_convert(d_x, B, m->dim[0], m->dim[0], m->H[0].p, train ? m->HT[0].p : nullptr, Bp, m->dpad[0],
+                          nullptr, m->st()));
+    for (int l = 0; l + 1 < m->L; ++l) {
+        MlpLayerArgs a = layer_args(m, l, Bp);
+        a.X = m->H[l + 1].p;
+        if (train) {
+            a.XT = m->HT[l + 1].p;
+            a.Z = m->Z[l].as<float>();
+        }
+        HIPTRY(c, mlp_hidden(a, train, m->st()));
     }
     return SQH_OK;
 }
 
-// Gradients into gW/gb from the output gradient already in dZf/dZb[L-1].
-int backward_layers(sqh_mlp* m, int B, int Bp) {
+// The hidden layers' output gradients from the last layer's in dZ[L-1].
+int backward_data(sqh_mlp* m, int Bp) {
+    sqh_ctx* c = m->ctx;
+    for (int l = m->L - 1; l > 0; --l) {
+        MlpLayerArgs a;
+        a.A = m->dZ[l].p;
+        a.B = m->WbT[l].p;
+        a.M = Bp;
+        a.N = m->dpad[l];
+        a.K = m->dpad[l + 1];
+        a.Z = m->Z[l - 1].as<float>();
+        a.X = m->dZ[l - 1].p;
+        a.XT = m->dZT[l - 1].p;
+        a.bpart = m->bpart[l - 1].as<float>();
+        m->parts[l - 1] = Bp / mlp_tile_rows(a.M, a.N);
+        HIPTRY(c, mlp_backward_data(a, m->st()));
+    }
+    return SQH_OK;
+}
+
+// Weight and bias gradients of every layer: applied by one Adam step of rate lr, or
+// (adam = false) stored in gW / gb.  After backward_data, which reads the old weights.
+int weights(sqh_mlp* m, int Bp, bool adam, float lr) {
+    sqh_ctx* c = m->ctx;
+    if (adam) m->step++;
+    const float b1 = 0.9f, b2 = 0.999f;
+    MlpWeightsArgs g;
+    g.batch = Bp;
+    g.adam = {lr, b1, b2, 1e-8f, 1.0f - powf(b1, (float)m->step), 1.0f - powf(b2, (float)m->step)};
+    for (int l0 = 0; l0 < m->L; l0 += kMlpGroup) {
+        g.layers = std::min(kMlpGroup, m->L - l0);
+        for (int k = 0; k < g.layers; ++k) {
+            const int l = l0 + k;
+            if (!adam) {
+                HIPTRY(c, m->gW[l].ensure((size_t)m->dpad[l + 1] * m->dpad[l] * 4));
+                HIPTRY(c, m->gb[l].ensure((size_t)m->dpad[l + 1] * 4));
+            }
+            g.w[k] = {m->dZT[l].p,          m->HT[l].p,          m->W[l].as<float>(),  m->mW[l].as<float>(),
+                      m->vW[l].as<float>(), m->gW[l].as<float>(), m->Wb[l].p,           m->WbT[l].p,
+                      m->b[l].as<float>(),  m->mb[l].as<float>(), m->vb[l].as<float>(), m->gb[l].as<float>(),
+                      m->bpart[l].as<float>(), m->parts[l],       m->dpad[l],           m->dpad[l + 1]};
+        }
+        HIPTRY(c, mlp_weights(g, adam, m->st()));
+    }
+    return SQH_OK;
+}
+
+// Forward pass of a training step on the MSE loss and the output gradients of every
+// layer.
+int forward_backward(sqh_mlp* m, const float* d_x, const float* d_t, int B, int Bp) {
     sqh_ctx* c = m->ctx;
     const int L = m->L;
-    for (int l = L - 1; l >= 0; --l) {
-        HIPTRY(c, mlp_gemm_backward_weights(m->dZb[l].p, m->dpad[l + 1], m->H[l].p, m->dpad[l], Bp,
-                                            m->gW[l].as<float>(), m->st()));
-        HIPTRY(c, mlp_bias_grad(m->dZf[l].as<float>(), m->dpad[l + 1], B, m->dpad[l + 1], m->gb[l].as<float>(),
-                                m->st()));
-        if (l > 0)
-            HIPTRY(c, mlp_gemm_backward_data(m->dZb[l].p, m->dpad[l + 1], m->Wb[l].p, m->dpad[l], Bp,
-                                             m->Z[l - 1].as<float>(), m->dZf[l - 1].as<float>(), m->dZb[l - 1].p,
-                                             m->st()));
-    }
-    return SQH_OK;
-}
-
-int adam_step(sqh_mlp* m, float lr) {
-    sqh_ctx* c = m->ctx;
-    m->step++;
-    for (int l = 0; l < m->L; ++l) {
-        const size_t nw = (size_t)m->dpad[l + 1] * m->dpad[l];
-        HIPTRY(c, mlp_adam(m->W[l].as<float>(), m->Wb[l].p, m->gW[l].as<float>(), m->mW[l].as<float>(),
-                           m->vW[l].as<float>(), nw, lr, 0.9f, 0.999f, 1e-8f, m->step, m->st()));
-        HIPTRY(c, mlp_adam(m->b[l].as<float>(), nullptr, m->gb[l].as<float>(), m->mb[l].as<float>(),
-                           m->vb[l].as<float>(), (size_t)m->dpad[l + 1], lr, 0.9f, 0.999f, 1e-8f, m->step, m->st()));
-    }
-    return SQH_OK;
-}
-
-// Loss, gradients into gW/gb; the loss sum goes to *loss (synchronises).
-int backward(sqh_mlp* m, const float* d_t, int B, int Bp, double* loss) {
-    sqh_ctx* c = m->ctx;
-    const int L = m->L;
-    int nb = 0;
-    HIPTRY(c, mlp_mse(m->Z[L - 1].as<float>(), m->dpad[L], d_t, B, m->dim[L], Bp, m->dZf[L - 1].as<float>(),
-                      m->dZb[L - 1].p, m->part.as<double>(), &nb, m->st()));
-    int rc = backward_layers(m, B, Bp);
+    int rc = forward_hidden(m, d_x, B, Bp, true);
     if (rc) return rc;
-    if (loss) {
-        std::vector<double> part(nb);
-        HIPTRY(c, hipMemcpyAsync(part.data(), m->part.p, nb * sizeof(double), hipMemcpyDeviceToHost, m->st()));
-        HIPTRY(c, hipStreamSynchronize(m->st()));
-        double s = 0.0;
-        for (double v : part) s += v;
-        *loss = s / ((double)B * m->dim[L]);
-    }
+    MlpLayerArgs a = layer_args(m, L - 1, Bp);
+    a.t = d_t;
+    a.batch = B;
+    a.out = m->dim[L];
+    a.X = m->dZ[L - 1].p;
+    a.XT = m->dZT[L - 1].p;
+    a.bpart = m->bpart[L - 1].as<float>();
+    a.loss = m->loss.as<double>();
+    const int T = mlp_tile_rows(a.M, a.N);
+    m->parts[L - 1] = Bp / T;
+    m->loss_parts = (Bp / T) * (a.N / T);
+    HIPTRY(c, mlp_output_mse(a, m->st()));
+    return backward_data(m, Bp);
+}
+
+// The batch loss of the last forward_backward (synchronises).
+int read_loss(sqh_mlp* m, int B, double* loss) {
+    sqh_ctx* c = m->ctx;
+    std::vector<double> part(m->loss_parts);
+    HIPTRY(c, hipMemcpyAsync(part.data(), m->loss.p, part.size() * sizeof(double), hipMemcpyDeviceToHost, m->st()));
+    HIPTRY(c, hipStreamSynchronize(m->st()));
+    double s = 0.0;
+    for (double v : part) s += v;
+    *loss = s / ((double)B * m->dim[m->L]);
     return SQH_OK;
+}
+
+// The BF16 copies of layer l's master weights, in both orders.
+hipError_t convert_weights(sqh_mlp* m, int l) {
+    return mlp_convert(m->W[l].as<float>(), m->dpad[l + 1], m->dpad[l], m->dpad[l], m->Wb[l].p, m->WbT[l].p,
+                       m->dpad[l + 1], m->dpad[l], nullptr, m->st());
+}
+
+// He-style initialisation on the real block; the padding stays zero.
+__attribute__((noinline)) void he_init(std::mt19937_64& gen, std::normal_distribution<float>& nd, int no, int ni,
+                                       int kp, float* w) {
+    const float sd = std::sqrt(2.0f / (float)ni);
+    for (int o = 0; o < no; ++o)
+        for (int i = 0; i < ni; ++i) w[(size_t)o * kp + i] = sd * nd(gen);
 }
 
 // Host flat layout of parameters: per layer W (real out x real in, row-major), then b.
@@ -156,7 +211,7 @@ int copy_params(sqh_mlp* m, float* host, bool to_host, bool grads) {
         HIPTRY(c, mlp_pack_layer(Wd.as<float>(), bd.as<float>(), no, ni, kp, m->flat.as<float>() + off, to_host,
                                  m->st()));
         if (!to_host)
-            HIPTRY(c, mlp_f32_to_bf16(m->W[l].as<float>(), m->Wb[l].p, (size_t)m->dpad[l + 1] * kp, m->st()));
+            HIPTRY(c, convert_weights(m, l));
         return SQH_OK;
     });
     if (rc) return rc;
@@ -184,34 +239,32 @@ int sqh_mlp_create(sqh_ctx* c, int in_dim, int hidden, int n_hidden, int out_dim
     m->dim.push_back(out_dim);
     m->L = (int)m->dim.size() - 1;
     for (int d : m->dim) m->dpad.push_back(pad64(d));
-    for (auto* v : {&m->W, &m->Wb, &m->b, &m->mW, &m->vW, &m->mb, &m->vb, &m->gW, &m->gb, &m->Z, &m->dZf, &m->dZb})
+    for (auto* v : {&m->W, &m->Wb, &m->WbT, &m->b, &m->mW, &m->vW, &m->mb, &m->vb, &m->gW, &m->gb, &m->H, &m->HT,
+                    &m->Z, &m->dZ, &m->dZT, &m->bpart})
         v->resize(m->L);
-    m->H.resize(m->L + 1);
+    m->parts.assign(m->L, 0);
     std::mt19937_64 gen(seed);
     std::normal_distribution<float> nd(0.0f, 1.0f);
     for (int l = 0; l < m->L; ++l) {
         const int np = m->dpad[l + 1], kp = m->dpad[l];
         const size_t nw = (size_t)np * kp;
-        bool ok = m->W[l].ensure(nw * 4) == hipSuccess && m->Wb[l].ensure(nw * 2) == hipSuccess &&
+        bool ok = m->W[l].ensure(nw * 4) == hipSuccess && m->Wb[l].ensure((size_t)np * kp * 2) == hipSuccess &&
+                  m->WbT[l].ensure((size_t)kp * np * 2) == hipSuccess &&
                   m->mW[l].ensure(nw * 4) == hipSuccess && m->vW[l].ensure(nw * 4) == hipSuccess &&
-                  m->gW[l].ensure(nw * 4) == hipSuccess && m->b[l].ensure(np * 4) == hipSuccess &&
-                  m->mb[l].ensure(np * 4) == hipSuccess && m->vb[l].ensure(np * 4) == hipSuccess &&
-                  m->gb[l].ensure(np * 4) == hipSuccess;
+                  m->b[l].ensure(np * 4) == hipSuccess && m->mb[l].ensure(np * 4) == hipSuccess &&
+                  m->vb[l].ensure(np * 4) == hipSuccess;
         if (!ok) {
             delete m;
             return fail(c, SQH_ERR_NOMEM, "network allocation failed");
         }
-        // He-style initialisation on the real block, zeros in the padding.
         std::vector<float> w(nw, 0.0f);
-        const float sd = std::sqrt(2.0f / (float)m->dim[l]);
-        for (int o = 0; o < m->dim[l + 1]; ++o)
-            for (int i = 0; i < m->dim[l]; ++i) w[(size_t)o * kp + i] = sd * nd(gen);
+        he_init(gen, nd, m->dim[l + 1], m->dim[l], kp, w.data());
         hipError_t e = hipMemcpy(m->W[l].p, w.data(), nw * 4, hipMemcpyHostToDevice);
-        for (DevBuf* z : {&m->mW[l], &m->vW[l], &m->gW[l]})
+        for (DevBuf* z : {&m->mW[l], &m->vW[l]})
             if (e == hipSuccess) e = hipMemset(z->p, 0, nw * 4);
-        for (DevBuf* z : {&m->b[l], &m->mb[l], &m->vb[l], &m->gb[l]})
+        for (DevBuf* z : {&m->b[l], &m->mb[l], &m->vb[l]})
             if (e == hipSuccess) e = hipMemset(z->p, 0, (size_t)np * 4);
-        if (e == hipSuccess) e = mlp_f32_to_bf16(m->W[l].as<float>(), m->Wb[l].p, nw, c->stream);
+        if (e == hipSuccess) e = convert_weights(m, l);
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) {
             delete m;
@@ -257,11 +310,14 @@ int sqh_mlp_forward_dev(sqh_mlp* m, const float* d_x, int B, float* d_y) {
     std::lock_guard<std::mutex> lk(c->mu);
     HIPTRY(c, hipSetDevice(c->device));
     const int Bp = pad64(B);
-    int rc = ensure_batch(m, Bp);
+    int rc = ensure_batch(m, Bp, false);
     if (rc) return rc;
-    if ((rc = forward(m, d_x, B, Bp))) return rc;
-    HIPTRY(c, hipMemcpy2DAsync(d_y, (size_t)m->dim[m->L] * 4, m->Z[m->L - 1].p, (size_t)m->dpad[m->L] * 4,
-                               (size_t)m->dim[m->L] * 4, B, hipMemcpyDeviceToDevice, m->st()));
+    if ((rc = forward_hidden(m, d_x, B, Bp, false))) return rc;
+    MlpLayerArgs a = layer_args(m, m->L - 1, Bp);
+    a.y = d_y;
+    a.batch = B;
+    a.out = m->dim[m->L];
+    HIPTRY(c, mlp_output(a, m->st()));
     return SQH_OK;
 }
 
@@ -271,11 +327,11 @@ int sqh_mlp_train_step_dev(sqh_mlp* m, const float* d_x, const float* d_t, int B
     std::lock_guard<std::mutex> lk(c->mu);
     HIPTRY(c, hipSetDevice(c->device));
     const int Bp = pad64(B);
-    int rc = ensure_batch(m, Bp);
+    int rc = ensure_batch(m, Bp, true);
     if (rc) return rc;
-    if ((rc = forward(m, d_x, B, Bp))) return rc;
-    if ((rc = backward(m, d_t, B, Bp, loss))) return rc;
-    return adam_step(m, lr);
+    if ((rc = forward_backward(m, d_x, d_t, B, Bp))) return rc;
+    if ((rc = weights(m, Bp, true, lr))) return rc;
+    return loss ? read_loss(m, B, loss) : SQH_OK;
 }
 
 int sqh_mlp_backward_step_dev(sqh_mlp* m, const float* d_x, const float* d_dy, int B, float lr) {
@@ -283,15 +339,16 @@ int sqh_mlp_backward_step_dev(sqh_mlp* m, const float* d_x, const float* d_dy, i
     sqh_ctx* c = m->ctx;
     std::lock_guard<std::mutex> lk(c->mu);
     HIPTRY(c, hipSetDevice(c->device));
-    const int Bp = pad64(B);
-    int rc = ensure_batch(m, Bp);
+    const int Bp = pad64(B), L = m->L;
+    int rc = ensure_batch(m, Bp, true);
     if (rc) return rc;
-    if ((rc = forward(m, d_x, B, Bp))) return rc;
-    const int L = m->L;
-    HIPTRY(c, mlp_out_grad(d_dy, B, m->dim[L], m->dpad[L], Bp, m->dZf[L - 1].as<float>(), m->dZb[L - 1].p,
-                           m->st()));
-    if ((rc = backward_layers(m, B, Bp))) return rc;
-    return adam_step(m, lr);
+    // the output itself is not needed: its gradient is the caller's
+    if ((rc = forward_hidden(m, d_x, B, Bp, true))) return rc;
+    HIPTRY(c, mlp_convert(d_dy, B, m->dim[L], m->dim[L], m->dZ[L - 1].p, m->dZT[L - 1].p, Bp, m->dpad[L],
+                          m->bpart[L - 1].as<float>(), m->st()));
+    m->parts[L - 1] = Bp / 64;
+    if ((rc = backward_data(m, Bp))) return rc;
+    return weights(m, Bp, true, lr);
 }
 
 int sqh_mlp_gradients(sqh_mlp* m, const float* x, const float* t, int B, float* grads, double* loss) {
@@ -300,19 +357,17 @@ int sqh_mlp_gradients(sqh_mlp* m, const float* x, const float* t, int B, float* 
     std::lock_guard<std::mutex> lk(c->mu);
     HIPTRY(c, hipSetDevice(c->device));
     const int Bp = pad64(B);
-    int rc = ensure_batch(m, Bp);
+    int rc = ensure_batch(m, Bp, true);
     if (rc) return rc;
     DevBuf dx, dt;
     HIPTRY(c, dx.ensure((size_t)B * m->dim[0] * 4));
     HIPTRY(c, dt.ensure((size_t)B * m->dim[m->L] * 4));
     HIPTRY(c, hipMemcpyAsync(dx.p, x, (size_t)B * m->dim[0] * 4, hipMemcpyHostToDevice, m->st()));
     HIPTRY(c, hipMemcpyAsync(dt.p, t, (size_t)B * m->dim[m->L] * 4, hipMemcpyHostToDevice, m->st()));
-    rc = forward(m, dx.as<float>(), B, Bp);
-    if (!rc) rc = backward(m, dt.as<float>(), B, Bp, loss);
-    if (!rc) {
-        (void)hipStreamSynchronize(m->st());
-        rc = copy_params(m, grads, true, true);
-    }
+    rc = forward_backward(m, dx.as<float>(), dt.as<float>(), B, Bp);
+    if (!rc) rc = weights(m, Bp, false, 0.0f);
+    if (!rc && loss) rc = read_loss(m, B, loss);
+    if (!rc) rc = copy_params(m, grads, true, true);
     (void)hipStreamSynchronize(m->st());
     dx.release();
     dt.release();
