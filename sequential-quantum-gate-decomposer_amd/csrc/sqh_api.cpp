@@ -221,22 +221,34 @@ bool fused_cost_applies(const sqh_ctx* c, bool grad, const TraceSpec& ts) {
     return !grad && ts.nch == 0 && fused_pass_applies(c);
 }
 
-// Costs of B parameter vectors by the tile-resident fused-block kernels: block
-// matrices (from the kernel table kern, or each gate's 2x2 kernel computed from d_params
-// while staging) -> one launch over every column -> trace entries into diag.  U: the
-// target (rows x m, row stride m), or with in_index element b's target at
-// U + in_index[b] * in_bstride.
-int fused_cost_eval(sqh_ctx* c, bool f32, int B, const void* kern, const double* d_params, double* diag, int trace_off,
-                    const void* U, int m, const int* in_index, long long in_bstride) {
+// The 2x2 kernels of a batch computed from its parameters where they are used.
+GateKernels gate_kernels(const sqh_ctx* c, const double* d_params, int pstride) {
+    GateKernels g;
+    g.params = d_params;
+    g.pstride = pstride;
+    g.slots = c->d_slots.as<Slot>();
+    return g;
+}
+
+// The same from kernel tables.
+GateKernels gate_table(const void* kern, long long bstride) {
+    GateKernels g;
+    g.kern = kern;
+    g.kern_bstride = bstride;
+    return g;
+}
+
+// Costs of B parameter vectors by the tile-resident fused-block kernels: block matrices
+// -> one launch over every column -> trace entries into diag.  U: the target (rows x m,
+// row stride m), or with in_index element b's target at U + in_index[b] * in_bstride.
+int fused_cost_eval(sqh_ctx* c, bool f32, int B, const double* d_params, double* diag, int trace_off, const void* U, int m,
+                    const int* in_index, long long in_bstride) {
     const FusionPlan& fp = c->fplan;
-    const int nb = (int)fp.qubits.size(), ns = (int)c->prog.slots.size();
+    const int nb = (int)fp.qubits.size();
     const size_t esz = f32 ? 8 : 16;
     HIPTRY(c, c->d_fused.ensure((size_t)B * nb * 256 * esz));
-    // the block matrices from the kernel table kern, or with d_params straight from the
-    // parameters (no kernel table)
-    HIPTRY(c, launch_fuse_blocks(f32, c->d_fgates.p, c->d_ffirst.as<int>(), nb, kern, (long long)ns * 4, B,
-                                 c->d_fused.p, c->stream, nullptr, nullptr, d_params, c->prog.P,
-                                 c->d_slots.as<Slot>()));
+    HIPTRY(c, launch_fuse_blocks(f32, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb,
+                                 gate_kernels(c, d_params, c->prog.P), B, c->d_fused.p, c->stream));
     FusedCostArgs a;
     a.U = U;
     a.in_index = in_index;
@@ -304,7 +316,7 @@ bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, 
 // Costs and gradients of B parameter vectors through the fused blocks on stream st:
 // block matrices (into fused), the forward + backward kernel (trace entries into diag,
 // per-workgroup correlation partials into mpart), then each block's gate correlations
-// into corr ([B][ns][8]) for k_finish.  kern: the [B][ns][4] kernel tables; U: the
+// into corr ([B][ns][8]) for k_finish.  g: the gates' kernels; U: the
 // target (m columns, row stride m), or with bi.count the optimiser's per-run targets
 // (element e's at U + run_target[elem_run[e]] * tgt_stride, *count live elements).
 // The buffers hold the plan's sizes; nothing is allocated.
@@ -320,12 +332,11 @@ bool fused_grad_uses_chain(const sqh_ctx* c) {
     return S == (1u << c->prog.N) - 1u;
 }
 
-int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, const void* kern, const void* U,
+int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, const GateKernels& g, const void* U,
                    double* diag, int trace_off, void* fused, double* mpart, double* corr, const BatchIndex& bi,
                    hipStream_t st, bool timed) {
     const int N = c->prog.N, nb = (int)c->fplan.qubits.size(), ns = (int)c->prog.slots.size();
-    HIPTRY(c, launch_fuse_blocks(f32, c->d_fgates.p, c->d_ffirst.as<int>(), nb, kern, (long long)ns * 4, B, fused, st,
-                                 bi.count));
+    HIPTRY(c, launch_fuse_blocks(f32, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb, g, B, fused, st, bi.count));
     FusedGradArgs a;
     a.U = U;
     a.m = m;
@@ -348,24 +359,23 @@ int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, c
     } else {
         HIPTRY(c, launch_fused_grad(f32, N, a, p.T, p.waves, st));
     }
-    HIPTRY(c, launch_fused_block_corr(f32, c->d_fgates.p, c->d_ffirst.as<int>(), nb, kern, (long long)ns * 4, fused,
-                                      mpart, p.wgs, B, corr, ns, st, bi.count));
+    HIPTRY(c, launch_fused_block_corr(f32, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb, g, fused, mpart, p.wgs,
+                                      B, corr, ns, st, bi.count));
     return SQH_OK;
 }
 
 // The circuit as fused dense blocks (<= 4 qubits each): one HBM pass per block,
-// matrix cores for the 4-qubit FP64 blocks.  kern holds the kernel tables built for
-// this call (per matrix when kern_bstride != 0).
+// matrix cores.  Matrix b's parameters at d_params + b * pbstride (0: shared).
 int fused_apply(sqh_ctx* c, void* mats, int rows, int cols, int stride, long long bstride, int B, bool f32,
-                long long kern_bstride) {
+                const double* d_params, int pbstride) {
     const FusionPlan& fp = c->fplan;
     const int nb = (int)fp.qubits.size();
     if (nb == 0) return SQH_OK;
-    const int Bk = kern_bstride ? B : 1;
+    const int Bk = pbstride ? B : 1;
     const size_t esz = f32 ? 8 : 16;
     HIPTRY(c, c->d_fused.ensure((size_t)Bk * nb * 256 * esz));
-    HIPTRY(c, launch_fuse_blocks(f32, c->d_fgates.p, c->d_ffirst.as<int>(), nb, c->d_kern.p, kern_bstride, Bk,
-                                 c->d_fused.p, c->stream));
+    HIPTRY(c, launch_fuse_blocks(f32, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb,
+                                 gate_kernels(c, d_params, pbstride), Bk, c->d_fused.p, c->stream));
     BlockCfg cfg;
     int rc = block_config(c, f32, rows, cols, B, &cfg);
     if (rc) return rc;
@@ -408,14 +418,16 @@ int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double*
     const bool hs_corr = ts.nch > 0 && !uses_offset(c->variant);
     void* kern = nullptr;
     double* diag = nullptr;
-    // cost-only batches on the fused blocks build their 2x2 kernels inside the block build
+    // the fused blocks' kernels compute their 2x2 kernels from the parameters: no table
+    FusedGradPlan fgp;
+    const bool fused_grad = d_grad && !fixed && fused_grad_applies(c, ts, f32, B, m, &fgp);
     const bool fused_costs = !fixed && fused_cost_applies(c, d_grad != nullptr, ts);
     if (fixed) {
         kern = fixed->kern;
         diag = fixed->diag;
         HIPTRY(c, launch_build_kernels(f32, d_params, c->prog.P, B, c->d_slots.as<Slot>(), ns, kern, c->stream));
     } else {
-        if (!fused_costs && (rc = build_kernels(c, d_params, B, f32))) return rc;
+        if (!fused_costs && !fused_grad && N <= kMaxTileQubits && (rc = build_kernels(c, d_params, B, f32))) return rc;
         HIPTRY(c, c->d_diag.ensure((size_t)(ts.nch + 1) * B * m * 2 * sizeof(double)));
         kern = c->d_kern.p;
         diag = c->d_diag.as<double>();
@@ -429,12 +441,12 @@ int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double*
         return tile_launch(c, t, kind, fixed == nullptr);
     };
     const void* U = f32 ? c->d_U32.p : c->d_U64.p;
-    FusedGradPlan fgp;
-    if (d_grad && !fixed && fused_grad_applies(c, ts, f32, B, m, &fgp)) {
+    if (fused_grad) {
         HIPTRY(c, c->d_fused.ensure(fgp.fused_bytes));
         HIPTRY(c, c->d_mpart.ensure(fgp.mpart_bytes));
         HIPTRY(c, c->d_fcorr.ensure(fgp.corr_bytes));
-        if ((rc = fused_grad_run(c, f32, fgp, B, m, kern, U, diag, off, c->d_fused.p, c->d_mpart.as<double>(),
+        if ((rc = fused_grad_run(c, f32, fgp, B, m, gate_kernels(c, d_params, c->prog.P), U, diag, off, c->d_fused.p,
+                                 c->d_mpart.as<double>(),
                                  c->d_fcorr.as<double>(), BatchIndex(), c->stream, true)))
             return rc;
         HIPTRY(c, launch_finish(diag, m, B, c->variant, d_costs, c->d_fcorr.as<double>(), 1, ns, c->d_slots.as<Slot>(),
@@ -442,7 +454,7 @@ int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double*
         return SQH_OK;
     }
     if (fused_costs) {
-        if ((rc = fused_cost_eval(c, f32, B, nullptr, d_params, diag, off, U, m, nullptr, 0))) return rc;
+        if ((rc = fused_cost_eval(c, f32, B, d_params, diag, off, U, m, nullptr, 0))) return rc;
         HIPTRY(c, launch_finish(diag, m, B, c->variant, d_costs, nullptr, 0, ns, c->d_slots.as<Slot>(), d_params,
                                 c->prog.P, nullptr, c->stream, BatchIndex(), ts));
         return SQH_OK;
@@ -512,7 +524,7 @@ int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double*
     const long long msz = (long long)c->rows * m;
     HIPTRY(c, c->d_mat.ensure((size_t)B * msz * esz));
     HIPTRY(c, launch_broadcast_copy(f32, U, c->rows, m, m, c->d_mat.p, msz, B, c->stream));
-    if ((rc = fused_apply(c, c->d_mat.p, c->rows, m, m, msz, B, f32, (long long)ns * 4))) return rc;
+    if ((rc = fused_apply(c, c->d_mat.p, c->rows, m, m, msz, B, f32, d_params, c->prog.P))) return rc;
     HIPTRY(c, launch_extract_diag(f32, c->d_mat.p, msz, m, m, B, off, c->d_diag.as<double>(), N, ts, c->stream));
     HIPTRY(c, launch_finish(c->d_diag.as<double>(), m, B, c->variant, d_costs, nullptr, 0, ns, c->d_slots.as<Slot>(),
                             d_params, c->prog.P, nullptr, c->stream, BatchIndex(), ts));
@@ -533,7 +545,7 @@ int eval_targets(sqh_ctx* c, const double* d_params, int B, const void* d_target
         return fail(c, SQH_ERR_ARG, "targets must be %d x m with m + trace offset <= %d", 1 << N, 1 << N);
     const TraceSpec ts = trace_spec(c, B, m);
     const bool fused_costs = fused_cost_applies(c, false, ts);
-    if ((rc = build_kernels(c, d_params, B, false))) return rc;
+    if (!fused_costs && (rc = build_kernels(c, d_params, B, false))) return rc;
     HIPTRY(c, c->d_diag.ensure((size_t)(ts.nch + 1) * B * m * 2 * sizeof(double)));
     TileLaunch t = base_launch(c, false);
     t.in = d_targets;
@@ -549,8 +561,7 @@ int eval_targets(sqh_ctx* c, const double* d_params, int B, const void* d_target
     t.ts = ts;
     t.mode = 1;
     if (fused_costs) {
-        if ((rc = fused_cost_eval(c, false, B, c->d_kern.p, nullptr, t.diag, off, d_targets, m, d_index,
-                                  t.in_bstride)))
+        if ((rc = fused_cost_eval(c, false, B, d_params, t.diag, off, d_targets, m, d_index, t.in_bstride)))
             return rc;
     } else {
         TimedLaunch tl(c);
@@ -575,17 +586,19 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
     if (pbstride != 0 && pbstride != c->prog.P) return fail(c, SQH_ERR_ARG, "parameter batch stride must be 0 or P");
     const int ns = (int)c->prog.slots.size();
     const int Bk = pbstride ? B : 1;
-    if ((rc = build_kernels(c, d_params, Bk, f32))) return rc;
     const long long kb = pbstride ? (long long)ns * 4 : 0;
-    if (path == 0 && N > kMaxTileQubits) path = N >= 4 ? 2 : 1;
-    if (path == 0 && fused_pass_applies(c)) {
+    if (path == 0 && N > kMaxTileQubits) path = 2;
+    if (path == 2) return fused_apply(c, d_inout, rows, cols, stride, bstride, B, f32, d_params, pbstride);
+    const bool fused = path == 0 && fused_pass_applies(c);
+    if (!fused && (rc = build_kernels(c, d_params, Bk, f32))) return rc;
+    if (fused) {
         // the circuit's fused 4-qubit blocks on the matrix cores, every column resident
         const FusionPlan& fp = c->fplan;
         const int nb = (int)fp.qubits.size();
         const size_t esz = f32 ? 8 : 16;
         HIPTRY(c, c->d_fused.ensure((size_t)Bk * nb * 256 * esz));
-        HIPTRY(c, launch_fuse_blocks(f32, c->d_fgates.p, c->d_ffirst.as<int>(), nb, c->d_kern.p, kb, Bk, c->d_fused.p,
-                                     c->stream));
+        HIPTRY(c, launch_fuse_blocks(f32, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb,
+                                     gate_kernels(c, d_params, pbstride), Bk, c->d_fused.p, c->stream));
         FusedCostArgs a;
         a.U = d_inout;
         a.in_bstride = bstride;
@@ -620,7 +633,6 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
         HIPTRY(c, launch_tile_forward(t, c->stream));
         return SQH_OK;
     }
-    if (path == 2) return fused_apply(c, d_inout, rows, cols, stride, bstride, B, f32, kb);
     return stream_apply(c, d_inout, rows, cols, stride, bstride, B, f32, kb);
 }
 
@@ -652,8 +664,9 @@ int deriv_dev(sqh_ctx* c, const double* d_params, const void* d_in, int rows, in
         // per-parameter kernel tables), every column resident on the chip
         const int nb = (int)c->fplan.qubits.size();
         HIPTRY(c, c->d_fused.ensure((size_t)P * nb * 256 * 16));
-        HIPTRY(c, launch_fuse_blocks(false, c->d_fgates.p, c->d_ffirst.as<int>(), nb, c->d_dtab.p, (long long)ns * 4, P,
-                                     c->d_fused.p, c->stream, nullptr, controlled ? c->d_zslot.as<int>() : nullptr));
+        HIPTRY(c, launch_fuse_blocks(false, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb,
+                                     gate_table(c->d_dtab.p, (long long)ns * 4), P, c->d_fused.p, c->stream, nullptr,
+                                     controlled ? c->d_zslot.as<int>() : nullptr));
         FusedCostArgs a;
         a.U = d_in;
         a.in_stride = stride;
@@ -765,11 +778,10 @@ int sqh_set_circuit(sqh_ctx* c, int qbit_num, const sqh_gate* gates, int n_gates
     if (!p.slots.empty())
         HIPTRY(c, hipMemcpy(c->d_slots.p, p.slots.data(), p.slots.size() * sizeof(Slot), hipMemcpyHostToDevice));
     FusionPlan fp = plan_fusion(qbit_num, g, p.gate_slot);
-    static_assert(sizeof(FusedRec) == 8, "fused record layout");
-    HIPTRY(c, c->d_fgates.ensure(std::max<size_t>(fp.gates.size(), 1) * sizeof(FusedRec)));
+    HIPTRY(c, c->d_quads.ensure(std::max<size_t>(fp.quads.size(), 1) * sizeof(uint32_t)));
     HIPTRY(c, c->d_ffirst.ensure(fp.first.size() * sizeof(int)));
-    if (!fp.gates.empty())
-        HIPTRY(c, hipMemcpy(c->d_fgates.p, fp.gates.data(), fp.gates.size() * sizeof(FusedRec), hipMemcpyHostToDevice));
+    if (!fp.quads.empty())
+        HIPTRY(c, hipMemcpy(c->d_quads.p, fp.quads.data(), fp.quads.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     HIPTRY(c, hipMemcpy(c->d_ffirst.p, fp.first.data(), fp.first.size() * sizeof(int), hipMemcpyHostToDevice));
     if (qbit_num >= 4 && qbit_num <= kFusedCostMaxQubits && fp.k == 4 && !fp.qubits.empty()) {
         const std::vector<int> maps = fused_row_maps(qbit_num, fp);

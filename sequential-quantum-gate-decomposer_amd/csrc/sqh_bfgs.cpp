@@ -128,7 +128,8 @@ int enqueue_round(sqh_ctx* c, BatchBufs& bb, std::vector<Group>& groups, const B
             if (gr.fused[p]) {
                 // the fused blocks' adjoint: block matrices on the matrix cores forward and
                 // backward, each block's correlations resolved to its gates
-                const int rc = fused_grad_run(c, t.f32, gr.fplan[p], gr.B, gr.cols, t.kern, t.in, t.diag, t.trace_off,
+                const int rc = fused_grad_run(c, t.f32, gr.fplan[p], gr.B, gr.cols,
+                                              gate_table(t.kern, t.kern_bstride), t.in, t.diag, t.trace_off,
                                               gr.ffused.p, gr.fmpart.as<double>(), gr.fcorr.as<double>(), t.bi, st,
                                               false);
                 if (rc) return rc;

@@ -81,7 +81,7 @@ struct sqh_ctx {
 
     // Dense-block fusion of the circuit for the streaming path.
     sqh::FusionPlan fplan;
-    sqh::DevBuf d_fgates, d_ffirst, d_fused;
+    sqh::DevBuf d_quads, d_ffirst, d_fused;
     // Row tables of the tile-resident fused-block cost kernel ([blocks][kFusedMapStride];
     // present for 4 <= N <= 10) and its switch (sqh_set_fused_cost).
     sqh::DevBuf d_fmaps;
@@ -123,7 +123,7 @@ struct sqh_ctx {
             (void)hipEventDestroy(e.second);
         }
         for (sqh::DevBuf* b : {&d_ops, &d_lays, &d_slots, &d_U64, &d_U32, &d_params, &d_kern, &d_diag, &d_mpart,
-                               &d_res, &d_mat, &d_out, &d_fgates, &d_ffirst, &d_fused, &d_fmaps, &d_tmaps, &d_fcorr, &d_idx, &d_seed, &d_dtab, &d_zslot})
+                               &d_res, &d_mat, &d_out, &d_quads, &d_ffirst, &d_fused, &d_fmaps, &d_tmaps, &d_fcorr, &d_idx, &d_seed, &d_dtab, &d_zslot})
             b->release();
         for (hipStream_t s : side) (void)hipStreamDestroy(s);
         for (hipEvent_t e : side_ev) (void)hipEventDestroy(e);
@@ -183,7 +183,8 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
               long long bstride, int B, bool f32, int path);
 int deriv_dev(sqh_ctx* c, const double* d_params, const void* d_in, int rows, int cols, int stride, void* d_out);
 int fused_apply(sqh_ctx* c, void* mats, int rows, int cols, int stride, long long bstride, int B, bool f32,
-                long long kern_bstride);
+                const double* d_params, int pbstride);
+GateKernels gate_table(const void* kern, long long bstride);
 // Run-time specialised kernel for the current program: kind 0 forward store, 1
 // forward diagonal, 2 gradient (sqh_jit.cpp).
 // With compile = false a kernel that is not compiled yet is not compiled: the call
@@ -208,13 +209,6 @@ hipError_t launch_block_apply(bool f32, bool use_mfma, void* mats, long long bst
 // the tuned one for this shape, or (tuning on, not under graph capture) tuned now by
 // timing every candidate on a scratch batch of the same shape (sqh_tune.cpp).
 int block_config(sqh_ctx* c, bool f32, int rows, int m, int B, BlockCfg* out);
-// With params (and slots), each element's 2x2 kernels are computed from its P
-// parameters while staging (kern unused): the cost pass needs no kernel table.
-hipError_t launch_fuse_blocks(bool f32, const void* fg, const int* block_first, int nblocks, const void* kern,
-                              long long kern_bstride, int Bk, void* out, hipStream_t s, const int* count = nullptr,
-                              const int* zslot = nullptr, const double* params = nullptr, int P = 0,
-                              const Slot* slots = nullptr);
-size_t fused_gate_bytes();
 // Fused-block cost + gradient (sqh_api.cpp): launch shape and scratch sizes, the
 // applicability rule, and the enqueue (no allocation) on a stream.
 struct FusedGradPlan {
@@ -223,7 +217,7 @@ struct FusedGradPlan {
 };
 bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, FusedGradPlan& p);
 bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, int m, FusedGradPlan* plan);
-int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, const void* kern, const void* U,
+int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, const GateKernels& g, const void* U,
                    double* diag, int trace_off, void* fused, double* mpart, double* corr, const BatchIndex& bi,
                    hipStream_t st, bool timed);
 // The fused-block cost launch with the context's launch shape (forced, tuned or default).

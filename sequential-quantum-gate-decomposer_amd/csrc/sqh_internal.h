@@ -48,6 +48,20 @@ enum OpKind : uint8_t {
     OP_NOP = 5,    // padding around the program (never executed, only prefetched)
 };
 
+// A gate of a fused block as the block kernels walk it: kind, the pair of local qubits
+// (a, b) whose rows a lane holds while the gate runs, kernel-table slot + 1 (0: none).
+enum QuadKind : uint32_t {
+    QK_UA = 0,   // 2x2 on a
+    QK_UB = 1,   // 2x2 on b
+    QK_XA = 2,   // CNOT: target a, control b
+    QK_XB = 3,   // CNOT: target b, control a
+    QK_Z = 4,    // CZ
+    QK_CUA = 5,  // controlled 2x2: target a, control b
+    QK_CUB = 6,  // controlled 2x2: target b, control a
+};
+constexpr int kQuadPairShift = 4;  // a, then b in the next two bits
+constexpr int kQuadSlotShift = 8;
+
 // Padding records on each side of the device copy of a program, so the kernels'
 // look-ahead loads need no bounds checks.
 constexpr int kOpPad = 2;

@@ -1,7 +1,6 @@
 // sqh_k_block.hip -- dense 2^k x 2^k blocks on k qubits, applied in one HBM pass
 // (apply_large_kernel_to_input, apply_large_kernel_to_input.cpp:82-102, 124+: local
-// index bit i <-> the i-th smallest involved qubit), and the fusion of gate runs into
-// such blocks.
+// index bit i <-> the i-th smallest involved qubit).
 //
 // k = 4 runs on the matrix cores: a wavefront computes a 16 x 16 output tile Y = F X
 // for 16 columns with 16 MFMAs (four real products, K = 16 in steps of 4):
@@ -164,92 +163,6 @@ __global__ __launch_bounds__(256) void k_block_mfma4(cpx<R>* __restrict__ mats, 
     }
 }
 
-// Fused block matrices: the block's gates (FusedGate: local qubits 0..3, the block's
-// slots) applied to the unit columns e_j.
-
-// Gates staged per pass and batch elements per workgroup (x 16 block columns = one
-// wavefront) of k_fuse_blocks.
-constexpr int kFuseChunk = 32;
-constexpr int kFuseElems = 4;
-
-// Workgroup -> (block, 16 batch elements); thread -> (element, column j of the block).
-// The block's gate records and the elements' 2x2 kernels of those gates are staged in
-// LDS a chunk at a time (all loads in flight together), then every thread applies the
-// gates to its unit column e_j.
-template <typename R>
-__global__ __launch_bounds__(16 * kFuseElems) void k_fuse_blocks(const FusedGate* __restrict__ fg,
-                                                     const int* __restrict__ block_first, int nblocks,
-                                                     const cpx<R>* __restrict__ kern, long long kern_bstride, int Bk,
-                                                     cpx<R>* __restrict__ out, const int* __restrict__ count,
-                                                     const int* __restrict__ zslot, const double* __restrict__ params,
-                                                     int P, const Slot* __restrict__ slots) {
-    __shared__ FusedGate srec[kFuseChunk];
-    __shared__ cpx<R> skern[kFuseElems][kFuseChunk][4];
-    const int blk = blockIdx.x % nblocks;
-    const int b0 = (blockIdx.x / nblocks) * kFuseElems;
-    if (count) Bk = min(*count, Bk);  // live elements (the optimiser's rounds)
-    if (b0 >= Bk) return;             // the whole workgroup
-    const int le = threadIdx.x >> 4, j = threadIdx.x & 15;
-    // apply_derivate_to: the element's differentiated controlled gate (or -1) runs with
-    // its control-0 block zeroed (the derivative of a controlled kernel)
-    const int zs = (zslot && b0 + le < Bk) ? zslot[b0 + le] : -1;
-    cpx<R> v[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = mk<R>(i == j ? (R)1 : (R)0, (R)0);
-    const int first = block_first[blk], last = block_first[blk + 1];
-    for (int p0 = first; p0 < last; p0 += kFuseChunk) {
-        const int cnt = min(kFuseChunk, last - p0);
-        __syncthreads();  // the previous chunk is consumed
-        for (int i = threadIdx.x; i < cnt; i += blockDim.x) srec[i] = fg[p0 + i];
-        __syncthreads();
-        if (params) {
-            // the 2x2 kernels from the elements' parameters (as k_build_kernels computes them)
-            for (int i = threadIdx.x; i < kFuseElems * cnt; i += blockDim.x) {
-                const int e = i / cnt, gi = i % cnt;
-                const int slot = srec[gi].slot;
-                if (slot >= 0 && b0 + e < Bk) {
-                    const Slot sl = slots[slot];
-                    cpx<double> k4[4];
-                    dev_gate_kernel(sl.type, params + (long long)(b0 + e) * P + sl.param_start, k4);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) skern[e][gi][k] = cvt<R>(k4[k]);
-                }
-            }
-        } else {
-            for (int i = threadIdx.x; i < kFuseElems * cnt * 4; i += blockDim.x) {
-                const int e = i / (cnt * 4), gi = (i / 4) % cnt, k = i % 4;
-                const int slot = srec[gi].slot;
-                if (slot >= 0 && b0 + e < Bk) skern[e][gi][k] = kern[(long long)(b0 + e) * kern_bstride + 4 * slot + k];
-            }
-        }
-        __syncthreads();
-        for (int gi = 0; gi < cnt; ++gi) {
-            const FusedGate gt = srec[gi];
-            Op op;
-            op.kind = (uint8_t)gt.kind;
-            op.t = (uint8_t)gt.t;
-            op.cmode = gt.c >= 0 ? CM_REG : CM_NONE;
-            op.c = (uint8_t)(gt.c >= 0 ? gt.c : 0);
-            op.idx = gt.slot;
-            cpx<R> k[4] = {mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0)};
-            if (gt.slot >= 0) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) k[e] = skern[le][gi][e];
-            }
-            if (gt.slot == zs && op.kind == OP_CU)
-                exec_gate<4, true, R>(v, op, k, 0);
-            else
-                exec_gate<4, false, R>(v, op, k, 0);
-        }
-    }
-    const int b = b0 + le;
-    if (b >= Bk) return;
-    // out[b][blk][i][j]
-    cpx<R>* o = out + ((long long)b * nblocks + blk) * 256;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) o[i * 16 + j] = v[i];
-}
-
 // Launchers -----------------------------------------------------------------------
 
 template <typename R, int K>
@@ -320,23 +233,5 @@ hipError_t launch_block_apply(bool f32, bool use_mfma, void* mats, long long bst
     return f32 ? launch_fma<float>(mats, bstride, stride, rows, m, B, F, fbstride, bq, s)
                : launch_fma<double>(mats, bstride, stride, rows, m, B, F, fbstride, bq, s);
 }
-
-hipError_t launch_fuse_blocks(bool f32, const void* fg, const int* block_first, int nblocks, const void* kern,
-                              long long kern_bstride, int Bk, void* out, hipStream_t s, const int* count,
-                              const int* zslot, const double* params, int P, const Slot* slots) {
-    if (params && !slots) return hipErrorInvalidValue;
-    if ((long long)Bk * nblocks == 0) return hipSuccess;
-    const long long grid = (long long)nblocks * ((Bk + kFuseElems - 1) / kFuseElems);
-    const int threads = 16 * kFuseElems;
-    if (f32)
-        hipLaunchKernelGGL(k_fuse_blocks<float>, dim3((unsigned)grid), dim3(threads), 0, s, (const FusedGate*)fg,
-                           block_first, nblocks, (const cpx<float>*)kern, kern_bstride, Bk, (cpx<float>*)out, count, zslot, params, P, slots);
-    else
-        hipLaunchKernelGGL(k_fuse_blocks<double>, dim3((unsigned)grid), dim3(threads), 0, s, (const FusedGate*)fg,
-                           block_first, nblocks, (const cpx<double>*)kern, kern_bstride, Bk, (cpx<double>*)out, count, zslot, params, P, slots);
-    return hipGetLastError();
-}
-
-size_t fused_gate_bytes() { return sizeof(FusedGate); }
 
 }  // namespace sqh

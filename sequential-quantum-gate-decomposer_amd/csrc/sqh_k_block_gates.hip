@@ -1,0 +1,382 @@
+// sqh_k_block_gates.hip -- the gates inside the fused 4-qubit blocks: the blocks' 16 x 16
+// matrices (k_fuse_blocks) and, for the gradient, each gate's 2 x 2 correlations from its
+// block's 16 x 16 correlation (k_fused_block_corr).
+//
+// Both walk a block's gates on 16-row vectors, one wavefront per (block, element), with
+// the 16 columns' 256 entries as 4 rows per lane: lane = column + 16 z holds the quad of
+// rows that differ in the two qubits (a, b) a run of gates acts on, z numbering the other
+// two qubits.  Gates on a and b, CNOTs between them included, work on the lane's own four
+// values; when the pair changes, the rows go through LDS once.  The host orders a block's
+// gates into runs per pair (quad_ops): a run of a CNOT layer is the CNOT and two U3.
+//
+// What bounds these kernels is latency (a block has some twenty dependent gates), so the
+// code that a gate runs is kept short enough to stay in the instruction cache: the same
+// few operations for every pair, where a walk with every target and control of a 16-row
+// register column unrolled took 27 us a block build and 74 us a correlation walk with the
+// partials' sum (8 qubits, one element; 30 and 100 for 512).  Now 12 and 22 (16 and 61),
+// with the kernel table's launch gone: gradient of one 8-qubit vector 209 -> 117 us.
+#include <hip/hip_runtime.h>
+
+#include "sqh_device.h"
+#include "sqh_kernels.h"
+
+namespace sqh {
+
+namespace {
+
+__device__ __forceinline__ void quad_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// Rows of the lane's quad for the pair in an op word: row0 | (k & 1 ? u : 0) | (k & 2 ? v : 0).
+struct QuadRows {
+    int row0, u, v;
+};
+__device__ __forceinline__ QuadRows quad_rows(uint32_t pair, int z) {
+    const int qa = pair & 3, qb = pair >> 2;
+    const int rest = 15 ^ (1 << qa) ^ (1 << qb);
+    const int c = __builtin_ctz(rest), d = 31 - __builtin_clz(rest);
+    return {((z & 1) << c) | ((z >> 1) << d), 1 << qa, 1 << qb};
+}
+__device__ __forceinline__ int quad_row(const QuadRows& q, int k) {
+    return q.row0 | ((k & 1) ? q.u : 0) | ((k & 2) ? q.v : 0);
+}
+
+template <typename R>
+__device__ __forceinline__ void quad_store(const cpx<R> (&v)[4], const QuadRows& q, int col, cpx<R>* s) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s[quad_row(q, k) * 16 + col] = v[k];
+}
+template <typename R>
+__device__ __forceinline__ void quad_load(cpx<R> (&v)[4], const QuadRows& q, int col, const cpx<R>* s) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = s[quad_row(q, k) * 16 + col];
+}
+
+template <typename R>
+__device__ __forceinline__ void quad_pair(cpx<R>& x0, cpx<R>& x1, const cpx<R> (&k)[4]) {
+    const cpx<R> a = mac2(k[0], x0, k[1], x1), b = mac2(k[2], x0, k[3], x1);
+    x0 = a;
+    x1 = b;
+}
+
+template <typename R>
+__device__ __forceinline__ void quad_swap(cpx<R>& a, cpx<R>& b) {
+    const cpx<R> t = a;
+    a = b;
+    b = t;
+}
+
+// A gate backwards on a pair of rows: x <- G^dagger x, acc += y x^T, y <- G^T y.
+template <typename R>
+__device__ __forceinline__ void quad_back(cpx<R>& x0, cpx<R>& x1, cpx<R>& y0, cpx<R>& y1, const cpx<R> (&kd)[4],
+                                          const cpx<R> (&kt)[4], cpx<R> (&acc)[4]) {
+    quad_pair(x0, x1, kd);
+    cacc(acc[0], y0, x0);
+    cacc(acc[1], y0, x1);
+    cacc(acc[2], y1, x0);
+    cacc(acc[3], y1, x1);
+    quad_pair(y0, y1, kt);
+}
+
+// The 2 x 2 kernels of a chunk's gates for one element into tab[gate][4], a gate per lane:
+// computed from the element's parameters as k_build_kernels does (FP64, then converted),
+// or taken from the element's kernel table.
+template <typename R>
+__device__ __forceinline__ void quad_stage(uint32_t w, bool live, const cpx<R>* kern, const double* params,
+                                           const Slot* slots, int lane, cpx<R>* tab) {
+    const int slot = (int)(w >> kQuadSlotShift) - 1;
+    if (live && slot >= 0) {
+        if (params) {
+            const Slot sl = slots[slot];
+            cpx<double> k4[4];
+            dev_gate_kernel(sl.type, params + sl.param_start, k4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) tab[4 * lane + k] = cvt<R>(k4[k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) tab[4 * lane + k] = kern[4 * slot + k];
+        }
+    }
+}
+
+// Sums of eight values over the wavefront: on return lanes 0, 16, 32, 48 hold the sums of
+// values {0, 2, 1, 3} in lo and of values {4, 6, 5, 7} in hi.  The first two steps halve
+// the values held per lane while they add across lane halves and rows
+// (v_permlane32_swap / v_permlane16_swap exchange one value's upper half with another's
+// lower), so eight sums take 42 instructions where a butterfly for each takes 144.
+__device__ __forceinline__ double lane_halves(double a, double b, bool rows) {
+    const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    unsigned p[2], q[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const unsigned xs = (unsigned)(x >> (32 * h)), ys = (unsigned)(y >> (32 * h));
+        const auto r = rows ? __builtin_amdgcn_permlane16_swap(xs, ys, false, false)
+                            : __builtin_amdgcn_permlane32_swap(xs, ys, false, false);
+        p[h] = r[0];
+        q[h] = r[1];
+    }
+    return __longlong_as_double((unsigned long long)p[0] | ((unsigned long long)p[1] << 32)) +
+           __longlong_as_double((unsigned long long)q[0] | ((unsigned long long)q[1] << 32));
+}
+__device__ __forceinline__ double row_sum(double v) {
+    v += dpp_f64<0x128>(v);  // row_ror:8
+    v += dpp_f64<0x124>(v);  // row_ror:4
+    v += dpp_f64<0x122>(v);  // row_ror:2
+    v += dpp_f64<0x121>(v);  // row_ror:1
+    return v;
+}
+__device__ __forceinline__ void wave_sum8(const double (&r)[8], double& lo, double& hi) {
+    double s[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = lane_halves(r[2 * i], r[2 * i + 1], false);
+    lo = row_sum(lane_halves(s[0], s[1], true));
+    hi = row_sum(lane_halves(s[2], s[3], true));
+}
+
+}  // namespace
+
+constexpr int kQuadWaves = 4;  // elements per workgroup of the block build
+
+template <typename R>
+__global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t* __restrict__ ops,
+                                                                 const int* __restrict__ first, int nb,
+                                                                 const cpx<R>* __restrict__ kern,
+                                                                 long long kern_bstride,
+                                                                 const double* __restrict__ params, int pstride,
+                                                                 const Slot* __restrict__ slots, int B,
+                                                                 cpx<R>* __restrict__ out,
+                                                                 const int* __restrict__ count,
+                                                                 const int* __restrict__ zslot) {
+    __shared__ cpx<R> state[kQuadWaves][256];
+    __shared__ cpx<R> table[kQuadWaves][64 * 4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int blk = blockIdx.x % nb, e = (blockIdx.x / nb) * kQuadWaves + wave;
+    if (count) B = min(*count, B);  // live elements (the optimiser's rounds)
+    if (e >= B) return;             // the whole wavefront; the waves share nothing
+    const int col = lane & 15, z = lane >> 4;
+    cpx<R>* s = state[wave];
+    cpx<R>* tab = table[wave];
+    // apply_derivate_to: the element's differentiated controlled gate (or -1) runs with its
+    // control-0 rows zeroed (the derivative of a controlled kernel)
+    const int zs = zslot ? zslot[e] : -1;
+    const int p0 = first[blk], p1 = first[blk + 1];
+    uint32_t pair = 4;  // qubits 0 and 1
+    QuadRows q = quad_rows(pair, z);
+    cpx<R> v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = mk<R>(quad_row(q, k) == col ? (R)1 : (R)0, (R)0);
+    for (int p = p0; p < p1; p += 64) {
+        const int cnt = min(64, p1 - p);
+        const uint32_t w = lane < cnt ? ops[p + lane] : 0;
+        quad_fence();  // the previous chunk's table is read
+        quad_stage<R>(w, lane < cnt, kern + e * kern_bstride, params ? params + (long long)e * pstride : nullptr, slots,
+                      lane, tab);
+        quad_fence();
+        for (int i = 0; i < cnt; ++i) {
+            const uint32_t op = __builtin_amdgcn_readlane(w, i);
+            const uint32_t pr = (op >> kQuadPairShift) & 15;
+            cpx<R> k[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) k[t] = tab[4 * i + t];
+            if (pr != pair) {
+                quad_store(v, q, col, s);
+                quad_fence();
+                pair = pr;
+                q = quad_rows(pair, z);
+                quad_load(v, q, col, s);
+                quad_fence();
+            }
+            switch (op & 15) {
+            case QK_UA:
+                quad_pair(v[0], v[1], k);
+                quad_pair(v[2], v[3], k);
+                break;
+            case QK_UB:
+                quad_pair(v[0], v[2], k);
+                quad_pair(v[1], v[3], k);
+                break;
+            case QK_XA: quad_swap(v[2], v[3]); break;
+            case QK_XB: quad_swap(v[1], v[3]); break;
+            case QK_Z: v[3] = mk<R>(-v[3].re, -v[3].im); break;
+            case QK_CUA:
+                quad_pair(v[2], v[3], k);
+                if ((int)(op >> kQuadSlotShift) - 1 == zs) v[0] = v[1] = mk<R>(0, 0);
+                break;
+            default:  // QK_CUB
+                quad_pair(v[1], v[3], k);
+                if ((int)(op >> kQuadSlotShift) - 1 == zs) v[0] = v[2] = mk<R>(0, 0);
+                break;
+            }
+        }
+    }
+    cpx<R>* o = out + ((long long)e * nb + blk) * 256;  // out[e][blk][row][col]
+    quad_store(v, q, col, o);
+}
+
+// Sums the workgroup partials of the block's correlation M_b (SPLIT: a workgroup per (block,
+// element), each of its four wavefronts every fourth partial, then only the first goes on;
+// else a wavefront per (block, element), four elements per workgroup), starts from x = the
+// columns of F_b and y = the columns of M_b and walks the gates backwards: x <- G^dagger x,
+// the pair correlations of y and x summed over the wavefront, y <- G^T y.
+// corr[e][slot][8] is the register-tile adjoint's layout.
+template <typename R, bool SPLIT>
+__global__ __launch_bounds__(256) void k_fused_block_corr(const uint32_t* __restrict__ ops,
+                                                          const int* __restrict__ first, int nb,
+                                                          const cpx<R>* __restrict__ kern, long long kern_bstride,
+                                                          const double* __restrict__ params, int pstride,
+                                                          const Slot* __restrict__ slots, const cpx<R>* __restrict__ F,
+                                                          const double* __restrict__ mpart, int wgs, int B,
+                                                          double* __restrict__ corr, int ns,
+                                                          const int* __restrict__ count) {
+    constexpr int E = SPLIT ? 1 : 4;  // elements per workgroup
+    __shared__ cpx<double> sums[4][256];
+    __shared__ cpx<R> states[E][512], tables[E][64 * 4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int blk = blockIdx.x % nb, e = (blockIdx.x / nb) * E + (SPLIT ? 0 : wave);
+    if (count) B = min(*count, B);
+    if (e >= B) return;  // the whole workgroup, or a wavefront that shares nothing
+    {
+        const cpx<double>* M = reinterpret_cast<const cpx<double>*>(mpart) + ((long long)e * wgs * nb + blk) * 256;
+        cpx<double> acc[4] = {mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0)};
+#pragma unroll 4
+        for (int p = SPLIT ? wave : 0; p < wgs; p += SPLIT ? 4 : 1) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const cpx<double> t = M[(long long)p * nb * 256 + 64 * i + lane];
+                acc[i].re += t.re;
+                acc[i].im += t.im;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sums[wave][64 * i + lane] = acc[i];
+    }
+    if constexpr (SPLIT) {
+        __syncthreads();
+        if (wave != 0) return;
+    } else {
+        quad_fence();
+    }
+    const int col = lane & 15, z = lane >> 4;
+    cpx<R>* sx = states[SPLIT ? 0 : wave];
+    cpx<R>* sy = sx + 256;
+    cpx<R>* tab = tables[SPLIT ? 0 : wave];
+    const cpx<R>* Fb = F + ((long long)e * nb + blk) * 256;
+    const int p0 = first[blk], p1 = first[blk + 1];
+    uint32_t pair = 4;
+    QuadRows q = quad_rows(pair, z);
+    cpx<R> x[4], y[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int at = quad_row(q, k) * 16 + col;
+        x[k] = Fb[at];
+        cpx<double> a = sums[SPLIT ? 0 : wave][at];
+        if constexpr (SPLIT) {
+            const cpx<double> b = sums[1][at], c = sums[2][at], d = sums[3][at];
+            a = mk((a.re + b.re) + (c.re + d.re), (a.im + b.im) + (c.im + d.im));
+        }
+        y[k] = mk<R>((R)a.re, (R)a.im);
+    }
+    for (int pe = p1; pe > p0; pe -= 64) {
+        const int p = max(p0, pe - 64), cnt = pe - p;
+        const uint32_t w = lane < cnt ? ops[p + lane] : 0;
+        quad_fence();
+        quad_stage<R>(w, lane < cnt, kern + e * kern_bstride, params ? params + (long long)e * pstride : nullptr, slots,
+                      lane, tab);
+        quad_fence();
+        for (int i = cnt - 1; i >= 0; --i) {
+            const uint32_t op = __builtin_amdgcn_readlane(w, i);
+            const uint32_t pr = (op >> kQuadPairShift) & 15;
+            cpx<R> k[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) k[t] = tab[4 * i + t];
+            if (pr != pair) {
+                quad_store(x, q, col, sx);
+                quad_store(y, q, col, sy);
+                quad_fence();
+                pair = pr;
+                q = quad_rows(pair, z);
+                quad_load(x, q, col, sx);
+                quad_load(y, q, col, sy);
+                quad_fence();
+            }
+            const cpx<R> kd[4] = {mk(k[0].re, -k[0].im), mk(k[2].re, -k[2].im), mk(k[1].re, -k[1].im),
+                                  mk(k[3].re, -k[3].im)};
+            const cpx<R> kt[4] = {k[0], k[2], k[1], k[3]};
+            cpx<R> acc[4] = {mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0)};
+            // CNOT and CZ are their own adjoint and transpose
+            switch (op & 15) {
+            case QK_UA:
+                quad_back(x[0], x[1], y[0], y[1], kd, kt, acc);
+                quad_back(x[2], x[3], y[2], y[3], kd, kt, acc);
+                break;
+            case QK_UB:
+                quad_back(x[0], x[2], y[0], y[2], kd, kt, acc);
+                quad_back(x[1], x[3], y[1], y[3], kd, kt, acc);
+                break;
+            case QK_CUA: quad_back(x[2], x[3], y[2], y[3], kd, kt, acc); break;
+            case QK_CUB: quad_back(x[1], x[3], y[1], y[3], kd, kt, acc); break;
+            case QK_XA:
+                quad_swap(x[2], x[3]);
+                quad_swap(y[2], y[3]);
+                continue;
+            case QK_XB:
+                quad_swap(x[1], x[3]);
+                quad_swap(y[1], y[3]);
+                continue;
+            default:  // QK_Z
+                x[3] = mk<R>(-x[3].re, -x[3].im);
+                y[3] = mk<R>(-y[3].re, -y[3].im);
+                continue;
+            }
+            double r[8], lo, hi;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                r[2 * t] = (double)acc[t].re;
+                r[2 * t + 1] = (double)acc[t].im;
+            }
+            wave_sum8(r, lo, hi);
+            if (col == 0) {
+                double* d = corr + ((long long)e * ns + (int)(op >> kQuadSlotShift) - 1) * 8;
+                const int at = ((z & 1) << 1) | (z >> 1);  // values 0, 2, 1, 3 for z = 0 .. 3
+                d[at] = lo;
+                d[4 + at] = hi;
+            }
+        }
+    }
+}
+
+hipError_t launch_fuse_blocks(bool f32, const uint32_t* ops, const int* first, int nb, const GateKernels& g, int B,
+                              void* out, hipStream_t s, const int* count, const int* zslot) {
+    if ((long long)B * nb == 0) return hipSuccess;
+    const unsigned grid = (unsigned)(nb * (long long)((B + kQuadWaves - 1) / kQuadWaves));
+    if (f32)
+        hipLaunchKernelGGL(k_fuse_blocks<float>, dim3(grid), dim3(64 * kQuadWaves), 0, s, ops, first, nb,
+                           (const cpx<float>*)g.kern, g.kern_bstride, g.params, g.pstride, g.slots, B, (cpx<float>*)out,
+                           count, zslot);
+    else
+        hipLaunchKernelGGL(k_fuse_blocks<double>, dim3(grid), dim3(64 * kQuadWaves), 0, s, ops, first, nb,
+                           (const cpx<double>*)g.kern, g.kern_bstride, g.params, g.pstride, g.slots, B,
+                           (cpx<double>*)out, count, zslot);
+    return hipGetLastError();
+}
+
+hipError_t launch_fused_block_corr(bool f32, const uint32_t* ops, const int* first, int nb, const GateKernels& g,
+                                   const void* F, const double* mpart, int wgs, int B, double* corr, int ns,
+                                   hipStream_t s, const int* count) {
+    if ((long long)B * nb == 0) return hipSuccess;
+    // With a wavefront per SIMD's worth of (block, element) pairs each sums its own
+    // partials; below that, as with one vector, the sum is the longer part and is split.
+    const bool split = (long long)B * nb < 1024;
+    const unsigned grid = (unsigned)(nb * (long long)(split ? B : (B + 3) / 4));
+#define SQH_CORR(R, SP)                                                                                       \
+    hipLaunchKernelGGL((k_fused_block_corr<R, SP>), dim3(grid), dim3(256), 0, s, ops, first, nb,               \
+                       (const cpx<R>*)g.kern, g.kern_bstride, g.params, g.pstride, g.slots, (const cpx<R>*)F,  \
+                       mpart, wgs, B, corr, ns, count)
+    if (f32 && split) SQH_CORR(float, true);
+    else if (f32) SQH_CORR(float, false);
+    else if (split) SQH_CORR(double, true);
+    else SQH_CORR(double, false);
+#undef SQH_CORR
+    return hipGetLastError();
+}
+
+}  // namespace sqh

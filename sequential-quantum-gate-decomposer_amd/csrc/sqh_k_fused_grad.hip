@@ -520,126 +520,6 @@ __global__ __launch_bounds__(512) void k_fused_grad_chain(FusedGradArgs a) {
     for (int b = 1; b + 1 < a.nb; ++b) step(b, false);
 }
 
-// The workgroup partials of every (element, block) M summed in a fixed order, in place
-// into the first partial: thread per double, consecutive threads on consecutive
-// entries.
-__global__ __launch_bounds__(256) void k_fused_sum_partials(double* __restrict__ mpart, int wgs, int nb,
-                                                            long long total, const int* __restrict__ count) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;  // total = B * nb * 512
-    const long long per_e = (long long)nb * 512;
-    const long long e = i / per_e, r = i % per_e;
-    if (count && e >= *count) return;
-    double* base = mpart + e * wgs * per_e + r;
-    double sum = base[0];
-    for (int v = 1; v < wgs; ++v) sum += base[(long long)v * per_e];
-    base[0] = sum;
-}
-
-// Gates staged per pass and batch elements per workgroup (x 16 block columns = one
-// wavefront) of k_fused_block_corr.
-constexpr int kCorrChunk = 32;
-constexpr int kCorrElems = 4;
-
-// Workgroup -> (block, 4 batch elements); thread -> (element, column k of the block).
-// Thread k starts from x = F_b e_k (column k of the block matrix) and y = column k of
-// M_b (the workgroup partials, summed into the first) and walks the block's gates
-// backwards: x <- G^dagger x, the pair correlations of y and x, y <- G^T y.  The 16
-// threads of an element sum their correlations in a fixed butterfly order, giving each
-// parametric gate's 2x2 correlations in corr[e][slot][8] (the register-tile adjoint's
-// layout).  Gate records and the elements' 2x2 kernels are staged in LDS a chunk at a
-// time (from the block's end), so the walk issues no dependent global loads.
-template <typename R>
-__global__ __launch_bounds__(16 * kCorrElems) void k_fused_block_corr(const FusedGate* __restrict__ fg,
-                                                         const int* __restrict__ block_first, int nb,
-                                                         const cpx<R>* __restrict__ kern, long long kern_bstride,
-                                                         const cpx<R>* __restrict__ F, const double* __restrict__ mpart,
-                                                         int wgs, int B, double* __restrict__ corr, int ns,
-                                                         const int* __restrict__ count) {
-    __shared__ FusedGate srec[kCorrChunk];
-    __shared__ cpx<R> skern[kCorrElems][kCorrChunk][4];
-    const int blk = blockIdx.x % nb;
-    const int e0 = (blockIdx.x / nb) * kCorrElems;
-    if (count) B = min(*count, B);
-    if (e0 >= B) return;  // the whole workgroup
-    const int le = threadIdx.x >> 4, k = threadIdx.x & 15;
-    const int e = e0 + le;
-    const bool live = e < B;
-    cpx<R> x[16], y[16];
-    {
-        const cpx<R>* Fb = F + ((long long)(live ? e : 0) * nb + blk) * 256;
-        const double* Mb = mpart + ((long long)(live ? e : 0) * wgs * nb + blk) * 512;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            x[i] = live ? Fb[i * 16 + k] : mk<R>(0, 0);
-            y[i] = live ? mk<R>((R)Mb[(i * 16 + k) * 2], (R)Mb[(i * 16 + k) * 2 + 1]) : mk<R>(0, 0);
-        }
-    }
-    const int first = block_first[blk], last = block_first[blk + 1];
-    for (int p1 = last; p1 > first; p1 -= kCorrChunk) {
-        const int p0 = max(first, p1 - kCorrChunk), cnt = p1 - p0;
-        __syncthreads();  // the previous chunk is consumed
-        for (int i = threadIdx.x; i < cnt; i += blockDim.x) srec[i] = fg[p0 + i];
-        __syncthreads();
-        for (int i = threadIdx.x; i < kCorrElems * cnt * 4; i += blockDim.x) {
-            const int el = i / (cnt * 4), gi = (i / 4) % cnt, t = i % 4;
-            const int slot = srec[gi].slot;
-            if (slot >= 0 && e0 + el < B) skern[el][gi][t] = kern[(long long)(e0 + el) * kern_bstride + 4 * slot + t];
-        }
-        __syncthreads();
-        for (int gi = cnt - 1; gi >= 0; --gi) {
-            const FusedGate gt = srec[gi];
-            Op op;
-            op.kind = (uint8_t)gt.kind;
-            op.t = (uint8_t)gt.t;
-            op.cmode = gt.c >= 0 ? CM_REG : CM_NONE;
-            op.c = (uint8_t)(gt.c >= 0 ? gt.c : 0);
-            op.idx = gt.slot;
-            cpx<R> kk[4] = {mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0)};
-            if (gt.slot >= 0) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) kk[t] = skern[le][gi][t];
-            }
-            if (op.kind == OP_X || op.kind == OP_Z) {
-                // self-inverse real symmetric: G^dagger = G^T = G
-                exec_gate<4, false, R>(x, op, kk, 0);
-                exec_gate<4, false, R>(y, op, kk, 0);
-                continue;
-            }
-            cpx<R> kd[4] = {mk(kk[0].re, -kk[0].im), mk(kk[2].re, -kk[2].im), mk(kk[1].re, -kk[1].im),
-                            mk(kk[3].re, -kk[3].im)};
-            cpx<R> kt[4] = {kk[0], kk[2], kk[1], kk[3]};
-            cpx<R> acc[4] = {mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0)};
-            switch (op.kind * 4 + op.t) {
-                SQH_ARMS(OP_U, 4, (pairs_apply<T, false, false>(x, kd, 0u), pairs_corr<T>(y, x, acc, 0u, false),
-                                   pairs_apply<T, false, false>(y, kt, 0u)))
-                SQH_ARMS(OP_CU, 4,
-                         (pairs_apply<T, true, false>(x, kd, ctrl_mask<4>(op.cmode, op.c, 0)),
-                          pairs_corr<T>(y, x, acc, ctrl_mask<4>(op.cmode, op.c, 0), true),
-                          pairs_apply<T, true, false>(y, kt, ctrl_mask<4>(op.cmode, op.c, 0))))
-            default:
-                break;
-            }
-            double r[8];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                r[2 * t] = (double)acc[t].re;
-                r[2 * t + 1] = (double)acc[t].im;
-            }
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-#pragma unroll
-                for (int off = 8; off >= 1; off >>= 1) r[t] += __shfl_xor(r[t], off, 16);
-            }
-            if (live && k == 0 && gt.slot >= 0) {
-                double* d = corr + ((long long)e * ns + gt.slot) * 8;
-#pragma unroll
-                for (int t = 0; t < 8; ++t) d[t] = r[t];
-            }
-        }
-    }
-}
-
 size_t fused_grad_lds_bytes(bool f32, int nb, int T, int waves) {
     // both row tables (the chain kernel's too), then one region per wavefront
     const size_t esz = f32 ? 8 : 16;
@@ -699,27 +579,6 @@ hipError_t launch_fused_grad(bool f32, int N, FusedGradArgs a, int T, int waves,
     const size_t shm = fused_grad_lds_bytes(f32, a.nb, T, waves);
     return f32 ? launch_fg<float>(N, a, T, grid, 64 * waves, shm, s)
                : launch_fg<double>(N, a, T, grid, 64 * waves, shm, s);
-}
-
-hipError_t launch_fused_block_corr(bool f32, const void* fg, const int* block_first, int nb, const void* kern,
-                                   long long kern_bstride, const void* F, double* mpart, int wgs, int B, double* corr,
-                                   int ns, hipStream_t s, const int* count) {
-    const long long pairs = (long long)B * nb;
-    if (pairs == 0) return hipSuccess;
-    if (wgs > 1) {
-        const long long total = pairs * 512;
-        hipLaunchKernelGGL(k_fused_sum_partials, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                           mpart, wgs, nb, total, count);
-    }
-    const long long groups = (B + kCorrElems - 1) / kCorrElems;
-    const unsigned grid = (unsigned)(groups * nb);
-    if (f32)
-        hipLaunchKernelGGL(k_fused_block_corr<float>, dim3(grid), dim3(16 * kCorrElems), 0, s, (const FusedGate*)fg, block_first,
-                           nb, (const cpx<float>*)kern, kern_bstride, (const cpx<float>*)F, mpart, wgs, B, corr, ns, count);
-    else
-        hipLaunchKernelGGL(k_fused_block_corr<double>, dim3(grid), dim3(16 * kCorrElems), 0, s, (const FusedGate*)fg, block_first,
-                           nb, (const cpx<double>*)kern, kern_bstride, (const cpx<double>*)F, mpart, wgs, B, corr, ns, count);
-    return hipGetLastError();
 }
 
 }  // namespace sqh

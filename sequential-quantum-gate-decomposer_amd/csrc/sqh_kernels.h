@@ -114,12 +114,21 @@ struct FusedCostArgs {
     int out_stride = 0;
     int groups = 0;  // column groups per element (set by the launcher)
 };
-// A gate of a fused block: OP_U / OP_CU / OP_X / OP_Z, local target, local control (-1
-// none), parametric slot (kernel table index) or -1 (the host's FusedRec layout).
-struct FusedGate {
-    int8_t kind, t, c, pad;
-    int32_t slot;
+// 2 x 2 kernels of the parametric gates of a batch: element e's computed from its P
+// parameters at params + e * pstride, or (params null) read from its table at
+// kern + e * kern_bstride ([slot][4]).
+struct GateKernels {
+    const void* kern = nullptr;
+    long long kern_bstride = 0;
+    const double* params = nullptr;
+    int pstride = 0;
+    const Slot* slots = nullptr;
 };
+// The 16 x 16 matrices of the fused blocks (out[B][nb][16][16]) from their gates (quad
+// ops, quad_ops).  count: live elements; zslot: per element the controlled slot whose
+// control-0 rows are zeroed, or -1.
+hipError_t launch_fuse_blocks(bool f32, const uint32_t* ops, const int* first, int nb, const GateKernels& g, int B,
+                              void* out, hipStream_t s, const int* count = nullptr, const int* zslot = nullptr);
 
 // Cost and gradient through the fused blocks (sqh_k_fused_grad.hip): the forward pass
 // and trace entries as the cost kernel, then the blocks backwards with the trace
@@ -156,9 +165,9 @@ hipError_t launch_fused_grad(bool f32, int N, FusedGradArgs a, int T, int waves,
 // 16-dimensional vectors (from the columns of F, the block matrices [B][nb][16][16]),
 // giving each parametric slot's 2x2 correlations in corr[B][ns][8] (the register-tile
 // adjoint's layout, one partial per element).
-hipError_t launch_fused_block_corr(bool f32, const void* fg, const int* block_first, int nb, const void* kern,
-                                   long long kern_bstride, const void* F, double* mpart, int wgs, int B, double* corr,
-                                   int ns, hipStream_t s, const int* count = nullptr);
+hipError_t launch_fused_block_corr(bool f32, const uint32_t* ops, const int* first, int nb, const GateKernels& g,
+                                   const void* F, const double* mpart, int wgs, int B, double* corr, int ns,
+                                   hipStream_t s, const int* count = nullptr);
 
 // Launch shape: tiles per wavefront (2 or 4), LDS exchange groups per block (1, or 2
 // with 4 tiles and prefetch), waves per workgroup (1, 2 or 4), next block's matrix

@@ -351,6 +351,52 @@ bool compile_program(int N, const std::vector<GateRec>& gates, Program& prog, st
     return true;
 }
 
+std::vector<uint32_t> quad_ops(const FusionPlan& fp) {
+    std::vector<uint32_t> out;
+    for (size_t b = 0; b + 1 < fp.first.size(); ++b) {
+        std::vector<FusedRec> left(fp.gates.begin() + fp.first[b], fp.gates.begin() + fp.first[b + 1]);
+        // the gates of left that run on qubits (x, y) before any that needs another qubit
+        auto run = [&](int x, int y, std::vector<FusedRec>* taken) {
+            bool blocked[4] = {false, false, false, false};
+            int n = 0;
+            std::vector<FusedRec> rest;
+            for (const FusedRec& g : left) {
+                auto inside = [&](int q) { return q < 0 || q == x || q == y; };
+                const bool ok = inside(g.t) && inside(g.c) && !blocked[g.t] && (g.c < 0 || !blocked[g.c]);
+                if (ok) {
+                    ++n;
+                    if (taken) taken->push_back(g);
+                } else {
+                    blocked[g.t] = true;
+                    if (g.c >= 0) blocked[g.c] = true;
+                    if (taken) rest.push_back(g);
+                }
+            }
+            if (taken) left.swap(rest);
+            return n;
+        };
+        while (!left.empty()) {
+            int bx = 0, by = 1, best = -1;
+            for (int x = 0; x < 4; ++x)
+                for (int y = x + 1; y < 4; ++y) {
+                    const int n = run(x, y, nullptr);
+                    if (n > best) best = n, bx = x, by = y;
+                }
+            std::vector<FusedRec> taken;
+            run(bx, by, &taken);
+            for (const FusedRec& g : taken) {
+                const bool a = g.t == bx;
+                const uint32_t kind = g.kind == OP_U ? (a ? QK_UA : QK_UB)
+                                      : g.kind == OP_X ? (a ? QK_XA : QK_XB)
+                                      : g.kind == OP_Z ? QK_Z : (a ? QK_CUA : QK_CUB);
+                out.push_back(kind | (uint32_t)(bx | by << 2) << kQuadPairShift |
+                              (uint32_t)(g.slot + 1) << kQuadSlotShift);
+            }
+        }
+    }
+    return out;
+}
+
 FusionPlan plan_fusion(int N, const std::vector<GateRec>& gates, const std::vector<int>& gate_slot) {
     FusionPlan fp;
     const int kmax = N < 4 ? N : 4;
@@ -416,6 +462,7 @@ FusionPlan plan_fusion(int N, const std::vector<GateRec>& gates, const std::vect
         if (!members.empty()) emit(cur, members);
     }
     fp.first.push_back((int)fp.gates.size());
+    if (fp.k == 4) fp.quads = quad_ops(fp);
     return fp;
 }
 

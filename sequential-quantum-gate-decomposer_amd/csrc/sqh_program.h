@@ -36,11 +36,17 @@ struct FusionPlan {
     std::vector<int> first;             // block b covers gates[first[b] .. first[b+1])
     std::vector<std::array<int, 4>> qubits;  // sorted qubits of each block
     int k = 0;                          // qubits per block
+    std::vector<uint32_t> quads;        // the same gates in the order the block kernels run them (quad_ops)
 };
 
 // Up to this many qubits the blocks are packed by dependency scheduling (a search over
 // the C(N, 4) qubit sets per block); above it, in gate-list order.
 constexpr int kFuseScheduleMaxQubits = 16;
+
+// The op words of each 4-qubit block's gates (same ranges as gates), ordered into runs on
+// one pair of local qubits: repeatedly the pair on which the most gates can run next.
+// Every qubit keeps its gates' order.
+std::vector<uint32_t> quad_ops(const FusionPlan& fp);
 
 // gate_slot: the kernel-table index of each parametric gate (Program::gate_slot).
 FusionPlan plan_fusion(int N, const std::vector<GateRec>& gates, const std::vector<int>& gate_slot);
