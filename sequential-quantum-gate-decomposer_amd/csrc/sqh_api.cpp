@@ -181,6 +181,42 @@ std::vector<int> fused_trace_maps(int N, const FusionPlan& fp) {
     return maps;
 }
 
+// Lane tables of the fused kernels (LT_*, sqh_kernels.h) from the two row tables.
+std::vector<int> fused_lane_tabs(int N, const FusionPlan& fp) {
+    const int nb = (int)fp.qubits.size(), D = 1 << N, O = D >> 4;
+    const std::vector<int> full = fused_row_maps(N, fp), chain = fused_trace_maps(N, fp);
+    std::vector<int> tabs((size_t)nb * kLaneTab, 0);
+    auto slot = [&](int j) {  // fc_slot
+        int h = N <= 4 ? 0 : j >> 4;
+        if (N > 8) h ^= h >> 4;
+        return j ^ (h & 15);
+    };
+    for (int b = 0; b < nb; ++b) {
+        int* t = tabs.data() + (size_t)b * kLaneTab;
+        const int* off = full.data() + (size_t)b * kFusedMapStride;
+        const int* kb = off + 16;
+        const int* cm = chain.data() + (size_t)b * kTraceMapStride;
+        const int lg = cm[80];
+        for (int l = 0; l < 64; ++l) {
+            const int nl = l & 15, g = l >> 4;
+            t[LT_ROW + l] = kb[nl % O] | off[g];
+            t[LT_LANE + l] = slot(t[LT_ROW + l]) ^ (nl / O * D);
+            t[LT_SLANE + l] = slot(cm[16 + (nl & ((1 << lg) - 1))] | off[g]);
+        }
+        for (int k = 0; k < 4; ++k) {
+            t[LT_RS + k] = off[4 * k];
+            t[LT_S + k] = slot(off[4 * k]);
+            // tile k: with 16 outer groups or fewer whole columns per tile, else 16 groups of one
+            t[LT_RT + k] = O > 16 ? kb[16 * (k % (O / 16))] : 0;
+            t[LT_T + k] = O > 16 ? slot(t[LT_RT + k]) ^ (k / (O / 16) * D) : k * (16 / O) * D;
+            t[LT_ST + k] = lg > 4 ? slot(cm[16 + 16 * (k & ((1 << (lg - 4)) - 1))]) : 0;
+        }
+        t[LT_LG] = lg;
+        t[LT_NS] = cm[81];
+    }
+    return tabs;
+}
+
 // The circuit fuses into 4-qubit blocks the fused kernels take (4 to 10 qubits).
 bool fused_plan_fits(const sqh_ctx* c) {
     const int N = c->prog.N;
@@ -261,6 +297,7 @@ int fused_cost_eval(sqh_ctx* c, bool f32, int B, const double* d_params, double*
     a.nb = nb;
     a.F = c->d_fused.p;
     a.maps = c->d_fmaps.as<int>();
+    a.tabs = c->d_ftabs.as<int>();
     a.diag = diag;
     TimedLaunch tl(c);
     return fused_cost_launch(c, f32, a);
@@ -290,7 +327,7 @@ bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, FusedGradPlan& p)
         }
     }
     if (!p.T) return false;
-    p.wgs = fused_grad_wgs(N, m, p.T, p.waves);
+    p.wgs = fused_grad_wgs(N, m, p.T, B);
     p.fused_bytes = (size_t)B * nb * 256 * (f32 ? 8 : 16);
     p.mpart_bytes = (size_t)B * p.wgs * nb * 512 * sizeof(double);
     p.corr_bytes = (size_t)B * std::max(ns, 1) * 8 * sizeof(double);
@@ -345,6 +382,7 @@ int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, c
     a.nb = nb;
     a.F = fused;
     a.maps = c->d_fmaps.as<int>();
+    a.tabs = c->d_ftabs.as<int>();
     a.diag = diag;
     a.mpart = mpart;
     a.wgs = p.wgs;
@@ -609,6 +647,7 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
         a.F = c->d_fused.p;
         a.F_bstride = Bk > 1 ? (long long)nb * 256 : 0;
         a.maps = c->d_fmaps.as<int>();
+    a.tabs = c->d_ftabs.as<int>();
         a.out = d_inout;
         a.out_bstride = bstride;
         a.out_stride = stride;
@@ -636,11 +675,10 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
     return stream_apply(c, d_inout, rows, cols, stride, bstride, B, f32, kb);
 }
 
-// Gates_block::apply_derivate_to: a forward store pass over P elements that share the
-// input, element k running the circuit with parameter k's gate replaced by its
-// derivative kernel (per-element kernel tables; a controlled gate's control-0 block
-// zeroed) -- through the fused blocks where that path applies (fused_pass_applies),
-// else the register-tile store kernel.  Output k is at d_out + k * rows * cols, row
+// Gates_block::apply_derivate_to: a forward store pass over P elements, element k running
+// the circuit with parameter k's gate replaced by its derivative kernel (a controlled
+// gate's control-0 block zeroed) -- through the fused blocks where that path applies
+// (fused_pass_applies), else the register-tile store kernel on per-element kernel tables.  Output k is at d_out + k * rows * cols, row
 // stride cols.
 int deriv_dev(sqh_ctx* c, const double* d_params, const void* d_in, int rows, int cols, int stride, void* d_out) {
     int rc = require_circuit(c);
@@ -652,6 +690,41 @@ int deriv_dev(sqh_ctx* c, const double* d_params, const void* d_in, int rows, in
         return fail(c, SQH_ERR_ARG, "apply_derivate_to supports up to %d qubits", kMaxTileQubits);
     if (c->prog.slots.empty()) return SQH_OK;
     const int ns = (int)c->prog.slots.size(), P = c->prog.P;
+    if (fused_pass_applies(c)) {
+        // Through the fused blocks: a derivative shares the blocks before its gate's with
+        // the others, so the products F_{b-1} ... F_0 in are formed once per block and
+        // element k starts from its block's, with that block differentiated.  The 8-qubit
+        // ansatz: 3.5 block products per element instead of 6.
+        const int nb = (int)c->fplan.qubits.size();
+        const long long msz = (long long)rows * cols;
+        HIPTRY(c, c->d_fused.ensure((size_t)(nb + P) * 256 * 16));
+        HIPTRY(c, c->d_dtab.ensure((size_t)nb * msz * 16));
+        HIPTRY(c, launch_fuse_deriv_blocks(c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb, d_params,
+                                           c->d_slots.as<Slot>(), c->d_dinfo.as<int>(), P, c->d_fused.p, c->stream));
+        FusedCostArgs a;
+        a.U = d_in;
+        a.in_stride = stride;
+        a.m = cols;
+        a.B = nb;
+        a.nb = nb;
+        a.F = c->d_fused.p;
+        a.maps = c->d_fmaps.as<int>();
+        a.tabs = c->d_ftabs.as<int>();
+        a.prefix = true;
+        a.out = c->d_dtab.p;
+        a.out_bstride = msz;
+        a.out_stride = cols;
+        if ((rc = fused_cost_launch(c, false, a))) return rc;
+        a.prefix = false;
+        a.dinfo = c->d_dinfo.as<int>();
+        a.U = c->d_dtab.p;
+        a.in_bstride = msz;
+        a.in_stride = cols;
+        a.B = P;
+        a.out = d_out;
+        TimedLaunch tl(c);
+        return fused_cost_launch(c, false, a);
+    }
     bool controlled = false;
     for (const Op& op : c->prog.ops) controlled |= op.kind == OP_CU;
     if ((rc = build_kernels(c, d_params, 1, false))) return rc;
@@ -659,29 +732,6 @@ int deriv_dev(sqh_ctx* c, const double* d_params, const void* d_in, int rows, in
     HIPTRY(c, c->d_zslot.ensure((size_t)P * sizeof(int)));
     HIPTRY(c, launch_deriv_tables(c->d_kern.p, c->d_slots.as<Slot>(), ns, d_params, P, c->d_dtab.p,
                                   c->d_zslot.as<int>(), c->stream));
-    if (fused_pass_applies(c)) {
-        // the fused blocks' store pass over the P elements (block matrices from the
-        // per-parameter kernel tables), every column resident on the chip
-        const int nb = (int)c->fplan.qubits.size();
-        HIPTRY(c, c->d_fused.ensure((size_t)P * nb * 256 * 16));
-        HIPTRY(c, launch_fuse_blocks(false, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb,
-                                     gate_table(c->d_dtab.p, (long long)ns * 4), P, c->d_fused.p, c->stream, nullptr,
-                                     controlled ? c->d_zslot.as<int>() : nullptr));
-        FusedCostArgs a;
-        a.U = d_in;
-        a.in_stride = stride;
-        a.m = cols;
-        a.B = P;
-        a.nb = nb;
-        a.F = c->d_fused.p;
-        a.F_bstride = (long long)nb * 256;
-        a.maps = c->d_fmaps.as<int>();
-        a.out = d_out;
-        a.out_bstride = (long long)rows * cols;
-        a.out_stride = cols;
-        TimedLaunch tl(c);
-        return fused_cost_launch(c, false, a);
-    }
     TileLaunch t = base_launch(c, false);
     t.kern = c->d_dtab.p;
     t.kern_bstride = (long long)ns * 4;
@@ -787,6 +837,26 @@ int sqh_set_circuit(sqh_ctx* c, int qbit_num, const sqh_gate* gates, int n_gates
         const std::vector<int> maps = fused_row_maps(qbit_num, fp);
         HIPTRY(c, c->d_fmaps.ensure(maps.size() * sizeof(int)));
         HIPTRY(c, hipMemcpy(c->d_fmaps.p, maps.data(), maps.size() * sizeof(int), hipMemcpyHostToDevice));
+        // per parameter: its gate's block, slot, which of the gate's parameters it is, and
+        // whether the gate is controlled
+        std::vector<int> dinfo((size_t)std::max(p.P, 1) * 4, 0);
+        for (size_t b = 0; b < fp.qubits.size(); ++b)
+            for (int i = fp.first[b]; i < fp.first[b + 1]; ++i) {
+                if (fp.gates[i].slot < 0) continue;
+                const Slot& sl = p.slots[fp.gates[i].slot];
+                for (int k = 0; k < sl.nparam; ++k) {
+                    int* d = dinfo.data() + 4 * (size_t)(sl.param_start + k);
+                    d[0] = (int)b;
+                    d[1] = fp.gates[i].slot;
+                    d[2] = k;
+                    d[3] = fp.gates[i].kind == OP_CU;
+                }
+            }
+        HIPTRY(c, c->d_dinfo.ensure(dinfo.size() * sizeof(int)));
+        HIPTRY(c, hipMemcpy(c->d_dinfo.p, dinfo.data(), dinfo.size() * sizeof(int), hipMemcpyHostToDevice));
+        const std::vector<int> tabs = fused_lane_tabs(qbit_num, fp);
+        HIPTRY(c, c->d_ftabs.ensure(tabs.size() * sizeof(int)));
+        HIPTRY(c, hipMemcpy(c->d_ftabs.p, tabs.data(), tabs.size() * sizeof(int), hipMemcpyHostToDevice));
         const std::vector<int> tmaps = fused_trace_maps(qbit_num, fp);
         HIPTRY(c, c->d_tmaps.ensure(tmaps.size() * sizeof(int)));
         HIPTRY(c, hipMemcpy(c->d_tmaps.p, tmaps.data(), tmaps.size() * sizeof(int), hipMemcpyHostToDevice));

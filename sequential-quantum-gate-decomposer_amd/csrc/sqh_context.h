@@ -75,7 +75,7 @@ struct sqh_ctx {
 
     sqh::DevBuf d_params, d_kern, d_diag, d_mpart, d_res, d_mat, d_out;
     sqh::DevBuf d_seed;  // [B][3] complex adjoint seed weights of the HS correction variants
-    sqh::DevBuf d_dtab, d_zslot;  // apply_derivate_to: per-parameter kernel tables, derivative slots
+    sqh::DevBuf d_dtab, d_zslot;  // apply_derivate_to: per-parameter kernel tables (or prefix products), derivative slots
     sqh::DevBuf d_idx;  // [count][0..B) identity element list of the per-target evaluation
     int idx_B = -1;
 
@@ -85,6 +85,8 @@ struct sqh_ctx {
     // Row tables of the tile-resident fused-block cost kernel ([blocks][kFusedMapStride];
     // present for 4 <= N <= 10) and its switch (sqh_set_fused_cost).
     sqh::DevBuf d_fmaps;
+    sqh::DevBuf d_dinfo;  // per parameter its gate's block, slot, index in the gate, controlled
+    sqh::DevBuf d_ftabs;  // lane tables of the fused kernels ([blocks][kLaneTab])
     // Row tables of the transposed-chain cost kernel ([blocks][kTraceMapStride]) and its
     // switch (sqh_set_fused_cost_chain; on by default): the cost pass builds the rows of
     // the circuit matrix the trace needs instead of running the target's columns forward.
@@ -123,7 +125,7 @@ struct sqh_ctx {
             (void)hipEventDestroy(e.second);
         }
         for (sqh::DevBuf* b : {&d_ops, &d_lays, &d_slots, &d_U64, &d_U32, &d_params, &d_kern, &d_diag, &d_mpart,
-                               &d_res, &d_mat, &d_out, &d_quads, &d_ffirst, &d_fused, &d_fmaps, &d_tmaps, &d_fcorr, &d_idx, &d_seed, &d_dtab, &d_zslot})
+                               &d_res, &d_mat, &d_out, &d_quads, &d_ffirst, &d_fused, &d_fmaps, &d_ftabs, &d_dinfo, &d_tmaps, &d_fcorr, &d_idx, &d_seed, &d_dtab, &d_zslot})
             b->release();
         for (hipStream_t s : side) (void)hipStreamDestroy(s);
         for (hipEvent_t e : side_ev) (void)hipEventDestroy(e);

@@ -594,6 +594,32 @@ __device__ __forceinline__ double dpp_f64(double v) {
     return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
 }
 
+// Two values a, b over the wavefront's halves (or, with rows, over the even and odd rows of
+// 16 lanes): lanes of the lower half (even rows) get a's sum over both, the others b's.
+// v_permlane32_swap exchanges its first operand's upper half with the second's lower one,
+// v_permlane16_swap the odd rows with the even ones.
+__device__ __forceinline__ double lane_halves(double a, double b, bool rows) {
+    const unsigned long long x = __builtin_bit_cast(unsigned long long, a), y = __builtin_bit_cast(unsigned long long, b);
+    unsigned p[2], q[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const unsigned xs = (unsigned)(x >> (32 * h)), ys = (unsigned)(y >> (32 * h));
+        const auto r = rows ? __builtin_amdgcn_permlane16_swap(xs, ys, false, false)
+                            : __builtin_amdgcn_permlane32_swap(xs, ys, false, false);
+        p[h] = r[0];
+        q[h] = r[1];
+    }
+    return __builtin_bit_cast(double, (unsigned long long)p[0] | ((unsigned long long)p[1] << 32)) +
+           __builtin_bit_cast(double, (unsigned long long)q[0] | ((unsigned long long)q[1] << 32));
+}
+__device__ __forceinline__ double row_sum(double v) {
+    v += dpp_f64<0x128>(v);  // row_ror:8
+    v += dpp_f64<0x124>(v);  // row_ror:4
+    v += dpp_f64<0x122>(v);  // row_ror:2
+    v += dpp_f64<0x121>(v);  // row_ror:1
+    return v;
+}
+
 // Sum over all 64 lanes of the wavefront with DPP row operations (no LDS round
 // trips): pairs within quads, half rows, rows, then rows 0+1 into 1 and 2+3 into 3
 // by row broadcasts, and 0..2 into 3; the total lands in lane 63 and is read back

@@ -80,15 +80,17 @@ __device__ __forceinline__ void quad_back(cpx<R>& x0, cpx<R>& x1, cpx<R>& y0, cp
 // The 2 x 2 kernels of a chunk's gates for one element into tab[gate][4], a gate per lane:
 // computed from the element's parameters as k_build_kernels does (FP64, then converted),
 // or taken from the element's kernel table.
+// Gate dslot gets its derivative with respect to its parameter dparam.
 template <typename R>
 __device__ __forceinline__ void quad_stage(uint32_t w, bool live, const cpx<R>* kern, const double* params,
-                                           const Slot* slots, int lane, cpx<R>* tab) {
+                                           const Slot* slots, int lane, cpx<R>* tab, int dslot = -1, int dparam = 0) {
     const int slot = (int)(w >> kQuadSlotShift) - 1;
     if (live && slot >= 0) {
         if (params) {
             const Slot sl = slots[slot];
             cpx<double> k4[4];
-            dev_gate_kernel(sl.type, params + sl.param_start, k4);
+            if (slot == dslot) dev_deriv_kernel(sl.type, params + sl.param_start, dparam, k4);
+            else dev_gate_kernel(sl.type, params + sl.param_start, k4);
 #pragma unroll
             for (int k = 0; k < 4; ++k) tab[4 * lane + k] = cvt<R>(k4[k]);
         } else {
@@ -101,29 +103,7 @@ __device__ __forceinline__ void quad_stage(uint32_t w, bool live, const cpx<R>* 
 // Sums of eight values over the wavefront: on return lanes 0, 16, 32, 48 hold the sums of
 // values {0, 2, 1, 3} in lo and of values {4, 6, 5, 7} in hi.  The first two steps halve
 // the values held per lane while they add across lane halves and rows
-// (v_permlane32_swap / v_permlane16_swap exchange one value's upper half with another's
-// lower), so eight sums take 42 instructions where a butterfly for each takes 144.
-__device__ __forceinline__ double lane_halves(double a, double b, bool rows) {
-    const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
-    unsigned p[2], q[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const unsigned xs = (unsigned)(x >> (32 * h)), ys = (unsigned)(y >> (32 * h));
-        const auto r = rows ? __builtin_amdgcn_permlane16_swap(xs, ys, false, false)
-                            : __builtin_amdgcn_permlane32_swap(xs, ys, false, false);
-        p[h] = r[0];
-        q[h] = r[1];
-    }
-    return __longlong_as_double((unsigned long long)p[0] | ((unsigned long long)p[1] << 32)) +
-           __longlong_as_double((unsigned long long)q[0] | ((unsigned long long)q[1] << 32));
-}
-__device__ __forceinline__ double row_sum(double v) {
-    v += dpp_f64<0x128>(v);  // row_ror:8
-    v += dpp_f64<0x124>(v);  // row_ror:4
-    v += dpp_f64<0x122>(v);  // row_ror:2
-    v += dpp_f64<0x121>(v);  // row_ror:1
-    return v;
-}
+// (lane_halves), so eight sums take 42 instructions where a butterfly for each takes 144.
 __device__ __forceinline__ void wave_sum8(const double (&r)[8], double& lo, double& hi) {
     double s[4];
 #pragma unroll
@@ -136,7 +116,9 @@ __device__ __forceinline__ void wave_sum8(const double (&r)[8], double& lo, doub
 
 constexpr int kQuadWaves = 4;  // elements per workgroup of the block build
 
-template <typename R>
+// A wavefront per (block, element); DERIV: per block of the one parameter vector, then per
+// parameter with its gate differentiated (launch_fuse_deriv_blocks; B is nb + P then).
+template <typename R, bool DERIV>
 __global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t* __restrict__ ops,
                                                                  const int* __restrict__ first, int nb,
                                                                  const cpx<R>* __restrict__ kern,
@@ -145,19 +127,25 @@ __global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t*
                                                                  const Slot* __restrict__ slots, int B,
                                                                  cpx<R>* __restrict__ out,
                                                                  const int* __restrict__ count,
-                                                                 const int* __restrict__ zslot) {
+                                                                 const int* __restrict__ dinfo) {
     __shared__ cpx<R> state[kQuadWaves][256];
     __shared__ cpx<R> table[kQuadWaves][64 * 4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int blk = blockIdx.x % nb, e = (blockIdx.x / nb) * kQuadWaves + wave;
+    const int e = (DERIV ? blockIdx.x : blockIdx.x / nb) * kQuadWaves + wave;
     if (count) B = min(*count, B);  // live elements (the optimiser's rounds)
     if (e >= B) return;             // the whole wavefront; the waves share nothing
+    int blk = DERIV ? e : blockIdx.x % nb, dslot = -1, dparam = 0;
+    bool zero = false;  // the differentiated gate is controlled: its control-0 rows become zero
+    if (DERIV && e >= nb) {
+        const int* d = dinfo + 4 * (e - nb);
+        blk = __builtin_amdgcn_readfirstlane(d[0]);
+        dslot = __builtin_amdgcn_readfirstlane(d[1]);
+        dparam = d[2];
+        zero = d[3] != 0;
+    }
     const int col = lane & 15, z = lane >> 4;
     cpx<R>* s = state[wave];
     cpx<R>* tab = table[wave];
-    // apply_derivate_to: the element's differentiated controlled gate (or -1) runs with its
-    // control-0 rows zeroed (the derivative of a controlled kernel)
-    const int zs = zslot ? zslot[e] : -1;
     const int p0 = first[blk], p1 = first[blk + 1];
     uint32_t pair = 4;  // qubits 0 and 1
     QuadRows q = quad_rows(pair, z);
@@ -169,7 +157,7 @@ __global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t*
         const uint32_t w = lane < cnt ? ops[p + lane] : 0;
         quad_fence();  // the previous chunk's table is read
         quad_stage<R>(w, lane < cnt, kern + e * kern_bstride, params ? params + (long long)e * pstride : nullptr, slots,
-                      lane, tab);
+                      lane, tab, dslot, dparam);
         quad_fence();
         for (int i = 0; i < cnt; ++i) {
             const uint32_t op = __builtin_amdgcn_readlane(w, i);
@@ -199,27 +187,27 @@ __global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t*
             case QK_Z: v[3] = mk<R>(-v[3].re, -v[3].im); break;
             case QK_CUA:
                 quad_pair(v[2], v[3], k);
-                if ((int)(op >> kQuadSlotShift) - 1 == zs) v[0] = v[1] = mk<R>(0, 0);
+                if (zero && (int)(op >> kQuadSlotShift) - 1 == dslot) v[0] = v[1] = mk<R>(0, 0);
                 break;
             default:  // QK_CUB
                 quad_pair(v[1], v[3], k);
-                if ((int)(op >> kQuadSlotShift) - 1 == zs) v[0] = v[2] = mk<R>(0, 0);
+                if (zero && (int)(op >> kQuadSlotShift) - 1 == dslot) v[0] = v[2] = mk<R>(0, 0);
                 break;
             }
         }
     }
-    cpx<R>* o = out + ((long long)e * nb + blk) * 256;  // out[e][blk][row][col]
+    cpx<R>* o = out + (DERIV ? (long long)e : (long long)e * nb + blk) * 256;  // [row][col]
     quad_store(v, q, col, o);
 }
 
 // Sums the workgroup partials of the block's correlation M_b (SPLIT: a workgroup per (block,
-// element), each of its four wavefronts every fourth partial, then only the first goes on;
+// element), each of its eight wavefronts every eighth partial, then only the first goes on;
 // else a wavefront per (block, element), four elements per workgroup), starts from x = the
 // columns of F_b and y = the columns of M_b and walks the gates backwards: x <- G^dagger x,
 // the pair correlations of y and x summed over the wavefront, y <- G^T y.
 // corr[e][slot][8] is the register-tile adjoint's layout.
 template <typename R, bool SPLIT>
-__global__ __launch_bounds__(256) void k_fused_block_corr(const uint32_t* __restrict__ ops,
+__global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const uint32_t* __restrict__ ops,
                                                           const int* __restrict__ first, int nb,
                                                           const cpx<R>* __restrict__ kern, long long kern_bstride,
                                                           const double* __restrict__ params, int pstride,
@@ -228,26 +216,22 @@ __global__ __launch_bounds__(256) void k_fused_block_corr(const uint32_t* __rest
                                                           double* __restrict__ corr, int ns,
                                                           const int* __restrict__ count) {
     constexpr int E = SPLIT ? 1 : 4;  // elements per workgroup
-    __shared__ cpx<double> sums[4][256];
+    __shared__ double sums[SPLIT ? 8 : 4][512];  // 256 real, then 256 imaginary parts
     __shared__ cpx<R> states[E][512], tables[E][64 * 4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int blk = blockIdx.x % nb, e = (blockIdx.x / nb) * E + (SPLIT ? 0 : wave);
     if (count) B = min(*count, B);
     if (e >= B) return;  // the whole workgroup, or a wavefront that shares nothing
     {
-        const cpx<double>* M = reinterpret_cast<const cpx<double>*>(mpart) + ((long long)e * wgs * nb + blk) * 256;
-        cpx<double> acc[4] = {mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0)};
+        const double* M = mpart + ((long long)e * wgs * nb + blk) * 512;
+        double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll 4
-        for (int p = SPLIT ? wave : 0; p < wgs; p += SPLIT ? 4 : 1) {
+        for (int p = SPLIT ? wave : 0; p < wgs; p += SPLIT ? 8 : 1) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const cpx<double> t = M[(long long)p * nb * 256 + 64 * i + lane];
-                acc[i].re += t.re;
-                acc[i].im += t.im;
-            }
+            for (int i = 0; i < 8; ++i) acc[i] += M[(long long)p * nb * 512 + 64 * i + lane];
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) sums[wave][64 * i + lane] = acc[i];
+        for (int i = 0; i < 8; ++i) sums[wave][64 * i + lane] = acc[i];
     }
     if constexpr (SPLIT) {
         __syncthreads();
@@ -268,12 +252,16 @@ __global__ __launch_bounds__(256) void k_fused_block_corr(const uint32_t* __rest
     for (int k = 0; k < 4; ++k) {
         const int at = quad_row(q, k) * 16 + col;
         x[k] = Fb[at];
-        cpx<double> a = sums[SPLIT ? 0 : wave][at];
+        const double* sw = sums[SPLIT ? 0 : wave];
+        double yr = sw[at], yi = sw[256 + at];
         if constexpr (SPLIT) {
-            const cpx<double> b = sums[1][at], c = sums[2][at], d = sums[3][at];
-            a = mk((a.re + b.re) + (c.re + d.re), (a.im + b.im) + (c.im + d.im));
+#pragma unroll
+            for (int w = 1; w < 8; ++w) {
+                yr += sums[w][at];
+                yi += sums[w][256 + at];
+            }
         }
-        y[k] = mk<R>((R)a.re, (R)a.im);
+        y[k] = mk<R>((R)yr, (R)yi);
     }
     for (int pe = p1; pe > p0; pe -= 64) {
         const int p = max(p0, pe - 64), cnt = pe - p;
@@ -345,17 +333,26 @@ __global__ __launch_bounds__(256) void k_fused_block_corr(const uint32_t* __rest
 }
 
 hipError_t launch_fuse_blocks(bool f32, const uint32_t* ops, const int* first, int nb, const GateKernels& g, int B,
-                              void* out, hipStream_t s, const int* count, const int* zslot) {
+                              void* out, hipStream_t s, const int* count) {
     if ((long long)B * nb == 0) return hipSuccess;
     const unsigned grid = (unsigned)(nb * (long long)((B + kQuadWaves - 1) / kQuadWaves));
     if (f32)
-        hipLaunchKernelGGL(k_fuse_blocks<float>, dim3(grid), dim3(64 * kQuadWaves), 0, s, ops, first, nb,
+        hipLaunchKernelGGL((k_fuse_blocks<float, false>), dim3(grid), dim3(64 * kQuadWaves), 0, s, ops, first, nb,
                            (const cpx<float>*)g.kern, g.kern_bstride, g.params, g.pstride, g.slots, B, (cpx<float>*)out,
-                           count, zslot);
+                           count, nullptr);
     else
-        hipLaunchKernelGGL(k_fuse_blocks<double>, dim3(grid), dim3(64 * kQuadWaves), 0, s, ops, first, nb,
+        hipLaunchKernelGGL((k_fuse_blocks<double, false>), dim3(grid), dim3(64 * kQuadWaves), 0, s, ops, first, nb,
                            (const cpx<double>*)g.kern, g.kern_bstride, g.params, g.pstride, g.slots, B,
-                           (cpx<double>*)out, count, zslot);
+                           (cpx<double>*)out, count, nullptr);
+    return hipGetLastError();
+}
+
+hipError_t launch_fuse_deriv_blocks(const uint32_t* ops, const int* first, int nb, const double* params,
+                                    const Slot* slots, const int* dinfo, int P, void* out, hipStream_t s) {
+    const int n = nb + P;
+    hipLaunchKernelGGL((k_fuse_blocks<double, true>), dim3((n + kQuadWaves - 1) / kQuadWaves), dim3(64 * kQuadWaves), 0,
+                       s, ops, first, nb, (const cpx<double>*)nullptr, 0LL, params, 0, slots, n, (cpx<double>*)out,
+                       (const int*)nullptr, dinfo);
     return hipGetLastError();
 }
 
@@ -368,7 +365,7 @@ hipError_t launch_fused_block_corr(bool f32, const uint32_t* ops, const int* fir
     const bool split = (long long)B * nb < 1024;
     const unsigned grid = (unsigned)(nb * (long long)(split ? B : (B + 3) / 4));
 #define SQH_CORR(R, SP)                                                                                       \
-    hipLaunchKernelGGL((k_fused_block_corr<R, SP>), dim3(grid), dim3(256), 0, s, ops, first, nb,               \
+    hipLaunchKernelGGL((k_fused_block_corr<R, SP>), dim3(grid), dim3(SP ? 512 : 256), 0, s, ops, first, nb,    \
                        (const cpx<R>*)g.kern, g.kern_bstride, g.params, g.pstride, g.slots, (const cpx<R>*)F,  \
                        mpart, wgs, B, corr, ns, count)
     if (f32 && split) SQH_CORR(float, true);

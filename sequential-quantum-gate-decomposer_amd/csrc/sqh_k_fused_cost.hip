@@ -40,182 +40,131 @@ namespace sqh {
 // Workgroups are ordered for the XCDs: hardware workgroup i runs on XCD i mod 8, and the
 // logical order gives each XCD a contiguous range of (element, column group) work, so
 // an element's block matrices and the target stay in one XCD's L2.
+//
+// The columns come in and go out through the LDS regions with a workgroup's threads along
+// the rows of the matrix (W columns per wavefront, 128 contiguous bytes a row for four
+// wavefronts at 8 qubits): in the operand layout each lane of a load takes another row, and
+// the addresses, a cache line per lane, took as long as the blocks.
 template <typename R, int N, int T, int H, bool PF>
-__global__ __launch_bounds__(256) void k_fused_cost(FusedCostArgs a) {
+__global__ __launch_bounds__(256, 2) void k_fused_cost(FusedCostArgs a, const int* __restrict__ tabs) {
     typedef FcMfma<R> MF;
-    constexpr int D = 1 << N;
-    constexpr int O = D >> 4;      // outer groups per column
-    constexpr int W = 16 * T / O;  // columns per wavefront
-    constexpr int TH = T / H;      // tiles per exchange group
+    typedef FcRegion<R, N, T> Reg;
+    constexpr int D = Reg::D, O = Reg::O, W = Reg::W;
+    constexpr int TH = T / H;  // tiles per exchange group
     static_assert(W >= 1 && (16 * TH) % O == 0, "an exchange group holds whole columns");
     extern __shared__ __align__(16) unsigned char fc_smem[];
-    int* smap = reinterpret_cast<int*>(fc_smem);
-    const int nmap = a.nb * kFusedMapStride;
-    cpx<R>* region = reinterpret_cast<cpx<R>*>(fc_smem + (((size_t)nmap * sizeof(int) + 15) & ~(size_t)15));
-    for (int i = threadIdx.x; i < nmap; i += blockDim.x) smap[i] = a.maps[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
+    R* const region = reinterpret_cast<R*>(fc_smem);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nw = blockDim.x >> 6;
     const long long per_xcd = gridDim.x >> 3;  // the grid is a multiple of 8
     const long long lwg = (long long)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    const long long wave = lwg * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (wave >= (long long)a.B * a.groups) return;
-    const int e = (int)(wave / a.groups);
-    const int c0 = (int)(wave % a.groups) * W;
-    cpx<R>* lds = region + (threadIdx.x >> 6) * (16 * T * 16);
-    const int nl = lane & 15, g = lane >> 4;
-    // vector column 16 t + nl of tile t: column c0 + w[t], outer group o[t]
-    int w[T], o[T];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int n = 16 * t + nl;
-        w[t] = n / O;
-        o[t] = n % O;
-    }
-    const cpx<R>* U =
-        static_cast<const cpx<R>*>(a.U) + (a.in_index ? (long long)a.in_index[e] : (long long)e) * a.in_bstride;
-    const int m = a.m, ist = a.in_stride;
-    // B operand of step s, tile t: X[4 s + g][16 t + nl] (block 0's grouping, from U)
-    R xr[T][4], xi[T][4];
+    const long long total = (long long)a.B * a.groups;
+    const int m = a.m;
+    // the thread's column in the passes over rows: column cq of element eq, in wavefront
+    // q / W's region; it takes rows tid / (W nw) + k 64 / W
+    const int q = threadIdx.x & (W * nw - 1), v = q / W, wq = q % W;
+    const long long first = lwg * nw;  // the workgroup's first (element, column group)
+    const int e0 = (int)(first / a.groups), g0 = (int)(first % a.groups);
+    const int eq = e0 + (g0 + v) / a.groups, cq = (g0 + v) % a.groups * W + wq;
+    const bool okq = first + v < total && cq < m;
+    const Reg ldsq{region + v * 512 * T};
+    const int row_q = threadIdx.x / (W * nw);
     {
-        const int* mp = smap;
+        const long long src = a.in_index ? (long long)a.in_index[okq ? eq : 0]
+                              : a.dinfo ? (long long)a.dinfo[4 * (okq ? eq : 0)] : (long long)eq;
+        const cpx<R>* p = static_cast<const cpx<R>*>(a.U) + src * a.in_bstride + (long long)row_q * a.in_stride + cq;
+        const long long step = (long long)(64 / W) * a.in_stride;
+        cpx<R> u[4 * T];
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const int col = c0 + w[t];
-            const int base = mp[16 + o[t]];
+        for (int k = 0; k < 4 * T; ++k) u[k] = okq ? p[k * step] : mk<R>(0, 0);
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int j = base + mp[4 * s + g];
-                const cpx<R> v = col < m ? U[(long long)j * ist + col] : mk<R>(0, 0);
-                xr[t][s] = v.re;
-                xi[t][s] = v.im;
-            }
-        }
+        for (int k = 0; k < 4 * T; ++k) ldsq.put(fc_slot<N>(row_q + k * (64 / W)) + wq * D, u[k].re, u[k].im);
     }
-    const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.F_bstride;
-    // A operand of step s: F_b[nl][4 s + g] (with PF, block b + 1's is loaded while
-    // block b runs)
-    R far[4], fai[4];
-    if constexpr (PF) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const cpx<R> f = Fe[nl * 16 + 4 * s + g];
-            far[s] = f.re;
-            fai[s] = f.im;
+    __syncthreads();
+    const long long wave = first + wv;
+    const int e = e0 + (g0 + wv) / a.groups;
+    const int c0 = (g0 + wv) % a.groups * W;
+    const Reg lds{region + wv * 512 * T};
+    const int nl = lane & 15, g = lane >> 4;
+    if (wave < total) {
+        const cpx<R>* F = static_cast<const cpx<R>*>(a.F);
+        const cpx<R>* Fe = F + (long long)e * a.F_bstride;
+        // Blocks lo .. hi - 1: all of them; up to the element's own number (the prefixes of
+        // the derivatives); or from the differentiated one, which is the element's own, on.
+        // The cost pass stops before the last block: of it only row c + trace_off of each
+        // column c is needed (below).
+        int lo = 0, hi = a.out ? a.nb : a.nb - 1;
+        const cpx<R>* F0 = Fe;
+        if (a.prefix) hi = e;
+        if (a.dinfo) {
+            lo = __builtin_amdgcn_readfirstlane(a.dinfo[4 * e]);
+            F0 = F + (long long)(a.nb + e) * 256;
         }
-    }
-    // the cost pass stops before the last block: of it only row c + trace_off of each
-    // column c is needed (below)
-    const int nbl = a.out ? a.nb : a.nb - 1;
-    for (int b = 0; b < nbl; ++b) {
-        R ar[4], ai[4], ain[4];
-        if constexpr (PF) {
+        // A operand of the running block (with PF, the next block's is loaded meanwhile)
+        FcA<R> A, An;
+        const int* tab = tabs + lo * kLaneTab;
+        int entry = tab[LT_LANE + lane];
+        if (lo < hi) A.load_n(a.dinfo ? F0 : Fe + (long long)lo * 256, nl, g);
+        for (int b = lo; b < hi; ++b) {
+            int at[4];
+            Reg::full_at(at, tab, entry);
+            if (PF && b + 1 < hi) An.load_n(Fe + (long long)(b + 1) * 256, nl, g);
+            if (b + 1 < a.nb) entry = tab[kLaneTab + LT_LANE + lane];
+            // each exchange group reads and stores its own columns only
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                ar[s] = far[s];
-                ai[s] = fai[s];
-                ain[s] = -fai[s];
-            }
-            if (b + 1 < nbl) {
+            for (int h = 0; h < H; ++h) {
+                R vr[TH][4], vi[TH][4];
+                typename MF::V yr[TH], yi[TH];
 #pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const cpx<R> f = Fe[(long long)(b + 1) * 256 + nl * 16 + 4 * s + g];
-                    far[s] = f.re;
-                    fai[s] = f.im;
-                }
-            }
-        } else {
+                for (int u = 0; u < TH; ++u)
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const cpx<R> f = Fe[(long long)b * 256 + nl * 16 + 4 * s + g];
-                ar[s] = f.re;
-                ai[s] = f.im;
-                ain[s] = -f.im;
-            }
-        }
-        const int* mp = smap + b * kFusedMapStride;
-        const int* mn = mp + kFusedMapStride;
-#pragma unroll
-        for (int h = 0; h < H; ++h) {
-            typename MF::V yr[TH], yi[TH];
-#pragma unroll
-            for (int u = 0; u < TH; ++u) {
-                yr[u] = typename MF::V{0, 0, 0, 0};
-                yi[u] = typename MF::V{0, 0, 0, 0};
-            }
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-#pragma unroll
-                for (int u = 0; u < TH; ++u) {
-                    const int t = h * TH + u;
-                    yr[u] = MF::op(ar[s], xr[t][s], yr[u]);
-                    yi[u] = MF::op(ar[s], xi[t][s], yi[u]);
-                }
-#pragma unroll
-                for (int u = 0; u < TH; ++u) {
-                    const int t = h * TH + u;
-                    yr[u] = MF::op(ain[s], xi[t][s], yr[u]);
-                    yi[u] = MF::op(ai[s], xr[t][s], yi[u]);
-                }
-            }
-            if (b + 1 < a.nb) {
-                // through LDS in natural row order, back in block b + 1's grouping
-#pragma unroll
-                for (int u = 0; u < TH; ++u) {
-                    const int t = h * TH + u;
-                    const int base = mp[16 + o[t]];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int j = base + mp[MF::row(r, g)];
-                        lds[w[t] * D + fc_slot<N>(j)] = mk<R>(yr[u][r], yi[u][r]);
-                    }
-                }
+                    for (int s = 0; s < 4; ++s) lds.get(Reg::full(at, tab, h * TH + u, s), vr[u][s], vi[u][s]);
                 fc_wave_fence();
-#pragma unroll
-                for (int u = 0; u < TH; ++u) {
-                    const int t = h * TH + u;
-                    const int base = mn[16 + o[t]];
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const cpx<R> v = lds[w[t] * D + fc_slot<N>(base + mn[4 * s + g])];
-                        xr[t][s] = v.re;
-                        xi[t][s] = v.im;
-                    }
-                }
-                fc_wave_fence();
-            } else {
-                // apply_to: the transformed columns back to HBM (each wavefront writes
-                // only the columns it read, so the pass may run in place)
-                cpx<R>* O = static_cast<cpx<R>*>(a.out) + (long long)e * a.out_bstride;
-#pragma unroll
-                for (int u = 0; u < TH; ++u) {
-                    const int t = h * TH + u;
-                    const int col = c0 + w[t];
-                    const int base = mp[16 + o[t]];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int j = base + mp[MF::row(r, g)];
-                        if (col < m) O[(long long)j * a.out_stride + col] = mk<R>(yr[u][r], yi[u][r]);
-                    }
-                }
+                fc_mma<R, TH, TH>(A, vr, vi, yr, yi);
+                if (h == 0) lds.template store_full<TH, 0>(at, tab, yr, yi);
+                else lds.template store_full<TH, (H > 1 ? TH : 0)>(at, tab, yr, yi);
             }
+            tab += kLaneTab;
+            if constexpr (PF) A = An;
+            else if (b + 1 < hi) A.load_n(Fe + (long long)(b + 1) * 256, nl, g);
         }
     }
-    if (a.out) return;
+    if (a.out) {
+        // apply_to: the columns back to HBM (a workgroup writes only the columns it read,
+        // after it has read them all, so the pass may run in place)
+        __syncthreads();
+        if (okq) {
+            cpx<R>* p = static_cast<cpx<R>*>(a.out) + (long long)eq * a.out_bstride + (long long)row_q * a.out_stride + cq;
+            const long long step = (long long)(64 / W) * a.out_stride;
+#pragma unroll
+            for (int k = 0; k < 4 * T; ++k) {
+                cpx<R> y;
+                ldsq.get(fc_slot<N>(row_q + k * (64 / W)) + wq * D, y.re, y.im);
+                p[k * step] = y;
+            }
+        }
+        return;
+    }
+    if (wave >= total) return;
     // cost pass, last block: one 16-term dot product with row c + trace_off of F per
     // column c.  X is in the block's grouping; the vector column whose outer group holds
     // the row contributes, its 4 lane groups summing their 4 entries each.
     {
-        const int* mp = smap + (a.nb - 1) * kFusedMapStride;
+        const int* tab = tabs + (a.nb - 1) * kLaneTab;
+        R xr[T][4], xi[T][4];
+        int at[4];
+        Reg::full_at(at, tab, tab[LT_LANE + lane]);
+        lds.load_full(at, tab, xr, xi);
+        const int* mp = a.maps + (a.nb - 1) * kFusedMapStride;
         const int mask = mp[15];  // the block's four row bits (off of local index 15)
-        const cpx<R>* Fl = Fe + (long long)(a.nb - 1) * 256;
+        const cpx<R>* Fl = static_cast<const cpx<R>*>(a.F) + (long long)e * a.F_bstride + (long long)(a.nb - 1) * 256;
 #pragma unroll
         for (int t = 0; t < T; ++t) {
-            const int col = c0 + w[t];
+            const int col = c0 + (16 * t + nl) / O;
             const int jt = col + a.trace_off;
-            const bool hit = col < m && (jt & ~mask) == mp[16 + o[t]];
+            const bool hit = col < m && (jt & ~mask) == ((tab[LT_ROW + lane] & ~mask) | tab[LT_RT + t]);
             // local index of row jt: its bits at the block's qubits
-            const int is = ((jt & mp[1]) ? 1 : 0) | ((jt & mp[2]) ? 2 : 0) | ((jt & mp[4]) ? 4 : 0) |
-                           ((jt & mp[8]) ? 8 : 0);
+            const int is = ft_local(mp, jt);
             R sr = 0, si = 0;
             if (hit) {
 #pragma unroll
@@ -263,249 +212,99 @@ __global__ __launch_bounds__(256) void k_fused_cost(FusedCostArgs a) {
 // same order: results are bit-identical across shapes.
 
 template <typename R, int N, int T, bool PF>
-__global__ __launch_bounds__(256) void k_fused_trace(FusedCostArgs a) {
+__global__ __launch_bounds__(256, 2) void k_fused_trace(FusedCostArgs a, const int* __restrict__ tabs,
+                                                        const int* __restrict__ tmaps) {
     typedef FcMfma<R> MF;
-    constexpr int D = 1 << N;
-    constexpr int O = D >> 4;      // outer groups per column
-    constexpr int W = 16 * T / O;  // columns per wavefront
+    typedef FcRegion<R, N, T> Reg;
+    constexpr int D = Reg::D, O = Reg::O, W = Reg::W;
     static_assert(W >= 1, "a wavefront holds whole columns");
     extern __shared__ __align__(16) unsigned char fc_smem[];
-    int* smap = reinterpret_cast<int*>(fc_smem);
-    const int nmap = a.nb * kTraceMapStride;
-    cpx<R>* region = reinterpret_cast<cpx<R>*>(fc_smem + (((size_t)nmap * sizeof(int) + 15) & ~(size_t)15));
-    for (int i = threadIdx.x; i < nmap; i += blockDim.x) smap[i] = a.maps[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long per_xcd = gridDim.x >> 3;  // the grid is a multiple of 8
     const long long lwg = (long long)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    const long long wave = lwg * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const long long wave = lwg * (blockDim.x >> 6) + wv;
     if (wave >= (long long)a.B * a.groups) return;
     const int e = (int)(wave / a.groups);
     const int c0 = (int)(wave % a.groups) * W;
-    cpx<R>* lds = region + (threadIdx.x >> 6) * (16 * T * 16);
+    const Reg lds{reinterpret_cast<R*>(fc_smem) + wv * 512 * T};
     const int nl = lane & 15, g = lane >> 4;
     const int m = a.m;
-    // the row of V column c0 + w needs (columns past m take row trace_off and write
-    // nothing; trace_off + m <= 2^N)
-    auto rho_of = [&](int w) { return (c0 + w < m ? c0 + w : 0) + a.trace_off; };
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.F_bstride;
-    // X of block bn (B operand of step s, tile t: X[4 s + g][16 t + nl] in its grouping)
-    // from the LDS region, for the tiles holding its support's groups; vector columns
-    // past the wavefront's columns read column 0 (their products are never stored)
     R xr[T][4], xi[T][4];
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) xr[t][s] = xi[t][s] = 0;
-    auto load_x = [&](int bn) {
-        const int* mn = smap + bn * kTraceMapStride;
-        const int lgn = mn[80], nSn = mn[81];
-        const int tsn = ((W << lgn) + 15) >> 4;
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            if (t < tsn) {
-                const int n = 16 * t + nl;
-                const int w = n >> lgn < W ? n >> lgn : 0;
-                const int base = mn[16 + (n & ((1 << lgn) - 1))] | (rho_of(w) & nSn);
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const cpx<R> v = lds[w * D + fc_slot<N>(base + mn[4 * s + g])];
-                    xr[t][s] = v.re;
-                    xi[t][s] = v.im;
-                }
-            }
-        }
-        fc_wave_fence();
-    };
-    // The region starts at zero (rows outside a block's support are never stored and
-    // read as zero; the supports only grow), then holds F_{nb-1}^T e_rho per column:
-    // row loc(rho) of F_{nb-1} on the rows that agree with rho outside its qubits.
-    for (int i = lane; i < W * D; i += 64) lds[i] = mk<R>(0, 0);
-    fc_wave_fence();
-    {
-        const int* mq = smap + (a.nb - 1) * kTraceMapStride;
-        const cpx<R>* Fq = Fe + (long long)(a.nb - 1) * 256;
-        for (int p = lane; p < 16 * W; p += 64) {
-            const int w = p >> 4, i = p & 15;
-            const int rho = rho_of(w);
-            lds[w * D + fc_slot<N>((rho & mq[81]) | mq[i])] = Fq[ft_local(mq, rho) * 16 + i];
-        }
-    }
-    fc_wave_fence();
-    load_x(a.nb - 2);
-    // A operand of step s: F_b^T[nl][4 s + g] = F_b[4 s + g][nl] (with PF, block b - 1's
-    // is loaded while block b runs)
-    R far[4], fai[4];
-    if constexpr (PF) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const cpx<R> f = Fe[(long long)(a.nb - 2) * 256 + (4 * s + g) * 16 + nl];
-            far[s] = f.re;
-            fai[s] = f.im;
-        }
-    }
-    // A operand of block b into ar / ai / ain (with PF from far / fai, block b - 1's then
-    // loaded into them)
-    auto a_operand = [&](int b, R (&ar)[4], R (&ai)[4], R (&ain)[4]) {
-        if constexpr (PF) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                ar[s] = far[s];
-                ai[s] = fai[s];
-                ain[s] = -fai[s];
-            }
-            if (b > 0) {
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const cpx<R> f = Fe[(long long)(b - 1) * 256 + (4 * s + g) * 16 + nl];
-                    far[s] = f.re;
-                    fai[s] = f.im;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const cpx<R> f = Fe[(long long)b * 256 + (4 * s + g) * 16 + nl];
-                ar[s] = f.re;
-                ai[s] = f.im;
-                ain[s] = -f.im;
-            }
-        }
-    };
-    // block b's output Y (its support's tiles) through LDS in natural row order, back in
-    // block b - 1's grouping
-    auto exchange = [&](int b, int lg, int nS, int ts, const typename MF::V (&yr)[T], const typename MF::V (&yi)[T]) {
-        const int* mp = smap + b * kTraceMapStride;
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const int n = 16 * t + nl;
-            const int w = n >> lg;
-            if (t < ts && w < W) {
-                const int base = mp[16 + (n & ((1 << lg) - 1))] | (rho_of(w) & nS);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int j = base + mp[MF::row(r, g)];
-                    lds[w * D + fc_slot<N>(j)] = mk<R>(yr[t][r], yi[t][r]);
-                }
-            }
-        }
-        fc_wave_fence();
-        load_x(b - 1);
-    };
-    // The supports only grow along the chain: first the blocks whose support fills
-    // fewer than T tiles (1, or 2 of 4), then the dense ones.  (Separate loops keep the
-    // tile-count variants' registers apart.)
-    int b = a.nb - 2;
-    for (; b > 0; --b) {
-        const int* mp = smap + b * kTraceMapStride;
-        const int lg = mp[80], nS = mp[81];
-        const int ts = ((W << lg) + 15) >> 4;
-        if (ts >= T) break;
-        R ar[4], ai[4], ain[4];
-        a_operand(b, ar, ai, ain);
-        typename MF::V yr[T], yi[T];
-        if (T >= 4 && ts >= 2) ft_mma<R, T, (T >= 4 ? 2 : 1)>(ar, ai, ain, xr, xi, yr, yi);
-        else ft_mma<R, T, 1>(ar, ai, ain, xr, xi, yr, yi);
-        exchange(b, lg, nS, ts, yr, yi);
-    }
-    // Blocks of full support (no row outside it): vector column 16 t + nl is column
-    // wd[t], outer group od[t], as in the forward pass -- no predicates, no row of V.
-    int wd[T], od[T];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        wd[t] = (16 * t + nl) / O;
-        od[t] = (16 * t + nl) % O;
-    }
-    for (; b > 0; --b) {
-        const int* mp = smap + b * kTraceMapStride;
-        const int* mn = mp - kTraceMapStride;
-        R ar[4], ai[4], ain[4];
-        a_operand(b, ar, ai, ain);
-        typename MF::V yr[T], yi[T];
-        ft_mma<R, T, T>(ar, ai, ain, xr, xi, yr, yi);
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const int base = mp[16 + od[t]];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                lds[wd[t] * D + fc_slot<N>(base + mp[MF::row(r, g)])] = mk<R>(yr[t][r], yi[t][r]);
-        }
-        fc_wave_fence();
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const int base = mn[16 + od[t]];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const cpx<R> v = lds[wd[t] * D + fc_slot<N>(base + mn[4 * s + g])];
-                xr[t][s] = v.re;
-                xi[t][s] = v.im;
-            }
-        }
-        fc_wave_fence();
-    }
+    FcA<R> A;
+    fused_chain_to_block0<R, N, T, PF>(tabs, tmaps, a.nb, lds, Fe, c0, m, a.trace_off, lane, xr, xi, A);
     // block 0, then row rho of V times column c of U: per lane its rows of the column,
-    // then the lanes of the column (the four lane groups and, below 16 support groups,
-    // the column's lanes of the tile); a column spanning several tiles accumulates them
-    // first
-    const int* mp = smap;
-    const int lg0 = mp[80], nS = mp[81];
+    // then the lanes of the column
     typename MF::V yr[T], yi[T];
-    {
-        // all T tiles (those past the support's hold zeros when it stays short)
-        R ar[4], ai[4], ain[4];
-        a_operand(0, ar, ai, ain);
-        ft_mma<R, T, T>(ar, ai, ain, xr, xi, yr, yi);
-    }
+    fc_mma<R, T, T>(A, xr, xi, yr, yi);  // (a support short of the register leaves zeros in the last tiles)
     const cpx<R>* U =
         static_cast<const cpx<R>*>(a.U) + (a.in_index ? (long long)a.in_index[e] : (long long)e) * a.in_bstride;
-    const int ist = a.in_stride;
-    auto dot = [&](auto full_support) {
-        constexpr bool FULL = decltype(full_support)::value;
-        const int lg = FULL ? N - 4 : lg0;
-        const int ng = 1 << lg, seg = ng < 16 ? ng : 16;
-        const int ts = ((W << lg) + 15) >> 4;
-        double sr = 0, si = 0;
+    const unsigned ist = (unsigned)a.in_stride;
+    const int lg0 = tabs[LT_LG];
+    double* dg = a.diag + 2 * ((long long)e * m + c0);
+    if (lg0 == N - 4) {
+        // vector column 16 t + nl is column (16 t + nl) / O; its rows' offsets in U fit 32
+        // bits (at most 1024 x 1024 entries)
+        constexpr int C = O > 16 ? W : T;  // sums: per column, or per tile of whole columns
+        double sr[C], si[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) sr[c] = si[c] = 0;
+        const unsigned row0 = (unsigned)tabs[LT_ROW + lane] * ist;
 #pragma unroll
         for (int t = 0; t < T; ++t) {
-            if (t < ts) {
-                const int n = 16 * t + nl;
-                const int w = FULL ? wd[t] : n >> lg;
-                const int col = c0 + w;
-                if (w < W && col < m) {
-                    const int base = FULL ? mp[16 + od[t]] : mp[16 + (n & (ng - 1))] | (rho_of(w) & nS);
+            const int c = O > 16 ? t / (O / 16 ? O / 16 : 1) : t;
+            const int col = c0 + (O > 16 ? c : (16 * t + nl) / O);
+            const unsigned at = row0 + (unsigned)tabs[LT_RT + t] * ist + (unsigned)(col < m ? col : 0);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int j = base + mp[MF::row(r, g)];
-                        const cpx<R> u = U[(long long)j * ist + col];
-                        sr += (double)yr[t][r] * (double)u.re - (double)yi[t][r] * (double)u.im;
-                        si += (double)yr[t][r] * (double)u.im + (double)yi[t][r] * (double)u.re;
-                    }
-                }
-                if (lg < 4 || (((t + 1) << 4) & (ng - 1)) == 0) {
-                    sr += __shfl_xor(sr, 16, 64);
-                    si += __shfl_xor(si, 16, 64);
-                    sr += __shfl_xor(sr, 32, 64);
-                    si += __shfl_xor(si, 32, 64);
-#pragma unroll
-                    for (int d = 1; d < 16; d <<= 1) {
-                        if (d < seg) {
-                            sr += __shfl_xor(sr, d, 64);
-                            si += __shfl_xor(si, d, 64);
-                        }
-                    }
-                    if (g == 0 && (nl & (seg - 1)) == 0 && w < W && col < m) {
-                        double* dg = a.diag + 2 * ((long long)e * m + col);
-                        dg[0] = sr;
-                        dg[1] = si;
-                    }
-                    sr = 0;
-                    si = 0;
-                }
+            for (int r = 0; r < 4; ++r) {
+                const cpx<R> u = U[at + (unsigned)tabs[LT_RS + r] * ist];
+                sr[c] += (double)yr[t][r] * (double)u.re - (double)yi[t][r] * (double)u.im;
+                si[c] += (double)yr[t][r] * (double)u.im + (double)yi[t][r] * (double)u.re;
             }
         }
-    };
-    if (lg0 == N - 4) dot(std::true_type{});
-    else dot(std::false_type{});
+        fc_column_sums<N, T>(sr, si, dg, c0, m, lane);
+        return;
+    }
+    // blocks that leave qubits out: the support layout of block 0, rows outside the support
+    // those of rho
+    const int* mp = tmaps;
+    const int nS = mp[81], ng = 1 << lg0, seg = ng < 16 ? ng : 16;
+    const int ts = ((W << lg0) + 15) >> 4;
+    double sr = 0, si = 0;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        if (t < ts) {
+            const int n = 16 * t + nl, w = n >> lg0, col = c0 + w;
+            if (w < W && col < m) {
+                const int base = mp[16 + (n & (ng - 1))] | ((col + a.trace_off) & nS);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const cpx<R> u = U[(unsigned)(base + mp[4 * r + g]) * ist + (unsigned)col];
+                    sr += (double)yr[t][r] * (double)u.re - (double)yi[t][r] * (double)u.im;
+                    si += (double)yr[t][r] * (double)u.im + (double)yi[t][r] * (double)u.re;
+                }
+            }
+            if (lg0 < 4 || (((t + 1) << 4) & (ng - 1)) == 0) {
+                sr += __shfl_xor(sr, 16, 64);
+                si += __shfl_xor(si, 16, 64);
+                sr += __shfl_xor(sr, 32, 64);
+                si += __shfl_xor(si, 32, 64);
+#pragma unroll
+                for (int d = 1; d < 16; d <<= 1) {
+                    if (d < seg) {
+                        sr += __shfl_xor(sr, d, 64);
+                        si += __shfl_xor(si, d, 64);
+                    }
+                }
+                if (g == 0 && (nl & (seg - 1)) == 0 && w < W && col < m) {
+                    dg[2 * w] = sr;
+                    dg[2 * w + 1] = si;
+                }
+                sr = 0;
+                si = 0;
+            }
+        }
+    }
 }
 
 bool fused_trace_cfg_valid(int N, bool f32, int nb, FusedCostCfg cfg) {
@@ -517,8 +316,8 @@ bool fused_trace_cfg_valid(int N, bool f32, int nb, FusedCostCfg cfg) {
 }
 
 size_t fused_trace_lds_bytes(bool f32, int nb, FusedCostCfg cfg) {
-    return (((size_t)nb * kTraceMapStride * sizeof(int) + 15) & ~(size_t)15) +
-           (size_t)cfg.waves * cfg.tiles * 256 * (f32 ? 8 : 16);
+    (void)nb;
+    return (size_t)cfg.waves * cfg.tiles * 256 * (f32 ? 8 : 16);
 }
 
 template <typename R, int N>
@@ -526,15 +325,15 @@ static void launch_ft_n(const FusedCostArgs& a, FusedCostCfg cfg, int grid, size
     const int threads = 64 * cfg.waves;
     if constexpr (16 * 4 >= ((1 << N) >> 4)) {
         if (cfg.tiles == 4 && cfg.prefetch)
-            hipLaunchKernelGGL((k_fused_trace<R, N, 4, true>), dim3(grid), dim3(threads), shm, s, a);
+            hipLaunchKernelGGL((k_fused_trace<R, N, 4, true>), dim3(grid), dim3(threads), shm, s, a, a.tabs, a.maps);
         else if (cfg.tiles == 4)
-            hipLaunchKernelGGL((k_fused_trace<R, N, 4, false>), dim3(grid), dim3(threads), shm, s, a);
+            hipLaunchKernelGGL((k_fused_trace<R, N, 4, false>), dim3(grid), dim3(threads), shm, s, a, a.tabs, a.maps);
     }
     if constexpr (16 * 2 >= ((1 << N) >> 4)) {
         if (cfg.tiles == 2 && cfg.prefetch)
-            hipLaunchKernelGGL((k_fused_trace<R, N, 2, true>), dim3(grid), dim3(threads), shm, s, a);
+            hipLaunchKernelGGL((k_fused_trace<R, N, 2, true>), dim3(grid), dim3(threads), shm, s, a, a.tabs, a.maps);
         else if (cfg.tiles == 2)
-            hipLaunchKernelGGL((k_fused_trace<R, N, 2, false>), dim3(grid), dim3(threads), shm, s, a);
+            hipLaunchKernelGGL((k_fused_trace<R, N, 2, false>), dim3(grid), dim3(threads), shm, s, a, a.tabs, a.maps);
     }
 }
 
@@ -578,14 +377,14 @@ bool fused_cost_cfg_valid(int N, bool f32, int nb, FusedCostCfg cfg) {
 }
 
 size_t fused_cost_lds_bytes(bool f32, int nb, FusedCostCfg cfg) {
-    return (((size_t)nb * kFusedMapStride * sizeof(int) + 15) & ~(size_t)15) +
-           (size_t)cfg.waves * cfg.tiles * 256 * (f32 ? 8 : 16);
+    (void)nb;
+    return (size_t)cfg.waves * cfg.tiles * 256 * (f32 ? 8 : 16);
 }
 
 template <typename R, int N, int T, int H, bool PF>
 static void launch_fc_shape(const FusedCostArgs& a, int grid, int threads, size_t shm, hipStream_t s) {
     if constexpr (16 * T >= ((1 << N) >> 4) && (16 * T / H) % ((1 << N) >> 4) == 0)
-        hipLaunchKernelGGL((k_fused_cost<R, N, T, H, PF>), dim3(grid), dim3(threads), shm, s, a);
+        hipLaunchKernelGGL((k_fused_cost<R, N, T, H, PF>), dim3(grid), dim3(threads), shm, s, a, a.tabs);
 }
 
 template <typename R, int N>

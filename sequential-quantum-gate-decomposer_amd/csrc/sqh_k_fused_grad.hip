@@ -21,266 +21,231 @@
 // B operand of step s holds rows 4 s + lane / 16, the D layout rows row(r, lane / 16).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "sqh_device.h"
 #include "sqh_fused_chain.h"
 #include "sqh_kernels.h"
 
 namespace sqh {
 
-typedef double fg_f64x4 __attribute__((ext_vector_type(4)));
-typedef float fg_f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename R>
-struct FgMfma;
-template <>
-struct FgMfma<double> {
-    typedef fg_f64x4 V;
-    static __device__ __forceinline__ V op(double a, double b, V c) {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int r, int g) { return 4 * r + g; }
-};
-template <>
-struct FgMfma<float> {
-    typedef fg_f32x4 V;
-    static __device__ __forceinline__ V op(float a, float b, V c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int r, int g) { return 4 * g + r; }
-};
-
-template <int N>
-__device__ __forceinline__ int fg_slot(int j) {
-    if constexpr (N <= 4) {
-        return j;
-    } else {
-        int h = j >> 4;
-        if constexpr (N > 8) h ^= h >> 4;
-        return j ^ (h & 15);
-    }
-}
-
-__device__ __forceinline__ void fg_wave_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+namespace {
 
 // Entry (r, c) of a 16 x 16 tile in LDS, columns rotated by the row (XOR) so that both a
 // row-wise and a column-wise sweep of 16 lanes touch 16 different bank groups.
 __device__ __forceinline__ int fg_tile(int r, int c) { return r * 16 + (c ^ r); }
 
-// Complex 16x16 tile product Y = A X for T tiles: A given by (ar, ai, ain = -ai) per
-// step, X the B operand (xr, xi) per tile and step; result in the D layout.
-template <typename R, int T>
-__device__ __forceinline__ void fg_product(const R (&ar)[4], const R (&ai)[4], const R (&ain)[4], const R (&xr)[T][4],
-                                           const R (&xi)[T][4], typename FgMfma<R>::V (&yr)[T],
-                                           typename FgMfma<R>::V (&yi)[T]) {
-    typedef FgMfma<R> MF;
+// Y = A X (CONJ: with A's conjugate) on all tiles.
+template <typename R, int T, bool CONJ>
+__device__ __forceinline__ void fg_mma(const FcA<R>& A, const R (&xr)[T][4], const R (&xi)[T][4],
+                                       typename FcMfma<R>::V (&yr)[T], typename FcMfma<R>::V (&yi)[T]) {
+    typedef FcMfma<R> MF;
+    if constexpr (!CONJ) {
+        fc_mma<R, T, T>(A, xr, xi, yr, yi);
+    } else {
 #pragma unroll
-    for (int t = 0; t < T; ++t) {
-        yr[t] = typename MF::V{0, 0, 0, 0};
-        yi[t] = typename MF::V{0, 0, 0, 0};
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            yr[t] = MF::op(ar[s], xr[t][s], yr[t]);
-            yi[t] = MF::op(ar[s], xi[t][s], yi[t]);
-        }
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            yr[t] = MF::op(ain[s], xi[t][s], yr[t]);
-            yi[t] = MF::op(ai[s], xr[t][s], yi[t]);
-        }
-    }
-}
-
-// D-layout tiles (block b's grouping, tables mp) through the wavefront's LDS region into
-// B-layout operands of the grouping of tables mn.
-template <typename R, int N, int T>
-__device__ __forceinline__ void fg_remap(const typename FgMfma<R>::V (&dr)[T], const typename FgMfma<R>::V (&di)[T],
-                                         R (&xr)[T][4], R (&xi)[T][4], const int* mp, const int* mn, const int (&w)[T],
-                                         const int (&o)[T], int g, cpx<R>* lds) {
-    typedef FgMfma<R> MF;
-    constexpr int D = 1 << N;
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int base = mp[16 + o[t]];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) lds[w[t] * D + fg_slot<N>(base + mp[MF::row(r, g)])] = mk<R>(dr[t][r], di[t][r]);
-    }
-    fg_wave_fence();
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int base = mn[16 + o[t]];
+        for (int t = 0; t < T; ++t) yr[t] = yi[t] = typename MF::V{0, 0, 0, 0};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const cpx<R> v = lds[w[t] * D + fg_slot<N>(base + mn[4 * s + g])];
-            xr[t][s] = v.re;
-            xi[t][s] = v.im;
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                yr[t] = MF::op(A.re[s], xr[t][s], yr[t]);
+                yi[t] = MF::op(A.re[s], xi[t][s], yi[t]);
+            }
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                yr[t] = MF::op(A.im[s], xi[t][s], yr[t]);
+                yi[t] = MF::op_neg(A.im[s], xr[t][s], yi[t]);
+            }
         }
     }
-    fg_wave_fence();
 }
 
-template <typename R, int N, int T>
-__global__ __launch_bounds__(512) void k_fused_grad(FusedGradArgs a) {
-    typedef FgMfma<R> MF;
-    constexpr int D = 1 << N;
-    constexpr int O = D >> 4;
-    constexpr int W = 16 * T / O;
-    static_assert(W >= 1, "a wavefront holds whole columns");
-    // Per wavefront one LDS region of RG complex entries, used in turn by the remaps, the
-    // two transposed tiles of the correlation product (2 x 256 entries) and the
-    // workgroup's reduction of M_b (512 doubles).
-    constexpr int RG = 16 * T * 16;
-    static_assert(RG >= 512 && RG * sizeof(cpx<R>) >= 512 * sizeof(double), "the region holds the tiles");
-    extern __shared__ __align__(16) unsigned char fg_smem[];
-    const int nwv = blockDim.x >> 6;
-    int* smap = reinterpret_cast<int*>(fg_smem);
-    const int nmap = a.nb * kFusedMapStride;
-    cpx<R>* region = reinterpret_cast<cpx<R>*>(fg_smem + (((size_t)nmap * sizeof(int) + 15) & ~(size_t)15));
-    for (int i = threadIdx.x; i < nmap; i += blockDim.x) smap[i] = a.maps[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+// What a wavefront of the gradient kernels works on: element e and the column groups
+// first .. last - 1 of it, whose correlations it sums in partial slot `slot`.
+struct FgTask {
+    int e, slot, first, last;
+    bool live;
+};
+__device__ __forceinline__ FgTask fg_task(const FusedGradArgs& a, int wv) {
     // XCD-ordered workgroups (the grid is a multiple of 8); with a live count (the
     // optimiser's rounds) the plain order, so the live elements spread over the XCDs
     int B = a.B;
     long long lwg = blockIdx.x;
-    if (a.count) {
-        B = min(*a.count, a.B);
-    } else {
-        const long long per_xcd = gridDim.x >> 3;
-        lwg = (long long)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    }
-    const long long wave = lwg * nwv + wv;
-    // whole workgroups past the batch leave together (the workgroups of one element
-    // hold whole column groups: groups % waves == 0)
-    if (lwg * nwv >= (long long)B * a.groups) return;
-    const int e = (int)(wave / a.groups);
-    const int cg = (int)(wave % a.groups);
-    const int c0 = cg * W;
-    const int wgi = cg / nwv;  // the workgroup's index within its element
-    cpx<R>* lds = region + (size_t)wv * RG;
-    cpx<R>* ys = lds;
-    cpx<R>* xs = lds + 256;
-    const int nl = lane & 15, g = lane >> 4;
-    int w[T], o[T];
+    if (a.count) B = min(*a.count, a.B);
+    else lwg = (long long)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const long long task = lwg * (blockDim.x >> 6) + wv;
+    FgTask t;
+    t.e = (int)(task / a.wgs);
+    t.slot = (int)(task % a.wgs);
+    t.first = t.slot * a.per;
+    t.last = min(t.first + a.per, a.groups);
+    t.live = t.e < B;
+    return t;
+}
+
+// X = the target's columns c0 + w in a block's full layout (tab), zero past column m.
+template <typename R, int N, int T>
+__device__ __forceinline__ void fg_load_target(const cpx<R>* __restrict__ U, const int* tab, int c0, int m, int lane,
+                                               R (&xr)[T][4], R (&xi)[T][4]) {
+    constexpr int O = (1 << N) >> 4;
+    const unsigned row0 = (unsigned)tab[LT_ROW + lane] * (unsigned)m;
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        const int n = 16 * t + nl;
-        w[t] = n / O;
-        o[t] = n % O;
+        const int col = c0 + (O > 16 ? t / (O / 16 ? O / 16 : 1) : (16 * t + (lane & 15)) / O);
+        const unsigned at = row0 + (unsigned)tab[LT_RT + t] * (unsigned)m + (unsigned)(col < m ? col : 0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const cpx<R> v = U[at + (unsigned)tab[LT_RS + s] * (unsigned)m];
+            xr[t][s] = col < m ? v.re : (R)0;
+            xi[t][s] = col < m ? v.im : (R)0;
+        }
     }
+}
+
+// M += Y X^T over the wavefront's vector columns (Y and X: item i of tile t is row 4 i +
+// lane / 16 of its vector columns), tile by tile through the region as two transposed
+// tiles, added to the wavefront's own partial of the block at M: [256] real, then [256]
+// imaginary parts.  The partial stays in the caches between the column groups, and no
+// wavefront waits for another: summing four wavefronts' correlations in LDS behind two
+// barriers per block kept them in step, all in their exchanges while the matrix cores idled.
+template <typename R, int T, typename Y>
+__device__ __forceinline__ void fg_correlate(R* lds, const Y& yr, const Y& yi, const R (&xr)[T][4],
+                                             const R (&xi)[T][4], double* __restrict__ M, bool first, int lane) {
+    typedef FcMfma<R> MF;
+    const int nl = lane & 15, g = lane >> 4;
+    constexpr bool D64 = sizeof(R) == 8;
+    typename MF::V mr, mi;
+    double pr[4], pi[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int idx = MF::row(r, g) * 16 + nl;
+        pr[r] = first ? 0.0 : M[idx];
+        pi[r] = first ? 0.0 : M[256 + idx];
+        mr[r] = D64 ? (R)pr[r] : (R)0;
+        mi[r] = D64 ? (R)pi[r] : (R)0;
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        R* yb = lds + (T >= 4 && (t & 1) ? 1024 : 0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int at = fg_tile(4 * s + g, nl);
+            yb[at] = yr[t][s];
+            yb[256 + at] = yi[t][s];
+            yb[512 + at] = xr[t][s];
+            yb[768 + at] = xi[t][s];
+        }
+        fc_wave_fence();
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int at = fg_tile(nl, 4 * s + g);
+            const R yvr = yb[at], yvi = yb[256 + at], xvr = yb[512 + at], xvi = yb[768 + at];
+            mr = MF::op(yvr, xvr, mr);
+            mi = MF::op(yvr, xvi, mi);
+            mr = MF::op_neg(yvi, xvi, mr);
+            mi = MF::op(yvi, xvr, mi);
+        }
+        fc_wave_fence();
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int idx = MF::row(r, g) * 16 + nl;
+        M[idx] = D64 ? (double)mr[r] : pr[r] + (double)mr[r];
+        M[256 + idx] = D64 ? (double)mi[r] : pi[r] + (double)mi[r];
+    }
+}
+
+}  // namespace
+
+template <typename R, int N, int T>
+__global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const int* __restrict__ tabs) {
+    typedef FcMfma<R> MF;
+    typedef FcRegion<R, N, T> Reg;
+    constexpr int O = Reg::O, W = Reg::W;
+    static_assert(W >= 1, "a wavefront holds whole columns");
+    extern __shared__ __align__(16) unsigned char fg_smem[];
+    int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const FgTask task = fg_task(a, wv);
+    if (!task.live) return;
+    const int e = task.e, m = a.m;
+    const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 512 * T};
     const cpx<R>* U = static_cast<const cpx<R>*>(a.U);
     if (a.count) U += (long long)a.run_target[a.elem_run[e]] * a.tgt_stride;
-    const int m = a.m;
-    R xr[T][4], xi[T][4];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int col = c0 + w[t];
-        const int base = smap[16 + o[t]];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const cpx<R> v = col < m ? U[(long long)(base + smap[4 * s + g]) * m + col] : mk<R>(0, 0);
-            xr[t][s] = v.re;
-            xi[t][s] = v.im;
-        }
-    }
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.nb * 256;
-    typename MF::V dr[T], di[T];
-    // forward
-    for (int b = 0; b < a.nb; ++b) {
-        R ar[4], ai[4], ain[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const cpx<R> f = Fe[(long long)b * 256 + nl * 16 + 4 * s + g];
-            ar[s] = f.re;
-            ai[s] = f.im;
-            ain[s] = -f.im;
+    double* const part = a.mpart + ((long long)e * a.wgs + task.slot) * a.nb * 512;
+    for (int cg = task.first; cg < task.last; ++cg) {
+        const int c0 = cg * W;
+        const int nl = lane & 15, g = lane >> 4;
+        R xr[T][4], xi[T][4], yr[T][4], yi[T][4];
+        FcA<R> A;
+        typename MF::V dr[T], di[T];
+        fg_load_target<R, N, T>(U, tabs, c0, m, lane, xr, xi);
+        // forward; after the last block X stays in its own grouping
+        for (int b = 0; b < a.nb; ++b) {
+            const int* tab = tabs + b * kLaneTab;
+            A.load_n(Fe + (long long)b * 256, nl, g);
+            fg_mma<R, T, false>(A, xr, xi, dr, di);
+            if (b + 1 < a.nb) {
+                int at[4];
+                Reg::full_at(at, tab, tab[LT_LANE + lane]);
+                lds.template store_full<T>(at, tab, dr, di);
+                const int* tn = tab + kLaneTab;
+                Reg::full_at(at, tn, tn[LT_LANE + lane]);
+                lds.load_full(at, tn, xr, xi);
+            }
         }
-        fg_product<R, T>(ar, ai, ain, xr, xi, dr, di);
-        const int* mp = smap + b * kFusedMapStride;
-        // next block's grouping, or for the last block its own B layout
-        fg_remap<R, N, T>(dr, di, xr, xi, mp, b + 1 < a.nb ? mp + kFusedMapStride : mp, w, o, g, lds);
-    }
-    // trace entries from X (B layout of the last block) and the selector Y
-    R yr_[T][4], yi_[T][4];
-    {
-        const int* mp = smap + (a.nb - 1) * kFusedMapStride;
+        // trace entries from X and the selector Y (1 at row c + trace_off of column c)
+        {
+            const int* tab = tabs + (a.nb - 1) * kLaneTab;
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const int col = c0 + w[t];
-            const int base = mp[16 + o[t]];
+            for (int t = 0; t < T; ++t) {
+                const int col = c0 + (16 * t + nl) / O;
+                const int row = tab[LT_ROW + lane] | tab[LT_RT + t];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const bool hit = col < m && base + mp[4 * s + g] == col + a.trace_off;
-                if (hit) {
-                    double* d = a.diag + 2 * ((long long)e * m + col);
-                    d[0] = (double)xr[t][s];
-                    d[1] = (double)xi[t][s];
+                for (int s = 0; s < 4; ++s) {
+                    xr[t][s] = dr[t][s];
+                    xi[t][s] = di[t][s];
+                    const bool hit = col < m && (row | tab[LT_RS + s]) == col + a.trace_off;
+                    if (hit) {
+                        double* d = a.diag + 2 * ((long long)e * m + col);
+                        d[0] = (double)xr[t][s];
+                        d[1] = (double)xi[t][s];
+                    }
+                    yr[t][s] = hit ? (R)1 : (R)0;
+                    yi[t][s] = (R)0;
                 }
-                yr_[t][s] = hit ? (R)1 : (R)0;
-                yi_[t][s] = (R)0;
             }
         }
-    }
-    // backward
-    for (int b = a.nb - 1; b >= 0; --b) {
-        // F_b^T as the A operand: A[i][k] = F[k][i]; F^dagger: its conjugate
-        R tr_[4], ti_[4], tin_[4];
+        // backward: X_{b-1} = F^dagger X_b, M_b += Y_b X_{b-1}^T, Y_{b-1} = F^T Y_b
+        for (int b = a.nb - 1; b >= 0; --b) {
+            const int* tab = tabs + b * kLaneTab;
+            A.load_t(Fe + (long long)b * 256, nl, g);
+            fg_mma<R, T, true>(A, xr, xi, dr, di);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const cpx<R> f = Fe[(long long)b * 256 + (4 * s + g) * 16 + nl];
-            tr_[s] = f.re;
-            ti_[s] = f.im;
-            tin_[s] = -f.im;
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    xr[t][s] = dr[t][s];
+                    xi[t][s] = di[t][s];
+                }
+            fg_correlate<R, T>(lds.p, yr, yi, xr, xi, part + b * 512, cg == task.first, lane);
+            if (b == 0) break;
+            fg_mma<R, T, false>(A, yr, yi, dr, di);
+            const int* tn = tab - kLaneTab;
+            int at[4], an[4];
+            Reg::full_at(at, tab, tab[LT_LANE + lane]);
+            Reg::full_at(an, tn, tn[LT_LANE + lane]);
+            lds.template store_full<T>(at, tab, dr, di);
+            lds.load_full(an, tn, yr, yi);
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) lds.put(Reg::full(at, tab, t, s), xr[t][s], xi[t][s]);
+            fc_wave_fence();
+            lds.load_full(an, tn, xr, xi);
         }
-        // X_{b-1} = F^dagger X_b (A = conj(F^T): imaginary part negated)
-        fg_product<R, T>(tr_, tin_, ti_, xr, xi, dr, di);
-        // M_b += Y_b X_{b-1}^T over the wavefront's vector columns, tile by tile through
-        // the transposed buffers: ys[i][vc] from Y (B layout), xs[k][vc] from X_{b-1}
-        typename MF::V mr = typename MF::V{0, 0, 0, 0}, mi = typename MF::V{0, 0, 0, 0};
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) ys[fg_tile(4 * s + g, nl)] = mk<R>(yr_[t][s], yi_[t][s]);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) xs[fg_tile(MF::row(r, g), nl)] = mk<R>(dr[t][r], di[t][r]);
-            fg_wave_fence();
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const cpx<R> yv = ys[fg_tile(nl, 4 * s + g)];
-                const cpx<R> xv = xs[fg_tile(nl, 4 * s + g)];
-                mr = MF::op(yv.re, xv.re, mr);
-                mi = MF::op(yv.re, xv.im, mi);
-                mr = MF::op(-yv.im, xv.im, mr);
-                mi = MF::op(yv.im, xv.re, mi);
-            }
-            fg_wave_fence();
-        }
-        // the workgroup's wavefronts sum their M_b in a fixed order (each wavefront's
-        // region as 512 doubles: [256][re, im])
-        double* red = reinterpret_cast<double*>(lds);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = MF::row(r, g) * 16 + nl;
-            red[idx * 2] = (double)mr[r];
-            red[idx * 2 + 1] = (double)mi[r];
-        }
-        __syncthreads();
-        for (int i = threadIdx.x; i < 512; i += blockDim.x) {
-            double sum = 0.0;
-            for (int v = 0; v < nwv; ++v) sum += reinterpret_cast<const double*>(region + (size_t)v * RG)[i];
-            a.mpart[(((long long)e * a.wgs + wgi) * a.nb + b) * 512 + i] = sum;
-        }
-        __syncthreads();
-        if (b == 0) break;
-        // Y_{b-1} = F^T Y_b, then both to the grouping of block b - 1
-        typename MF::V er[T], ei[T];
-        fg_product<R, T>(tr_, ti_, tin_, yr_, yi_, er, ei);
-        const int* mp = smap + b * kFusedMapStride;
-        const int* mn = mp - kFusedMapStride;
-        fg_remap<R, N, T>(dr, di, xr, xi, mp, mn, w, o, g, lds);
-        fg_remap<R, N, T>(er, ei, yr_, yi_, mp, mn, w, o, g, lds);
     }
 }
 
@@ -297,234 +262,114 @@ __global__ __launch_bounds__(512) void k_fused_grad(FusedGradArgs a) {
 // k_fused_grad.  Needs nb >= 2 and block 0's support to cover every qubit (the chain
 // then ends in the forward layout).
 template <typename R, int N, int T>
-__global__ __launch_bounds__(512) void k_fused_grad_chain(FusedGradArgs a) {
-    typedef FgMfma<R> MF;
-    constexpr int D = 1 << N;
-    constexpr int O = D >> 4;
-    constexpr int W = 16 * T / O;
+__global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, const int* __restrict__ tabs,
+                                                             const int* __restrict__ tmaps) {
+    typedef FcMfma<R> MF;
+    typedef FcRegion<R, N, T> Reg;
+    constexpr int O = Reg::O, W = Reg::W;
     static_assert(W >= 1, "a wavefront holds whole columns");
-    constexpr int RG = 16 * T * 16;
-    static_assert(RG >= 512 && RG * sizeof(cpx<R>) >= 512 * sizeof(double), "the region holds the tiles");
     extern __shared__ __align__(16) unsigned char fg_smem[];
-    const int nwv = blockDim.x >> 6;
-    int* smap = reinterpret_cast<int*>(fg_smem);
-    int* tmap = smap + a.nb * kFusedMapStride;
-    const int nmap = a.nb * (kFusedMapStride + kTraceMapStride);
-    cpx<R>* region = reinterpret_cast<cpx<R>*>(fg_smem + (((size_t)nmap * sizeof(int) + 15) & ~(size_t)15));
-    for (int i = threadIdx.x; i < a.nb * kFusedMapStride; i += blockDim.x) smap[i] = a.maps[i];
-    for (int i = threadIdx.x; i < a.nb * kTraceMapStride; i += blockDim.x) tmap[i] = a.tmaps[i];
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int B = a.B;
-    long long lwg = blockIdx.x;
-    if (a.count) {
-        B = min(*a.count, a.B);
-    } else {
-        const long long per_xcd = gridDim.x >> 3;
-        lwg = (long long)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    }
-    const long long wave = lwg * nwv + wv;
-    if (lwg * nwv >= (long long)B * a.groups) return;  // whole workgroups
-    const int e = (int)(wave / a.groups);
-    const int cg = (int)(wave % a.groups);
-    const int c0 = cg * W;
-    const int wgi = cg / nwv;
-    cpx<R>* lds = region + (size_t)wv * RG;
-    cpx<R>* ys = lds;
-    cpx<R>* xs = lds + 256;
-    const int nl = lane & 15, g = lane >> 4;
-    int w[T], o[T];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        w[t] = (16 * t + nl) / O;
-        o[t] = (16 * t + nl) % O;
-    }
+    int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const FgTask task = fg_task(a, wv);
+    if (!task.live) return;
+    const int e = task.e, m = a.m;
+    const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 512 * T};
     const cpx<R>* U = static_cast<const cpx<R>*>(a.U);
     if (a.count) U += (long long)a.run_target[a.elem_run[e]] * a.tgt_stride;
-    const int m = a.m;
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.nb * 256;
-    // phase 1: Z_1 in block 0's grouping (B layout)
-    R zr[T][4], zi[T][4], far[4], fai[4];
-    fused_chain_to_block0<R, N, T, false>(tmap, a.nb, lds, Fe, c0, m, a.trace_off, lane, zr, zi, far, fai);
-    typename MF::V er[T], ei[T];
-    {
-        // Z_0 = F_0^T Z_1, times the target's columns: the trace entries
-        R ar[4], ai[4], ain[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const cpx<R> f = Fe[(4 * s + g) * 16 + nl];
-            ar[s] = f.re;
-            ai[s] = f.im;
-            ain[s] = -f.im;
-        }
-        fg_product<R, T>(ar, ai, ain, zr, zi, er, ei);
-        constexpr int seg = O < 16 ? O : 16;
-        double sr = 0, si = 0;
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const int col = c0 + w[t];
-            if (col < m) {
-                const int base = smap[16 + o[t]];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const cpx<R> u = U[(long long)(base + smap[MF::row(r, g)]) * m + col];
-                    sr += (double)er[t][r] * (double)u.re - (double)ei[t][r] * (double)u.im;
-                    si += (double)er[t][r] * (double)u.im + (double)ei[t][r] * (double)u.re;
-                }
-            }
-            if (O < 16 || ((t + 1) * 16) % O == 0) {
-                sr += __shfl_xor(sr, 16, 64);
-                si += __shfl_xor(si, 16, 64);
-                sr += __shfl_xor(sr, 32, 64);
-                si += __shfl_xor(si, 32, 64);
-#pragma unroll
-                for (int d = 1; d < seg; d <<= 1) {
-                    sr += __shfl_xor(sr, d, 64);
-                    si += __shfl_xor(si, d, 64);
-                }
-                if (g == 0 && (nl & (seg - 1)) == 0 && col < m) {
-                    double* dg = a.diag + 2 * ((long long)e * m + col);
-                    dg[0] = sr;
-                    dg[1] = si;
-                }
-                sr = 0;
-                si = 0;
-            }
-        }
-    }
-    // phase 2: X_{-1} = the target's columns in block 0's grouping (B layout)
-    R xr[T][4], xi[T][4];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        const int col = c0 + w[t];
-        const int base = smap[16 + o[t]];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const cpx<R> v = col < m ? U[(long long)(base + smap[4 * s + g]) * m + col] : mk<R>(0, 0);
-            xr[t][s] = v.re;
-            xi[t][s] = v.im;
-        }
-    }
-    // M_bb += Y X^T over the wavefront's vector columns, Y in the B layout (ZB) or the D
-    // layout (er / ei), X in the B layout; then the workgroup's partial of block bb
-    auto correlate = [&](int bb, bool zb) __attribute__((always_inline)) {
-        typename MF::V mr = typename MF::V{0, 0, 0, 0}, mi = typename MF::V{0, 0, 0, 0};
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            if (zb) {
-#pragma unroll
-                for (int s = 0; s < 4; ++s) ys[fg_tile(4 * s + g, nl)] = mk<R>(zr[t][s], zi[t][s]);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) ys[fg_tile(MF::row(r, g), nl)] = mk<R>(er[t][r], ei[t][r]);
-            }
-#pragma unroll
-            for (int s = 0; s < 4; ++s) xs[fg_tile(4 * s + g, nl)] = mk<R>(xr[t][s], xi[t][s]);
-            fg_wave_fence();
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const cpx<R> yv = ys[fg_tile(nl, 4 * s + g)];
-                const cpx<R> xv = xs[fg_tile(nl, 4 * s + g)];
-                mr = MF::op(yv.re, xv.re, mr);
-                mi = MF::op(yv.re, xv.im, mi);
-                mr = MF::op(-yv.im, xv.im, mr);
-                mi = MF::op(yv.im, xv.re, mi);
-            }
-            fg_wave_fence();
-        }
-        double* red = reinterpret_cast<double*>(lds);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int idx = MF::row(r, g) * 16 + nl;
-            red[idx * 2] = (double)mr[r];
-            red[idx * 2 + 1] = (double)mi[r];
-        }
-        __syncthreads();
-        for (int i = threadIdx.x; i < 512; i += blockDim.x) {
-            double sum = 0.0;
-            for (int v = 0; v < nwv; ++v) sum += reinterpret_cast<const double*>(region + (size_t)v * RG)[i];
-            a.mpart[(((long long)e * a.wgs + wgi) * a.nb + bb) * 512 + i] = sum;
-        }
-        __syncthreads();
-    };
-    correlate(0, true);
-    typename MF::V dr[T], di[T];
-    // one step up: X_b into block b + 1's grouping, Z_{b+2} (D layout, block b + 1's
-    // grouping) from Z_{b+1} -- in the B layout of block 0 for the first step (zb), in
-    // the D layout of block b after it -- then M_{b+1}.  The first step runs on its own
-    // so the B-layout Z is not live through the loop.
-    auto step = [&](int b, bool zb) __attribute__((always_inline)) {
-        const int* mp = smap + b * kFusedMapStride;
-        const int* mn = mp + kFusedMapStride;
+    double* const part = a.mpart + ((long long)e * a.wgs + task.slot) * a.nb * 512;
+    for (int cg = task.first; cg < task.last; ++cg) {
+        const int c0 = cg * W;
+        const bool first = cg == task.first;
+        asm volatile("" : "+v"(lane));  // no lane's addresses kept in registers from group to group
+        const int nl = lane & 15, g = lane >> 4;
+        // phase 1: Z_1 in block 0's grouping, X = the target's columns there, and the trace
+        // entries from Z_0 = F_0^T Z_1
+        R zr[T][4], zi[T][4], xr[T][4], xi[T][4];
+        typename MF::V er[T], ei[T];
+        FcA<R> A;
+        fused_chain_to_block0<R, N, T, false>(tabs, tmaps, a.nb, lds, Fe, c0, m, a.trace_off, lane, zr, zi, A);
+        fg_mma<R, T, false>(A, zr, zi, er, ei);
         {
-            R ar[4], ai[4], ain[4];
+            constexpr int C = O > 16 ? W : T;  // sums: per column, or per tile of whole columns
+            double sr[C], si[C];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const cpx<R> f = Fe[(long long)b * 256 + nl * 16 + 4 * s + g];
-                ar[s] = f.re;
-                ai[s] = f.im;
-                ain[s] = -f.im;
-            }
-            fg_product<R, T>(ar, ai, ain, xr, xi, dr, di);
-            fg_remap<R, N, T>(dr, di, xr, xi, mp, mn, w, o, g, lds);
-        }
-        if (b + 2 < a.nb) {
-            if (zb) {
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    const int base = mp[16 + o[t]];
-#pragma unroll
-                    for (int s = 0; s < 4; ++s)
-                        lds[w[t] * D + fg_slot<N>(base + mp[4 * s + g])] = mk<R>(zr[t][s], zi[t][s]);
-                }
-                fg_wave_fence();
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    const int base = mn[16 + o[t]];
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const cpx<R> v = lds[w[t] * D + fg_slot<N>(base + mn[4 * s + g])];
-                        zr[t][s] = v.re;
-                        zi[t][s] = v.im;
-                    }
-                }
-                fg_wave_fence();
-            } else {
-                fg_remap<R, N, T>(er, ei, zr, zi, mp, mn, w, o, g, lds);
-            }
-            R ar[4], ai[4], ain[4];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const cpx<R> f = Fe[(long long)(b + 1) * 256 + nl * 16 + 4 * s + g];
-                ar[s] = f.re;
-                ai[s] = -f.im;
-                ain[s] = f.im;
-            }
-            fg_product<R, T>(ar, ai, ain, zr, zi, er, ei);
-        } else {
-            // Z_nb: the selector, row rho = c + trace_off of column c (D layout)
+            for (int c = 0; c < C; ++c) sr[c] = si[c] = 0;
+            const unsigned row0 = (unsigned)tabs[LT_ROW + lane] * (unsigned)m;
 #pragma unroll
             for (int t = 0; t < T; ++t) {
-                const int col = c0 + w[t];
-                const int base = mn[16 + o[t]];
+                const int c = O > 16 ? t / (O / 16 ? O / 16 : 1) : t;
+                const int col = c0 + (16 * t + nl) / O;
+                const unsigned at = row0 + (unsigned)tabs[LT_RT + t] * (unsigned)m + (unsigned)(col < m ? col : 0);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    er[t][r] = (col < m && base + mn[MF::row(r, g)] == col + a.trace_off) ? (R)1 : (R)0;
-                    ei[t][r] = (R)0;
+                    const cpx<R> u = U[at + (unsigned)tabs[LT_RS + r] * (unsigned)m];
+                    sr[c] += (double)er[t][r] * (double)u.re - (double)ei[t][r] * (double)u.im;
+                    si[c] += (double)er[t][r] * (double)u.im + (double)ei[t][r] * (double)u.re;
                 }
             }
+            fc_column_sums<N, T>(sr, si, a.diag + 2 * ((long long)e * m + c0), c0, m, lane);
         }
-        correlate(b + 1, false);
-    };
-    step(0, true);
-    for (int b = 1; b + 1 < a.nb; ++b) step(b, false);
+        fg_load_target<R, N, T>(U, tabs, c0, m, lane, xr, xi);
+        fg_correlate<R, T>(lds.p, zr, zi, xr, xi, part, first, lane);
+        // phase 2, one step up: X_b into block b + 1's grouping, Z_{b+2} (block b + 1's
+        // grouping, as a result) from Z_{b+1} -- block 0's operand for the first step, the
+        // last step's result after it -- then M_{b+1}.  The first step runs on its own, so
+        // that its operand is not live through the loop.
+        auto step = [&](int b, auto first_step) __attribute__((always_inline)) {
+            constexpr bool ZB = decltype(first_step)::value;
+            const int* tab = tabs + b * kLaneTab;
+            const int* tn = tab + kLaneTab;
+            int at[4], an[4];
+            Reg::full_at(at, tab, tab[LT_LANE + lane]);
+            Reg::full_at(an, tn, tn[LT_LANE + lane]);
+            {
+                FcA<R> An;
+                An.load_n(Fe + (long long)b * 256, nl, g);
+                typename MF::V dr[T], di[T];
+                fg_mma<R, T, false>(An, xr, xi, dr, di);
+                lds.template store_full<T>(at, tab, dr, di);
+                lds.load_full(an, tn, xr, xi);
+            }
+            if (b + 2 < a.nb) {
+                if constexpr (ZB) {
+#pragma unroll
+                    for (int t = 0; t < T; ++t)
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) lds.put(Reg::full(at, tab, t, s), zr[t][s], zi[t][s]);
+                    fc_wave_fence();
+                } else {
+                    lds.template store_full<T>(at, tab, er, ei);
+                }
+                R vr[T][4], vi[T][4];
+                lds.load_full(an, tn, vr, vi);
+                FcA<R> An;
+                An.load_n(Fe + (long long)(b + 1) * 256, nl, g);
+                fg_mma<R, T, true>(An, vr, vi, er, ei);
+            } else {
+                // Z_nb: the selector, row rho = c + trace_off of column c
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    const int col = c0 + (16 * t + nl) / O;
+                    const int row = tn[LT_ROW + lane] | tn[LT_RT + t];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        er[t][r] = (col < m && (row | tn[LT_RS + r]) == col + a.trace_off) ? (R)1 : (R)0;
+                        ei[t][r] = (R)0;
+                    }
+                }
+            }
+            fg_correlate<R, T>(lds.p, er, ei, xr, xi, part + (b + 1) * 512, first, lane);
+        };
+        step(0, std::true_type{});
+        for (int b = 1; b + 1 < a.nb; ++b) step(b, std::false_type{});
+    }
 }
 
 size_t fused_grad_lds_bytes(bool f32, int nb, int T, int waves) {
-    // both row tables (the chain kernel's too), then one region per wavefront
-    const size_t esz = f32 ? 8 : 16;
-    return (((size_t)nb * (kFusedMapStride + kTraceMapStride) * sizeof(int) + 15) & ~(size_t)15) +
-           esz * (size_t)(16 * T * 16) * waves;
+    (void)nb;
+    return (f32 ? 8 : 16) * (size_t)(256 * T) * waves;  // a region per wavefront
 }
 
 template <typename R>
@@ -532,9 +377,9 @@ static hipError_t launch_fg(int N, const FusedGradArgs& a, int T, int grid, int 
 #define SQH_FG_CASE(n, t)                                                                                    \
     if (N == n && T == t) {                                                                                  \
         if (a.tmaps)                                                                                         \
-            hipLaunchKernelGGL((k_fused_grad_chain<R, n, t>), dim3(grid), dim3(threads), shm, s, a);         \
+            hipLaunchKernelGGL((k_fused_grad_chain<R, n, t>), dim3(grid), dim3(threads), shm, s, a, a.tabs, a.tmaps); \
         else                                                                                                 \
-            hipLaunchKernelGGL((k_fused_grad<R, n, t>), dim3(grid), dim3(threads), shm, s, a);               \
+            hipLaunchKernelGGL((k_fused_grad<R, n, t>), dim3(grid), dim3(threads), shm, s, a, a.tabs);       \
         return hipGetLastError();                                                                            \
     }
     SQH_FG_CASE(4, 4)
@@ -568,13 +413,25 @@ bool fused_grad_shape_valid(bool f32, int N, int m, int nb, int T, int waves) {
     return groups > 0 && groups % waves == 0 && fused_grad_lds_bytes(f32, nb, T, waves) <= device_max_lds();
 }
 
-int fused_grad_wgs(int N, int m, int T, int waves) { return fg_groups(N, m, T) / waves; }
+// Column groups a wavefront takes one after another, adding to one partial: as many as
+// leave two wavefronts per SIMD (2048), the most that are resident with four tiles.  Fewer
+// partials are then written and summed; a small batch keeps a group per wavefront.
+int fused_grad_per(int N, int m, int T, int B) {
+    const long long total = (long long)fg_groups(N, m, T) * B;
+    return (int)std::max<long long>(1, std::min<long long>(total / 2048, fg_groups(N, m, T)));
+}
+
+int fused_grad_wgs(int N, int m, int T, int B) {
+    const int per = fused_grad_per(N, m, T, B);
+    return (fg_groups(N, m, T) + per - 1) / per;
+}
 
 hipError_t launch_fused_grad(bool f32, int N, FusedGradArgs a, int T, int waves, hipStream_t s) {
     if (a.B <= 0 || !fused_grad_shape_valid(f32, N, a.m, a.nb, T, waves)) return hipErrorInvalidValue;
     a.groups = fg_groups(N, a.m, T);
-    if (a.wgs != a.groups / waves) return hipErrorInvalidValue;  // the partials' layout the caller sized
-    const long long wgs_total = (long long)a.B * a.wgs;
+    a.per = fused_grad_per(N, a.m, T, a.B);
+    if (a.wgs != fused_grad_wgs(N, a.m, T, a.B)) return hipErrorInvalidValue;  // the partials' layout the caller sized
+    const long long wgs_total = ((long long)a.B * a.wgs + waves - 1) / waves;
     const int grid = (int)((wgs_total + 7) / 8 * 8);
     const size_t shm = fused_grad_lds_bytes(f32, a.nb, T, waves);
     return f32 ? launch_fg<float>(N, a, T, grid, 64 * waves, shm, s)

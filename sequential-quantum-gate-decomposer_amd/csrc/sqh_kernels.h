@@ -98,6 +98,16 @@ hipError_t launch_convert(bool to_f32, const void* src, void* dst, long long nre
 // F + b * F_bstride (0: shared).  diag receives the B x m trace entries (complex, as
 // double pairs).
 constexpr int kFusedMapStride = 16 + 64;
+// Lane tables of the fused kernels, kLaneTab ints per block (fused_lane_tabs): where lane l
+// = nl + 16 g of a wavefront finds row 4 s + g of vector column 16 t + nl of the block.  A
+// row's LDS slot is linear over XOR (fc_slot) and the bits of a row's parts are disjoint, so
+// a slot is the lane's entry XOR a uniform part of s XOR a uniform part of t:
+//   LT_LANE[64], LT_S[4], LT_T[4]   full layout: slot (column included) of the lane, s, t
+//   LT_ROW[64], LT_RS[4], LT_RT[4]  the same as plain rows (columns excluded)
+//   LT_SLANE[64], LT_ST[4]          the chain's support layout: slots of the lane and t
+//   LT_LG, LT_NS                    its log2 of groups per column, row bits outside it
+constexpr int LT_LANE = 0, LT_S = 64, LT_T = 68, LT_ROW = 72, LT_RS = 136, LT_RT = 140, LT_SLANE = 144, LT_ST = 208,
+              LT_LG = 212, LT_NS = 213, kLaneTab = 216;
 constexpr int kFusedCostMaxQubits = 10;
 struct FusedCostArgs {
     const void* U = nullptr;  // input: element b's at U + (in_index ? in_index[b] : b) * in_bstride
@@ -108,11 +118,16 @@ struct FusedCostArgs {
     const void* F = nullptr;
     long long F_bstride = 0;
     const int* maps = nullptr;
+    const int* tabs = nullptr;  // lane tables [nb][kLaneTab]
     double* diag = nullptr;
     void* out = nullptr;  // non-null: store element b's result at out + b * out_bstride (row stride out_stride)
     long long out_bstride = 0;
     int out_stride = 0;
     int groups = 0;  // column groups per element (set by the launcher)
+    bool prefix = false;  // store pass: element e runs only blocks 0 .. e - 1
+    // store pass of apply_derivate_to: element e starts with block dinfo[4 e], whose matrix is
+    // number nb + e of F, from input dinfo[4 e]
+    const int* dinfo = nullptr;
 };
 // 2 x 2 kernels of the parametric gates of a batch: element e's computed from its P
 // parameters at params + e * pstride, or (params null) read from its table at
@@ -125,15 +140,20 @@ struct GateKernels {
     const Slot* slots = nullptr;
 };
 // The 16 x 16 matrices of the fused blocks (out[B][nb][16][16]) from their gates (quad
-// ops, quad_ops).  count: live elements; zslot: per element the controlled slot whose
-// control-0 rows are zeroed, or -1.
+// ops, quad_ops).  count: live elements.
 hipError_t launch_fuse_blocks(bool f32, const uint32_t* ops, const int* first, int nb, const GateKernels& g, int B,
-                              void* out, hipStream_t s, const int* count = nullptr, const int* zslot = nullptr);
+                              void* out, hipStream_t s, const int* count = nullptr);
+// The nb block matrices of one parameter vector and, after them, for every parameter k the
+// matrix of its gate's block with that gate differentiated (out[nb + P][16][16],
+// complex128).  dinfo[k]: block, slot, parameter within the gate, whether the gate is
+// controlled (its control-0 rows are then zeroed).
+hipError_t launch_fuse_deriv_blocks(const uint32_t* ops, const int* first, int nb, const double* params,
+                                    const Slot* slots, const int* dinfo, int P, void* out, hipStream_t s);
 
 // Cost and gradient through the fused blocks (sqh_k_fused_grad.hip): the forward pass
 // and trace entries as the cost kernel, then the blocks backwards with the trace
-// selector, writing per workgroup and block the 16x16 correlation partials
-// mpart[B][wgs][nb][256] (complex, as double pairs).  T: 16-column tiles per wavefront.
+// selector, writing per wavefront and block the 16x16 correlation partials
+// mpart[B][wgs][nb][512] (256 real, then 256 imaginary parts).  T: 16-column tiles per wavefront.
 struct FusedGradArgs {
     const void* U = nullptr;  // target, rows = 2^N, m columns, row stride m
     int m = 0, trace_off = 0, B = 0, nb = 0;
@@ -141,8 +161,10 @@ struct FusedGradArgs {
     const int* maps = nullptr;
     double* diag = nullptr;
     double* mpart = nullptr;
-    int wgs = 0;     // workgroups per element (the partials' layout)
+    int wgs = 0;     // partials per element
     int groups = 0;  // column groups per element (set by the launcher)
+    int per = 1;     // column groups per partial (set by the launcher)
+    const int* tabs = nullptr;  // lane tables [nb][kLaneTab]
     // optional optimiser indirection: live elements *count (of B), element e's target at
     // U + run_target[elem_run[e]] * tgt_stride
     const int* count = nullptr;
@@ -155,10 +177,10 @@ struct FusedGradArgs {
     const int* tmaps = nullptr;
 };
 // Launch shape: T 16-column tiles per wavefront (2 or 4; 4 at 10 qubits), waves 1, 2, 4
-// or 8 per workgroup dividing the element's column groups; wgs = workgroups per element
-// (the partials' count).
+// or 8 per workgroup dividing the element's column groups; wgs = partials per element of a
+// batch of B.
 bool fused_grad_shape_valid(bool f32, int N, int m, int nb, int T, int waves);
-int fused_grad_wgs(int N, int m, int T, int waves);
+int fused_grad_wgs(int N, int m, int T, int B);
 size_t fused_grad_lds_bytes(bool f32, int nb, int T, int waves);
 hipError_t launch_fused_grad(bool f32, int N, FusedGradArgs a, int T, int waves, hipStream_t s);
 // Per (element, block): the partials summed, then the block's gates run backwards on

@@ -150,6 +150,12 @@ int fused_cost_launch(sqh_ctx* c, bool f32, const FusedCostArgs& a_in) {
     auto launch = [&](const FusedCostArgs& x, FusedCostCfg cfg) {
         return chain ? launch_fused_trace(f32, N, x, cfg, c->stream) : launch_fused_cost(f32, N, x, cfg, c->stream);
     };
+    if (a.prefix) {
+        // a few matrices once per call: the smallest work per wavefront, not tuned
+        const FusedCostCfg small{2, 1, 4, 0};
+        HIPTRY(c, launch(a, valid(small) ? small : fused_default(N, f32, nb, chain)));
+        return SQH_OK;
+    }
     if (c->fused_force.tiles != 0) {
         if (!valid(c->fused_force))
             return fail(c, SQH_ERR_ARG,
