@@ -319,12 +319,13 @@ int sqh_get_jit_stats(sqh_ctx* ctx, double* compile_ms, int* compiles);
  * as MFMA tiles, LDS exchanges between blocks, trace entries at the end).  Applies for
  * 4 to 10 qubits and costs without correction channels; elsewhere the tile kernels
  * run.  Results agree with the tile kernels to rounding (the blocks reassociate the
- * products).  mode: SQH_FUSED_COST_OFF, _ON, or _AUTO (the default: on from 7 qubits,
- * or from 5 when the run-time specialised kernels are off -- where it measured faster
- * than the tile kernels -- when the blocks do no more arithmetic than the gates).  The
- * same mode selects the fused blocks' adjoint for cost + gradient batches
- * (sqh_optimization_problem_combined_batch[_dev]; _AUTO: from 6 qubits, with the same
- * arithmetic condition): forward and backward block products on the matrix cores, each
+ * products).  mode: SQH_FUSED_COST_OFF, _ON, or _AUTO (the default: where it measured
+ * faster than the tile kernels, by the qubits and the blocks' arithmetic over the gates' --
+ * against the run-time specialised kernels from 7 qubits when the blocks do no more;
+ * against the generic ones from 4 qubits for deep circuits and from 6 for all but shallow
+ * ones).  The same mode selects the fused blocks' adjoint for cost + gradient batches
+ * (sqh_optimization_problem_combined_batch[_dev]; _AUTO: from 6 qubits against the
+ * specialised kernels): forward and backward block products on the matrix cores, each
  * block's correlations then resolved to its gates.  sqh_decompose_batch's lockstep
  * rounds use the fused adjoint with _ON only.  apply_derivate_to follows the cost pass's
  * rule (one fused store pass over the P derivative elements).  No counterpart in the reference: it

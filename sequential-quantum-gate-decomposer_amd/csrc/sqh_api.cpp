@@ -231,30 +231,49 @@ double tile_gate_flops(const sqh_ctx* c) {
     return w;
 }
 
-// Whether the fused blocks do less arithmetic than the gate-by-gate kernels (128 flop
-// per element per dense block; the cost + gradient: 4 nb - 1 block products against
-// (3 + 8/7) x the forward gate arithmetic).  Shallow circuits, with few gates per
-// block, stay on the tile kernels in the automatic mode.
-bool fused_pays(const sqh_ctx* c, bool grad) {
+// Arithmetic of the fused blocks over that of the gate-by-gate kernels (128 flop per
+// element per dense block; the cost + gradient: 4 nb - 1 block products against
+// (3 + 8/7) x the forward gate arithmetic).  Large for shallow circuits, with few gates
+// per block.
+double fused_ratio(const sqh_ctx* c, bool grad) {
     const double nb = (double)c->fplan.qubits.size(), w = tile_gate_flops(c);
-    return grad ? (4.0 * nb - 1.0) * 128.0 <= (3.0 + 8.0 / 7.0) * w : nb * 128.0 <= w;
+    return grad ? (4.0 * nb - 1.0) * 128.0 / ((3.0 + 8.0 / 7.0) * w) : nb * 128.0 / w;
 }
 
-// Whether a pass (costs, or the apply_to store pass) runs through the tile-resident
-// fused-block kernel: 4 <= N <= 10, the circuit has blocks, and the switch is on -- or
-// automatic (the default) where it measured faster on MI355X than the register-tile
-// kernels: from 7 qubits, or from 5 when the circuit-specialised kernels are off, and
-// the blocks do no more arithmetic than the gates.  Costs also need no correction
-// channels (fused_cost_applies).
-bool fused_pass_applies(const sqh_ctx* c) {
+// The automatic choice of the fused kernels, where they measured faster on MI355X than the
+// register-tile kernels.  Against the circuit-specialised ones: from 7 qubits (with a
+// gradient from 6), when the blocks do no more arithmetic than the gates.  Against the
+// generic ones the line is the arithmetic ratio up to which both precisions gain at
+// B = 1 to 4096 (time of the tile kernels over that of the fused ones); it does not look at
+// B, so that a vector's result does not depend on the batch it came in:
+//   gradients  8+ qubits: 2.5 (1.3 - 3.2 at 1.9 - 2.4, 2.0 - 6.1 below 1.2)
+//              6, 7:      1.5 (1.1 - 1.9 at 1.3, 0.85 at 2.6)
+//              5:         1   (1.2 - 3.0 below, 0.85 at 1.5)
+//              4:         0.3 (0.95 - 2.5 below; 0.81 at 0.41 and B = 4096)
+//   costs      8+: 1.5, 6 and 7: 1.2, 5: 1 (1.0 - 4.2 below these, 0.8 - 1.2 at 2.3)
+//              4:  0.25 (1.0 - 1.7 below; 0.89 at 0.33 and B = 4096)
+//   store pass 7+: 1.2, 5 and 6: 1 (0.9 - 3.5 below, 0.5 - 1.3 at 2.3)
+//              4:  0.25 (1.3 - 1.7 below; 0.9 at 0.57)
+enum FusedKind { FUSED_COST_PASS, FUSED_STORE_PASS, FUSED_GRAD_PASS };
+bool fused_auto(const sqh_ctx* c, FusedKind kind) {
     const int N = c->prog.N;
+    const double r = fused_ratio(c, kind == FUSED_GRAD_PASS);
+    if (c->jit) return N >= (kind == FUSED_GRAD_PASS ? 6 : 7) && r <= 1.0;
+    static const double line[3][5] = {{0.25, 1.0, 1.2, 1.2, 1.5}, {0.25, 1.0, 1.0, 1.2, 1.2}, {0.3, 1.0, 1.5, 1.5, 2.5}};
+    return r <= line[kind][std::min(N, 8) - 4];
+}
+
+// Whether a pass (costs, or the apply_to store pass) runs through the tile-resident fused-block kernel: 4 <= N <= 10, the circuit has blocks, and the switch is
+// on, or automatic (the default) and the rule above holds.  Costs also need no correction
+// channels (fused_cost_applies).
+bool fused_pass_applies(const sqh_ctx* c, bool store) {
     if (!fused_plan_fits(c)) return false;
-    if (c->fused_cost == SQH_FUSED_COST_AUTO) return (N >= 7 || (N >= 5 && !c->jit)) && fused_pays(c, false);
+    if (c->fused_cost == SQH_FUSED_COST_AUTO) return fused_auto(c, store ? FUSED_STORE_PASS : FUSED_COST_PASS);
     return c->fused_cost == SQH_FUSED_COST_ON;
 }
 
 bool fused_cost_applies(const sqh_ctx* c, bool grad, const TraceSpec& ts) {
-    return !grad && ts.nch == 0 && fused_pass_applies(c);
+    return !grad && ts.nch == 0 && fused_pass_applies(c, false);
 }
 
 // The 2x2 kernels of a batch computed from its parameters where they are used.
@@ -334,18 +353,17 @@ bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, FusedGradPlan& p)
     return true;
 }
 
-// Whether a cost + gradient evaluation of B elements of m columns runs through the
-// fused blocks: the switch on (SQH_FUSED_COST_ON, or _AUTO from 6 qubits when the blocks
-// do less arithmetic than the gates -- where it measured faster than the register-tile
-// adjoint at every batch size), 4 <= N <= 10, no correction channels, and a launch
-// shape fits.
+// Whether a cost + gradient evaluation of B elements of m columns runs through the fused
+// blocks: the switch on, or automatic and the rule of fused_auto, 4 <= N <= 10, no
+// correction channels, and a launch shape fits.  Below 6 qubits, where the blocks' scratch
+// is several times the tile kernels', automatic batches keep it within 4 GiB.
 bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, int m, FusedGradPlan* plan) {
     if (ts.nch != 0 || !fused_plan_fits(c)) return false;
-    if (c->fused_cost == SQH_FUSED_COST_OFF ||
-        (c->fused_cost == SQH_FUSED_COST_AUTO && (c->prog.N < 6 || !fused_pays(c, true))))
-        return false;
+    const bool automatic = c->fused_cost == SQH_FUSED_COST_AUTO;
+    if (c->fused_cost == SQH_FUSED_COST_OFF || (automatic && !fused_auto(c, FUSED_GRAD_PASS))) return false;
     FusedGradPlan p;
     if (!fused_grad_plan(c, f32, B, m, p)) return false;
+    if (automatic && c->prog.N < 6 && p.fused_bytes + p.mpart_bytes + p.corr_bytes > (size_t)4 << 30) return false;
     if (plan) *plan = p;
     return true;
 }
@@ -627,7 +645,7 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
     const long long kb = pbstride ? (long long)ns * 4 : 0;
     if (path == 0 && N > kMaxTileQubits) path = 2;
     if (path == 2) return fused_apply(c, d_inout, rows, cols, stride, bstride, B, f32, d_params, pbstride);
-    const bool fused = path == 0 && fused_pass_applies(c);
+    const bool fused = path == 0 && fused_pass_applies(c, true);
     if (!fused && (rc = build_kernels(c, d_params, Bk, f32))) return rc;
     if (fused) {
         // the circuit's fused 4-qubit blocks on the matrix cores, every column resident
@@ -690,7 +708,7 @@ int deriv_dev(sqh_ctx* c, const double* d_params, const void* d_in, int rows, in
         return fail(c, SQH_ERR_ARG, "apply_derivate_to supports up to %d qubits", kMaxTileQubits);
     if (c->prog.slots.empty()) return SQH_OK;
     const int ns = (int)c->prog.slots.size(), P = c->prog.P;
-    if (fused_pass_applies(c)) {
+    if (fused_pass_applies(c, true)) {
         // Through the fused blocks: a derivative shares the blocks before its gate's with
         // the others, so the products F_{b-1} ... F_0 in are formed once per block and
         // element k starts from its block's, with that block differentiated.  The 8-qubit

@@ -15,6 +15,8 @@
 // register column unrolled took 27 us a block build and 74 us a correlation walk with the
 // partials' sum (8 qubits, one element; 30 and 100 for 512).  Now 12 and 22 (16 and 61),
 // with the kernel table's launch gone: gradient of one 8-qubit vector 209 -> 117 us.
+// Both compute in FP64 in either precision: a complex64 block matrix is then rounded once,
+// not after each of its gates.
 #include <hip/hip_runtime.h>
 
 #include "sqh_device.h"
@@ -23,6 +25,11 @@
 namespace sqh {
 
 namespace {
+
+template <typename R>
+__device__ __forceinline__ cpx<double> widen(cpx<R> a) {
+    return mk((double)a.re, (double)a.im);
+}
 
 __device__ __forceinline__ void quad_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
@@ -78,12 +85,12 @@ __device__ __forceinline__ void quad_back(cpx<R>& x0, cpx<R>& x1, cpx<R>& y0, cp
 }
 
 // The 2 x 2 kernels of a chunk's gates for one element into tab[gate][4], a gate per lane:
-// computed from the element's parameters as k_build_kernels does (FP64, then converted),
-// or taken from the element's kernel table.
+// computed from the element's parameters, or taken from the element's kernel table.
 // Gate dslot gets its derivative with respect to its parameter dparam.
 template <typename R>
 __device__ __forceinline__ void quad_stage(uint32_t w, bool live, const cpx<R>* kern, const double* params,
-                                           const Slot* slots, int lane, cpx<R>* tab, int dslot = -1, int dparam = 0) {
+                                           const Slot* slots, int lane, cpx<double>* tab, int dslot = -1,
+                                           int dparam = 0) {
     const int slot = (int)(w >> kQuadSlotShift) - 1;
     if (live && slot >= 0) {
         if (params) {
@@ -92,10 +99,10 @@ __device__ __forceinline__ void quad_stage(uint32_t w, bool live, const cpx<R>* 
             if (slot == dslot) dev_deriv_kernel(sl.type, params + sl.param_start, dparam, k4);
             else dev_gate_kernel(sl.type, params + sl.param_start, k4);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) tab[4 * lane + k] = cvt<R>(k4[k]);
+            for (int k = 0; k < 4; ++k) tab[4 * lane + k] = k4[k];
         } else {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) tab[4 * lane + k] = kern[4 * slot + k];
+            for (int k = 0; k < 4; ++k) tab[4 * lane + k] = widen(kern[4 * slot + k]);
         }
     }
 }
@@ -128,8 +135,8 @@ __global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t*
                                                                  cpx<R>* __restrict__ out,
                                                                  const int* __restrict__ count,
                                                                  const int* __restrict__ dinfo) {
-    __shared__ cpx<R> state[kQuadWaves][256];
-    __shared__ cpx<R> table[kQuadWaves][64 * 4];
+    __shared__ cpx<double> state[kQuadWaves][256];
+    __shared__ cpx<double> table[kQuadWaves][64 * 4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int e = (DERIV ? blockIdx.x : blockIdx.x / nb) * kQuadWaves + wave;
     if (count) B = min(*count, B);  // live elements (the optimiser's rounds)
@@ -144,14 +151,14 @@ __global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t*
         zero = d[3] != 0;
     }
     const int col = lane & 15, z = lane >> 4;
-    cpx<R>* s = state[wave];
-    cpx<R>* tab = table[wave];
+    cpx<double>* s = state[wave];
+    cpx<double>* tab = table[wave];
     const int p0 = first[blk], p1 = first[blk + 1];
     uint32_t pair = 4;  // qubits 0 and 1
     QuadRows q = quad_rows(pair, z);
-    cpx<R> v[4];
+    cpx<double> v[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = mk<R>(quad_row(q, k) == col ? (R)1 : (R)0, (R)0);
+    for (int k = 0; k < 4; ++k) v[k] = mk(quad_row(q, k) == col ? 1.0 : 0.0, 0.0);
     for (int p = p0; p < p1; p += 64) {
         const int cnt = min(64, p1 - p);
         const uint32_t w = lane < cnt ? ops[p + lane] : 0;
@@ -162,7 +169,7 @@ __global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t*
         for (int i = 0; i < cnt; ++i) {
             const uint32_t op = __builtin_amdgcn_readlane(w, i);
             const uint32_t pr = (op >> kQuadPairShift) & 15;
-            cpx<R> k[4];
+            cpx<double> k[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) k[t] = tab[4 * i + t];
             if (pr != pair) {
@@ -184,20 +191,21 @@ __global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t*
                 break;
             case QK_XA: quad_swap(v[2], v[3]); break;
             case QK_XB: quad_swap(v[1], v[3]); break;
-            case QK_Z: v[3] = mk<R>(-v[3].re, -v[3].im); break;
+            case QK_Z: v[3] = mk(-v[3].re, -v[3].im); break;
             case QK_CUA:
                 quad_pair(v[2], v[3], k);
-                if (zero && (int)(op >> kQuadSlotShift) - 1 == dslot) v[0] = v[1] = mk<R>(0, 0);
+                if (zero && (int)(op >> kQuadSlotShift) - 1 == dslot) v[0] = v[1] = mk(0.0, 0.0);
                 break;
             default:  // QK_CUB
                 quad_pair(v[1], v[3], k);
-                if (zero && (int)(op >> kQuadSlotShift) - 1 == dslot) v[0] = v[2] = mk<R>(0, 0);
+                if (zero && (int)(op >> kQuadSlotShift) - 1 == dslot) v[0] = v[2] = mk(0.0, 0.0);
                 break;
             }
         }
     }
     cpx<R>* o = out + (DERIV ? (long long)e : (long long)e * nb + blk) * 256;  // [row][col]
-    quad_store(v, q, col, o);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[quad_row(q, k) * 16 + col] = cvt<R>(v[k]);
 }
 
 // Sums the workgroup partials of the block's correlation M_b (SPLIT: a workgroup per (block,
@@ -217,7 +225,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
                                                           const int* __restrict__ count) {
     constexpr int E = SPLIT ? 1 : 4;  // elements per workgroup
     __shared__ double sums[SPLIT ? 8 : 4][512];  // 256 real, then 256 imaginary parts
-    __shared__ cpx<R> states[E][512], tables[E][64 * 4];
+    __shared__ cpx<double> states[E][512], tables[E][64 * 4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int blk = blockIdx.x % nb, e = (blockIdx.x / nb) * E + (SPLIT ? 0 : wave);
     if (count) B = min(*count, B);
@@ -240,18 +248,18 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
         quad_fence();
     }
     const int col = lane & 15, z = lane >> 4;
-    cpx<R>* sx = states[SPLIT ? 0 : wave];
-    cpx<R>* sy = sx + 256;
-    cpx<R>* tab = tables[SPLIT ? 0 : wave];
+    cpx<double>* sx = states[SPLIT ? 0 : wave];
+    cpx<double>* sy = sx + 256;
+    cpx<double>* tab = tables[SPLIT ? 0 : wave];
     const cpx<R>* Fb = F + ((long long)e * nb + blk) * 256;
     const int p0 = first[blk], p1 = first[blk + 1];
     uint32_t pair = 4;
     QuadRows q = quad_rows(pair, z);
-    cpx<R> x[4], y[4];
+    cpx<double> x[4], y[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const int at = quad_row(q, k) * 16 + col;
-        x[k] = Fb[at];
+        x[k] = widen(Fb[at]);
         const double* sw = sums[SPLIT ? 0 : wave];
         double yr = sw[at], yi = sw[256 + at];
         if constexpr (SPLIT) {
@@ -261,7 +269,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
                 yi += sums[w][256 + at];
             }
         }
-        y[k] = mk<R>((R)yr, (R)yi);
+        y[k] = mk(yr, yi);
     }
     for (int pe = p1; pe > p0; pe -= 64) {
         const int p = max(p0, pe - 64), cnt = pe - p;
@@ -273,7 +281,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
         for (int i = cnt - 1; i >= 0; --i) {
             const uint32_t op = __builtin_amdgcn_readlane(w, i);
             const uint32_t pr = (op >> kQuadPairShift) & 15;
-            cpx<R> k[4];
+            cpx<double> k[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) k[t] = tab[4 * i + t];
             if (pr != pair) {
@@ -286,10 +294,10 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
                 quad_load(y, q, col, sy);
                 quad_fence();
             }
-            const cpx<R> kd[4] = {mk(k[0].re, -k[0].im), mk(k[2].re, -k[2].im), mk(k[1].re, -k[1].im),
+            const cpx<double> kd[4] = {mk(k[0].re, -k[0].im), mk(k[2].re, -k[2].im), mk(k[1].re, -k[1].im),
                                   mk(k[3].re, -k[3].im)};
-            const cpx<R> kt[4] = {k[0], k[2], k[1], k[3]};
-            cpx<R> acc[4] = {mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0), mk<R>(0, 0)};
+            const cpx<double> kt[4] = {k[0], k[2], k[1], k[3]};
+            cpx<double> acc[4] = {mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0)};
             // CNOT and CZ are their own adjoint and transpose
             switch (op & 15) {
             case QK_UA:
@@ -311,15 +319,15 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
                 quad_swap(y[1], y[3]);
                 continue;
             default:  // QK_Z
-                x[3] = mk<R>(-x[3].re, -x[3].im);
-                y[3] = mk<R>(-y[3].re, -y[3].im);
+                x[3] = mk(-x[3].re, -x[3].im);
+                y[3] = mk(-y[3].re, -y[3].im);
                 continue;
             }
             double r[8], lo, hi;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                r[2 * t] = (double)acc[t].re;
-                r[2 * t + 1] = (double)acc[t].im;
+                r[2 * t] = acc[t].re;
+                r[2 * t + 1] = acc[t].im;
             }
             wave_sum8(r, lo, hi);
             if (col == 0) {

@@ -312,8 +312,7 @@ class Context:
     def set_fused_cost(self, mode=True):
         """Batched evaluations through the fused 4-qubit blocks on the matrix cores
         (4-10 qubits, costs without correction channels): True / False, or "auto" (the
-        default: costs from 7 qubits, or from 5 without specialised kernels; costs with
-        gradients from 6 qubits)."""
+        default: where it measured faster than the register-tile kernels in use)."""
         m = FUSED_COST_AUTO if mode == "auto" else (FUSED_COST_ON if mode else FUSED_COST_OFF)
         self.check(self._L.sqh_set_fused_cost(self.h, m))
 

@@ -1,0 +1,52 @@
+"""The automatic choice between the fused blocks and the register-tile kernels: on both
+sides of every line of the rule (qubits 4 to 10, deep and shallow circuits) costs,
+gradients and apply_to agree with the forced paths to rounding, strided rows included,
+and do not depend on the batch a vector comes in by more."""
+import numpy as np
+import pytest
+import torch
+
+from squander_hip import _native as nat
+from squander_hip import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def _evaluate(ctx, ps, M, stride, mode):
+    ctx.set_fused_cost(mode)
+    B, P = ps.shape
+    c, f, g = np.empty(B), np.empty(B), np.empty((B, P))
+    ctx.check(ctx._L.sqh_optimization_problem_batch(ctx.h, ps.ctypes.data, B, nat.PREC_F64, c.ctypes.data))
+    ctx.check(ctx._L.sqh_optimization_problem_combined_batch(ctx.h, ps.ctypes.data, B, nat.PREC_F64, f.ctypes.data,
+                                                             g.ctypes.data))
+    dp, dM = torch.from_numpy(ps).cuda(), torch.from_numpy(M).cuda()
+    torch.cuda.synchronize()
+    d, cols = M.shape[1], M.shape[2] - stride
+    ctx.check(ctx._L.sqh_apply_to_dev(ctx.h, dp.data_ptr(), P, dM.data_ptr(), d, cols, M.shape[2], d * M.shape[2], B, 0))
+    ctx.synchronize()
+    return c, f, g, dM.cpu().numpy()
+
+
+@pytest.mark.parametrize("n", [4, 5, 6, 8, 10])
+@pytest.mark.parametrize("layers", [0, 1, 3, 14])
+def test_automatic_equals_both_paths(n, layers):
+    print(n, layers, flush=True)
+    gates = W.ansatz_layers(n, W.alternating_pairs(n, layers))
+    d, P, B, cols, pad = 1 << n, W.param_count(gates), 3, (1 << n) - 3, 2
+    rng = np.random.default_rng(n)
+    U = W.haar_unitary(d, 3)[:, :cols].copy()
+    ps = W.random_params(P, 4, batch=B)
+    M = rng.standard_normal((B, d, cols + pad)) + 1j * rng.standard_normal((B, d, cols + pad))
+    ctx = nat.Context(0)
+    ctx.set_circuit(n, gates)
+    ctx.set_target(U)
+    ctx.set_trace_offset(2)
+    c, f, g, R = _evaluate(ctx, ps, M, pad, "auto")
+    for mode in (True, False):
+        c2, f2, g2, R2 = _evaluate(ctx, ps, M, pad, mode)
+        assert np.abs(c - c2).max() < 1e-12 and np.abs(f - f2).max() < 1e-12
+        assert np.abs(g - g2).max() < 1e-12
+        assert np.linalg.norm(R - R2) <= 1e-12 * np.linalg.norm(R)
+        assert np.array_equal(R2[:, :, cols:], M[:, :, cols:])
+    one = _evaluate(ctx, ps[1:2].copy(), M[1:2].copy(), pad, "auto")
+    assert abs(one[0][0] - c[1]) < 1e-12 and np.abs(one[2][0] - g[1]).max() < 1e-12
