@@ -217,6 +217,35 @@ std::vector<int> fused_lane_tabs(int N, const FusionPlan& fp) {
     return tabs;
 }
 
+// Lane tables of the store pass with whole columns in LDS (BT_*, sqh_kernels.h).
+std::vector<int> fused_big_tabs(int N, const FusionPlan& fp) {
+    const int nb = (int)fp.qubits.size();
+    std::vector<int> tabs((size_t)nb * kBigTab, 0);
+    for (int b = 0; b < nb; ++b) {
+        int* t = tabs.data() + (size_t)b * kBigTab;
+        const auto& q = fp.qubits[b];
+        int outer[16], no = 0;
+        for (int k = 0; k < N; ++k)
+            if (k != q[0] && k != q[1] && k != q[2] && k != q[3]) outer[no++] = k;
+        auto group = [&](int o) {
+            int r = 0;
+            for (int k = 0; k < no; ++k)
+                if ((o >> k) & 1) r |= 1 << outer[k];
+            return r;
+        };
+        auto local = [&](int i) {
+            int r = 0;
+            for (int k = 0; k < 4; ++k)
+                if ((i >> k) & 1) r |= 1 << q[k];
+            return r;
+        };
+        for (int l = 0; l < 64; ++l) t[BT_LANE + l] = fused_big_slot(group(l & 15) | local(l >> 4));
+        for (int s = 0; s < 4; ++s) t[BT_S + s] = fused_big_slot(local(4 * s));
+        for (int o = 0; o < (1 << (N - 8)); ++o) t[BT_T + o] = fused_big_slot(group(16 * o));
+    }
+    return tabs;
+}
+
 // The circuit fuses into 4-qubit blocks the fused kernels take (4 to 10 qubits).
 bool fused_plan_fits(const sqh_ctx* c) {
     const int N = c->prog.N;
@@ -448,6 +477,34 @@ int fused_apply(sqh_ctx* c, void* mats, int rows, int cols, int stride, long lon
     return SQH_OK;
 }
 
+// apply_to through the blocks with whole columns in LDS (fused_big_fits): matrix b of rows x
+// cols from in + b * in_bstride (0: the same input) to out + b * out_bstride; in place when
+// they are the same.
+int fused_big_apply(sqh_ctx* c, const void* in, int in_stride, long long in_bstride, void* out, int out_stride,
+                    long long out_bstride, int cols, int B, bool f32, const double* d_params, int pbstride) {
+    const FusionPlan& fp = c->fplan;
+    const int nb = (int)fp.qubits.size(), Bk = pbstride ? B : 1;
+    HIPTRY(c, c->d_fused.ensure((size_t)Bk * nb * 256 * (f32 ? 8 : 16)));
+    HIPTRY(c, launch_fuse_blocks(f32, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb,
+                                 gate_kernels(c, d_params, pbstride), Bk, c->d_fused.p, c->stream));
+    FusedCostArgs a;
+    a.U = in;
+    a.in_stride = in_stride;
+    a.in_bstride = in_bstride;
+    a.m = cols;
+    a.B = B;
+    a.nb = nb;
+    a.F = c->d_fused.p;
+    a.F_bstride = Bk > 1 ? (long long)nb * 256 : 0;
+    a.tabs = c->d_ftabs.as<int>();
+    a.out = out;
+    a.out_stride = out_stride;
+    a.out_bstride = out_bstride;
+    TimedLaunch tl(c);
+    HIPTRY(c, launch_fused_big(f32, c->prog.N, a, c->stream));
+    return SQH_OK;
+}
+
 void eval_scratch_bytes(sqh_ctx* c, int B, bool f32, bool grad, size_t bytes[4]) {
     const int N = c->prog.N, m = c->cols, ns = std::max((int)c->prog.slots.size(), 1);
     const TraceSpec ts = trace_spec(c, B, m);
@@ -575,12 +632,17 @@ int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double*
         return SQH_OK;
     }
     if (d_grad) return fail(c, SQH_ERR_ARG, "gradient evaluation supports up to %d qubits", kMaxTileQubits);
-    // Streaming path: B copies of the target, one pass per gate, then the diagonal.
+    // B copies of the target through the blocks (above 13 qubits, 14 in complex64, a pass over
+    // HBM per block), then the diagonal.
     const size_t esz = f32 ? 8 : 16;
     const long long msz = (long long)c->rows * m;
     HIPTRY(c, c->d_mat.ensure((size_t)B * msz * esz));
-    HIPTRY(c, launch_broadcast_copy(f32, U, c->rows, m, m, c->d_mat.p, msz, B, c->stream));
-    if ((rc = fused_apply(c, c->d_mat.p, c->rows, m, m, msz, B, f32, d_params, c->prog.P))) return rc;
+    if (fused_big_fits(f32, N) && !c->fplan.qubits.empty()) {
+        if ((rc = fused_big_apply(c, U, m, 0, c->d_mat.p, m, msz, m, B, f32, d_params, c->prog.P))) return rc;
+    } else {
+        HIPTRY(c, launch_broadcast_copy(f32, U, c->rows, m, m, c->d_mat.p, msz, B, c->stream));
+        if ((rc = fused_apply(c, c->d_mat.p, c->rows, m, m, msz, B, f32, d_params, c->prog.P))) return rc;
+    }
     HIPTRY(c, launch_extract_diag(f32, c->d_mat.p, msz, m, m, B, off, c->d_diag.as<double>(), N, ts, c->stream));
     HIPTRY(c, launch_finish(c->d_diag.as<double>(), m, B, c->variant, d_costs, nullptr, 0, ns, c->d_slots.as<Slot>(),
                             d_params, c->prog.P, nullptr, c->stream, BatchIndex(), ts));
@@ -643,6 +705,8 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
     const int ns = (int)c->prog.slots.size();
     const int Bk = pbstride ? B : 1;
     const long long kb = pbstride ? (long long)ns * 4 : 0;
+    if (path == 0 && fused_big_fits(f32, N) && !c->fplan.qubits.empty())
+        return fused_big_apply(c, d_inout, stride, bstride, d_inout, stride, bstride, cols, B, f32, d_params, pbstride);
     if (path == 0 && N > kMaxTileQubits) path = 2;
     if (path == 2) return fused_apply(c, d_inout, rows, cols, stride, bstride, B, f32, d_params, pbstride);
     const bool fused = path == 0 && fused_pass_applies(c, true);
@@ -878,6 +942,11 @@ int sqh_set_circuit(sqh_ctx* c, int qbit_num, const sqh_gate* gates, int n_gates
         const std::vector<int> tmaps = fused_trace_maps(qbit_num, fp);
         HIPTRY(c, c->d_tmaps.ensure(tmaps.size() * sizeof(int)));
         HIPTRY(c, hipMemcpy(c->d_tmaps.p, tmaps.data(), tmaps.size() * sizeof(int), hipMemcpyHostToDevice));
+    }
+    if (fused_big_fits(true, qbit_num) && fp.k == 4 && !fp.qubits.empty()) {
+        const std::vector<int> tabs = fused_big_tabs(qbit_num, fp);
+        HIPTRY(c, c->d_ftabs.ensure(tabs.size() * sizeof(int)));
+        HIPTRY(c, hipMemcpy(c->d_ftabs.p, tabs.data(), tabs.size() * sizeof(int), hipMemcpyHostToDevice));
     }
     c->fplan = std::move(fp);
     c->fused_tuned.clear();

@@ -191,6 +191,15 @@ hipError_t launch_fused_block_corr(bool f32, const uint32_t* ops, const int* fir
                                    const void* F, const double* mpart, int wgs, int B, double* corr, int ns,
                                    hipStream_t s, const int* count = nullptr);
 
+// The store pass above kFusedCostMaxQubits with whole columns in a workgroup's LDS
+// (sqh_k_fused_big.hip): up to 13 qubits in complex128, 14 in complex64.  a.tabs: kBigTab
+// ints per block, the slot of row 4 s + g of group 16 tile + nl being the XOR of
+// BT_LANE[nl + 16 g], BT_S[s] and BT_T[tile].  May run in place.
+constexpr int BT_LANE = 0, BT_S = 64, BT_T = 68, kBigTab = 132;
+int fused_big_slot(int row);
+bool fused_big_fits(bool f32, int N);
+hipError_t launch_fused_big(bool f32, int N, const FusedCostArgs& a, hipStream_t s);
+
 // Launch shape: tiles per wavefront (2 or 4), LDS exchange groups per block (1, or 2
 // with 4 tiles and prefetch), waves per workgroup (1, 2 or 4), next block's matrix
 // prefetched (0 or 1).  Every valid shape gives bit-identical results.
