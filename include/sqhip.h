@@ -113,8 +113,8 @@ int sqh_apply_to(sqh_ctx* ctx, const void* params, void* inout, int rows, int co
  * kernels, or -- where sqh_set_fused_cost selects it (by default from 7 qubits) -- the
  * tile-resident pass of the circuit's fused 4-qubit blocks on the matrix cores, which
  * writes each column back to where it read it; above 10 qubits the same pass with
- * whole columns in a workgroup's LDS (to 13 qubits, 14 in complex64), then the fused
- * streaming path. */
+ * whole columns in a workgroup's LDS (to 13 qubits, 14 in complex64) where that is the
+ * faster way, else the fused streaming path. */
 int sqh_apply_to_dev(sqh_ctx* ctx, const double* d_params, int pbstride, void* d_inout, int rows, int cols,
                      int stride, long long bstride, int B, int is_f32);
 /* The same result computed by one streaming HBM pass per gate (the unfused path). */

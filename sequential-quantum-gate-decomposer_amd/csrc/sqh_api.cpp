@@ -477,7 +477,22 @@ int fused_apply(sqh_ctx* c, void* mats, int rows, int cols, int stride, long lon
     return SQH_OK;
 }
 
-// apply_to through the blocks with whole columns in LDS (fused_big_fits): matrix b of rows x
+// Whether the store pass with whole columns in LDS runs B matrices of m columns: it fits, and
+// it is not where a pass per block measured faster on MI355X.  Those are shallow circuits
+// (fewer than 6 blocks) on a few matrices of 4 or more columns (0.64 - 1.1 times; a
+// streamed block is then little more than its launch) and columns of 128 KiB, one workgroup
+// per CU, when there are fewer than 64 (0.85 - 1.1).  Elsewhere 1.0 - 3 times, and 2.7 - 11
+// for many matrices of one column.
+bool fused_big_applies(const sqh_ctx* c, bool f32, int m, int B) {
+    const int N = c->prog.N;
+    if (!fused_big_fits(f32, N) || c->fplan.k != 4 || c->fplan.qubits.empty()) return false;
+    const long long columns = (long long)B * m;
+    if (columns >= 512) return true;
+    const bool enough = ((size_t)(f32 ? 8 : 16) << N) <= 65536 || columns >= 64;
+    return c->fplan.qubits.size() >= 6 ? m < 4 || enough : m < 4 && enough;
+}
+
+// apply_to through the blocks with whole columns in LDS (fused_big_applies): matrix b of rows x
 // cols from in + b * in_bstride (0: the same input) to out + b * out_bstride; in place when
 // they are the same.
 int fused_big_apply(sqh_ctx* c, const void* in, int in_stride, long long in_bstride, void* out, int out_stride,
@@ -637,7 +652,7 @@ int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double*
     const size_t esz = f32 ? 8 : 16;
     const long long msz = (long long)c->rows * m;
     HIPTRY(c, c->d_mat.ensure((size_t)B * msz * esz));
-    if (fused_big_fits(f32, N) && !c->fplan.qubits.empty()) {
+    if (fused_big_applies(c, f32, m, B)) {
         if ((rc = fused_big_apply(c, U, m, 0, c->d_mat.p, m, msz, m, B, f32, d_params, c->prog.P))) return rc;
     } else {
         HIPTRY(c, launch_broadcast_copy(f32, U, c->rows, m, m, c->d_mat.p, msz, B, c->stream));
@@ -705,7 +720,7 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
     const int ns = (int)c->prog.slots.size();
     const int Bk = pbstride ? B : 1;
     const long long kb = pbstride ? (long long)ns * 4 : 0;
-    if (path == 0 && fused_big_fits(f32, N) && !c->fplan.qubits.empty())
+    if (path == 0 && fused_big_applies(c, f32, cols, B))
         return fused_big_apply(c, d_inout, stride, bstride, d_inout, stride, bstride, cols, B, f32, d_params, pbstride);
     if (path == 0 && N > kMaxTileQubits) path = 2;
     if (path == 2) return fused_apply(c, d_inout, rows, cols, stride, bstride, B, f32, d_params, pbstride);

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n,f32", [(11, False), (11, True), (12, False), (12, True), (13, False), (13, True),
                                    (14, True)])
-@pytest.mark.parametrize("cols,pad,B", [(1, 0, 1), (3, 2, 2), (17, 0, 3)])
+@pytest.mark.parametrize("cols,pad,B", [(1, 0, 1), (3, 2, 2), (17, 0, 4)])
 def test_big_store_pass(n, f32, cols, pad, B):
     print(n, f32, cols, pad, B, flush=True)
     gates = np.concatenate([W.mixed_gate_circuit(n, 40, n), [[nat.GATE_CNOT, 0, n - 1, 0]]]).astype(np.int32)
