@@ -29,6 +29,8 @@ hipError_t launch_bfgs_advance(void* st, double* vecs, double* Z, const double* 
                                int* lists, int* counts, const int* run_group, const BfgsOpts& o, int B,
                                hipStream_t s);
 size_t bfgs_state_bytes();
+hipError_t launch_bfgs_collect(const void* st, const double* vecs, int B, int Ps, double* x, RunResult* res,
+                               hipStream_t s);
 int bfgs_max_params();
 
 namespace {
@@ -61,17 +63,27 @@ struct Group {
     }
 };
 
-struct BatchBufs {
-    DevBuf run_target, run_group, run_P, run_prog, x0, states, vecs, Z, fe, ge, xt, lists, counts, jitter;
-    ~BatchBufs() {
-        for (DevBuf* b : {&run_target, &run_group, &run_P, &run_prog, &x0, &states, &vecs, &Z, &fe, &ge, &xt, &lists,
-                          &counts, &jitter})
-            b->release();
+// Gives the call's buffers back when it ends: the context keeps them for the next call
+// after a call that went through and used no more than kRunBufsKept, else they are freed
+// (which also waits for whatever a failed call left running).
+struct RunBufsGuard {
+    sqh_ctx* c;
+    Group* g;  // single circuit: the group that borrows the kept target buffers (or null)
+    bool done = false;
+    RunBufsGuard(sqh_ctx* ctx, Group* grp) : c(ctx), g(grp) { lend(); }
+    ~RunBufsGuard() {
+        lend();
+        if (!done || c->run.bytes() > kRunBufsKept) c->run.release();
+    }
+    void lend() {
+        if (!g) return;
+        std::swap(g->tgt64, c->run.tgt64);
+        std::swap(g->tgt32, c->run.tgt32);
     }
 };
 
 // The evaluation launch of group g in precision p (f32 when p == 1).
-TileLaunch group_launch(sqh_ctx* c, BatchBufs& bb, Group& gr, int g, int p, int B, bool grouped) {
+TileLaunch group_launch(sqh_ctx* c, RunBufs& bb, Group& gr, int g, int p, int B, bool grouped) {
     const bool f32 = p == 1;
     TileLaunch t;
     t.N = gr.N;
@@ -106,7 +118,7 @@ TileLaunch group_launch(sqh_ctx* c, BatchBufs& bb, Group& gr, int g, int p, int 
 // several qubit-count groups the groups' evaluation chains are independent (disjoint
 // runs, their own scratch), so the round forks them onto side streams after the
 // advance and joins them before the next round's advance.
-int enqueue_round(sqh_ctx* c, BatchBufs& bb, std::vector<Group>& groups, const BfgsOpts& o, int B, bool mixed,
+int enqueue_round(sqh_ctx* c, RunBufs& bb, std::vector<Group>& groups, const BfgsOpts& o, int B, bool mixed,
                   bool grouped) {
     const int G = (int)groups.size();
     HIPTRY(c, launch_bfgs_reset_counts(bb.counts.as<int>(), G, c->stream));
@@ -193,7 +205,7 @@ const char* persistent_blocker(sqh_ctx* c, const std::vector<Group>& groups, int
 // groups keeps the streams within the hardware queues a process gets by default (four,
 // one taken by the default stream), where launches on a shared queue would run one
 // after the other.
-int solve_persistent(sqh_ctx* c, std::vector<Group>& groups, BatchBufs& bb, const BfgsOpts& o, int B,
+int solve_persistent(sqh_ctx* c, std::vector<Group>& groups, RunBufs& bb, const BfgsOpts& o, int B,
                      const int* run_group, bool grouped, long long max_evals) {
     const int G = (int)groups.size();
     std::vector<std::vector<int>> queue(G);
@@ -255,7 +267,7 @@ int solve_persistent(sqh_ctx* c, std::vector<Group>& groups, BatchBufs& bb, cons
                 flat_n.push_back(groups[g].N);
             }
     }
-    DevBuf d_queue, d_queue_n, d_next;
+    DevBuf &d_queue = bb.queue, &d_queue_n = bb.queue_n, &d_next = bb.next;
     HIPTRY(c, d_queue.ensure(std::max<size_t>(flat.size(), 1) * sizeof(int)));
     HIPTRY(c, d_queue_n.ensure(std::max<size_t>(flat.size(), 1) * sizeof(int)));
     HIPTRY(c, d_next.ensure((size_t)std::max(U, 1) * sizeof(int)));
@@ -321,23 +333,23 @@ int jitter_count(const sqh_decompose_options* opts) {
 
 // Reads the runs' results back.  rounds < 0: report the largest evaluation count of a
 // run (the persistent solver has no lockstep rounds).
-int collect(sqh_ctx* c, BatchBufs& bb, int B, int Ps, double* x_out, int x_stride, double* f_out, int* status_out,
-            long long* evals_out, long long* rounds_out, long long rounds) {
-    std::vector<char> st((size_t)B * bfgs_state_bytes());
-    HIPTRY(c, hipMemcpy(st.data(), bb.states.p, st.size(), hipMemcpyDeviceToHost));
-    std::vector<double> vecs((size_t)B * RV_COUNT * Ps);
-    HIPTRY(c, hipMemcpy(vecs.data(), bb.vecs.p, vecs.size() * sizeof(double), hipMemcpyDeviceToHost));
+int collect(sqh_ctx* c, RunBufs& bb, int B, int Ps, double* x_out, double* f_out, int* status_out, long long* evals_out,
+            long long* rounds_out, long long rounds) {
+    // packed on the device: the whole states and vectors are ten times as much to copy
+    const size_t xb = (size_t)B * Ps * sizeof(double);
+    HIPTRY(c, bb.out.ensure(xb + (size_t)B * sizeof(RunResult)));
+    RunResult* d_res = reinterpret_cast<RunResult*>(bb.out.as<char>() + xb);
+    HIPTRY(c, launch_bfgs_collect(bb.states.p, bb.vecs.as<double>(), B, Ps, bb.out.as<double>(), d_res, c->stream));
+    std::vector<RunResult> res(B);
+    HIPTRY(c, hipMemcpyAsync(x_out, bb.out.p, xb, hipMemcpyDeviceToHost, c->stream));
+    HIPTRY(c, hipMemcpyAsync(res.data(), d_res, res.size() * sizeof(RunResult), hipMemcpyDeviceToHost, c->stream));
+    HIPTRY(c, hipStreamSynchronize(c->stream));
     long long most = 0;
     for (int r = 0; r < B; ++r) {
-        RunState S;
-        std::memcpy(&S, st.data() + (size_t)r * bfgs_state_bytes(), sizeof(RunState));
-        std::memcpy(x_out + (size_t)r * x_stride, vecs.data() + ((size_t)r * RV_COUNT + RV_BEST) * Ps,
-                    (size_t)S.P * sizeof(double));
-        f_out[r] = S.cur_min;
-        const long long ev = S.total_calls + (S.finished ? 0 : S.calls);
-        if (status_out) status_out[r] = S.finished ? S.status : -1;
-        if (evals_out) evals_out[r] = ev;
-        most = std::max(most, ev);
+        f_out[r] = res[r].f;
+        if (status_out) status_out[r] = res[r].status;
+        if (evals_out) evals_out[r] = res[r].evals;
+        most = std::max(most, res[r].evals);
     }
     if (rounds_out) *rounds_out = rounds >= 0 ? rounds : most;
     return SQH_OK;
@@ -350,12 +362,29 @@ int collect(sqh_ctx* c, BatchBufs& bb, int B, int Ps, double* x_out, int x_strid
 // rows of stride Ps.
 int run_batch(sqh_ctx* c, std::vector<Group>& groups, int B, int Ps, const int* run_target, const int* run_P,
               const int* run_group, const double* x0, const std::vector<double>& jitter,
-              const sqh_decompose_options* opts, double* x_out, int x_stride, double* f_out, int* status_out,
+              const sqh_decompose_options* opts, double* x_out, double* f_out, int* status_out,
               long long* evals_out, long long* rounds_out) {
     const bool grouped = run_group != nullptr;
     const bool mixed = opts->mixed_precision != 0;
     const int G = (int)groups.size();
+    const long long max_rounds =
+        opts->max_rounds > 0 ? opts->max_rounds
+                             : (long long)opts->max_outer_iterations * loops_of(opts) *
+                                   (opts->max_inner_iterations + 2) * (mixed ? 2 : 1);
+    const char* blocker = persistent_blocker(c, groups, Ps, max_rounds);
+    if (opts->engine == SQH_ENGINE_PERSISTENT && *blocker)
+        return fail(c, SQH_ERR_ARG, "persistent solver unavailable: %s", blocker);
+    // Automatic choice: the persistent solver where it measured faster than the lockstep
+    // rounds (every run on at most kSolveAutoQubits qubits; at 6 qubits with four
+    // wavefronts per run, one per column slab), and where it applies (no correction
+    // channels, the LDS a workgroup may allocate).
+    bool auto_persistent = true;
+    for (const Group& g : groups) auto_persistent = auto_persistent && g.N <= kSolveAutoQubits;
+    const bool persistent = opts->engine == SQH_ENGINE_PERSISTENT ||
+                            (opts->engine == SQH_ENGINE_AUTO && !*blocker && auto_persistent);
+    // the rounds' own scratch (the persistent solver evaluates in LDS)
     for (Group& g : groups) {
+        if (persistent) break;
         const size_t kern_elems = (size_t)g.B * std::max(g.ns, 1) * 4;
         HIPTRY(c, g.kern64.ensure(kern_elems * 16));
         HIPTRY(c, g.kern32.ensure(kern_elems * 8));
@@ -395,17 +424,19 @@ int run_batch(sqh_ctx* c, std::vector<Group>& groups, int B, int Ps, const int* 
             c->side_ev.push_back(e);
         }
     }
-    BatchBufs bb;
+    RunBufs& bb = c->run;
     HIPTRY(c, bb.run_target.ensure((size_t)B * sizeof(int)));
     HIPTRY(c, bb.x0.ensure((size_t)B * Ps * sizeof(double)));
     HIPTRY(c, bb.states.ensure((size_t)B * bfgs_state_bytes()));
     HIPTRY(c, bb.vecs.ensure((size_t)B * RV_COUNT * Ps * sizeof(double)));
     HIPTRY(c, bb.Z.ensure((size_t)B * Ps * Ps * sizeof(double)));
-    HIPTRY(c, bb.fe.ensure((size_t)B * sizeof(double)));
-    HIPTRY(c, bb.ge.ensure((size_t)B * Ps * sizeof(double)));
-    HIPTRY(c, bb.xt.ensure((size_t)B * Ps * sizeof(double)));
-    HIPTRY(c, bb.lists.ensure((size_t)2 * G * B * sizeof(int)));
-    HIPTRY(c, bb.counts.ensure((size_t)(4 + 2 * G) * sizeof(int)));
+    if (!persistent) {
+        HIPTRY(c, bb.fe.ensure((size_t)B * sizeof(double)));
+        HIPTRY(c, bb.ge.ensure((size_t)B * Ps * sizeof(double)));
+        HIPTRY(c, bb.xt.ensure((size_t)B * Ps * sizeof(double)));
+        HIPTRY(c, bb.lists.ensure((size_t)2 * G * B * sizeof(int)));
+        HIPTRY(c, bb.counts.ensure((size_t)(4 + 2 * G) * sizeof(int)));
+    }
     HIPTRY(c, hipMemcpyAsync(bb.run_target.p, run_target, (size_t)B * sizeof(int), hipMemcpyHostToDevice, c->stream));
     if (grouped) {
         HIPTRY(c, bb.run_group.ensure((size_t)B * sizeof(int)));
@@ -414,9 +445,10 @@ int run_batch(sqh_ctx* c, std::vector<Group>& groups, int B, int Ps, const int* 
         HIPTRY(c, hipMemcpyAsync(bb.run_P.p, run_P, (size_t)B * sizeof(int), hipMemcpyHostToDevice, c->stream));
     }
     HIPTRY(c, hipMemcpyAsync(bb.x0.p, x0, (size_t)B * Ps * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPTRY(c, launch_bfgs_init(bb.states.p, bb.vecs.as<double>(), bb.x0.as<double>(), B, Ps,
-                               grouped ? bb.run_P.as<int>() : nullptr, mixed ? 1 : 0, bb.counts.as<int>(), G,
-                               c->stream));
+    if (!persistent)  // which starts its runs itself
+        HIPTRY(c, launch_bfgs_init(bb.states.p, bb.vecs.as<double>(), bb.x0.as<double>(), B, Ps,
+                                   grouped ? bb.run_P.as<int>() : nullptr, mixed ? 1 : 0, bb.counts.as<int>(), G,
+                                   c->stream));
 
     BfgsOpts o;
     o.max_calls = opts->max_inner_iterations;
@@ -437,27 +469,12 @@ int run_batch(sqh_ctx* c, std::vector<Group>& groups, int B, int Ps, const int* 
         o.jitter = bb.jitter.as<double>();
     }
 
-    const int R = opts->rounds_per_graph > 0 ? opts->rounds_per_graph : 16;
-    const long long max_rounds =
-        opts->max_rounds > 0 ? opts->max_rounds
-                             : (long long)opts->max_outer_iterations * loops_of(opts) *
-                                   (opts->max_inner_iterations + 2) * (mixed ? 2 : 1);
-    const char* blocker = persistent_blocker(c, groups, Ps, max_rounds);
-    if (opts->engine == SQH_ENGINE_PERSISTENT && *blocker)
-        return fail(c, SQH_ERR_ARG, "persistent solver unavailable: %s", blocker);
-    // Automatic choice: the persistent solver where it measured faster than the lockstep
-    // rounds (every run on at most kSolveAutoQubits qubits; at 6 qubits with four
-    // wavefronts per run, one per column slab), and where it applies (no correction
-    // channels, the LDS a workgroup may allocate).
-    bool auto_persistent = true;
-    for (const Group& g : groups) auto_persistent = auto_persistent && g.N <= kSolveAutoQubits;
-    const bool persistent = opts->engine == SQH_ENGINE_PERSISTENT ||
-                            (opts->engine == SQH_ENGINE_AUTO && !*blocker && auto_persistent);
     if (persistent) {
         int rc = solve_persistent(c, groups, bb, o, B, run_group, grouped, max_rounds);
         if (rc) return rc;
-        return collect(c, bb, B, Ps, x_out, x_stride, f_out, status_out, evals_out, rounds_out, -1);
+        return collect(c, bb, B, Ps, x_out, f_out, status_out, evals_out, rounds_out, -1);
     }
+    const int R = opts->rounds_per_graph > 0 ? opts->rounds_per_graph : 16;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     if (!grouped && jit_wants(c, 2)) {
@@ -503,7 +520,7 @@ int run_batch(sqh_ctx* c, std::vector<Group>& groups, int B, int Ps, const int* 
     if (h_counts) (void)hipHostFree(h_counts);
     if (e != hipSuccess) return fail(c, SQH_ERR_DEVICE, "batched optimisation: %s", hipGetErrorString(e));
 
-    return collect(c, bb, B, Ps, x_out, x_stride, f_out, status_out, evals_out, rounds_out, rounds);
+    return collect(c, bb, B, Ps, x_out, f_out, status_out, evals_out, rounds_out, rounds);
 }
 
 int check_opts(sqh_ctx* c, const sqh_decompose_options* opts) {
@@ -521,11 +538,11 @@ void copy_jitter(std::vector<double>& dst, int r, int J, int Ps, const double* s
         std::memcpy(&dst[((size_t)r * J + j) * Ps], src + (size_t)j * P, (size_t)P * sizeof(double));
 }
 
-// Uploads n_targets complex128 targets of a group and their complex64 copies.
-int upload_targets(sqh_ctx* c, Group& g, const double* const* targets) {
+// Uploads n_targets complex128 targets of a group and, for mixed precision, makes their
+// complex64 copies.
+int upload_targets(sqh_ctx* c, Group& g, const double* const* targets, bool mixed) {
     const size_t msz = (size_t)g.rows * g.cols;
     HIPTRY(c, g.tgt64.ensure((size_t)g.n_targets * msz * 16));
-    HIPTRY(c, g.tgt32.ensure((size_t)g.n_targets * msz * 8));
     // targets adjacent in host memory go up in one copy (a batch of single-circuit
     // targets is one copy instead of one per target)
     for (int i = 0; i < g.n_targets;) {
@@ -535,7 +552,10 @@ int upload_targets(sqh_ctx* c, Group& g, const double* const* targets) {
                                  hipMemcpyHostToDevice, c->stream));
         i = j;
     }
-    HIPTRY(c, launch_convert(true, g.tgt64.p, g.tgt32.p, (long long)g.n_targets * msz * 2, c->stream));
+    if (mixed) {
+        HIPTRY(c, g.tgt32.ensure((size_t)g.n_targets * msz * 8));
+        HIPTRY(c, launch_convert(true, g.tgt64.p, g.tgt32.p, (long long)g.n_targets * msz * 2, c->stream));
+    }
     return SQH_OK;
 }
 
@@ -570,6 +590,7 @@ extern "C" int sqh_decompose_batch(sqh_ctx* c, const double* targets, int n_targ
 
     std::vector<Group> groups(1);
     Group& g = groups[0];
+    RunBufsGuard guard(c, &g);
     g.N = N;
     g.rows = rows;
     g.cols = cols;
@@ -586,12 +607,14 @@ extern "C" int sqh_decompose_batch(sqh_ctx* c, const double* targets, int n_targ
     g.slots = pr.slots.empty() ? nullptr : c->d_slots.as<Slot>();
     std::vector<const double*> tp(n_targets);
     for (int i = 0; i < n_targets; ++i) tp[i] = targets + (size_t)i * rows * cols * 2;
-    if ((rc = upload_targets(c, g, tp.data()))) return rc;
+    if ((rc = upload_targets(c, g, tp.data(), opts->mixed_precision != 0))) return rc;
     std::vector<double> jitter;
     if (jitter_count(opts) > 0)
         jitter.assign(opts->restart_jitter, opts->restart_jitter + (size_t)n_runs * jitter_count(opts) * P);
-    return run_batch(c, groups, n_runs, P, run_target, nullptr, nullptr, x0, jitter, opts, x_out, P, f_out,
-                     status_out, evals_out, rounds_out);
+    rc = run_batch(c, groups, n_runs, P, run_target, nullptr, nullptr, x0, jitter, opts, x_out, f_out, status_out,
+                   evals_out, rounds_out);
+    guard.done = rc == SQH_OK;
+    return rc;
 }
 
 extern "C" int sqh_decompose_problems(sqh_ctx* c, const sqh_problem* problems, int n_problems,
@@ -626,6 +649,7 @@ extern "C" int sqh_decompose_problems(sqh_ctx* c, const sqh_problem* problems, i
     }
     HIPTRY(c, hipSetDevice(c->device));
     std::vector<Group> groups(by_n.size());
+    RunBufsGuard guard(c, nullptr);
     std::vector<int> run_target(n_problems), run_group(n_problems), run_P(n_problems);
     std::vector<ProgRef> refs(n_problems);
     std::vector<double> x0((size_t)n_problems * Ps, 0.0);
@@ -690,7 +714,7 @@ extern "C" int sqh_decompose_problems(sqh_ctx* c, const sqh_problem* problems, i
         g.nops = 0;
         g.lays = g.d_lays.as<Layout>();
         g.slots = g.d_slots.as<Slot>();
-        if ((rc = upload_targets(c, g, tp.data()))) return rc;
+        if ((rc = upload_targets(c, g, tp.data(), opts->mixed_precision != 0))) return rc;
         ++gi;
     }
     std::vector<double> jitter;
@@ -710,8 +734,9 @@ extern "C" int sqh_decompose_problems(sqh_ctx* c, const sqh_problem* problems, i
     for (Group& g : groups) g.run_prog = d_refs.as<ProgRef>();
     std::vector<double> xo((size_t)n_problems * Ps);
     rc = run_batch(c, groups, n_problems, Ps, run_target.data(), run_P.data(), run_group.data(), x0.data(), jitter,
-                   opts, xo.data(), Ps, f_out, status_out, evals_out, rounds_out);
+                   opts, xo.data(), f_out, status_out, evals_out, rounds_out);
     if (rc == SQH_OK) {
+        guard.done = true;
         size_t o = 0;
         for (int i = 0; i < n_problems; ++i) {
             std::memcpy(x_out + o, &xo[(size_t)i * Ps], (size_t)run_P[i] * sizeof(double));

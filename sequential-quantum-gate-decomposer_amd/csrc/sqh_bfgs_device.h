@@ -62,6 +62,13 @@ struct alignas(16) RunState {
     double minvec[kMinWindow];
 };
 
+// What a run reports: smallest cost, evaluations, status (-1: unfinished).
+struct RunResult {
+    double f;
+    long long evals;
+    int status, pad;
+};
+
 // Per-run vectors, each P doubles.
 enum RunVec : int { RV_X = 0, RV_G, RV_D, RV_X0, RV_G0, RV_GBEST, RV_ZTG, RV_BEST, RV_DELTA, RV_GAMMA, RV_COUNT };
 

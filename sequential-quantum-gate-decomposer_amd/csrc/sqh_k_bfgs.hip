@@ -84,6 +84,18 @@ __global__ __launch_bounds__(kBfgsThreads) void k_bfgs_advance(RunState* __restr
     if (tid == 0) states[r] = S;
 }
 
+// The results of run blockIdx.x packed for the host: its best point and RunResult.
+__global__ void k_bfgs_collect(const RunState* __restrict__ st, const double* __restrict__ vecs, int Ps,
+                               double* __restrict__ x, RunResult* __restrict__ res) {
+    const int r = blockIdx.x;
+    const double* best = vecs + ((size_t)r * RV_COUNT + RV_BEST) * Ps;
+    for (int k = threadIdx.x; k < Ps; k += blockDim.x) x[(size_t)r * Ps + k] = best[k];
+    if (threadIdx.x == 0) {
+        const RunState& S = st[r];
+        res[r] = {S.cur_min, S.total_calls + (S.finished ? 0 : S.calls), S.finished ? S.status : -1, 0};
+    }
+}
+
 hipError_t launch_bfgs_init(void* st, double* vecs, const double* x0, int B, int Ps, const int* run_P, int mixed,
                             int* counts, int n_groups, hipStream_t s) {
     hipLaunchKernelGGL(k_bfgs_init, dim3(B), dim3(256), 0, s, (RunState*)st, vecs, x0, B, Ps, run_P, mixed, counts,
@@ -102,6 +114,12 @@ hipError_t launch_bfgs_advance(void* st, double* vecs, double* Z, const double* 
     const size_t shm = sizeof(double) * (size_t)o.P * (3 + kBfgsThreads / 64);
     hipLaunchKernelGGL(k_bfgs_advance, dim3(B), dim3(kBfgsThreads), shm, s, (RunState*)st, vecs, Z, fe, ge, xt,
                        lists, counts, run_group, o, B);
+    return hipGetLastError();
+}
+
+hipError_t launch_bfgs_collect(const void* st, const double* vecs, int B, int Ps, double* x, RunResult* res,
+                               hipStream_t s) {
+    hipLaunchKernelGGL(k_bfgs_collect, dim3(B), dim3(64), 0, s, (const RunState*)st, vecs, Ps, x, res);
     return hipGetLastError();
 }
 
