@@ -137,6 +137,8 @@ struct sqh_ctx {
     bool tile_forced = false;
     double tune_ms = 0.0;
 
+    double* h_small = nullptr;  // pinned: parameters and results of small host-array calls (small_host)
+
     sqh::RunBufs run;  // batched optimiser (under mu, as every call)
 
     // Kernel timers: HIP events around the dominant kernel of each call.
@@ -153,6 +155,7 @@ struct sqh_ctx {
                                &d_res, &d_mat, &d_out, &d_quads, &d_ffirst, &d_fused, &d_fmaps, &d_ftabs, &d_dinfo, &d_tmaps, &d_fcorr, &d_idx, &d_seed, &d_dtab, &d_zslot})
             b->release();
         run.release();
+        if (h_small) (void)hipHostFree(h_small);
         for (hipStream_t s : side) (void)hipStreamDestroy(s);
         for (hipEvent_t e : side_ev) (void)hipEventDestroy(e);
         if (stream) (void)hipStreamDestroy(stream);
