@@ -929,6 +929,12 @@ int sqh_set_circuit(sqh_ctx* c, int qbit_num, const sqh_gate* gates, int n_gates
     HIPTRY(c, c->d_ffirst.ensure(fp.first.size() * sizeof(int)));
     if (!fp.quads.empty())
         HIPTRY(c, hipMemcpy(c->d_quads.p, fp.quads.data(), fp.quads.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    const std::vector<uint32_t> sq = quad_program(p);
+    c->n_squads = (int)sq.size();
+    if (!sq.empty()) {
+        HIPTRY(c, c->d_squads.ensure(sq.size() * sizeof(uint32_t)));
+        HIPTRY(c, hipMemcpy(c->d_squads.p, sq.data(), sq.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    }
     HIPTRY(c, hipMemcpy(c->d_ffirst.p, fp.first.data(), fp.first.size() * sizeof(int), hipMemcpyHostToDevice));
     if (qbit_num >= 4 && qbit_num <= kFusedCostMaxQubits && fp.k == 4 && !fp.qubits.empty()) {
         const std::vector<int> maps = fused_row_maps(qbit_num, fp);

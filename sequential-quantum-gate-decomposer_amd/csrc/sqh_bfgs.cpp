@@ -311,6 +311,11 @@ int solve_persistent(sqh_ctx* c, std::vector<Group>& groups, RunBufs& bb, const 
             const int rc = jit_launch_solve(c, a, grid, solve_lds_bytes(groups[g].N, o.P, a.ns_max), st);
             if (rc) return rc;
         } else {
+            // one circuit of 3 or 4 qubits: four rows per lane, where its table fits in LDS
+            if (!grouped && c->n_squads && solve_quad_lds_bytes(o.P, a.ns_max) <= device_max_lds()) {
+                a.quads = c->d_squads.as<uint32_t>();
+                a.nquads = c->n_squads;
+            }
             HIPTRY(c, launch_solve(groups[g].N, a, grid, st));
         }
     }

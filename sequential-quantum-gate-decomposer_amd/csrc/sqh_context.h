@@ -105,6 +105,8 @@ struct sqh_ctx {
     // Dense-block fusion of the circuit for the streaming path.
     sqh::FusionPlan fplan;
     sqh::DevBuf d_quads, d_ffirst, d_fused;
+    sqh::DevBuf d_squads;  // the persistent solver's op words (quad_program; n_squads, 0: none)
+    int n_squads = 0;
     // Row tables of the tile-resident fused-block cost kernel ([blocks][kFusedMapStride];
     // present for 4 <= N <= 10) and its switch (sqh_set_fused_cost).
     sqh::DevBuf d_fmaps;
@@ -152,7 +154,7 @@ struct sqh_ctx {
             (void)hipEventDestroy(e.second);
         }
         for (sqh::DevBuf* b : {&d_ops, &d_lays, &d_slots, &d_U64, &d_U32, &d_params, &d_kern, &d_diag, &d_mpart,
-                               &d_res, &d_mat, &d_out, &d_quads, &d_ffirst, &d_fused, &d_fmaps, &d_ftabs, &d_dinfo, &d_tmaps, &d_fcorr, &d_idx, &d_seed, &d_dtab, &d_zslot})
+                               &d_res, &d_mat, &d_out, &d_quads, &d_squads, &d_ffirst, &d_fused, &d_fmaps, &d_ftabs, &d_dinfo, &d_tmaps, &d_fcorr, &d_idx, &d_seed, &d_dtab, &d_zslot})
             b->release();
         run.release();
         if (h_small) (void)hipHostFree(h_small);

@@ -13,10 +13,34 @@
 #include "sqh_bfgs_core.h"
 #include "sqh_device.h"
 #include "sqh_kernels.h"
+#include "sqh_quads.h"
 #include "sqh_solve.h"
 #include "sqh_solve_loop.h"
 
 namespace sqh {
+
+// The gradient from the correlations and each parameter's derivative kernel; returns the cost.
+__device__ __forceinline__ double wave_gradient(int variant, double tre, double tim, int m,
+                                                const Slot* __restrict__ slots, int ns, const double* xr, double* gr,
+                                                const double* mc) {
+    for (int sl = threadIdx.x; sl < ns; sl += 64) {
+        const Slot s = slots[sl];
+        const double* M = mc + (long long)sl * 8;
+        for (int q = 0; q < s.nparam; ++q) {
+            cpx<double> d[4];
+            dev_deriv_kernel(s.type, xr + s.param_start, q, d);
+            double kre = 0.0, kim = 0.0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                kre += d[e].re * M[2 * e] - d[e].im * M[2 * e + 1];
+                kim += d[e].re * M[2 * e + 1] + d[e].im * M[2 * e];
+            }
+            gr[s.param_start + q] = grad_of(variant, tre, tim, kre, kim, (double)m);
+        }
+    }
+    __syncthreads();
+    return cost_of(variant, tre, tim, (double)m);
+}
 
 // Cost and gradient of one run at xr (LDS) by the wavefront: f returned, gradient to gr
 // (LDS).  kt: LDS table of ns 2x2 kernels (complex128 slots; complex64 uses the first
@@ -144,24 +168,197 @@ __device__ double wave_eval(const cpx<R>* __restrict__ U, int m, int trace_off, 
     tre = wave_sum(tre);
     tim = wave_sum(tim);
     __syncthreads();
-    // gradient from the correlations and each parameter's derivative kernel
-    for (int sl = lane; sl < ns; sl += 64) {
-        const Slot s = slots[sl];
-        const double* M = mc + (long long)sl * 8;
-        for (int q = 0; q < s.nparam; ++q) {
-            cpx<double> d[4];
-            dev_deriv_kernel(s.type, xr + s.param_start, q, d);
-            double kre = 0.0, kim = 0.0;
+    return wave_gradient(variant, tre, tim, m, slots, ns, xr, gr, mc);
+}
+
+// The correlations of a gate on qubit t (control c, or -1) over the columns, each sum in
+// wave_eval's order, so that the line searches see the same bits: lane z of a column takes
+// the z-th of the four entries y_(z >> 1) x_(z & 1) over the pairs of rows in ascending order
+// (the rows come through s), then the columns are added as wave_sum adds them.  Returned in
+// every lane of a row of 16.
+template <typename R>
+__device__ __forceinline__ cpx<double> quad_corr(const cpx<R> (&x)[4], const cpx<R> (&y)[4], const QuadRows& q, int col,
+                                                 int z, int t, int c, cpx<R>* s) {
+    const int ty = (z >> 1) << t, tx = (z & 1) << t;
+    cpx<R> yr[8];
+    quad_store(y, q, col, s);
+    quad_fence();
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                kre += d[e].re * M[2 * e] - d[e].im * M[2 * e + 1];
-                kim += d[e].re * M[2 * e + 1] + d[e].im * M[2 * e];
-            }
-            gr[s.param_start + q] = grad_of(variant, tre, tim, kre, kim, (double)m);
-        }
+    for (int p = 0; p < 8; ++p) yr[p] = s[(((p >> t) << (t + 1)) | (p & ((1 << t) - 1)) | ty) * 16 + col];
+    quad_fence();
+    quad_store(x, q, col, s);
+    quad_fence();
+    cpx<R> acc = mk<R>(0, 0);
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+        const int i = ((p >> t) << (t + 1)) | (p & ((1 << t) - 1));
+        if (c < 0 || ((i >> c) & 1)) cacc(acc, yr[p], s[(i | tx) * 16 + col]);
+    }
+    quad_fence();
+    auto columns = [](double v) {
+        v += dpp_f64<0xb1>(v);   // quad_perm [1,0,3,2]
+        v += dpp_f64<0x4e>(v);   // quad_perm [2,3,0,1]
+        v += dpp_f64<0x141>(v);  // row_half_mirror
+        v += dpp_f64<0x140>(v);  // row_mirror
+        return v;
+    };
+    return mk(columns((double)acc.re), columns((double)acc.im));
+}
+
+// wave_eval on 3 and 4 qubits with four rows per lane (sqh_quads.h): a column per lane, as
+// wave_eval has it, keeps 8 or 16 of the 64 lanes busy and all 16 rows of x and y in
+// registers (one wavefront per SIMD); here a 16 x 16 target takes every lane (8 x 8: 16) and
+// a gate is a quarter of the operations.  The results are wave_eval's to the bit: the first
+// steps of a line search carry a rounding of 1e-15 to 1e-7 in some runs.  Costs of the order:
+eight rows of x and y per lane through LDS at each gate; summed as they lie they took 1.31
+ms where a call takes 1.37 now (2048 runs of 4 qubits, 6 evaluations; a column per lane: 2.33).
+// s: 256 complex entries for the changes of the pair and the correlations.
+template <int N, typename R>
+__device__ double quad_eval(const cpx<R>* __restrict__ U, int m, int trace_off, int variant,
+                            const uint32_t* __restrict__ ops, int nops, const Slot* __restrict__ slots, int ns,
+                            const double* xr, double* gr, cpx<double>* kt_raw, double* mc, cpx<R>* s) {
+    constexpr int D = 1 << N;
+    const int lane = threadIdx.x, col = lane & 15, z = lane >> 4;
+    cpx<R>* kt = reinterpret_cast<cpx<R>*>(kt_raw);
+    for (int sl = lane; sl < ns; sl += 64) {
+        const Slot sd = slots[sl];
+        cpx<double> k[4];
+        dev_gate_kernel(sd.type, xr + sd.param_start, k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kt[4 * sl + e] = cvt<R>(k[e]);
     }
     __syncthreads();
-    return cost_of(variant, tre, tim, (double)m);
+    uint32_t pair = 4;  // qubits 0 and 1
+    QuadRows q = quad_rows(pair, z);
+    cpx<R> x[4], y[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int row = quad_row(q, k);
+        x[k] = row < D && col < m ? U[(long long)row * m + col] : mk<R>(0, 0);
+    }
+    auto move_to = [&](uint32_t pr, bool both) {
+        if (pr == pair) return;
+        const QuadRows n = quad_rows(pr, z);
+        quad_store(x, q, col, s);
+        quad_fence();
+        quad_load(x, n, col, s);
+        quad_fence();
+        if (both) {
+            quad_store(y, q, col, s);
+            quad_fence();
+            quad_load(y, n, col, s);
+            quad_fence();
+        }
+        pair = pr;
+        q = n;
+    };
+    for (int p = 0; p < nops; p += 64) {
+        const int cnt = min(64, nops - p);
+        const uint32_t w = lane < cnt ? ops[p + lane] : 0;
+        for (int i = 0; i < cnt; ++i) {
+            const uint32_t op = __builtin_amdgcn_readlane(w, i);
+            const int slot = (int)(op >> kQuadSlotShift) - 1;
+            cpx<R> k[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) k[t] = slot >= 0 ? kt[4 * slot + t] : mk<R>(0, 0);
+            move_to((op >> kQuadPairShift) & 15, false);
+            switch (op & 15) {
+            case QK_UA:
+                quad_pair(x[0], x[1], k);
+                quad_pair(x[2], x[3], k);
+                break;
+            case QK_UB:
+                quad_pair(x[0], x[2], k);
+                quad_pair(x[1], x[3], k);
+                break;
+            case QK_XA: quad_swap(x[2], x[3]); break;
+            case QK_XB: quad_swap(x[1], x[3]); break;
+            case QK_Z: x[3] = mk(-x[3].re, -x[3].im); break;
+            case QK_CUA: quad_pair(x[2], x[3], k); break;
+            default: quad_pair(x[1], x[3], k); break;  // QK_CUB
+            }
+        }
+    }
+    double tre = 0.0, tim = 0.0;  // this lane's trace entries
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const bool hit = col < m && quad_row(q, k) == col + trace_off;
+        if (hit) {
+            tre += (double)x[k].re;
+            tim += (double)x[k].im;
+        }
+        y[k] = mk<R>(hit ? (R)1 : (R)0, (R)0);
+    }
+    for (int pe = nops; pe > 0; pe -= 64) {
+        const int p = max(0, pe - 64), cnt = pe - p;
+        const uint32_t w = lane < cnt ? ops[p + lane] : 0;
+        for (int i = cnt - 1; i >= 0; --i) {
+            const uint32_t op = __builtin_amdgcn_readlane(w, i);
+            const int slot = (int)(op >> kQuadSlotShift) - 1;
+            cpx<R> k[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) k[t] = slot >= 0 ? kt[4 * slot + t] : mk<R>(0, 0);
+            move_to((op >> kQuadPairShift) & 15, true);
+            const cpx<R> kd[4] = {mk(k[0].re, -k[0].im), mk(k[2].re, -k[2].im), mk(k[1].re, -k[1].im),
+                                  mk(k[3].re, -k[3].im)};
+            const cpx<R> ktr[4] = {k[0], k[2], k[1], k[3]};
+            // CNOT and CZ are their own adjoint and transpose
+            const uint32_t kind = op & 15;
+            switch (kind) {
+            case QK_UA:
+                quad_pair(x[0], x[1], kd);
+                quad_pair(x[2], x[3], kd);
+                break;
+            case QK_UB:
+                quad_pair(x[0], x[2], kd);
+                quad_pair(x[1], x[3], kd);
+                break;
+            case QK_CUA: quad_pair(x[2], x[3], kd); break;
+            case QK_CUB: quad_pair(x[1], x[3], kd); break;
+            case QK_XA:
+                quad_swap(x[2], x[3]);
+                quad_swap(y[2], y[3]);
+                continue;
+            case QK_XB:
+                quad_swap(x[1], x[3]);
+                quad_swap(y[1], y[3]);
+                continue;
+            default:  // QK_Z
+                x[3] = mk(-x[3].re, -x[3].im);
+                y[3] = mk(-y[3].re, -y[3].im);
+                continue;
+            }
+            const bool on_a = kind == QK_UA || kind == QK_CUA, ctl = kind == QK_CUA || kind == QK_CUB;
+            const int qa = pair & 3, qb = pair >> 2;
+            const cpx<double> sum = quad_corr(x, y, q, col, z, on_a ? qa : qb, ctl ? (on_a ? qb : qa) : -1, s);
+            if (col == 0) {  // every slot has one gate
+                mc[8 * slot + 2 * z] = sum.re;
+                mc[8 * slot + 2 * z + 1] = sum.im;
+            }
+            switch (kind) {
+            case QK_UA:
+                quad_pair(y[0], y[1], ktr);
+                quad_pair(y[2], y[3], ktr);
+                break;
+            case QK_UB:
+                quad_pair(y[0], y[2], ktr);
+                quad_pair(y[1], y[3], ktr);
+                break;
+            case QK_CUA: quad_pair(y[2], y[3], ktr); break;
+            default: quad_pair(y[1], y[3], ktr); break;  // QK_CUB
+            }
+        }
+    }
+    // a column's entry is in one of its four lanes: to all of them, then as wave_eval adds
+    tre += __shfl_xor(tre, 16, 64);
+    tre += __shfl_xor(tre, 32, 64);
+    tim += __shfl_xor(tim, 16, 64);
+    tim += __shfl_xor(tim, 32, 64);
+    if (z != 0) tre = tim = 0.0;
+    tre = wave_sum(tre);
+    tim = wave_sum(tim);
+    __syncthreads();
+    return wave_gradient(variant, tre, tim, m, slots, ns, xr, gr, mc);
 }
 
 // The wavefront's column slabs through its own LDS buffer in two column groups (half
@@ -400,6 +597,25 @@ __global__ __launch_bounds__(64, (N <= 2) ? 2 : 1) void k_solve(SolveArgs a) {
         });
 }
 
+// Four rows per lane: single-circuit calls on 3 and 4 qubits.
+constexpr int kQuadState = 256;
+
+template <int N>
+__global__ __launch_bounds__(64, 2) void k_solve_quad(SolveArgs a) {
+    const int m = a.m, toff = a.trace_off, var = a.variant, nq = a.nquads;
+    const uint32_t* quads = a.quads;
+    solve_runs<kQuadState>(
+        a,
+        [=](const cpx<double>* U, const Op*, int, const Layout*, const Slot* slots, int ns, const double* xr, double* gr,
+            cpx<double>* kt, double* mc, cpx<double>* lds) {
+            return quad_eval<N, double>(U, m, toff, var, quads, nq, slots, ns, xr, gr, kt, mc, lds);
+        },
+        [=](const cpx<float>* U, const Op*, int, const Layout*, const Slot* slots, int ns, const double* xr, double* gr,
+            cpx<double>* kt, double* mc, cpx<float>* lds) {
+            return quad_eval<N, float>(U, m, toff, var, quads, nq, slots, ns, xr, gr, kt, mc, lds);
+        });
+}
+
 // The runs of several groups of at most five qubits in one launch (one wavefront per
 // run): a combined queue, each run dispatched to its group's code.  Separate launches
 // per group would each need a stream of their own, and a process gets four hardware
@@ -461,7 +677,17 @@ size_t solve_lds_bytes(int N, int Ps, int ns_max) {
            sizeof(double) * (6 + RV_COUNT) * (size_t)Ps + sizeof(double) * 8 + sizeof(RunState);
 }
 
+size_t solve_quad_lds_bytes(int Ps, int ns_max) {
+    return solve_lds_bytes(4, Ps, ns_max) + sizeof(cpx<double>) * (kQuadState - 1);
+}
+
 hipError_t launch_solve(int N, const SolveArgs& a, int grid, hipStream_t s) {
+    if (a.quads) {
+        const size_t shm = solve_quad_lds_bytes(a.o.P, a.ns_max);
+        if (N == 3) hipLaunchKernelGGL(k_solve_quad<3>, dim3(grid), dim3(64), shm, s, a);
+        else hipLaunchKernelGGL(k_solve_quad<4>, dim3(grid), dim3(64), shm, s, a);
+        return hipGetLastError();
+    }
     const size_t shm = solve_lds_bytes(N, a.o.P, a.ns_max);
     switch (N) {
 #define SQH_SOLVE_CASE(n) \

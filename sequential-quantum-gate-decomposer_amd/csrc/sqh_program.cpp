@@ -397,6 +397,40 @@ std::vector<uint32_t> quad_ops(const FusionPlan& fp) {
     return out;
 }
 
+std::vector<uint32_t> quad_program(const Program& pr) {
+    if (pr.N < 3 || pr.N > 4 || pr.layouts.size() != 1) return {};
+    for (int t = 0; t < pr.N; ++t)
+        if (pr.layouts[0].reg_off[1 << t] != 1 << t) return {};
+    std::vector<uint32_t> out;
+    int x = 0, y = 1;  // the pair
+    for (size_t i = 0; i < pr.ops.size(); ++i) {
+        const Op& op = pr.ops[i];
+        if (op.kind == OP_REMAP || op.cmode == CM_LANE) return {};
+        if (op.kind == OP_NOP) continue;
+        const int t = op.t, c = op.cmode == CM_NONE ? -1 : op.c;
+        if ((t != x && t != y) || (c >= 0 && c != x && c != y)) {
+            int other = c;
+            // an uncontrolled gate: with the qubit of the next gate that shares one with it
+            for (size_t j = i + 1; j < pr.ops.size() && other < 0; ++j) {
+                const Op& n = pr.ops[j];
+                if (n.kind == OP_NOP || n.cmode == CM_NONE) continue;
+                if (n.t == t) other = n.c;
+                else if (n.c == t) other = n.t;
+            }
+            if (other < 0) other = t == 0 ? 1 : 0;
+            x = std::min(t, other);
+            y = std::max(t, other);
+        }
+        const bool a = t == x;
+        const uint32_t kind = op.kind == OP_U ? (a ? QK_UA : QK_UB)
+                              : op.kind == OP_X ? (a ? QK_XA : QK_XB)
+                              : op.kind == OP_Z ? QK_Z : (a ? QK_CUA : QK_CUB);
+        const uint32_t slot = op.kind == OP_U || op.kind == OP_CU ? op.idx + 1 : 0;
+        out.push_back(kind | (uint32_t)(x | y << 2) << kQuadPairShift | slot << kQuadSlotShift);
+    }
+    return out;
+}
+
 FusionPlan plan_fusion(int N, const std::vector<GateRec>& gates, const std::vector<int>& gate_slot) {
     FusionPlan fp;
     const int kmax = N < 4 ? N : 4;

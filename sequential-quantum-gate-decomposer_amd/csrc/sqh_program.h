@@ -48,6 +48,10 @@ constexpr int kFuseScheduleMaxQubits = 16;
 // Every qubit keeps its gates' order.
 std::vector<uint32_t> quad_ops(const FusionPlan& fp);
 
+// The op words of a 3- or 4-qubit program (one layout, register bit t = qubit t) in program
+// order, each with the pair it runs on; empty for other programs.
+std::vector<uint32_t> quad_program(const Program& pr);
+
 // gate_slot: the kernel-table index of each parametric gate (Program::gate_slot).
 FusionPlan plan_fusion(int N, const std::vector<GateRec>& gates, const std::vector<int>& gate_slot);
 

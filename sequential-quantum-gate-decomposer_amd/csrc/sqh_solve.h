@@ -24,6 +24,8 @@ struct SolveArgs {
     int ns = 0;
     int ns_max = 1;  // largest slot count of the launch's programs (LDS tables)
     const ProgRef* run_prog = nullptr;
+    const uint32_t* quads = nullptr;  // the one program of 3 or 4 qubits as quad_program words (or null)
+    int nquads = 0;
     const int* run_P = nullptr;       // per-run parameter count (null: o.P)
     // targets: run r reads target run_target[r] (null: 0), rows x m, tgt_stride entries apart
     const int* run_target = nullptr;
@@ -57,6 +59,8 @@ constexpr int kSolveSmallMaxQubits = 5;
 
 #ifndef __HIPCC_RTC__
 size_t solve_lds_bytes(int N, int Ps, int ns_max);
+// The same with four rows per lane (launch_solve with a.quads).
+size_t solve_quad_lds_bytes(int Ps, int ns_max);
 hipError_t launch_solve(int N, const SolveArgs& a, int grid, hipStream_t s);
 hipError_t launch_solve_small(const SolveSmallArgs& s, int grid, size_t shm, hipStream_t st);
 #endif
