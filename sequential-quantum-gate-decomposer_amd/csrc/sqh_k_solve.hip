@@ -210,8 +210,8 @@ __device__ __forceinline__ cpx<double> quad_corr(const cpx<R> (&x)[4], const cpx
 // registers (one wavefront per SIMD); here a 16 x 16 target takes every lane (8 x 8: 16) and
 // a gate is a quarter of the operations.  The results are wave_eval's to the bit: the first
 // steps of a line search carry a rounding of 1e-15 to 1e-7 in some runs.  Costs of the order:
-eight rows of x and y per lane through LDS at each gate; summed as they lie they took 1.31
-ms where a call takes 1.37 now (2048 runs of 4 qubits, 6 evaluations; a column per lane: 2.33).
+// eight rows of x and y per lane through LDS at each gate; summed as they lie they took 1.31
+// ms where a call takes 1.37 now (2048 runs of 4 qubits, 6 evaluations; a column per lane: 2.33).
 // s: 256 complex entries for the changes of the pair and the correlations.
 template <int N, typename R>
 __device__ double quad_eval(const cpx<R>* __restrict__ U, int m, int trace_off, int variant,
