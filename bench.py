@@ -460,7 +460,7 @@ def mlp_train_leg(samples=65536, epochs=4, batch=1024):
     """Training throughput of the warm-start network at its configured size (512 ->
     3 x 1024 GELU -> 168, BF16 weights and activations, FP32 accumulation and master
     weights, Adam) on synthetic inputs and targets: every layer's forward and both
-    backward products run on k_gemm_bf16 (v_mfma_f32_16x16x32_bf16).  Algorithmic
+    backward products run on v_mfma_f32_16x16x32_bf16 (k_mlp_layer, k_mlp_weights).  Algorithmic
     flops per sample and step: 2 * sum(in * out) forward, twice that backward."""
     import numpy as np
     import torch

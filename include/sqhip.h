@@ -110,7 +110,8 @@ int sqh_set_correction_weights(sqh_ctx* ctx, double prev_cost, double scale1, do
 int sqh_apply_to(sqh_ctx* ctx, const void* params, void* inout, int rows, int cols, int stride, int is_f32);
 /* Device variant: B matrices at inout + b*bstride elements, parameters shared
  * (pbstride = 0) or per matrix (pbstride = P).  Up to 10 qubits it runs the register-tile
- * kernels, or -- where sqh_set_fused_cost selects it (by default from 7 qubits) -- the
+ * kernels, or -- where sqh_set_fused_cost selects it (by default where the blocks
+ * do little enough arithmetic beside the gates) -- the
  * tile-resident pass of the circuit's fused 4-qubit blocks on the matrix cores, which
  * writes each column back to where it read it; above 10 qubits the same pass with
  * whole columns in a workgroup's LDS (to 13 qubits, 14 in complex64) where that is the

@@ -10,11 +10,10 @@
 //                                                              (MFMA on transposed tiles)
 //   Y_{b-1} = F_b^T Y_b                                        (MFMA)
 // so that dTr/dtheta = sum_ik (dF_b/dtheta)_ik M_b[i][k] for a parameter of block b.
-// The wavefronts of a workgroup (one batch element) sum their M_b in LDS in a fixed
-// order and write one partial per workgroup and block; k_fused_block_corr then sums the
-// partials and runs the block's gates on 16-dimensional vectors (x from e_k, y from
-// column k of M_b) backwards, producing each gate's 2x2 correlations in the layout of
-// the register-tile adjoint kernel, from which k_finish forms the gradient.
+// A wavefront sums its M_b over its column groups in registers and its own partial slot, so
+// no wavefront waits for another; k_fused_block_corr then sums the partials and runs the
+// block's gates backwards, producing each gate's 2x2 correlations in the layout of the
+// register-tile adjoint kernel, from which k_finish forms the gradient.
 //
 // Layouts follow sqh_k_fused_cost.hip: row j of a column under block b is
 // base_b[o] + off_b[i]; 16x16x4 MFMA operands A[l % 16][l / 16], B[l / 16][l % 16]; the
