@@ -855,6 +855,12 @@ extern "C" {
 
 const char* sqh_version(void) { return "sqhip 0.1 (gfx950)"; }
 
+// Doubles of a host-array call (parameters and results) that go through the context's pinned
+// buffer: k_finish then writes the results where the host reads them, and one wait ends the
+// call.  Two copies to pageable memory, each with its own wait, took 22 us of the 83 (117) us
+// of a 4 (8) qubit cost and gradient.  64 KiB: there the copies cost less than the kernels.
+constexpr size_t kSmallHost = 8192;
+
 int sqh_create(int device, sqh_ctx** out) {
     if (!out) return SQH_ERR_ARG;
     *out = nullptr;
@@ -872,6 +878,11 @@ int sqh_create(int device, sqh_ctx** out) {
     // the allocation-free entry point's scratch address on this device (its failure
     // is reported by that entry point, not here)
     (void)noalloc_scratch_init(device);
+    // without it such calls copy as larger ones do
+    if (hipHostMalloc((void**)&c->h_small, kSmallHost * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        c->h_small = nullptr;
+        (void)hipGetLastError();
+    }
     *out = c;
     return SQH_OK;
 }
@@ -917,29 +928,27 @@ int sqh_set_circuit(sqh_ctx* c, int qbit_num, const sqh_gate* gates, int n_gates
     nop.idx = 0;
     for (auto& o : padded) o = nop;
     std::copy(p.ops.begin(), p.ops.end(), padded.begin() + kOpPad);
-    HIPTRY(c, c->d_ops.ensure(padded.size() * sizeof(Op)));
-    HIPTRY(c, c->d_lays.ensure(p.layouts.size() * sizeof(Layout)));
-    HIPTRY(c, c->d_slots.ensure(std::max<size_t>(p.slots.size(), 1) * sizeof(Slot)));
-    HIPTRY(c, hipMemcpy(c->d_ops.p, padded.data(), padded.size() * sizeof(Op), hipMemcpyHostToDevice));
-    HIPTRY(c, hipMemcpy(c->d_lays.p, p.layouts.data(), p.layouts.size() * sizeof(Layout), hipMemcpyHostToDevice));
-    if (!p.slots.empty())
-        HIPTRY(c, hipMemcpy(c->d_slots.p, p.slots.data(), p.slots.size() * sizeof(Slot), hipMemcpyHostToDevice));
+    // The circuit's tables go up in one allocation and one copy (a copy each took 10 us).
+    std::vector<char> host;
+    std::vector<std::pair<DevTable*, size_t>> tables;
+    auto table = [&](DevTable& t, const auto& v) {
+        const size_t bytes = v.size() * sizeof(v[0]);
+        tables.push_back({&t, host.size()});
+        host.resize(host.size() + (std::max<size_t>(bytes, 1) + 255) / 256 * 256);
+        if (bytes) std::memcpy(host.data() + tables.back().second, v.data(), bytes);
+    };
+    table(c->d_ops, padded);
+    table(c->d_lays, p.layouts);
+    table(c->d_slots, p.slots);
     FusionPlan fp = plan_fusion(qbit_num, g, p.gate_slot);
-    HIPTRY(c, c->d_quads.ensure(std::max<size_t>(fp.quads.size(), 1) * sizeof(uint32_t)));
-    HIPTRY(c, c->d_ffirst.ensure(fp.first.size() * sizeof(int)));
-    if (!fp.quads.empty())
-        HIPTRY(c, hipMemcpy(c->d_quads.p, fp.quads.data(), fp.quads.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    table(c->d_quads, fp.quads);
     const std::vector<uint32_t> sq = quad_program(p);
     c->n_squads = (int)sq.size();
-    if (!sq.empty()) {
-        HIPTRY(c, c->d_squads.ensure(sq.size() * sizeof(uint32_t)));
-        HIPTRY(c, hipMemcpy(c->d_squads.p, sq.data(), sq.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-    }
-    HIPTRY(c, hipMemcpy(c->d_ffirst.p, fp.first.data(), fp.first.size() * sizeof(int), hipMemcpyHostToDevice));
+    table(c->d_squads, sq);
+    table(c->d_ffirst, fp.first);
     if (qbit_num >= 4 && qbit_num <= kFusedCostMaxQubits && fp.k == 4 && !fp.qubits.empty()) {
         const std::vector<int> maps = fused_row_maps(qbit_num, fp);
-        HIPTRY(c, c->d_fmaps.ensure(maps.size() * sizeof(int)));
-        HIPTRY(c, hipMemcpy(c->d_fmaps.p, maps.data(), maps.size() * sizeof(int), hipMemcpyHostToDevice));
+        table(c->d_fmaps, maps);
         // per parameter: its gate's block, slot, which of the gate's parameters it is, and
         // whether the gate is controlled
         std::vector<int> dinfo((size_t)std::max(p.P, 1) * 4, 0);
@@ -955,20 +964,23 @@ int sqh_set_circuit(sqh_ctx* c, int qbit_num, const sqh_gate* gates, int n_gates
                     d[3] = fp.gates[i].kind == OP_CU;
                 }
             }
-        HIPTRY(c, c->d_dinfo.ensure(dinfo.size() * sizeof(int)));
-        HIPTRY(c, hipMemcpy(c->d_dinfo.p, dinfo.data(), dinfo.size() * sizeof(int), hipMemcpyHostToDevice));
+        table(c->d_dinfo, dinfo);
         const std::vector<int> tabs = fused_lane_tabs(qbit_num, fp);
-        HIPTRY(c, c->d_ftabs.ensure(tabs.size() * sizeof(int)));
-        HIPTRY(c, hipMemcpy(c->d_ftabs.p, tabs.data(), tabs.size() * sizeof(int), hipMemcpyHostToDevice));
+        table(c->d_ftabs, tabs);
         const std::vector<int> tmaps = fused_trace_maps(qbit_num, fp);
-        HIPTRY(c, c->d_tmaps.ensure(tmaps.size() * sizeof(int)));
-        HIPTRY(c, hipMemcpy(c->d_tmaps.p, tmaps.data(), tmaps.size() * sizeof(int), hipMemcpyHostToDevice));
+        table(c->d_tmaps, tmaps);
     }
     if (fused_big_fits(true, qbit_num) && fp.k == 4 && !fp.qubits.empty()) {
         const std::vector<int> tabs = fused_big_tabs(qbit_num, fp);
-        HIPTRY(c, c->d_ftabs.ensure(tabs.size() * sizeof(int)));
-        HIPTRY(c, hipMemcpy(c->d_ftabs.p, tabs.data(), tabs.size() * sizeof(int), hipMemcpyHostToDevice));
+        table(c->d_ftabs, tabs);
     }
+    c->have_circuit = false;  // the tables go with the old circuit
+    for (DevTable* t : {&c->d_ops, &c->d_lays, &c->d_slots, &c->d_quads, &c->d_squads, &c->d_ffirst, &c->d_fmaps,
+                        &c->d_dinfo, &c->d_ftabs, &c->d_tmaps})
+        t->p = nullptr;
+    HIPTRY(c, c->d_tables.ensure(host.size()));
+    HIPTRY(c, hipMemcpy(c->d_tables.p, host.data(), host.size(), hipMemcpyHostToDevice));
+    for (const auto& [t, at] : tables) t->p = c->d_tables.as<char>() + at;
     c->fplan = std::move(fp);
     c->fused_tuned.clear();
     c->tile_tuned.clear();
@@ -1218,21 +1230,6 @@ int sqh_optimization_problem_combined_targets_dev(sqh_ctx* c, const double* d_ta
     return SQH_OK;
 }
 
-// Doubles of a host-array call (parameters and results) that go through the context's pinned
-// buffer: k_finish then writes the results where the host reads them, and one wait ends the
-// call.  Two copies to pageable memory, each with its own wait, took 22 us of the 83 (117) us
-// of a 4 (8) qubit cost and gradient.  64 KiB: there the copies cost less than the kernels.
-constexpr size_t kSmallHost = 8192;
-
-// That buffer, allocated by the first call that is small enough (null: not to be had).
-static double* small_host(sqh_ctx* c) {
-    if (!c->h_small && hipHostMalloc((void**)&c->h_small, kSmallHost * sizeof(double), hipHostMallocDefault) != hipSuccess) {
-        c->h_small = nullptr;
-        (void)hipGetLastError();
-    }
-    return c->h_small;
-}
-
 static int host_batch(sqh_ctx* c, const double* params, int B, int precision, double* costs, double* grad) {
     if (!c) return SQH_ERR_ARG;
     std::lock_guard<std::mutex> lk(c->mu);
@@ -1243,7 +1240,7 @@ static int host_batch(sqh_ctx* c, const double* params, int B, int precision, do
     const int P = c->prog.P;
     const size_t np = (size_t)B * std::max(P, 1), nr = (size_t)B + (grad ? np : 0);
     HIPTRY(c, c->d_params.ensure(np * sizeof(double)));
-    double* h = np + nr <= kSmallHost ? small_host(c) : nullptr;
+    double* const h = np + nr <= kSmallHost ? c->h_small : nullptr;
     if (h) {
         double* res = h + np;
         if (P > 0) {

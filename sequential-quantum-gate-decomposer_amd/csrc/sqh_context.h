@@ -67,6 +67,15 @@ struct RunBufs {
 };
 constexpr size_t kRunBufsKept = (size_t)512 << 20;
 
+// One table of the circuit within the context's d_tables.
+struct DevTable {
+    void* p = nullptr;
+    template <typename T>
+    T* as() const {
+        return static_cast<T*>(p);
+    }
+};
+
 struct JitCache;
 void jit_release(sqh_ctx* c);
 
@@ -86,7 +95,8 @@ struct sqh_ctx {
     long long prog_version = 0;  // bumped by every sqh_set_circuit (keys the run-time kernels)
     sqh::Program prog;
     std::vector<sqh::GateRec> gates;
-    sqh::DevBuf d_ops, d_lays, d_slots;
+    sqh::DevBuf d_tables;  // every table of the circuit, uploaded as one (sqh_set_circuit)
+    sqh::DevTable d_ops, d_lays, d_slots;
 
     bool have_target = false;
     int rows = 0, cols = 0;
@@ -104,18 +114,19 @@ struct sqh_ctx {
 
     // Dense-block fusion of the circuit for the streaming path.
     sqh::FusionPlan fplan;
-    sqh::DevBuf d_quads, d_ffirst, d_fused;
-    sqh::DevBuf d_squads;  // the persistent solver's op words (quad_program; n_squads, 0: none)
+    sqh::DevTable d_quads, d_ffirst;
+    sqh::DevBuf d_fused;
+    sqh::DevTable d_squads;  // the persistent solver's op words (quad_program; n_squads, 0: none)
     int n_squads = 0;
     // Row tables of the tile-resident fused-block cost kernel ([blocks][kFusedMapStride];
     // present for 4 <= N <= 10) and its switch (sqh_set_fused_cost).
-    sqh::DevBuf d_fmaps;
-    sqh::DevBuf d_dinfo;  // per parameter its gate's block, slot, index in the gate, controlled
-    sqh::DevBuf d_ftabs;  // lane tables of the fused kernels ([blocks][kLaneTab])
+    sqh::DevTable d_fmaps;
+    sqh::DevTable d_dinfo;  // per parameter its gate's block, slot, index in the gate, controlled
+    sqh::DevTable d_ftabs;  // lane tables of the fused kernels ([blocks][kLaneTab])
     // Row tables of the transposed-chain cost kernel ([blocks][kTraceMapStride]) and its
     // switch (sqh_set_fused_cost_chain; on by default): the cost pass builds the rows of
     // the circuit matrix the trace needs instead of running the target's columns forward.
-    sqh::DevBuf d_tmaps;
+    sqh::DevTable d_tmaps;
     bool fused_chain = true;
     sqh::DevBuf d_fcorr;  // [B][ns][8] gate correlations of the fused-block gradient
     int fused_cost = SQH_FUSED_COST_AUTO;
@@ -139,7 +150,7 @@ struct sqh_ctx {
     bool tile_forced = false;
     double tune_ms = 0.0;
 
-    double* h_small = nullptr;  // pinned: parameters and results of small host-array calls (small_host)
+    double* h_small = nullptr;  // pinned: parameters and results of small host-array calls (or null)
 
     sqh::RunBufs run;  // batched optimiser (under mu, as every call)
 
@@ -153,8 +164,8 @@ struct sqh_ctx {
             (void)hipEventDestroy(e.first);
             (void)hipEventDestroy(e.second);
         }
-        for (sqh::DevBuf* b : {&d_ops, &d_lays, &d_slots, &d_U64, &d_U32, &d_params, &d_kern, &d_diag, &d_mpart,
-                               &d_res, &d_mat, &d_out, &d_quads, &d_squads, &d_ffirst, &d_fused, &d_fmaps, &d_ftabs, &d_dinfo, &d_tmaps, &d_fcorr, &d_idx, &d_seed, &d_dtab, &d_zslot})
+        for (sqh::DevBuf* b : {&d_tables, &d_U64, &d_U32, &d_params, &d_kern, &d_diag, &d_mpart, &d_res, &d_mat,
+                               &d_out, &d_fused, &d_fcorr, &d_idx, &d_seed, &d_dtab, &d_zslot})
             b->release();
         run.release();
         if (h_small) (void)hipHostFree(h_small);
