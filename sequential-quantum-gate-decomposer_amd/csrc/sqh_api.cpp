@@ -428,7 +428,6 @@ int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, c
     a.B = B;
     a.nb = nb;
     a.F = fused;
-    a.maps = c->d_fmaps.as<int>();
     a.tabs = c->d_ftabs.as<int>();
     a.diag = diag;
     a.mpart = mpart;

@@ -158,7 +158,6 @@ struct FusedGradArgs {
     const void* U = nullptr;  // target, rows = 2^N, m columns, row stride m
     int m = 0, trace_off = 0, B = 0, nb = 0;
     const void* F = nullptr;  // [B][nb][16][16] block matrices
-    const int* maps = nullptr;
     double* diag = nullptr;
     double* mpart = nullptr;
     int wgs = 0;     // partials per element
