@@ -26,8 +26,8 @@ enum MlpEpi : int {
     EPI_HIDDEN = 0,    // z = acc + bias -> Z, H = bf16(gelu(z)) -> H, H^T
     EPI_HIDDEN_ONLY,   // the same, H alone (no backward pass follows)
     EPI_OUTPUT,        // y = acc + bias -> the caller's B x out array
-    EPI_MSE,           // y = acc + bias, dY = 2 (y - t) / (B out) -> dZ, dZ^T, bias partials, loss
-    EPI_BWD_DATA,      // dz = acc gelu'(Z) -> dZ, dZ^T, bias partials
+    EPI_MSE,           // y = acc + bias, dY = 2 (y - t) / (B out) -> dZ, dZ^T, FP32 dZ, loss
+    EPI_BWD_DATA,      // dz = acc gelu'(Z) -> dZ, dZ^T, FP32 dZ
 };
 
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
@@ -38,27 +38,30 @@ __device__ __forceinline__ float gelu_grad(float z) {
     return cdf + z * pdf;
 }
 
-// The product of one TM x TN tile by a workgroup of 4 wavefronts, left as four partial
-// tiles in LDS.  Wavefront w takes the 32-wide K steps w, w + 4, ... of the whole tile, so
-// each operand value is loaded once per workgroup, straight from global memory into the
-// MFMA operand registers (mlp_frag order): no LDS and no barrier in the loop, and D steps
-// of loads in flight per wavefront.  What bounds it is the operands' way from the L2 (a
-// CU takes 64 bytes a cycle: 1.7 us for K = 1024 at 64 x 64).  Tiles shared through LDS between 32 x 32 quarters, K in stages of 256 behind
-// barriers, took 12 us (both operands K-contiguous) and 20 us (transposed on the way into
-// LDS) for 1024 x 1024 x 1024; this form 7.5 us with its epilogue, 5 of them launch, first
-// loads, the partials' sum and the epilogue.  Eight wavefronts of an eighth of K each: 7.9.
-// A lane's result item r of tile (i, j) is C[16 i + 4 (lane / 16) + r][16 j + lane % 16].
-constexpr int kPitch = 4;  // floats of padding per partial-tile row
+// The product of one TM x TN tile by a workgroup of 4 wavefronts, left in LDS.  Each
+// wavefront computes a quarter of the tile over the whole K, every element as one FP32 sum
+// in ascending K: a sum's bits depend neither on the tile size nor on the workgroup.  (K split
+// over the wavefronts loads half as much and takes 8 us less of a training step of 112, but
+// its sums round differently, and Adam's first steps carry that to 5e-4 of the weights.)
+// Operands come straight from global memory into the MFMA operand registers (mlp_frag
+// order): no LDS and no barrier in the loop, D steps of loads in flight per wavefront.  What
+// bounds it is the operands' way from the L2: a CU takes 64 bytes a cycle, 3.4 us for K = 1024
+// at 64 x 64.  1024 x 1024 x 1024 with its epilogue takes 11.3 us, 6.8 of them launch, first
+// loads and the epilogue; the operands handed round through LDS, 12.4.
+// A lane's result item r of tile (i, j) is C[16 i + 4 (lane / 16) + r][16 j + lane % 16] of
+// its quarter.
+constexpr int kPitch = 4;  // floats of padding per tile row
 
-template <int TM, int TN>
-__device__ __forceinline__ void mlp_product(const bf16* __restrict__ A, const bf16* __restrict__ B, int K, int m0, int n0, float* __restrict__ red) {
-    constexpr int I = TM / 16, J = TN / 16, D = TM < 64 ? 8 : 3;
+template <int TM, int TN, int D>
+__device__ __forceinline__ void mlp_product(const bf16* __restrict__ A, const bf16* __restrict__ B, int K, int m0,
+                                            int n0, float* __restrict__ tile) {
+    constexpr int I = TM / 32, J = TN / 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nl = lane & 15, g = lane >> 4;
-    const int ks = K >> 5;                                     // 32-wide K steps
-    const int S = ks > wave ? (ks - wave + 3) / 4 : 0;  // this wavefront's
-    const bf16* pa = A + ((size_t)(m0 >> 4) * ks + wave) * 512 + lane * 8;
-    const bf16* pb = B + ((size_t)(n0 >> 4) * ks + wave) * 512 + lane * 8;
+    const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
+    const int S = K >> 5;  // 32-wide K steps
+    const bf16* pa = A + (size_t)((m0 + wm) >> 4) * S * 512 + lane * 8;
+    const bf16* pb = B + (size_t)((n0 + wn) >> 4) * S * 512 + lane * 8;
     f32x4 acc[I][J];
 #pragma unroll
     for (int i = 0; i < I; ++i)
@@ -67,9 +70,9 @@ __device__ __forceinline__ void mlp_product(const bf16* __restrict__ A, const bf
     bf16x8 a[D][I], b[D][J];
     auto load = [&](int d, int s) {
 #pragma unroll
-        for (int i = 0; i < I; ++i) a[d][i] = *reinterpret_cast<const bf16x8*>(pa + ((size_t)i * ks + 4 * s) * 512);
+        for (int i = 0; i < I; ++i) a[d][i] = *reinterpret_cast<const bf16x8*>(pa + ((size_t)i * S + s) * 512);
 #pragma unroll
-        for (int j = 0; j < J; ++j) b[d][j] = *reinterpret_cast<const bf16x8*>(pb + ((size_t)j * ks + 4 * s) * 512);
+        for (int j = 0; j < J; ++j) b[d][j] = *reinterpret_cast<const bf16x8*>(pb + ((size_t)j * S + s) * 512);
     };
 #pragma unroll
     for (int d = 0; d < D; ++d)
@@ -87,31 +90,25 @@ __device__ __forceinline__ void mlp_product(const bf16* __restrict__ A, const bf
             }
         }
     }
-    float* part = red + wave * TM * (TN + kPitch);
 #pragma unroll
     for (int i = 0; i < I; ++i)
 #pragma unroll
         for (int j = 0; j < J; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) part[(16 * i + 4 * g + r) * (TN + kPitch) + 16 * j + nl] = acc[i][j][r];
+            for (int r = 0; r < 4; ++r)
+                tile[(wm + 16 * i + 4 * g + r) * (TN + kPitch) + wn + 16 * j + nl] = acc[i][j][r];
     __syncthreads();
 }
 
 // Threads of the epilogue and the 4 x 4 block of the tile each holds: rows 4 rg .. + 3,
-// columns 4 cg .. + 3, the four wavefronts' partials summed in wavefront order.
+// columns 4 cg .. + 3.
 template <int TM, int TN>
-__device__ __forceinline__ bool mlp_block(const float* __restrict__ red, int& rg, int& cg, f32x4 (&v)[4]) {
+__device__ __forceinline__ bool mlp_block(const float* __restrict__ tile, int& rg, int& cg, f32x4 (&v)[4]) {
     if (threadIdx.x >= TM * TN / 16) return false;
     rg = threadIdx.x / (TN / 4);
     cg = threadIdx.x % (TN / 4);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const float* p = red + (4 * rg + r) * (TN + kPitch) + 4 * cg;
-        f32x4 s = *reinterpret_cast<const f32x4*>(p);
-#pragma unroll
-        for (int w = 1; w < 4; ++w) s += *reinterpret_cast<const f32x4*>(p + w * TM * (TN + kPitch));
-        v[r] = s;
-    }
+    for (int r = 0; r < 4; ++r) v[r] = *reinterpret_cast<const f32x4*>(tile + (4 * rg + r) * (TN + kPitch) + 4 * cg);
     return true;
 }
 
@@ -132,30 +129,14 @@ __device__ __forceinline__ void mlp_store_bf16(const f32x4 (&v)[4], int row, int
     }
 }
 
-// Column sums of a tile's dZ (each thread holds the sums of its four rows) into the
-// tile row's slice of the bias partials; sums in a fixed order.
-template <int TM, int TN>
-__device__ __forceinline__ void mlp_bias_partials(bool active, int rg, int cg, const f32x4 (&v)[4],
-                                                  float* __restrict__ red, float* __restrict__ bpart, int n0) {
-    __syncthreads();  // the partial tiles are consumed
-    if (active) *reinterpret_cast<f32x4*>(red + rg * TN + 4 * cg) = (v[0] + v[1]) + (v[2] + v[3]);
-    __syncthreads();
-    if (threadIdx.x < TN) {
-        float s = 0.f;
-#pragma unroll
-        for (int k = 0; k < TM / 4; ++k) s += red[k * TN + threadIdx.x];
-        bpart[n0 + threadIdx.x] = s;
-    }
-}
-
 template <int TM, int TN, int EPI>
 __global__ __launch_bounds__(256, 2) void k_mlp_layer(MlpLayerArgs a) {
-    __shared__ __align__(16) float red[4 * TM * (TN + kPitch)];
+    __shared__ __align__(16) float tile[TM * (TN + kPitch)];
     const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-    mlp_product<TM, TN>((const bf16*)a.A, (const bf16*)a.B, a.K, m0, n0, red);
+    mlp_product<TM, TN, (TM < 64 ? 16 : 12)>((const bf16*)a.A, (const bf16*)a.B, a.K, m0, n0, tile);
     int rg = 0, cg = 0;
     f32x4 v[4];
-    const bool active = mlp_block<TM, TN>(red, rg, cg, v);
+    const bool active = mlp_block<TM, TN>(tile, rg, cg, v);
     const int row = m0 + 4 * rg, col = n0 + 4 * cg;
     if constexpr (EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_ONLY) {
         if (active) {
@@ -199,10 +180,10 @@ __global__ __launch_bounds__(256, 2) void k_mlp_layer(MlpLayerArgs a) {
                     }
                     v[r][c] = gr;
                 }
+                *reinterpret_cast<f32x4*>(&a.Z[(size_t)(row + r) * a.N + col]) = v[r];
             }
             mlp_store_bf16(v, row, col, (bf16*)a.X, a.N, (bf16*)a.XT, a.M);
         }
-        mlp_bias_partials<TM, TN>(active, rg, cg, v, red, a.bpart + (size_t)blockIdx.y * a.N, n0);
         __shared__ double sh[4];
         for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o, 64);
         if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = l;
@@ -215,86 +196,109 @@ __global__ __launch_bounds__(256, 2) void k_mlp_layer(MlpLayerArgs a) {
                 const f32x4 z = *reinterpret_cast<const f32x4*>(&a.Z[(size_t)(row + r) * a.N + col]);
 #pragma unroll
                 for (int c = 0; c < 4; ++c) v[r][c] *= gelu_grad(z[c]);
+                *reinterpret_cast<f32x4*>(&a.Z[(size_t)(row + r) * a.N + col]) = v[r];
             }
             mlp_store_bf16(v, row, col, (bf16*)a.X, a.N, (bf16*)a.XT, a.M);
         }
-        mlp_bias_partials<TM, TN>(active, rg, cg, v, red, a.bpart + (size_t)blockIdx.y * a.N, n0);
     }
 }
 
-// Adam on an FP32 master weight.
+// Adam on an FP32 master weight.  The roundings are spelled out: left to the compiler, which
+// of a moment's two products is rounded changes with the code around it.
 __device__ __forceinline__ float mlp_adam(float w, float g, float& m, float& v, const MlpAdam& p) {
-    m = p.b1 * m + (1.0f - p.b1) * g;
-    v = p.b2 * v + (1.0f - p.b2) * g * g;
+    m = fmaf(1.0f - p.b1, g, p.b1 * m);
+    v = fmaf((1.0f - p.b2) * g, g, p.b2 * v);
     return w - p.lr * (m / p.c1) / (sqrtf(v / p.c2) + p.eps);
 }
 
 // Weight and bias gradients of up to kMlpGroup layers in one launch, each either applied
 // by Adam where it is formed (the gradient never travels through memory) or stored.  The
-// weights' and moments' 28 bytes a parameter bound it: 28 us for 2.8 M parameters at a batch
+// weights' and moments' 28 bytes a parameter bound it: 33 us for 2.8 M parameters at a batch
 // of 1024, where the products, the column sums and the updates of the four layers, a launch
-// each, took 148.
-// Workgroups: the layers' weight tiles, then 64 bias entries per workgroup.
+// each, took 148.  The bias workgroups come first: they wait for memory while the tiles run.
+// Workgroups, per layer: 16 bias entries each, then the weight tiles.
 template <int TM, int TN, bool ADAM>
-__global__ __launch_bounds__(256, 2) void k_mlp_weights(MlpWeightsArgs a) {
-    __shared__ __align__(16) float red[4 * TM * (TN + kPitch)];
+__global__ __launch_bounds__(256, 3) void k_mlp_weights(MlpWeightsArgs a) {
+    __shared__ __align__(16) float tile[TM * (TN + kPitch)];
     int t = blockIdx.x, l = 0;
     while (l + 1 < a.layers && t >= a.first[l + 1]) ++l;
     const MlpWeights& w = a.w[l];
     t -= a.first[l];
-    const int tn = w.in / TN, tiles = (w.out / TM) * tn;
-    if (t < tiles) {
-        const int m0 = t / tn * TM, n0 = t % tn * TN;
-        mlp_product<TM, TN>((const bf16*)w.dZT, (const bf16*)w.HT, a.batch, m0, n0, red);
-        int rg = 0, cg = 0;
-        f32x4 v[4];
-        if (!mlp_block<TM, TN>(red, rg, cg, v)) return;
-        const int row = m0 + 4 * rg, col = n0 + 4 * cg;
+    const int nbias = w.out / 16;
+    if (t < nbias) {
+        // 16 bias entries: 64 row slices, each summing every 64th row of dZ, then the slices in
+        // order (the sum is the same on every run and for every tile size)
+        constexpr int kSlices = 64;
+        const int c4 = threadIdx.x & 3, q = threadIdx.x >> 2;
+        const float* z = w.dZ + t * 16 + 4 * c4;
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 16
+        for (int r = q; r < a.rows; r += kSlices) s += *reinterpret_cast<const f32x4*>(z + (size_t)r * w.out);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const size_t o = (size_t)(row + r) * w.in + col;
-            if constexpr (ADAM) {
-                f32x4 x = *reinterpret_cast<f32x4*>(&w.W[o]);
-                f32x4 m = *reinterpret_cast<f32x4*>(&w.mW[o]);
-                f32x4 s = *reinterpret_cast<f32x4*>(&w.vW[o]);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    float mc = m[c], sc = s[c];
-                    x[c] = mlp_adam(x[c], v[r][c], mc, sc, a.adam);
-                    m[c] = mc;
-                    s[c] = sc;
-                }
-                *reinterpret_cast<f32x4*>(&w.W[o]) = x;
-                *reinterpret_cast<f32x4*>(&w.mW[o]) = m;
-                *reinterpret_cast<f32x4*>(&w.vW[o]) = s;
-                v[r] = x;
-            } else {
-                *reinterpret_cast<f32x4*>(&w.gW[o]) = v[r];
-            }
+        for (int i = 0; i < 4; ++i) tile[q * 17 + 4 * c4 + i] = s[i];
+        __syncthreads();
+        if (threadIdx.x < 16) {
+            const int c = threadIdx.x, n = t * 16 + c;
+            float g = 0.f;
+#pragma unroll 8
+            for (int k = 0; k < kSlices; ++k) g += tile[k * 17 + c];
+            if constexpr (ADAM) w.b[n] = mlp_adam(w.b[n], g, w.mb[n], w.vb[n], a.adam);
+            else w.gb[n] = g;
         }
-        if constexpr (ADAM) mlp_store_bf16(v, row, col, (bf16*)w.Wb, w.in, (bf16*)w.WbT, w.out);
         return;
     }
-    // bias entries: the partials of every tile row, four interleaved slices per entry
-    const int n = (t - tiles) * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;
-    float s = 0.f;
-    for (int k = q; k < w.parts; k += 4) s += w.bpart[(size_t)k * w.out + n];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    if (q == 0) {
-        const float g = (red[n & 63] + red[64 + (n & 63)]) + (red[128 + (n & 63)] + red[192 + (n & 63)]);
-        if constexpr (ADAM) w.b[n] = mlp_adam(w.b[n], g, w.mb[n], w.vb[n], a.adam);
-        else w.gb[n] = g;
+    t -= nbias;
+    const int tn = w.in / TN;
+    const int m0 = t / tn * TM, n0 = t % tn * TN;
+    // the thread's block of the tile (mlp_block); its weights and moments are on their way
+    // while the product runs
+    const int row = m0 + 4 * (threadIdx.x / (TN / 4)), col = n0 + 4 * (threadIdx.x % (TN / 4));
+    const bool mine = threadIdx.x < TM * TN / 16;
+    f32x4 x[4], mo[4], se[4];
+    if constexpr (ADAM) {
+        if (mine) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const size_t o = (size_t)(row + r) * w.in + col;
+                x[r] = *reinterpret_cast<f32x4*>(&w.W[o]);
+                mo[r] = *reinterpret_cast<f32x4*>(&w.mW[o]);
+                se[r] = *reinterpret_cast<f32x4*>(&w.vW[o]);
+            }
+        }
     }
+    mlp_product<TM, TN, (TM < 64 ? 8 : 4)>((const bf16*)w.dZT, (const bf16*)w.HT, a.batch, m0, n0, tile);
+    int rg = 0, cg = 0;
+    f32x4 v[4];
+    if (!mlp_block<TM, TN>(tile, rg, cg, v)) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const size_t o = (size_t)(row + r) * w.in + col;
+        if constexpr (ADAM) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                float mc = mo[r][c], sc = se[r][c];
+                x[r][c] = mlp_adam(x[r][c], v[r][c], mc, sc, a.adam);
+                mo[r][c] = mc;
+                se[r][c] = sc;
+            }
+            *reinterpret_cast<f32x4*>(&w.W[o]) = x[r];
+            *reinterpret_cast<f32x4*>(&w.mW[o]) = mo[r];
+            *reinterpret_cast<f32x4*>(&w.vW[o]) = se[r];
+            v[r] = x[r];
+        } else {
+            *reinterpret_cast<f32x4*>(&w.gW[o]) = v[r];
+        }
+    }
+    if constexpr (ADAM) mlp_store_bf16(v, row, col, (bf16*)w.Wb, w.in, (bf16*)w.WbT, w.out);
 }
 
 // An FP32 array (rows x cols real entries, row stride ldx) as zero-padded BF16 in both
-// orders: X[row][col] (Rp x Cp) and, when given, XT[col][row]; bpart (when given)
-// receives the column sums of each 64-row slice.  64 x 64 per workgroup: the network's
-// input batch, the caller's output gradient and the weights.
+// orders: X[row][col] (Rp x Cp) and, when given, XT[col][row]; P (when given) receives it
+// padded in FP32.  64 x 64 per workgroup: the network's input batch, the caller's output
+// gradient and the weights.
 __global__ __launch_bounds__(256) void k_mlp_convert(const float* __restrict__ x, int rows, int cols, int ldx,
                                                      bf16* __restrict__ X, bf16* __restrict__ XT, int Rp, int Cp,
-                                                     float* __restrict__ bpart) {
+                                                     float* __restrict__ P) {
     __shared__ __align__(16) float tile[64 * 65];
     const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
     for (int i = threadIdx.x; i < 64 * 64; i += 256) {
@@ -310,7 +314,10 @@ __global__ __launch_bounds__(256) void k_mlp_convert(const float* __restrict__ x
 #pragma unroll
         for (int c = 0; c < 4; ++c) v[r][c] = tile[(4 * rg + r) * 65 + 4 * cg + c];
     mlp_store_bf16(v, r0 + 4 * rg, c0 + 4 * cg, X, Cp, XT, Rp);
-    if (bpart) mlp_bias_partials<64, 64>(true, rg, cg, v, tile, bpart + (size_t)blockIdx.y * Cp, c0);
+    if (P) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) *reinterpret_cast<f32x4*>(&P[(size_t)(r0 + 4 * rg + r) * Cp + c0 + 4 * cg]) = v[r];
+    }
 }
 
 // One layer's parameters between the padded device layout (W [np][kp], b [np]) and the
@@ -329,9 +336,9 @@ __global__ __launch_bounds__(256) void k_pack_layer(float* __restrict__ W, float
 
 // Host launchers ------------------------------------------------------------------
 
-// 64 x 64 tiles load half the operand bytes per flop of 32 x 32 ones (7.5 against 8.6 us
+// 64 x 64 tiles load half the operand bytes per flop of 32 x 32 ones (11.3 against 14.3 us
 // for a 1024 x 1024 x 1024 product); below 256 of them, one per CU, the smaller tiles put
-// four times the CUs to work.
+// four times the CUs to work (1024 x 192 x 1024: 8.6 against 10.4 us).
 static bool small_tiles(long long tiles64) { return tiles64 < 256; }
 
 int mlp_tile_rows(int M, int N) { return small_tiles((long long)(M / 64) * (N / 64)) ? 32 : 64; }
@@ -366,7 +373,7 @@ hipError_t mlp_weights(MlpWeightsArgs a, bool adam, hipStream_t s) {
     int first = 0;
     for (int l = 0; l < a.layers; ++l) {
         a.first[l] = first;
-        first += (a.w[l].out / T) * (a.w[l].in / T) + a.w[l].out / 64;
+        first += (a.w[l].out / T) * (a.w[l].in / T) + a.w[l].out / 16;
     }
     if (T == 32 && adam) hipLaunchKernelGGL((k_mlp_weights<32, 32, true>), dim3(first), dim3(256), 0, s, a);
     else if (T == 32) hipLaunchKernelGGL((k_mlp_weights<32, 32, false>), dim3(first), dim3(256), 0, s, a);
@@ -375,11 +382,11 @@ hipError_t mlp_weights(MlpWeightsArgs a, bool adam, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t mlp_convert(const float* x, int rows, int cols, int ldx, void* X, void* XT, int Rp, int Cp, float* bpart,
+hipError_t mlp_convert(const float* x, int rows, int cols, int ldx, void* X, void* XT, int Rp, int Cp, float* P,
                        hipStream_t s) {
     if (Rp % 64 || Cp % 64 || Rp <= 0 || Cp <= 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_mlp_convert, dim3(Cp / 64, Rp / 64), dim3(256), 0, s, x, rows, cols, ldx, (bf16*)X, (bf16*)XT,
-                       Rp, Cp, bpart);
+                       Rp, Cp, P);
     return hipGetLastError();
 }
 

@@ -26,17 +26,16 @@ struct sqh_mlp {
     // FP32 master weights, their BF16 copies in both orders, Adam's moments, gradients
     // (kept only by sqh_mlp_gradients)
     std::vector<DevBuf> W, Wb, WbT, b, mW, vW, mb, vb, gW, gb;
-    // per layer for a batch: input activations and their transposes, pre-activations,
-    // output gradients and their transposes, bias gradient partials
-    std::vector<DevBuf> H, HT, Z, dZ, dZT, bpart;
-    std::vector<int> parts;          // slices of bpart the last backward pass wrote
+    // per layer for a batch: input activations and their transposes, pre-activations (then
+    // output gradients) in FP32, output gradients and their transposes
+    std::vector<DevBuf> H, HT, Z, dZ, dZT;
     DevBuf loss;                     // loss partials
     DevBuf flat;                     // the parameters in the caller's flat layout
     int loss_parts = 0;              // loss partials the last forward pass wrote
     int step = 0;
 
     ~sqh_mlp() {
-        for (auto* v : {&W, &Wb, &WbT, &b, &mW, &vW, &mb, &vb, &gW, &gb, &H, &HT, &Z, &dZ, &dZT, &bpart})
+        for (auto* v : {&W, &Wb, &WbT, &b, &mW, &vW, &mb, &vb, &gW, &gb, &H, &HT, &Z, &dZ, &dZT})
             for (auto& x : *v) x.release();
         loss.release();
         flat.release();
@@ -54,10 +53,9 @@ int ensure_batch(sqh_mlp* m, int Bp, bool train) {
         HIPTRY(c, m->H[l].ensure((size_t)Bp * in * 2));
         if (!train) continue;
         HIPTRY(c, m->HT[l].ensure(in * Bp * 2));
-        if (l + 1 < m->L) HIPTRY(c, m->Z[l].ensure(out * 4));
+        HIPTRY(c, m->Z[l].ensure(out * 4));
         HIPTRY(c, m->dZ[l].ensure((size_t)Bp * outd * 2));
         HIPTRY(c, m->dZT[l].ensure(outd * Bp * 2));
-        HIPTRY(c, m->bpart[l].ensure(out / 32 * 4));
     }
     if (train) HIPTRY(c, m->loss.ensure((size_t)Bp * m->dpad[m->L] / 1024 * sizeof(double)));
     return SQH_OK;
@@ -105,8 +103,6 @@ int backward_data(sqh_mlp* m, int Bp) {
         a.Z = m->Z[l - 1].as<float>();
         a.X = m->dZ[l - 1].p;
         a.XT = m->dZT[l - 1].p;
-        a.bpart = m->bpart[l - 1].as<float>();
-        m->parts[l - 1] = Bp / mlp_tile_rows(a.M, a.N);
         HIPTRY(c, mlp_backward_data(a, m->st()));
     }
     return SQH_OK;
@@ -114,12 +110,13 @@ int backward_data(sqh_mlp* m, int Bp) {
 
 // Weight and bias gradients of every layer: applied by one Adam step of rate lr, or
 // (adam = false) stored in gW / gb.  After backward_data, which reads the old weights.
-int weights(sqh_mlp* m, int Bp, bool adam, float lr) {
+int weights(sqh_mlp* m, int B, int Bp, bool adam, float lr) {
     sqh_ctx* c = m->ctx;
     if (adam) m->step++;
     const float b1 = 0.9f, b2 = 0.999f;
     MlpWeightsArgs g;
     g.batch = Bp;
+    g.rows = B;
     g.adam = {lr, b1, b2, 1e-8f, 1.0f - powf(b1, (float)m->step), 1.0f - powf(b2, (float)m->step)};
     for (int l0 = 0; l0 < m->L; l0 += kMlpGroup) {
         g.layers = std::min(kMlpGroup, m->L - l0);
@@ -132,7 +129,7 @@ int weights(sqh_mlp* m, int Bp, bool adam, float lr) {
             g.w[k] = {m->dZT[l].p,          m->HT[l].p,          m->W[l].as<float>(),  m->mW[l].as<float>(),
                       m->vW[l].as<float>(), m->gW[l].as<float>(), m->Wb[l].p,           m->WbT[l].p,
                       m->b[l].as<float>(),  m->mb[l].as<float>(), m->vb[l].as<float>(), m->gb[l].as<float>(),
-                      m->bpart[l].as<float>(), m->parts[l],       m->dpad[l],           m->dpad[l + 1]};
+                      m->Z[l].as<float>(),  m->dpad[l],           m->dpad[l + 1]};
         }
         HIPTRY(c, mlp_weights(g, adam, m->st()));
     }
@@ -152,10 +149,9 @@ int forward_backward(sqh_mlp* m, const float* d_x, const float* d_t, int B, int 
     a.out = m->dim[L];
     a.X = m->dZ[L - 1].p;
     a.XT = m->dZT[L - 1].p;
-    a.bpart = m->bpart[L - 1].as<float>();
+    a.Z = m->Z[L - 1].as<float>();
     a.loss = m->loss.as<double>();
     const int T = mlp_tile_rows(a.M, a.N);
-    m->parts[L - 1] = Bp / T;
     m->loss_parts = (Bp / T) * (a.N / T);
     HIPTRY(c, mlp_output_mse(a, m->st()));
     return backward_data(m, Bp);
@@ -240,9 +236,8 @@ int sqh_mlp_create(sqh_ctx* c, int in_dim, int hidden, int n_hidden, int out_dim
     m->L = (int)m->dim.size() - 1;
     for (int d : m->dim) m->dpad.push_back(pad64(d));
     for (auto* v : {&m->W, &m->Wb, &m->WbT, &m->b, &m->mW, &m->vW, &m->mb, &m->vb, &m->gW, &m->gb, &m->H, &m->HT,
-                    &m->Z, &m->dZ, &m->dZT, &m->bpart})
+                    &m->Z, &m->dZ, &m->dZT})
         v->resize(m->L);
-    m->parts.assign(m->L, 0);
     std::mt19937_64 gen(seed);
     std::normal_distribution<float> nd(0.0f, 1.0f);
     for (int l = 0; l < m->L; ++l) {
@@ -330,7 +325,7 @@ int sqh_mlp_train_step_dev(sqh_mlp* m, const float* d_x, const float* d_t, int B
     int rc = ensure_batch(m, Bp, true);
     if (rc) return rc;
     if ((rc = forward_backward(m, d_x, d_t, B, Bp))) return rc;
-    if ((rc = weights(m, Bp, true, lr))) return rc;
+    if ((rc = weights(m, B, Bp, true, lr))) return rc;
     return loss ? read_loss(m, B, loss) : SQH_OK;
 }
 
@@ -345,10 +340,9 @@ int sqh_mlp_backward_step_dev(sqh_mlp* m, const float* d_x, const float* d_dy, i
     // the output itself is not needed: its gradient is the caller's
     if ((rc = forward_hidden(m, d_x, B, Bp, true))) return rc;
     HIPTRY(c, mlp_convert(d_dy, B, m->dim[L], m->dim[L], m->dZ[L - 1].p, m->dZT[L - 1].p, Bp, m->dpad[L],
-                          m->bpart[L - 1].as<float>(), m->st()));
-    m->parts[L - 1] = Bp / 64;
+                          m->Z[L - 1].as<float>(), m->st()));
     if ((rc = backward_data(m, Bp))) return rc;
-    return weights(m, Bp, true, lr);
+    return weights(m, B, Bp, true, lr);
 }
 
 int sqh_mlp_gradients(sqh_mlp* m, const float* x, const float* t, int B, float* grads, double* loss) {
@@ -365,7 +359,7 @@ int sqh_mlp_gradients(sqh_mlp* m, const float* x, const float* t, int B, float* 
     HIPTRY(c, hipMemcpyAsync(dx.p, x, (size_t)B * m->dim[0] * 4, hipMemcpyHostToDevice, m->st()));
     HIPTRY(c, hipMemcpyAsync(dt.p, t, (size_t)B * m->dim[m->L] * 4, hipMemcpyHostToDevice, m->st()));
     rc = forward_backward(m, dx.as<float>(), dt.as<float>(), B, Bp);
-    if (!rc) rc = weights(m, Bp, false, 0.0f);
+    if (!rc) rc = weights(m, B, Bp, false, 0.0f);
     if (!rc && loss) rc = read_loss(m, B, loss);
     if (!rc) rc = copy_params(m, grads, true, true);
     (void)hipStreamSynchronize(m->st());

@@ -21,13 +21,14 @@ struct MlpLayerArgs {
     const void* B = nullptr;
     int M = 0, N = 0, K = 0;      // padded; M is the padded batch
     const float* bias = nullptr;  // [N] (forward)
-    float* Z = nullptr;           // pre-activations [M][N]: written forward, read backward
+    // FP32 [M][N]: the pre-activations, written forward; the data gradient reads them and
+    // leaves dZ in their place (the output layer: dZ), from which the bias gradient is summed
+    float* Z = nullptr;
     void* X = nullptr;            // BF16 result [M][N] (H or dZ)
     void* XT = nullptr;           // ... and transposed [N][M]
     float* y = nullptr;           // the caller's output [batch][out]
     const float* t = nullptr;     // the caller's training targets [batch][out]
     int batch = 0, out = 0;       // real rows and columns of y / t
-    float* bpart = nullptr;       // bias partials [M / tile rows][N]
     double* loss = nullptr;       // loss partials, one per workgroup
 };
 
@@ -42,9 +43,8 @@ struct MlpWeights {
     float *W, *mW, *vW, *gW;
     void *Wb, *WbT;
     float *b, *mb, *vb, *gb;
-    const float* bpart;
-    int parts;    // slices of bpart
-    int in, out;  // padded
+    const float* dZ;  // FP32 [batch][out]
+    int in, out;      // padded
 };
 
 constexpr int kMlpGroup = 8;  // layers per launch
@@ -54,10 +54,11 @@ struct MlpWeightsArgs {
     int first[kMlpGroup];  // first workgroup of each layer
     int layers;
     int batch;  // padded
+    int rows;   // real rows of the batch
     MlpAdam adam;
 };
 
-// Rows of the tiles a layer product over M x N runs with (the slice height of bpart).
+// Rows of the tiles a layer product over M x N runs with.
 int mlp_tile_rows(int M, int N);
 hipError_t mlp_hidden(const MlpLayerArgs& a, bool train, hipStream_t s);
 hipError_t mlp_output(const MlpLayerArgs& a, hipStream_t s);
@@ -65,7 +66,7 @@ hipError_t mlp_output_mse(const MlpLayerArgs& a, hipStream_t s);
 hipError_t mlp_backward_data(const MlpLayerArgs& a, hipStream_t s);
 // The layers' gradients applied by Adam, or (adam = false) stored in gW / gb.
 hipError_t mlp_weights(MlpWeightsArgs a, bool adam, hipStream_t s);
-hipError_t mlp_convert(const float* x, int rows, int cols, int ldx, void* X, void* XT, int Rp, int Cp, float* bpart,
+hipError_t mlp_convert(const float* x, int rows, int cols, int ldx, void* X, void* XT, int Rp, int Cp, float* P,
                        hipStream_t s);
 hipError_t mlp_pack_layer(float* W, float* b, int no, int ni, int kp, float* flat, bool to_flat, hipStream_t s);
 
