@@ -365,11 +365,11 @@ int sqh_get_fused_cost_config(sqh_ctx* ctx, int is_f32, int B, int* tiles_per_wa
  * Optimization_Interface.cpp:940-1033 and 1401-1450 compute). */
 int sqh_set_fused_cost_chain(sqh_ctx* ctx, int on);
 /* Launch shape of the fused-block cost + gradient kernel: 16-column tiles per
- * wavefront (2 or 4; 10 qubits need 4) and wavefronts per workgroup (1, 2, 4 or 8,
- * dividing the element's column groups).  Both zero (the default): a fixed rule per
- * qubit count.  A shape that does not fit the circuit, target or the device's LDS falls
- * back to the rule.  The shape sets how the correlation sums are grouped, so different
- * shapes agree to rounding (each shape is deterministic). */
+ * wavefront (2 or 4; 10 qubits need 4) and wavefronts per workgroup (1, 2, 4 or 8).  Both
+ * zero (the default): a fixed rule.  A shape that does not fit the circuit, target or the
+ * device's LDS falls back to the rule.  The correlation sums are added in one fixed order,
+ * so a vector's cost and gradient are the same bits at every shape and in every batch
+ * that these kernels run. */
 int sqh_set_fused_grad_config(sqh_ctx* ctx, int tiles_per_wave, int waves);
 /* Launch options of the register-tile kernels (the batched costs and gradients when
  * the fused-block path does not run).  waves_per_group: for the forward pass with one

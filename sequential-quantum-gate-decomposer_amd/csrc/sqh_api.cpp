@@ -274,7 +274,8 @@ double fused_ratio(const sqh_ctx* c, bool grad) {
 // gradient from 6), when the blocks do no more arithmetic than the gates.  Against the
 // generic ones the line is the arithmetic ratio up to which both precisions gain at
 // B = 1 to 4096 (time of the tile kernels over that of the fused ones); it does not look at
-// B, so that a vector's result does not depend on the batch it came in:
+// B, and neither do the fused kernels' sums, so that a vector's result does not depend on the
+// batch it came in:
 //   gradients  8+ qubits: 2.5 (1.3 - 3.2 at 1.9 - 2.4, 2.0 - 6.1 below 1.2)
 //              6, 7:      1.5 (1.1 - 1.9 at 1.3, 0.85 at 2.6)
 //              5:         1   (1.2 - 3.0 below, 0.85 at 1.5)
@@ -292,9 +293,10 @@ bool fused_auto(const sqh_ctx* c, FusedKind kind) {
     return r <= line[kind][std::min(N, 8) - 4];
 }
 
-// Whether a pass (costs, or the apply_to store pass) runs through the tile-resident fused-block kernel: 4 <= N <= 10, the circuit has blocks, and the switch is
-// on, or automatic (the default) and the rule above holds.  Costs also need no correction
-// channels (fused_cost_applies).
+// Whether a pass (costs, or the apply_to store pass) runs through the tile-resident
+// fused-block kernel: 4 <= N <= 10, the circuit has blocks, and the switch is on, or
+// automatic (the default) and the rule above holds.  Costs also need no correction channels
+// (fused_cost_applies).
 bool fused_pass_applies(const sqh_ctx* c, bool store) {
     if (!fused_plan_fits(c)) return false;
     if (c->fused_cost == SQH_FUSED_COST_AUTO) return fused_auto(c, store ? FUSED_STORE_PASS : FUSED_COST_PASS);
@@ -351,59 +353,6 @@ int fused_cost_eval(sqh_ctx* c, bool f32, int B, const double* d_params, double*
     return fused_cost_launch(c, f32, a);
 }
 
-// Launch plan of the fused-block gradient for the context's circuit, B elements of m
-// columns: the shape set by sqh_set_fused_grad_config when it fits, else four 16-column
-// tiles per wavefront from 9 qubits or from 64 elements (fewer, larger partials), two
-// below (more wavefronts for small batches), and the most wavefronts per workgroup, up
-// to four, that divide the column groups -- the fastest shapes measured on MI355X --
-// with the scratch it needs.  Returns false when no shape fits the device's LDS.
-bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, FusedGradPlan& p) {
-    const int N = c->prog.N, nb = (int)c->fplan.qubits.size(), ns = (int)c->prog.slots.size();
-    p.T = 0;
-    if (c->fg_force_tiles && fused_grad_shape_valid(f32, N, m, nb, c->fg_force_tiles, c->fg_force_waves)) {
-        p.T = c->fg_force_tiles;
-        p.waves = c->fg_force_waves;
-    } else {
-        for (int t : {N >= 9 || B >= 64 ? 4 : 2, 4}) {
-            for (int w : {4, 2, 1})
-                if (fused_grad_shape_valid(f32, N, m, nb, t, w)) {
-                    p.T = t;
-                    p.waves = w;
-                    break;
-                }
-            if (p.T) break;
-        }
-    }
-    if (!p.T) return false;
-    p.wgs = fused_grad_wgs(N, m, p.T, B);
-    p.fused_bytes = (size_t)B * nb * 256 * (f32 ? 8 : 16);
-    p.mpart_bytes = (size_t)B * p.wgs * nb * 512 * sizeof(double);
-    p.corr_bytes = (size_t)B * std::max(ns, 1) * 8 * sizeof(double);
-    return true;
-}
-
-// Whether a cost + gradient evaluation of B elements of m columns runs through the fused
-// blocks: the switch on, or automatic and the rule of fused_auto, 4 <= N <= 10, no
-// correction channels, and a launch shape fits.  Below 6 qubits, where the blocks' scratch
-// is several times the tile kernels', automatic batches keep it within 4 GiB.
-bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, int m, FusedGradPlan* plan) {
-    if (ts.nch != 0 || !fused_plan_fits(c)) return false;
-    const bool automatic = c->fused_cost == SQH_FUSED_COST_AUTO;
-    if (c->fused_cost == SQH_FUSED_COST_OFF || (automatic && !fused_auto(c, FUSED_GRAD_PASS))) return false;
-    FusedGradPlan p;
-    if (!fused_grad_plan(c, f32, B, m, p)) return false;
-    if (automatic && c->prog.N < 6 && p.fused_bytes + p.mpart_bytes + p.corr_bytes > (size_t)4 << 30) return false;
-    if (plan) *plan = p;
-    return true;
-}
-
-// Costs and gradients of B parameter vectors through the fused blocks on stream st:
-// block matrices (into fused), the forward + backward kernel (trace entries into diag,
-// per-workgroup correlation partials into mpart), then each block's gate correlations
-// into corr ([B][ns][8]) for k_finish.  g: the gates' kernels; U: the
-// target (m columns, row stride m), or with bi.count the optimiser's per-run targets
-// (element e's at U + run_target[elem_run[e]] * tgt_stride, *count live elements).
-// The buffers hold the plan's sizes; nothing is allocated.
 // Whether the fused gradient takes its adjoint vectors from the transposed chain
 // (k_fused_grad_chain): the chain switch on, at least two blocks, and the blocks'
 // qubits covering the register (the chain then ends in the forward layout).
@@ -416,6 +365,65 @@ bool fused_grad_uses_chain(const sqh_ctx* c) {
     return S == (1u << c->prog.N) - 1u;
 }
 
+// Launch plan of the fused-block gradient for the context's circuit, B elements of m
+// columns (live: at most B, counted on the device): the shape set by
+// sqh_set_fused_grad_config when it fits, else four 16-column tiles per wavefront from 9
+// qubits or from 64 elements (fewer partials), two below (more wavefronts for small
+// batches), and four wavefronts per workgroup, fewer where every wavefront can then have a
+// compute unit's LDS to itself (256 one-group tasks on 5 and 6 qubits: 62 and 83 us a call
+// instead of 71 and 90; from 1024 tasks on, small workgroups are packed on some of the
+// units: 117 instead of 91) -- the fastest shapes measured on MI355X -- with the scratch it
+// needs.  Returns false when no shape fits the device's LDS.
+bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, bool live, FusedGradPlan& p) {
+    const int N = c->prog.N, nb = (int)c->fplan.qubits.size(), ns = (int)c->prog.slots.size();
+    p.T = 0;
+    if (c->fg_force_tiles && fused_grad_shape_valid(f32, N, m, nb, c->fg_force_tiles, c->fg_force_waves)) {
+        p.T = c->fg_force_tiles;
+        p.waves = c->fg_force_waves;
+    } else {
+        for (int t : {N >= 9 || B >= 64 ? 4 : 2, 4}) {
+            const long long groups = (long long)B * fused_grad_groups(N, m, t);
+            for (int w : {live || groups > 512 ? 4 : groups > 256 ? 2 : 1, 1})
+                if (fused_grad_shape_valid(f32, N, m, nb, t, w)) {
+                    p.T = t;
+                    p.waves = w;
+                    break;
+                }
+            if (p.T) break;
+        }
+    }
+    if (!p.T) return false;
+    size_t pending = 0;
+    p.split = fused_grad_split(f32, N, m, nb, p.T, p.waves, fused_grad_uses_chain(c), B, live, &p.partials, &pending);
+    p.fused_bytes = (size_t)B * nb * 256 * (f32 ? 8 : 16);
+    p.mpart_bytes = (p.partials + pending) * nb * 512 * sizeof(double);
+    p.corr_bytes = (size_t)B * std::max(ns, 1) * 8 * sizeof(double);
+    return true;
+}
+
+// Whether a cost + gradient evaluation of B elements of m columns runs through the fused
+// blocks: the switch on, or automatic and the rule of fused_auto, 4 <= N <= 10, no
+// correction channels, and a launch shape fits.  Below 6 qubits, where the blocks' scratch
+// is several times the tile kernels', automatic batches keep it within 4 GiB.
+bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, int m, bool live,
+                        FusedGradPlan* plan) {
+    if (ts.nch != 0 || !fused_plan_fits(c)) return false;
+    const bool automatic = c->fused_cost == SQH_FUSED_COST_AUTO;
+    if (c->fused_cost == SQH_FUSED_COST_OFF || (automatic && !fused_auto(c, FUSED_GRAD_PASS))) return false;
+    FusedGradPlan p;
+    if (!fused_grad_plan(c, f32, B, m, live, p)) return false;
+    if (automatic && c->prog.N < 6 && p.bytes() > (size_t)4 << 30) return false;
+    if (plan) *plan = p;
+    return true;
+}
+
+// Costs and gradients of B parameter vectors through the fused blocks on stream st:
+// block matrices (into fused), the forward + backward kernel (trace entries into diag,
+// correlation partials into mpart), then each block's gate correlations
+// into corr ([B][ns][8]) for k_finish.  g: the gates' kernels; U: the
+// target (m columns, row stride m), or with bi.count the optimiser's per-run targets
+// (element e's at U + run_target[elem_run[e]] * tgt_stride, *count live elements).
+// The buffers hold the plan's sizes; nothing is allocated.
 int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, const GateKernels& g, const void* U,
                    double* diag, int trace_off, void* fused, double* mpart, double* corr, const BatchIndex& bi,
                    hipStream_t st, bool timed) {
@@ -431,7 +439,9 @@ int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, c
     a.tabs = c->d_ftabs.as<int>();
     a.diag = diag;
     a.mpart = mpart;
-    a.wgs = p.wgs;
+    a.pend = mpart + p.partials * nb * 512;
+    a.split = p.split;
+    a.live_tasks = p.partials;
     a.count = bi.count;
     a.elem_run = bi.elem_run;
     a.run_target = bi.run_target;
@@ -443,8 +453,8 @@ int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, c
     } else {
         HIPTRY(c, launch_fused_grad(f32, N, a, p.T, p.waves, st));
     }
-    HIPTRY(c, launch_fused_block_corr(f32, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb, g, fused, mpart, p.wgs,
-                                      B, corr, ns, st, bi.count));
+    HIPTRY(c, launch_fused_block_corr(f32, c->d_quads.as<uint32_t>(), c->d_ffirst.as<int>(), nb, g, fused, mpart,
+                                      p.split, p.T, B, corr, ns, st, bi.count));
     return SQH_OK;
 }
 
@@ -547,7 +557,7 @@ int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double*
     double* diag = nullptr;
     // the fused blocks' kernels compute their 2x2 kernels from the parameters: no table
     FusedGradPlan fgp;
-    const bool fused_grad = d_grad && !fixed && fused_grad_applies(c, ts, f32, B, m, &fgp);
+    const bool fused_grad = d_grad && !fixed && fused_grad_applies(c, ts, f32, B, m, false, &fgp);
     const bool fused_costs = !fixed && fused_cost_applies(c, d_grad != nullptr, ts);
     if (fixed) {
         kern = fixed->kern;

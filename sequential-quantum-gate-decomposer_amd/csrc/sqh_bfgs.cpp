@@ -404,7 +404,7 @@ int run_batch(sqh_ctx* c, std::vector<Group>& groups, int B, int Ps, const int* 
         size_t fb = 0, mb = 0, cb = 0;
         for (int p = 0; p < (mixed ? 2 : 1); ++p) {
             g.fused[p] = !grouped && c->fused_cost == SQH_FUSED_COST_ON &&
-                         fused_grad_applies(c, trace_spec(c, g.B, g.cols), p == 1, g.B, g.cols, &g.fplan[p]);
+                         fused_grad_applies(c, trace_spec(c, g.B, g.cols), p == 1, g.B, g.cols, true, &g.fplan[p]);
             if (g.fused[p]) {
                 fb = std::max(fb, g.fplan[p].fused_bytes);
                 mb = std::max(mb, g.fplan[p].mpart_bytes);

@@ -256,11 +256,16 @@ int block_config(sqh_ctx* c, bool f32, int rows, int m, int B, BlockCfg* out);
 // Fused-block cost + gradient (sqh_api.cpp): launch shape and scratch sizes, the
 // applicability rule, and the enqueue (no allocation) on a stream.
 struct FusedGradPlan {
-    int T = 0, waves = 0, wgs = 0;
+    int T = 0, waves = 0;
+    FusedGradSplit split;
+    size_t partials = 0;  // of 16 x 16 correlations, then the sums pending
     size_t fused_bytes = 0, mpart_bytes = 0, corr_bytes = 0;
+    size_t bytes() const { return fused_bytes + mpart_bytes + corr_bytes; }
 };
-bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, FusedGradPlan& p);
-bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, int m, FusedGradPlan* plan);
+// live: B is a bound of the count the device holds (the optimiser's rounds).
+bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, bool live, FusedGradPlan& p);
+bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, int m, bool live,
+                        FusedGradPlan* plan);
 int fused_grad_run(sqh_ctx* c, bool f32, const FusedGradPlan& p, int B, int m, const GateKernels& g, const void* U,
                    double* diag, int trace_off, void* fused, double* mpart, double* corr, const BatchIndex& bi,
                    hipStream_t st, bool timed);

@@ -139,9 +139,73 @@ __global__ __launch_bounds__(64 * kQuadWaves) void k_fuse_blocks(const uint32_t*
     for (int k = 0; k < 4; ++k) o[quad_row(q, k) * 16 + col] = cvt<R>(v[k]);
 }
 
-// Sums the workgroup partials of the block's correlation M_b (SPLIT: a workgroup per (block,
-// element), each of its eight wavefronts every eighth partial, then only the first goes on;
-// else a wavefront per (block, element), four elements per workgroup), starts from x = the
+// Entries M, M + step, ... of C partials (the first `left` of them, the others count as
+// zero), each entry's added as a binary tree.
+template <int C, int E>
+__device__ __forceinline__ void partial_nodes(const double* __restrict__ M, unsigned stride, int left, int step,
+                                              double (&v)[E]) {
+    double t[E][C];
+#pragma unroll
+    for (int k = 0; k < C; ++k)
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const double x = M[(k < left ? k : 0) * stride + i * step];
+            t[i][k] = k < left ? x : 0.0;
+        }
+#pragma unroll
+    for (int w = 1; w < C; w *= 2)
+#pragma unroll
+        for (int k = 0; k < C; k += 2 * w)
+#pragma unroll
+            for (int i = 0; i < E; ++i) t[i][k] += t[i][k + w];
+#pragma unroll
+    for (int i = 0; i < E; ++i) v[i] = t[i][0];
+}
+
+// Sums over an element's n partials, 1 << up of them per chunk: FusedGradSplit's tree from
+// the partials' level on, then its chunks in order.
+template <int E>
+__device__ __forceinline__ void partial_sum(const double* __restrict__ M, unsigned stride, int n, int up, int step,
+                                            double (&out)[E]) {
+    constexpr int C = E == 1 ? 64 : 16;  // as many partials at a time as registers hold
+#pragma unroll
+    for (int i = 0; i < E; ++i) out[i] = 0.0;
+    for (int c = 0; c < n; c += 1 << up) {
+        const int left = min(1 << up, n - c);
+        const double* P = M + (long long)c * stride;
+        double v[E];
+        if (left <= 4) {
+            partial_nodes<4>(P, stride, left, step, v);
+        } else if (left <= 16) {
+            partial_nodes<16>(P, stride, left, step, v);
+        } else {
+            double s[128 / C][E];
+#pragma unroll
+            for (int j = 0; j < 128 / C; ++j) {
+                if (C * j < left) {
+                    partial_nodes<C>(P + C * j * stride, stride, left - C * j, step, s[j]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < E; ++i) s[j][i] = 0.0;
+                }
+            }
+#pragma unroll
+            for (int w = 1; w < 128 / C; w *= 2)
+#pragma unroll
+                for (int j = 0; j < 128 / C; j += 2 * w)
+#pragma unroll
+                    for (int i = 0; i < E; ++i) s[j][i] += s[j + w][i];
+#pragma unroll
+            for (int i = 0; i < E; ++i) v[i] = s[0][i];
+        }
+#pragma unroll
+        for (int i = 0; i < E; ++i) out[i] += v[i];
+    }
+}
+
+// Sums the partials of the block's correlation M_b (SPLIT: a workgroup per (block,
+// element), an entry per thread, then only the first wavefront goes on; else a wavefront per
+// (block, element), four elements per workgroup), starts from x = the
 // columns of F_b and y = the columns of M_b and walks the gates backwards: x <- G^dagger x,
 // the pair correlations of y and x summed over the wavefront, y <- G^T y.
 // corr[e][slot][8] is the register-tile adjoint's layout.
@@ -151,32 +215,52 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
                                                           const cpx<R>* __restrict__ kern, long long kern_bstride,
                                                           const double* __restrict__ params, int pstride,
                                                           const Slot* __restrict__ slots, const cpx<R>* __restrict__ F,
-                                                          const double* __restrict__ mpart, int wgs, int B,
-                                                          double* __restrict__ corr, int ns,
+                                                          const double* __restrict__ mpart, FusedGradSplit sp, int T,
+                                                          int B, double* __restrict__ corr, int ns,
                                                           const int* __restrict__ count) {
     constexpr int E = SPLIT ? 1 : 4;  // elements per workgroup
-    __shared__ double sums[SPLIT ? 8 : 4][512];  // 256 real, then 256 imaginary parts
+    __shared__ double sums[E][512];  // 256 real, then 256 imaginary parts
     __shared__ cpx<double> states[E][512], tables[E][64 * 4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int blk = blockIdx.x % nb, e = (blockIdx.x / nb) * E + (SPLIT ? 0 : wave);
-    if (count) B = min(*count, B);
+    if (count) {
+        B = min(*count, B);
+        fused_grad_split_live(sp, B, T);
+    }
     if (e >= B) return;  // the whole workgroup, or a wavefront that shares nothing
     {
-        const double* M = mpart + ((long long)e * wgs * nb + blk) * 512;
-        double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll 4
-        for (int p = SPLIT ? wave : 0; p < wgs; p += SPLIT ? 8 : 1) {
+        const int l = e < sp.n0 ? sp.l0 : sp.l1, n = fused_grad_tasks(sp.groups, l);
+        const long long before = (long long)min(e, sp.n0) * fused_grad_tasks(sp.groups, sp.l0) +
+                                 (long long)max(e - sp.n0, 0) * n;
+        const double* M = mpart + (before * nb + blk) * 512;
+        const unsigned stride = (unsigned)nb * 512;  // 128 partials within 32 bits
+        const int up = fused_grad_levels(T) - l;
+        if constexpr (SPLIT) {
+            double v[1];
+            partial_sum(M + threadIdx.x, stride, n, up, 0, v);
+            sums[0][threadIdx.x] = v[0];
+            __syncthreads();
+            if (wave != 0) return;
+        } else {
+            double* s = sums[wave] + lane;
+            M += lane;
+            if (n <= 4 && n <= 1 << up) {
+                double v[8];
+                if (n == 1) partial_nodes<1>(M, stride, 1, 64, v);
+                else partial_nodes<4>(M, stride, n, 64, v);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc[i] += M[(long long)p * nb * 512 + 64 * i + lane];
+                for (int i = 0; i < 8; ++i) s[64 * i] = v[i];
+            } else {
+#pragma unroll 1
+                for (int i = 0; i < 8; i += 2) {
+                    double v[2];
+                    partial_sum(M + 64 * i, stride, n, up, 64, v);
+                    s[64 * i] = v[0];
+                    s[64 * i + 64] = v[1];
+                }
+            }
+            quad_fence();
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) sums[wave][64 * i + lane] = acc[i];
-    }
-    if constexpr (SPLIT) {
-        __syncthreads();
-        if (wave != 0) return;
-    } else {
-        quad_fence();
     }
     const int col = lane & 15, z = lane >> 4;
     cpx<double>* sx = states[SPLIT ? 0 : wave];
@@ -192,15 +276,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
         const int at = quad_row(q, k) * 16 + col;
         x[k] = widen(Fb[at]);
         const double* sw = sums[SPLIT ? 0 : wave];
-        double yr = sw[at], yi = sw[256 + at];
-        if constexpr (SPLIT) {
-#pragma unroll
-            for (int w = 1; w < 8; ++w) {
-                yr += sums[w][at];
-                yi += sums[w][256 + at];
-            }
-        }
-        y[k] = mk(yr, yi);
+        y[k] = mk(sw[at], sw[256 + at]);
     }
     for (int pe = p1; pe > p0; pe -= 64) {
         const int p = max(p0, pe - 64), cnt = pe - p;
@@ -296,8 +372,8 @@ hipError_t launch_fuse_deriv_blocks(const uint32_t* ops, const int* first, int n
 }
 
 hipError_t launch_fused_block_corr(bool f32, const uint32_t* ops, const int* first, int nb, const GateKernels& g,
-                                   const void* F, const double* mpart, int wgs, int B, double* corr, int ns,
-                                   hipStream_t s, const int* count) {
+                                   const void* F, const double* mpart, const FusedGradSplit& sp, int T, int B,
+                                   double* corr, int ns, hipStream_t s, const int* count) {
     if ((long long)B * nb == 0) return hipSuccess;
     // With a wavefront per SIMD's worth of (block, element) pairs each sums its own
     // partials; below that, as with one vector, the sum is the longer part and is split.
@@ -306,7 +382,7 @@ hipError_t launch_fused_block_corr(bool f32, const uint32_t* ops, const int* fir
 #define SQH_CORR(R, SP)                                                                                       \
     hipLaunchKernelGGL((k_fused_block_corr<R, SP>), dim3(grid), dim3(SP ? 512 : 256), 0, s, ops, first, nb,    \
                        (const cpx<R>*)g.kern, g.kern_bstride, g.params, g.pstride, g.slots, (const cpx<R>*)F,  \
-                       mpart, wgs, B, corr, ns, count)
+                       mpart, sp, T, B, corr, ns, count)
     if (f32 && split) SQH_CORR(float, true);
     else if (f32) SQH_CORR(float, false);
     else if (split) SQH_CORR(double, true);

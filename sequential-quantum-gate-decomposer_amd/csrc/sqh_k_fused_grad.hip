@@ -10,8 +10,8 @@
 //                                                              (MFMA on transposed tiles)
 //   Y_{b-1} = F_b^T Y_b                                        (MFMA)
 // so that dTr/dtheta = sum_ik (dF_b/dtheta)_ik M_b[i][k] for a parameter of block b.
-// A wavefront sums its M_b over its column groups in registers and its own partial slot, so
-// no wavefront waits for another; k_fused_block_corr then sums the partials and runs the
+// A wavefront sums its M_b over its column groups in registers and its own partials, so no
+// wavefront waits for another; k_fused_block_corr then sums the partials and runs the
 // block's gates backwards, producing each gate's 2x2 correlations in the layout of the
 // register-tile adjoint kernel, from which k_finish forms the gradient.
 //
@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "sqh_device.h"
 #include "sqh_fused_chain.h"
@@ -60,26 +61,44 @@ __device__ __forceinline__ void fg_mma(const FcA<R>& A, const R (&xr)[T][4], con
     }
 }
 
-// What a wavefront of the gradient kernels works on: element e and the column groups
-// first .. last - 1 of it, whose correlations it sums in partial slot `slot`.
+// What a wavefront of the gradient kernels works on: the column groups first .. last - 1 of
+// element e, a node of the summation tree (FusedGradSplit), whose correlations go to part;
+// sums pending at level l > 0 of the tree wait in pend + (l - 1) nb 512, at level 0 in part.
 struct FgTask {
-    int e, slot, first, last;
+    int e, first, last;
     bool live;
+    double *part, *pend;
 };
+template <int T>
 __device__ __forceinline__ FgTask fg_task(const FusedGradArgs& a, int wv) {
-    // XCD-ordered workgroups (the grid is a multiple of 8); with a live count (the
-    // optimiser's rounds) the plain order, so the live elements spread over the XCDs
-    int B = a.B;
-    long long lwg = blockIdx.x;
-    if (a.count) B = min(*a.count, a.B);
-    else lwg = (long long)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-    const long long task = lwg * (blockDim.x >> 6) + wv;
+    FusedGradSplit sp = a.split;
+    // The workgroups of either part of the split ordered for the XCDs (multiples of 8);
+    // with a live count (the optimiser's rounds) the plain order, so the live elements
+    // spread over the XCDs.
+    unsigned wg = blockIdx.x, wgs = a.wg0;
+    const bool rest = !a.count && wg >= wgs;
+    if (a.count) {
+        fused_grad_split_live(sp, min(*a.count, a.B), T);
+    } else {
+        if (rest) {
+            wg -= wgs;
+            wgs = gridDim.x - wgs;
+        }
+        wg = (wg & 7) * (wgs >> 3) + (wg >> 3);
+    }
+    const int per0 = fused_grad_tasks(sp.groups, sp.l0), l = rest ? sp.l1 : sp.l0;
+    const int per = fused_grad_tasks(sp.groups, l), n = rest ? a.B - sp.n0 : sp.n0;
+    const long long id = (long long)wg * (blockDim.x >> 6) + wv;
     FgTask t;
-    t.e = (int)(task / a.wgs);
-    t.slot = (int)(task % a.wgs);
-    t.first = t.slot * a.per;
-    t.last = min(t.first + a.per, a.groups);
-    t.live = t.e < B;
+    t.live = id < (long long)n * per;
+    const int k = (int)(id / per), c = (int)(id % per);
+    t.e = (rest ? sp.n0 : 0) + k;
+    t.first = c << l;
+    t.last = min((c + 1) << l, sp.groups);
+    const long long before = rest ? (long long)sp.n0 * per0 : 0;
+    const long long size = (long long)a.nb * 512;
+    t.part = a.mpart + (before + id) * size;
+    t.pend = a.pend + (before * max(sp.l0 - 1, 0) + id * max(l - 1, 0)) * size;
     return t;
 }
 
@@ -102,56 +121,82 @@ __device__ __forceinline__ void fg_load_target(const cpx<R>* __restrict__ U, con
     }
 }
 
-// M += Y X^T over the wavefront's vector columns (Y and X: item i of tile t is row 4 i +
-// lane / 16 of its vector columns), tile by tile through the region as two transposed
-// tiles, added to the wavefront's own partial of the block at M: [256] real, then [256]
-// imaginary parts.  The partial stays in the caches between the column groups, and no
-// wavefront waits for another: summing four wavefronts' correlations in LDS behind two
-// barriers per block kept them in step, all in their exchanges while the matrix cores idled.
+// M_b of a column group, Y X^T over the wavefront's vector columns (Y and X: item i of tile
+// t is row 4 i + lane / 16 of its vector columns), tile by tile through the region as two
+// transposed tiles, added to the task's sums of block b: [256] real, then [256] imaginary
+// parts.  No wavefront waits for another: summing four wavefronts' correlations in LDS behind
+// two barriers per block kept them in step, all in their exchanges while the matrix cores
+// idled.  idx: the group's number in the task; the sums pending are those of idx's set bits.
 template <typename R, int T, typename Y>
 __device__ __forceinline__ void fg_correlate(R* lds, const Y& yr, const Y& yi, const R (&xr)[T][4],
-                                             const R (&xi)[T][4], double* __restrict__ M, bool first, int lane) {
+                                             const R (&xi)[T][4], const FgTask& task, int nb, int b, int cg,
+                                             int lane) {
     typedef FcMfma<R> MF;
     const int nl = lane & 15, g = lane >> 4;
-    constexpr bool D64 = sizeof(R) == 8;
-    typename MF::V mr, mi;
-    double pr[4], pi[4];
+    const unsigned idx = cg - task.first;
+    const bool last = cg + 1 == task.last;
+    const unsigned carry = idx & ~(idx + 1);  // the levels whose second half this group completes
+    unsigned set = last ? idx : carry;
+    auto at_level = [&](int l) { return (l ? task.pend + (long long)(l - 1) * nb * 512 : task.part) + b * 512; };
+    double pr[4] = {0, 0, 0, 0}, pi[4] = {0, 0, 0, 0};  // the first of them, on its way while the tiles run
+    auto load = [&]() {
+        const double* M = at_level(__builtin_ctz(set));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int at = MF::row(r, g) * 16 + nl;
+            pr[r] = M[at];
+            pi[r] = M[256 + at];
+        }
+    };
+    if (set) load();
+    double vr[4], vi[4];
+#pragma unroll
+    for (int h = 0; h < T / 2; ++h) {
+        typename MF::V mr = {0, 0, 0, 0}, mi = {0, 0, 0, 0};
+#pragma unroll
+        for (int t = 2 * h; t < 2 * h + 2; ++t) {
+            R* yb = lds + (T >= 4 && (t & 1) ? 1024 : 0);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int at = fg_tile(4 * s + g, nl);
+                yb[at] = yr[t][s];
+                yb[256 + at] = yi[t][s];
+                yb[512 + at] = xr[t][s];
+                yb[768 + at] = xi[t][s];
+            }
+            fc_wave_fence();
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int at = fg_tile(nl, 4 * s + g);
+                const R yvr = yb[at], yvi = yb[256 + at], xvr = yb[512 + at], xvi = yb[768 + at];
+                mr = MF::op(yvr, xvr, mr);
+                mi = MF::op(yvr, xvi, mi);
+                mr = MF::op_neg(yvi, xvi, mr);
+                mi = MF::op(yvi, xvr, mi);
+            }
+            fc_wave_fence();
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            vr[r] = h ? vr[r] + (double)mr[r] : (double)mr[r];
+            vi[r] = h ? vi[r] + (double)mi[r] : (double)mi[r];
+        }
+    }
+    while (set) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            vr[r] = pr[r] + vr[r];
+            vi[r] = pi[r] + vi[r];
+        }
+        set &= set - 1;
+        if (set) load();
+    }
+    double* M = at_level(last ? 0 : __builtin_popcount(carry));
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const int idx = MF::row(r, g) * 16 + nl;
-        pr[r] = first ? 0.0 : M[idx];
-        pi[r] = first ? 0.0 : M[256 + idx];
-        mr[r] = D64 ? (R)pr[r] : (R)0;
-        mi[r] = D64 ? (R)pi[r] : (R)0;
-    }
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        R* yb = lds + (T >= 4 && (t & 1) ? 1024 : 0);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int at = fg_tile(4 * s + g, nl);
-            yb[at] = yr[t][s];
-            yb[256 + at] = yi[t][s];
-            yb[512 + at] = xr[t][s];
-            yb[768 + at] = xi[t][s];
-        }
-        fc_wave_fence();
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int at = fg_tile(nl, 4 * s + g);
-            const R yvr = yb[at], yvi = yb[256 + at], xvr = yb[512 + at], xvi = yb[768 + at];
-            mr = MF::op(yvr, xvr, mr);
-            mi = MF::op(yvr, xvi, mi);
-            mr = MF::op_neg(yvi, xvi, mr);
-            mi = MF::op(yvi, xvr, mi);
-        }
-        fc_wave_fence();
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int idx = MF::row(r, g) * 16 + nl;
-        M[idx] = D64 ? (double)mr[r] : pr[r] + (double)mr[r];
-        M[256 + idx] = D64 ? (double)mi[r] : pi[r] + (double)mi[r];
+        const int at = MF::row(r, g) * 16 + nl;
+        M[at] = vr[r];
+        M[256 + at] = vi[r];
     }
 }
 
@@ -166,14 +211,13 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const in
     extern __shared__ __align__(16) unsigned char fg_smem[];
     int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const FgTask task = fg_task(a, wv);
+    const FgTask task = fg_task<T>(a, wv);
     if (!task.live) return;
     const int e = task.e, m = a.m;
     const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 512 * T};
     const cpx<R>* U = static_cast<const cpx<R>*>(a.U);
     if (a.count) U += (long long)a.run_target[a.elem_run[e]] * a.tgt_stride;
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.nb * 256;
-    double* const part = a.mpart + ((long long)e * a.wgs + task.slot) * a.nb * 512;
     for (int cg = task.first; cg < task.last; ++cg) {
         const int c0 = cg * W;
         const int nl = lane & 15, g = lane >> 4;
@@ -218,9 +262,9 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const in
             }
         }
         // backward: X_{b-1} = F^dagger X_b, M_b += Y_b X_{b-1}^T, Y_{b-1} = F^T Y_b
+        A.load_t(Fe + (long long)(a.nb - 1) * 256, nl, g);
         for (int b = a.nb - 1; b >= 0; --b) {
             const int* tab = tabs + b * kLaneTab;
-            A.load_t(Fe + (long long)b * 256, nl, g);
             fg_mma<R, T, true>(A, xr, xi, dr, di);
 #pragma unroll
             for (int t = 0; t < T; ++t)
@@ -229,9 +273,10 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const in
                     xr[t][s] = dr[t][s];
                     xi[t][s] = di[t][s];
                 }
-            fg_correlate<R, T>(lds.p, yr, yi, xr, xi, part + b * 512, cg == task.first, lane);
+            fg_correlate<R, T>(lds.p, yr, yi, xr, xi, task, a.nb, b, cg, lane);
             if (b == 0) break;
             fg_mma<R, T, false>(A, yr, yi, dr, di);
+            A.load_t(Fe + (long long)(b - 1) * 256, nl, g);
             const int* tn = tab - kLaneTab;
             int at[4], an[4];
             Reg::full_at(at, tab, tab[LT_LANE + lane]);
@@ -270,17 +315,15 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
     extern __shared__ __align__(16) unsigned char fg_smem[];
     int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const FgTask task = fg_task(a, wv);
+    const FgTask task = fg_task<T>(a, wv);
     if (!task.live) return;
     const int e = task.e, m = a.m;
     const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 512 * T};
     const cpx<R>* U = static_cast<const cpx<R>*>(a.U);
     if (a.count) U += (long long)a.run_target[a.elem_run[e]] * a.tgt_stride;
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.nb * 256;
-    double* const part = a.mpart + ((long long)e * a.wgs + task.slot) * a.nb * 512;
     for (int cg = task.first; cg < task.last; ++cg) {
         const int c0 = cg * W;
-        const bool first = cg == task.first;
         asm volatile("" : "+v"(lane));  // no lane's addresses kept in registers from group to group
         const int nl = lane & 15, g = lane >> 4;
         // phase 1: Z_1 in block 0's grouping, X = the target's columns there, and the trace
@@ -311,7 +354,12 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
             fc_column_sums<N, T>(sr, si, a.diag + 2 * ((long long)e * m + c0), c0, m, lane);
         }
         fg_load_target<R, N, T>(U, tabs, c0, m, lane, xr, xi);
-        fg_correlate<R, T>(lds.p, zr, zi, xr, xi, part, first, lane);
+        // The block that X, then Z pass next, on its way before the branches of the sums; with
+        // two tiles it would cost a wavefront per SIMD.
+        constexpr bool AHEAD = T == 4;
+        FcA<R> An;
+        if constexpr (AHEAD) An.load_n(Fe, nl, g);
+        fg_correlate<R, T>(lds.p, zr, zi, xr, xi, task, a.nb, 0, cg, lane);
         // phase 2, one step up: X_b into block b + 1's grouping, Z_{b+2} (block b + 1's
         // grouping, as a result) from Z_{b+1} -- block 0's operand for the first step, the
         // last step's result after it -- then M_{b+1}.  The first step runs on its own, so
@@ -324,10 +372,10 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
             Reg::full_at(at, tab, tab[LT_LANE + lane]);
             Reg::full_at(an, tn, tn[LT_LANE + lane]);
             {
-                FcA<R> An;
-                An.load_n(Fe + (long long)b * 256, nl, g);
                 typename MF::V dr[T], di[T];
+                if constexpr (!AHEAD) An.load_n(Fe + (long long)b * 256, nl, g);
                 fg_mma<R, T, false>(An, xr, xi, dr, di);
+                if constexpr (AHEAD) An.load_n(Fe + (long long)(b + 1) * 256, nl, g);
                 lds.template store_full<T>(at, tab, dr, di);
                 lds.load_full(an, tn, xr, xi);
             }
@@ -343,8 +391,7 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
                 }
                 R vr[T][4], vi[T][4];
                 lds.load_full(an, tn, vr, vi);
-                FcA<R> An;
-                An.load_n(Fe + (long long)(b + 1) * 256, nl, g);
+                if constexpr (!AHEAD) An.load_n(Fe + (long long)(b + 1) * 256, nl, g);
                 fg_mma<R, T, true>(An, vr, vi, er, ei);
             } else {
                 // Z_nb: the selector, row rho = c + trace_off of column c
@@ -359,7 +406,7 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
                     }
                 }
             }
-            fg_correlate<R, T>(lds.p, er, ei, xr, xi, part + (b + 1) * 512, first, lane);
+            fg_correlate<R, T>(lds.p, er, ei, xr, xi, task, a.nb, b + 1, cg, lane);
         };
         step(0, std::true_type{});
         for (int b = 1; b + 1 < a.nb; ++b) step(b, std::false_type{});
@@ -371,16 +418,13 @@ size_t fused_grad_lds_bytes(bool f32, int nb, int T, int waves) {
     return (f32 ? 8 : 16) * (size_t)(256 * T) * waves;  // a region per wavefront
 }
 
+// The kernel of a shape, or null.
 template <typename R>
-static hipError_t launch_fg(int N, const FusedGradArgs& a, int T, int grid, int threads, size_t shm, hipStream_t s) {
-#define SQH_FG_CASE(n, t)                                                                                    \
-    if (N == n && T == t) {                                                                                  \
-        if (a.tmaps)                                                                                         \
-            hipLaunchKernelGGL((k_fused_grad_chain<R, n, t>), dim3(grid), dim3(threads), shm, s, a, a.tabs, a.tmaps); \
-        else                                                                                                 \
-            hipLaunchKernelGGL((k_fused_grad<R, n, t>), dim3(grid), dim3(threads), shm, s, a, a.tabs);       \
-        return hipGetLastError();                                                                            \
-    }
+static const void* fg_kernel(int N, int T, bool chain) {
+#define SQH_FG_CASE(n, t)                                                    \
+    if (N == n && T == t)                                                    \
+        return chain ? reinterpret_cast<const void*>(&k_fused_grad_chain<R, n, t>) \
+                     : reinterpret_cast<const void*>(&k_fused_grad<R, n, t>);
     SQH_FG_CASE(4, 4)
     SQH_FG_CASE(5, 4)
     SQH_FG_CASE(6, 4)
@@ -395,12 +439,15 @@ static hipError_t launch_fg(int N, const FusedGradArgs& a, int T, int grid, int 
     SQH_FG_CASE(8, 2)
     SQH_FG_CASE(9, 2)
 #undef SQH_FG_CASE
-    return hipErrorInvalidValue;
+    return nullptr;
+}
+static const void* fg_kernel(bool f32, int N, int T, bool chain) {
+    return f32 ? fg_kernel<float>(N, T, chain) : fg_kernel<double>(N, T, chain);
 }
 
 // Column groups (one per wavefront) of an element: 16 T vector columns per wavefront,
 // 2^N / 16 of them per matrix column.
-static int fg_groups(int N, int m, int T) {
+int fused_grad_groups(int N, int m, int T) {
     const int W = 16 * T / ((1 << N) >> 4);
     return W < 1 ? 0 : (m + W - 1) / W;
 }
@@ -408,33 +455,96 @@ static int fg_groups(int N, int m, int T) {
 bool fused_grad_shape_valid(bool f32, int N, int m, int nb, int T, int waves) {
     if (N < 4 || N > kFusedCostMaxQubits || (T != 2 && T != 4) || m <= 0 || nb <= 0) return false;
     if (waves != 1 && waves != 2 && waves != 4 && waves != 8) return false;
-    const int groups = fg_groups(N, m, T);
-    return groups > 0 && groups % waves == 0 && fused_grad_lds_bytes(f32, nb, T, waves) <= device_max_lds();
+    return fused_grad_groups(N, m, T) > 0 && fused_grad_lds_bytes(f32, nb, T, waves) <= device_max_lds();
 }
 
-// Column groups a wavefront takes one after another, adding to one partial: as many as
-// leave two wavefronts per SIMD (2048), the most that are resident with four tiles.  Fewer
-// partials are then written and summed; a small batch keeps a group per wavefront.
-int fused_grad_per(int N, int m, int T, int B) {
-    const long long total = (long long)fg_groups(N, m, T) * B;
-    return (int)std::max<long long>(1, std::min<long long>(total / 2048, fg_groups(N, m, T)));
+// Wavefronts of the kernel that are resident together on the current device.
+static int fg_resident(const void* kernel, size_t shm, int waves) {
+    int dev = 0, cus = 0, wgs = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&wgs, kernel, 64 * waves, shm) != hipSuccess || wgs < 1) {
+        (void)hipGetLastError();
+        return 2048;
+    }
+    return cus * wgs * waves;
 }
 
-int fused_grad_wgs(int N, int m, int T, int B) {
-    const int per = fused_grad_per(N, m, T, B);
-    return (fg_groups(N, m, T) + per - 1) / per;
+// The card runs a launch in rounds of its resident wavefronts, and a last round that is not
+// full costs as much as a full one.  So the bulk of the elements runs in the largest tasks
+// (few partials) that fill whole rounds, and the rest in smaller ones.  Unit of the estimate:
+// a column group on a full card (83 us at 8 qubits in complex128); a round with fewer
+// wavefronts per SIMD is shorter by less than their share, and a partial costs its way to
+// memory and back.  Gradients of 384, 512, 520, 640 and 1000 vectors (8 qubits, 264 angles,
+// complex128): 1.06, 1.40, 1.44, 1.85 and 2.75 ms; in equal tasks of total / 2048 groups,
+// rounded down, 1.56, 1.41, 2.08, 2.56 and 3.94; a wavefront per group, four summed in LDS,
+// 1.32, 1.72, 1.78, 2.13 and 3.30.
+constexpr double kFgPartialCost = 1e-4;
+FusedGradSplit fused_grad_split(bool f32, int N, int m, int nb, int T, int waves, bool chain, int B, bool live,
+                                size_t* partials, size_t* pending) {
+    FusedGradSplit s;
+    s.groups = fused_grad_groups(N, m, T);
+    s.resident = 2048;
+    s.n0 = B;
+    const long long total = (long long)B * s.groups;
+    const int levels = fused_grad_levels(T);
+    if (live || total > 1024)
+        s.resident = fg_resident(fg_kernel(f32, N, T, chain), fused_grad_lds_bytes(f32, nb, T, waves), waves);
+    const long long R = s.resident;
+    if (live) {
+        FusedGradSplit most = s;
+        fused_grad_split_live(most, B, T);
+        // most tasks of any count up to B (fused_grad_split_live)
+        *partials = (size_t)std::min(total, std::max(4 * R + B, (long long)B * fused_grad_tasks(s.groups, levels)));
+        *pending = *partials * std::max(most.l0 - 1, 0);
+        return s;
+    }
+    auto tasks = [&](long long n, int l) { return n * fused_grad_tasks(s.groups, l); };
+    if (total > R) {
+        const double w = std::max(1.0, R / 1024.0);  // wavefronts per SIMD
+        auto cost = [&](long long n, int l) {
+            const long long t = tasks(n, l), rounds = t / R, over = t % R;
+            const double part = over ? 0.3 + 0.7 * std::ceil(over * w / R) / w : 0.0;
+            return (rounds + part) * (1 << l) + kFgPartialCost * t;
+        };
+        double best = -1.0;
+        for (int l = 0; l <= levels; ++l) {
+            if (l > 0 && (1 << (l - 1)) >= s.groups) break;
+            const long long full = tasks(B, l) / R * R / fused_grad_tasks(s.groups, l);  // elements in whole rounds
+            for (long long n : {full, (long long)B}) {
+                for (int k = 0; k <= (n < B ? l : 0); ++k) {
+                    const double c = (n ? cost(n, l) : 0.0) + (n < B ? cost(B - n, k) : 0.0);
+                    if (best < 0.0 || c < best) {
+                        best = c;
+                        s.n0 = (int)n;
+                        s.l0 = l;
+                        s.l1 = k;
+                    }
+                }
+            }
+        }
+    }
+    *partials = (size_t)(tasks(s.n0, s.l0) + tasks(B - s.n0, s.l1));
+    *pending = (size_t)(tasks(s.n0, s.l0) * std::max(s.l0 - 1, 0) + tasks(B - s.n0, s.l1) * std::max(s.l1 - 1, 0));
+    return s;
 }
 
 hipError_t launch_fused_grad(bool f32, int N, FusedGradArgs a, int T, int waves, hipStream_t s) {
     if (a.B <= 0 || !fused_grad_shape_valid(f32, N, a.m, a.nb, T, waves)) return hipErrorInvalidValue;
-    a.groups = fg_groups(N, a.m, T);
-    a.per = fused_grad_per(N, a.m, T, a.B);
-    if (a.wgs != fused_grad_wgs(N, a.m, T, a.B)) return hipErrorInvalidValue;  // the partials' layout the caller sized
-    const long long wgs_total = ((long long)a.B * a.wgs + waves - 1) / waves;
-    const int grid = (int)((wgs_total + 7) / 8 * 8);
-    const size_t shm = fused_grad_lds_bytes(f32, a.nb, T, waves);
-    return f32 ? launch_fg<float>(N, a, T, grid, 64 * waves, shm, s)
-               : launch_fg<double>(N, a, T, grid, 64 * waves, shm, s);
+    const void* kernel = fg_kernel(f32, N, T, a.tmaps != nullptr);
+    if (!kernel || a.split.groups != fused_grad_groups(N, a.m, T) || a.split.resident <= 0) return hipErrorInvalidValue;
+    auto wgs = [&](long long tasks) { return (int)(((tasks + waves - 1) / waves + 7) / 8 * 8); };
+    int grid;
+    if (a.count) {
+        grid = wgs((long long)a.live_tasks);
+    } else {
+        a.wg0 = wgs((long long)a.split.n0 * fused_grad_tasks(a.split.groups, a.split.l0));
+        grid = a.wg0 + wgs((long long)(a.B - a.split.n0) * fused_grad_tasks(a.split.groups, a.split.l1));
+    }
+    const int* tabs = a.tabs;
+    const int* tmaps = a.tmaps;
+    void* args[] = {&a, &tabs, &tmaps};  // k_fused_grad takes the first two
+    return hipLaunchKernel(kernel, dim3(grid), dim3(64 * waves), args, fused_grad_lds_bytes(f32, a.nb, T, waves), s);
 }
 
 }  // namespace sqh

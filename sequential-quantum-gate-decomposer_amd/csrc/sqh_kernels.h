@@ -152,17 +152,42 @@ hipError_t launch_fuse_deriv_blocks(const uint32_t* ops, const int* first, int n
 
 // Cost and gradient through the fused blocks (sqh_k_fused_grad.hip): the forward pass
 // and trace entries as the cost kernel, then the blocks backwards with the trace
-// selector, writing per wavefront and block the 16x16 correlation partials
-// mpart[B][wgs][nb][512] (256 real, then 256 imaginary parts).  T: 16-column tiles per wavefront.
+// selector, writing 16x16 correlation partials [512] (256 real, then 256 imaginary parts).
+// T: 16-column tiles per wavefront; a column group is what a wavefront works on at a time.
+//
+// How the correlations of an element's column groups are summed, whoever computes them: the
+// groups of each chunk of 2^fused_grad_levels(T) as a binary tree over aligned pairs, then
+// the chunks in order.  A wavefront takes 2^l aligned groups, a node of the tree, as its
+// task and leaves the node's sum in a partial; k_fused_block_corr does the rest of the tree.
+// So the result's bits depend neither on l nor on the batch (nor on T: a group of four tiles
+// is a node of two groups of two).
+struct FusedGradSplit {
+    int groups = 0;        // column groups per element
+    int resident = 0;      // wavefronts of the kernel the card holds at once
+    int n0 = 0;            // the first n0 elements run in tasks of 2^l0 groups,
+    int l0 = 0, l1 = 0;    // the others in tasks of 2^l1
+};
+__host__ __device__ constexpr int fused_grad_levels(int T) { return T == 4 ? 6 : 7; }
+__host__ __device__ inline int fused_grad_tasks(int groups, int l) { return (groups + (1 << l) - 1) >> l; }
+// The split of a launch whose element count only the device knows: at least two tasks per
+// resident wavefront (up to a whole chunk per task).  The rounds of 512 runs on 8 qubits of
+// which 8 go on take 20 ms; with tasks sized for all 512, 44.
+__host__ __device__ inline void fused_grad_split_live(FusedGradSplit& s, int live, int T) {
+    const long long total = (long long)live * s.groups;
+    s.n0 = live;
+    s.l0 = s.l1 = 0;
+    while (s.l0 < fused_grad_levels(T) && (total >> (s.l0 + 1)) >= 2LL * s.resident) ++s.l0;
+}
 struct FusedGradArgs {
     const void* U = nullptr;  // target, rows = 2^N, m columns, row stride m
     int m = 0, trace_off = 0, B = 0, nb = 0;
     const void* F = nullptr;  // [B][nb][16][16] block matrices
     double* diag = nullptr;
-    double* mpart = nullptr;
-    int wgs = 0;     // partials per element
-    int groups = 0;  // column groups per element (set by the launcher)
-    int per = 1;     // column groups per partial (set by the launcher)
+    double* mpart = nullptr;  // [task][nb][512]
+    double* pend = nullptr;  // sums pending in a task, l - 1 partials per task (level 0's wait in mpart)
+    FusedGradSplit split;
+    int wg0 = 0;             // workgroups of the first n0 elements (set by the launcher)
+    size_t live_tasks = 0;   // with count: most tasks (the partials of fused_grad_split)
     const int* tabs = nullptr;  // lane tables [nb][kLaneTab]
     // optional optimiser indirection: live elements *count (of B), element e's target at
     // U + run_target[elem_run[e]] * tgt_stride
@@ -176,19 +201,23 @@ struct FusedGradArgs {
     const int* tmaps = nullptr;
 };
 // Launch shape: T 16-column tiles per wavefront (2 or 4; 4 at 10 qubits), waves 1, 2, 4
-// or 8 per workgroup dividing the element's column groups; wgs = partials per element of a
-// batch of B.
+// or 8 per workgroup.
 bool fused_grad_shape_valid(bool f32, int N, int m, int nb, int T, int waves);
-int fused_grad_wgs(int N, int m, int T, int B);
+int fused_grad_groups(int N, int m, int T);  // column groups per element
+// The split of a batch of B (live: of at most B, counted on the device) and the partials and
+// pending sums it needs.
+FusedGradSplit fused_grad_split(bool f32, int N, int m, int nb, int T, int waves, bool chain, int B, bool live,
+                                size_t* partials, size_t* pending);
 size_t fused_grad_lds_bytes(bool f32, int nb, int T, int waves);
 hipError_t launch_fused_grad(bool f32, int N, FusedGradArgs a, int T, int waves, hipStream_t s);
-// Per (element, block): the partials summed, then the block's gates run backwards on
+// Per (element, block): the partials summed (split as the kernel's), then the block's gates
+// run backwards on
 // 16-dimensional vectors (from the columns of F, the block matrices [B][nb][16][16]),
 // giving each parametric slot's 2x2 correlations in corr[B][ns][8] (the register-tile
 // adjoint's layout, one partial per element).
 hipError_t launch_fused_block_corr(bool f32, const uint32_t* ops, const int* first, int nb, const GateKernels& g,
-                                   const void* F, const double* mpart, int wgs, int B, double* corr, int ns,
-                                   hipStream_t s, const int* count = nullptr);
+                                   const void* F, const double* mpart, const FusedGradSplit& split, int T, int B,
+                                   double* corr, int ns, hipStream_t s, const int* count = nullptr);
 
 // The store pass above kFusedCostMaxQubits with whole columns in a workgroup's LDS
 // (sqh_k_fused_big.hip): up to 13 qubits in complex128, 14 in complex64.  a.tabs: kBigTab

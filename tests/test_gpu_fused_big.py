@@ -36,6 +36,13 @@ def test_big_store_pass(n, f32, cols, pad, B):
         tol = 5e-6 if f32 else 1e-13
         assert torch.linalg.norm(X - Y) <= tol * torch.linalg.norm(Y)
         assert torch.equal(X[:, d], M[:, d]) and torch.equal(X[:, :, cols:], M[:, :, cols:])
+        # the pass per block does the same products in the same order: which of the two runs
+        # (by batch and columns) does not show in the bits
+        Z = M.clone()
+        torch.cuda.synchronize()
+        ctx.check(ctx._L.sqh_apply_to_fused_dev(ctx.h, ps.data_ptr(), pb, Z.data_ptr(), d, cols, st, bs, B, int(f32)))
+        ctx.synchronize()
+        assert torch.equal(X, Z)
 
 
 def test_big_costs(oracle):
