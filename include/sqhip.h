@@ -369,7 +369,7 @@ int sqh_set_fused_cost_chain(sqh_ctx* ctx, int on);
  * zero (the default): a fixed rule.  A shape that does not fit the circuit, target or the
  * device's LDS falls back to the rule.  The correlation sums are added in one fixed order,
  * so a vector's cost and gradient are the same bits at every shape and in every batch
- * that these kernels run. */
+ * (large batches run in parts of about 4 GiB of scratch). */
 int sqh_set_fused_grad_config(sqh_ctx* ctx, int tiles_per_wave, int waves);
 /* Launch options of the register-tile kernels (the batched costs and gradients when
  * the fused-block path does not run).  waves_per_group: for the forward pass with one

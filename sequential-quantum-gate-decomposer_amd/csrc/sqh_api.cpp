@@ -403,8 +403,7 @@ bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, bool live, FusedG
 
 // Whether a cost + gradient evaluation of B elements of m columns runs through the fused
 // blocks: the switch on, or automatic and the rule of fused_auto, 4 <= N <= 10, no
-// correction channels, and a launch shape fits.  Below 6 qubits, where the blocks' scratch
-// is several times the tile kernels', automatic batches keep it within 4 GiB.
+// correction channels, and a launch shape fits.
 bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, int m, bool live,
                         FusedGradPlan* plan) {
     if (ts.nch != 0 || !fused_plan_fits(c)) return false;
@@ -412,7 +411,6 @@ bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, 
     if (c->fused_cost == SQH_FUSED_COST_OFF || (automatic && !fused_auto(c, FUSED_GRAD_PASS))) return false;
     FusedGradPlan p;
     if (!fused_grad_plan(c, f32, B, m, live, p)) return false;
-    if (automatic && c->prog.N < 6 && p.bytes() > (size_t)4 << 30) return false;
     if (plan) *plan = p;
     return true;
 }
@@ -538,6 +536,9 @@ void eval_scratch_bytes(sqh_ctx* c, int B, bool f32, bool grad, size_t bytes[4])
     bytes[3] = grad ? (size_t)B * 6 * sizeof(double) : 0;
 }
 
+// Scratch of one launch of the fused gradient; larger batches run in parts of about this size.
+constexpr size_t kFusedGradScratch = (size_t)4 << 30;
+
 // costs (and, with grad, the gradient) for B parameter vectors on the device; with
 // `fixed` into the caller's scratch memory (tile path only, nothing allocated).
 int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double* d_costs, double* d_grad,
@@ -559,6 +560,14 @@ int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double*
     FusedGradPlan fgp;
     const bool fused_grad = d_grad && !fixed && fused_grad_applies(c, ts, f32, B, m, false, &fgp);
     const bool fused_costs = !fixed && fused_cost_applies(c, d_grad != nullptr, ts);
+    if (fused_grad && fgp.bytes() > kFusedGradScratch && B > 1) {
+        // part by part; an element's result does not depend on the others
+        const int part = (int)std::max<size_t>(1, B / ((fgp.bytes() + kFusedGradScratch - 1) / kFusedGradScratch));
+        for (int b = 0; b < B && !rc; b += part)
+            rc = eval_batch(c, d_params + (size_t)b * c->prog.P, std::min(part, B - b), precision,
+                            d_costs ? d_costs + b : nullptr, d_grad + (size_t)b * c->prog.P, nullptr);
+        return rc;
+    }
     if (fixed) {
         kern = fixed->kern;
         diag = fixed->diag;

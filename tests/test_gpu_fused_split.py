@@ -2,7 +2,7 @@
 gradient are the same bits in every batch, at every launch shape, next to any companions in
 the optimiser's rounds, and agree with the oracle where the split changes form (one column
 group per task or many, whole rounds and a rest, partials summed by a workgroup per block
-or by a wavefront)."""
+or by a wavefront, batches beyond one launch's scratch)."""
 import numpy as np
 import pytest
 
@@ -73,3 +73,21 @@ def test_rounds_do_not_depend_on_companions(mixed):
         some = decompose_batch(ctx, T, index[pick], x0[pick], opts)
         assert np.array_equal(some["f"], all_of["f"][pick]) and np.array_equal(some["x"], all_of["x"][pick])
 
+
+def test_batch_beyond_one_launch(oracle):
+    """600,000 vectors of a one-block circuit (5 GB of block matrices and partials) run in
+    parts, automatically through the same kernels as a few."""
+    n, B = 4, 600001
+    gates = W.ansatz_layers(n, W.alternating_pairs(n, 12))
+    P = W.param_count(gates)
+    U = W.haar_unitary(16, 8)
+    ps = W.random_params(P, 9, batch=B)
+    ctx = nat.Context(0)
+    ctx.set_circuit(n, gates)
+    ctx.set_target(U)
+    f, g = combined(ctx, ps, nat.PREC_F64)
+    for first in (0, B // 2 - 3, B - 5):
+        f2, g2 = combined(ctx, ps[first:first + 5], nat.PREC_F64)
+        assert np.array_equal(f2, f[first:first + 5]) and np.array_equal(g2, g[first:first + 5])
+    fo, go = oracle.optimization_problem_combined(gates, U, n, ps[B - 1])
+    assert abs(f[B - 1] - fo) < 1e-12 and np.abs(g[B - 1] - go).max() < 1e-12
