@@ -166,8 +166,9 @@ int fused_cost_launch(sqh_ctx* c, bool f32, const FusedCostArgs& a_in) {
         return SQH_OK;
     }
     // the store pass (apply_to) moves the matrices through HBM, the chain is another
-    // kernel: their own keys
-    const std::array<long long, 4> key{(f32 ? 1 : 0) + (a.out ? 2 : 0) + (chain ? 4 : 0), N, a.m, a.B};
+    // kernel, the derivatives' elements run some of the blocks each: their own keys
+    const std::array<long long, 4> key{(f32 ? 1 : 0) + (a.out ? 2 : 0) + (chain ? 4 : 0) + (a.dinfo ? 8 : 0), N, a.m,
+                                       a.B};
     auto it = c->fused_tuned.find(key);
     if (it != c->fused_tuned.end() && valid(it->second)) {
         HIPTRY(c, launch(a, it->second));
@@ -198,6 +199,13 @@ int fused_cost_launch(sqh_ctx* c, bool f32, const FusedCostArgs& a_in) {
         if (scratch.ensure((size_t)ta.B * per) != hipSuccess) {
             (void)hipGetLastError();  // no room for the scratch copy: keep the default
             can_tune = false;
+        }
+        if (a.dinfo) {
+            // the parameters in the middle, which start at the middle blocks (the matrices of
+            // the blocks after the first are then others', which the time does not show)
+            const int mid = (a.B - ta.B) / 2;
+            ta.dinfo = a.dinfo + 4 * (size_t)mid;
+            ta.F = static_cast<const char*>(a.F) + (size_t)mid * 256 * (f32 ? 8 : 16);
         }
         ta.out = scratch.p;
         ta.out_stride = a.m;

@@ -50,3 +50,36 @@ def test_automatic_equals_both_paths(n, layers):
         assert np.array_equal(R2[:, :, cols:], M[:, :, cols:])
     one = _evaluate(ctx, ps[1:2].copy(), M[1:2].copy(), pad, "auto")
     assert abs(one[0][0] - c[1]) < 1e-12 and np.abs(one[2][0] - g[1]).max() < 1e-12
+
+
+def test_derivatives_and_apply_to_are_tuned_apart():
+    """The derivatives' pass runs some of the blocks per matrix, apply_to all: a batch of as
+    many matrices of the same shape measures its own launch shape."""
+    import ctypes
+    n, cols = 7, 40
+    gates = W.mixed_gate_circuit(n, 40, 7)
+    P, d = W.param_count(gates), 1 << n
+    ctx = nat.Context(0)
+    ctx.set_circuit(n, gates)
+    ctx.set_fused_cost(True)
+
+    def tuned_ms():
+        t, w, ms = ctypes.c_int(), ctypes.c_int(), ctypes.c_double()
+        ctx.check(ctx._L.sqh_get_block_config(ctx.h, 0, 256, 16, 1, ctypes.byref(t), ctypes.byref(w),
+                                              ctypes.byref(ms)))
+        return ms.value
+
+    tuned_ms()  # the shape asked for here is itself measured once
+    p = torch.from_numpy(W.random_params(P, 3)).cuda()
+    M = torch.randn((P, d, cols), dtype=torch.complex128, device="cuda")
+    D = torch.empty_like(M)
+    torch.cuda.synchronize()
+    times = [tuned_ms()]
+    for _ in range(2):
+        ctx.check(ctx._L.sqh_apply_derivate_to_dev(ctx.h, p.data_ptr(), M.data_ptr(), d, cols, cols, D.data_ptr()))
+        times.append(tuned_ms())
+    for _ in range(2):
+        ctx.check(ctx._L.sqh_apply_to_dev(ctx.h, p.data_ptr(), 0, M.data_ptr(), d, cols, cols, d * cols, P, 0))
+        times.append(tuned_ms())
+    ctx.synchronize()
+    assert times[0] < times[1] == times[2] < times[3] == times[4]
