@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <array>
+#include <climits>
 #include <cstring>
 #include <functional>
 #include <queue>
@@ -353,38 +354,55 @@ bool compile_program(int N, const std::vector<GateRec>& gates, Program& prog, st
 
 std::vector<uint32_t> quad_ops(const FusionPlan& fp) {
     std::vector<uint32_t> out;
+    out.reserve(fp.gates.size());
     for (size_t b = 0; b + 1 < fp.first.size(); ++b) {
-        std::vector<FusedRec> left(fp.gates.begin() + fp.first[b], fp.gates.begin() + fp.first[b + 1]);
-        // the gates of left that run on qubits (x, y) before any that needs another qubit
-        auto run = [&](int x, int y, std::vector<FusedRec>* taken) {
-            bool blocked[4] = {false, false, false, false};
+        // each local qubit's gates in order; those taken are the first head[q] of them
+        std::array<std::vector<int>, 4> on;
+        std::array<size_t, 4> head = {0, 0, 0, 0};
+        for (int i = fp.first[b]; i < fp.first[b + 1]; ++i) {
+            on[fp.gates[i].t].push_back(i);
+            if (fp.gates[i].c >= 0) on[fp.gates[i].c].push_back(i);
+        }
+        // The gates that run on qubits (x, y) before any that needs another qubit, in order.
+        // Only gates on x and y are looked at, and no more of them than can run and two.
+        auto run = [&](int x, int y, std::vector<int>* taken) {
+            size_t i = head[x], j = head[y];
+            bool bx = false, by = false;  // the qubit's next gate needs another qubit
             int n = 0;
-            std::vector<FusedRec> rest;
-            for (const FusedRec& g : left) {
-                auto inside = [&](int q) { return q < 0 || q == x || q == y; };
-                const bool ok = inside(g.t) && inside(g.c) && !blocked[g.t] && (g.c < 0 || !blocked[g.c]);
-                if (ok) {
+            for (;;) {
+                const int gx = !bx && i < on[x].size() ? on[x][i] : INT_MAX;
+                const int gy = !by && j < on[y].size() ? on[y][j] : INT_MAX;
+                if (gx == INT_MAX && gy == INT_MAX) break;
+                const bool one = fp.gates[std::min(gx, gy)].c < 0;
+                if (gx == gy || one) {
                     ++n;
-                    if (taken) taken->push_back(g);
+                    if (taken) taken->push_back(std::min(gx, gy));
+                    if (gx <= gy) ++i;
+                    if (gy <= gx) ++j;
+                } else if (gx < gy) {
+                    bx = true;
                 } else {
-                    blocked[g.t] = true;
-                    if (g.c >= 0) blocked[g.c] = true;
-                    if (taken) rest.push_back(g);
+                    by = true;
                 }
             }
-            if (taken) left.swap(rest);
+            if (taken) {
+                head[x] = i;
+                head[y] = j;
+            }
             return n;
         };
-        while (!left.empty()) {
+        for (int left = fp.first[b + 1] - fp.first[b]; left > 0;) {
             int bx = 0, by = 1, best = -1;
             for (int x = 0; x < 4; ++x)
                 for (int y = x + 1; y < 4; ++y) {
                     const int n = run(x, y, nullptr);
                     if (n > best) best = n, bx = x, by = y;
                 }
-            std::vector<FusedRec> taken;
+            std::vector<int> taken;
             run(bx, by, &taken);
-            for (const FusedRec& g : taken) {
+            left -= (int)taken.size();
+            for (int k : taken) {
+                const FusedRec& g = fp.gates[k];
                 const bool a = g.t == bx;
                 const uint32_t kind = g.kind == OP_U ? (a ? QK_UA : QK_UB)
                                       : g.kind == OP_X ? (a ? QK_XA : QK_XB)
@@ -402,21 +420,27 @@ std::vector<uint32_t> quad_program(const Program& pr) {
     for (int t = 0; t < pr.N; ++t)
         if (pr.layouts[0].reg_off[1 << t] != 1 << t) return {};
     std::vector<uint32_t> out;
-    int x = 0, y = 1;  // the pair
-    for (size_t i = 0; i < pr.ops.size(); ++i) {
+    out.reserve(pr.ops.size());
+    // per op the qubit that the next controlled gate on its target shares it with (-1: none)
+    std::vector<int> partner(pr.ops.size(), -1);
+    int next[4] = {-1, -1, -1, -1};
+    for (size_t i = pr.ops.size(); i-- > 0;) {
         const Op& op = pr.ops[i];
         if (op.kind == OP_REMAP || op.cmode == CM_LANE) return {};
         if (op.kind == OP_NOP) continue;
+        partner[i] = next[op.t];
+        if (op.cmode == CM_NONE) continue;
+        next[op.t] = op.c;
+        next[op.c] = op.t;
+    }
+    int x = 0, y = 1;  // the pair
+    for (size_t i = 0; i < pr.ops.size(); ++i) {
+        const Op& op = pr.ops[i];
+        if (op.kind == OP_NOP) continue;
         const int t = op.t, c = op.cmode == CM_NONE ? -1 : op.c;
         if ((t != x && t != y) || (c >= 0 && c != x && c != y)) {
-            int other = c;
             // an uncontrolled gate: with the qubit of the next gate that shares one with it
-            for (size_t j = i + 1; j < pr.ops.size() && other < 0; ++j) {
-                const Op& n = pr.ops[j];
-                if (n.kind == OP_NOP || n.cmode == CM_NONE) continue;
-                if (n.t == t) other = n.c;
-                else if (n.c == t) other = n.t;
-            }
+            int other = c >= 0 ? c : partner[i];
             if (other < 0) other = t == 0 ? 1 : 0;
             x = std::min(t, other);
             y = std::max(t, other);

@@ -183,6 +183,17 @@ def test_fusion_plan_in_list_order_above_sixteen_qubits(n):
             assert tg in qubits and (t not in (W.GATE_CNOT, W.GATE_CZ, W.GATE_CRY) or c in qubits)
 
 
+def test_planning_time_grows_with_the_circuit():
+    """One block of 40000 gates (4 qubits, random order) is planned in milliseconds: the
+    order of a block's gates takes time in proportion to them (quadratic: 12 s)."""
+    import time
+    gates = W.mixed_gate_circuit(4, 40000, seed=3)
+    start = time.perf_counter()
+    plan = nat.inspect_fusion(4, gates)
+    assert time.perf_counter() - start < 2.0
+    assert len(plan) == 1 and len(plan[0][1]) == 40000
+
+
 @pytest.mark.parametrize("which", ["8q_40", "10q_60", "6q_mixed"])
 def test_chain_flop_accounting_counts_the_rows_the_chain_touches(which):
     """bench.py's flops for the transposed chain (fused_cost_flops) against a brute-force
