@@ -52,3 +52,27 @@ def test_one_qubit_only(n):
     gates = np.asarray([[nat.GATE_U3, n - 1, -1, 0], [nat.GATE_RX, n - 1, -1, 3]], dtype=np.int32)
     a, b = both(n, gates, 1 << n, 0, False, 2)
     assert np.abs(a["f"] - b["f"]).max() < 1e-11 and np.abs(a["x"] - b["x"]).max() < 1e-11
+
+
+@pytest.mark.parametrize("n", [3, 4])
+@pytest.mark.parametrize("kind", ["ansatz", "mixed"])
+@pytest.mark.parametrize("mixed_precision", [False, True])
+def test_same_bits_as_a_column_per_lane(n, kind, mixed_precision):
+    """Problems of their own circuits are evaluated with a column per lane: the same runs
+    end at the same bits after the same evaluations, line searches included."""
+    from squander_hip import decompose_problems
+    gates = (W.ansatz_layers(n, W.alternating_pairs(n, 3 * n)) if kind == "ansatz"
+             else W.mixed_gate_circuit(n, 8 * n, 40 + n))
+    P, d, runs = W.param_count(gates), 1 << n, 64
+    rng = np.random.default_rng(n)
+    T = np.array([np.linalg.qr(rng.standard_normal((d, d)) + 1j * rng.standard_normal((d, d)))[0] for _ in range(5)])
+    x0 = W.random_params(P, 3, batch=runs)
+    index = (np.arange(runs) % 5).astype(np.int32)
+    opts = default_options(n, max_inner_iterations=9, max_outer_iterations=1, engine="persistent",
+                           mixed_precision=mixed_precision)
+    ctx = nat.Context(0)
+    ctx.set_circuit(n, gates)
+    a = decompose_batch(ctx, T, index, x0, opts)
+    b = decompose_problems(ctx, [(n, gates, T[index[r]], x0[r]) for r in range(runs)], opts)
+    assert np.array_equal(a["evals"], b["evals"]) and np.array_equal(a["f"], b["f"])
+    assert np.array_equal(a["x"], np.array(b["x"]))
