@@ -143,10 +143,22 @@ __device__ __forceinline__ void fc_mma(const FcA<R>& A, const R (&xr)[T][4], con
     }
 }
 
+// Entries between the columns of a region beyond 2^N, for passes whose lanes run along the
+// rows of the matrix: W columns then start 16 / W banks apart, four wavefronts' regions 16.
+__host__ __device__ constexpr int fc_pad(int N, int T) {
+    const int W = 16 * T / ((1 << N) >> 4);
+    return W < 1 || W > 16 ? 1 : 16 / W;
+}
+// Entries of a region's plane (padded).
+__host__ __device__ constexpr int fc_plane(int N, int T, bool padded) {
+    return 256 * T + (padded ? 16 * T / ((1 << N) >> 4) * fc_pad(N, T) + 8 : 0);
+}
+
 // A wavefront's region of W 2^N entries: real parts, then imaginary parts.
-template <typename R, int N, int T>
+template <typename R, int N, int T, bool PADDED = false>
 struct FcRegion {
-    static constexpr int D = 1 << N, O = D >> 4, W = 16 * T / O, PL = 256 * T;
+    static constexpr int D = 1 << N, O = D >> 4, W = 16 * T / O, PL = fc_plane(N, T, PADDED);
+    static constexpr int PAD = PADDED ? fc_pad(N, T) : 0, CS = D + PAD;  // column stride
     R* p;
     __device__ __forceinline__ void put(int i, R re, R im) const {
         p[i] = re;
@@ -159,12 +171,12 @@ struct FcRegion {
     // Slot of row 4 s + g of tile t's vector column in the full layout of a block: lane
     // entry at[s] (LT_LANE ^ LT_S), tile part constant up to 16 outer groups.
     static __device__ __forceinline__ int full(const int (&at)[4], const int* tab, int t, int s) {
-        if constexpr (O <= 16) return at[s] + t * (16 / O) * D;
-        return at[s] ^ tab[LT_T + t];
+        if constexpr (O <= 16) return at[s] + t * (16 / O) * CS;
+        return (at[s] ^ tab[LT_T + t]) + t / (O > 16 ? O / 16 : 1) * PAD;
     }
-    static __device__ __forceinline__ void full_at(int (&at)[4], const int* tab, int lane_entry) {
+    static __device__ __forceinline__ void full_at(int (&at)[4], const int* tab, int lane_entry, int lane = 0) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) at[s] = lane_entry ^ tab[LT_S + s];
+        for (int s = 0; s < 4; ++s) at[s] = (lane_entry ^ tab[LT_S + s]) + (PADDED && O < 16 ? (lane & 15) / O * PAD : 0);
     }
     __device__ __forceinline__ void load_full(const int (&at)[4], const int* tab, R (&xr)[T][4], R (&xi)[T][4]) const {
 #pragma unroll

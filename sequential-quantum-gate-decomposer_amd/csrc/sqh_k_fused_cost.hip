@@ -44,12 +44,15 @@ namespace sqh {
 // The columns come in and go out through the LDS regions with a workgroup's threads along
 // the rows of the matrix (W columns per wavefront, 128 contiguous bytes a row for four
 // wavefronts at 8 qubits): in the operand layout each lane of a load takes another row, and
-// the addresses, a cache line per lane, took as long as the blocks.
+// the addresses, a cache line per lane, took as long as the blocks.  For that pass the columns
+// are padded apart (fc_pad): unpadded, all of them start in the same bank, and at 5 qubits
+// the stores into LDS took half the launch (5 qubits, 2 blocks, 4096 matrices of 32 columns
+// in complex128: 64 us, 35 so; 20000 in complex64: 210 and 88).
 template <typename R, int N, int T, int H, bool PF>
 __global__ __launch_bounds__(256, 2) void k_fused_cost(FusedCostArgs a, const int* __restrict__ tabs) {
     typedef FcMfma<R> MF;
-    typedef FcRegion<R, N, T> Reg;
-    constexpr int D = Reg::D, O = Reg::O, W = Reg::W;
+    typedef FcRegion<R, N, T, true> Reg;
+    constexpr int O = Reg::O, W = Reg::W;
     constexpr int TH = T / H;  // tiles per exchange group
     static_assert(W >= 1 && (16 * TH) % O == 0, "an exchange group holds whole columns");
     extern __shared__ __align__(16) unsigned char fc_smem[];
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(256, 2) void k_fused_cost(FusedCostArgs a, const in
     const int e0 = (int)(first / a.groups), g0 = (int)(first % a.groups);
     const int eq = e0 + (g0 + v) / a.groups, cq = (g0 + v) % a.groups * W + wq;
     const bool okq = first + v < total && cq < m;
-    const Reg ldsq{region + v * 512 * T};
+    const Reg ldsq{region + v * 2 * Reg::PL};
     const int row_q = threadIdx.x / (W * nw);
     {
         const long long src = a.in_index ? (long long)a.in_index[okq ? eq : 0]
@@ -78,13 +81,13 @@ __global__ __launch_bounds__(256, 2) void k_fused_cost(FusedCostArgs a, const in
 #pragma unroll
         for (int k = 0; k < 4 * T; ++k) u[k] = okq ? p[k * step] : mk<R>(0, 0);
 #pragma unroll
-        for (int k = 0; k < 4 * T; ++k) ldsq.put(fc_slot<N>(row_q + k * (64 / W)) + wq * D, u[k].re, u[k].im);
+        for (int k = 0; k < 4 * T; ++k) ldsq.put(fc_slot<N>(row_q + k * (64 / W)) + wq * Reg::CS, u[k].re, u[k].im);
     }
     __syncthreads();
     const long long wave = first + wv;
     const int e = e0 + (g0 + wv) / a.groups;
     const int c0 = (g0 + wv) % a.groups * W;
-    const Reg lds{region + wv * 512 * T};
+    const Reg lds{region + wv * 2 * Reg::PL};
     const int nl = lane & 15, g = lane >> 4;
     if (wave < total) {
         const cpx<R>* F = static_cast<const cpx<R>*>(a.F);
@@ -107,7 +110,7 @@ __global__ __launch_bounds__(256, 2) void k_fused_cost(FusedCostArgs a, const in
         if (lo < hi) A.load_n(a.dinfo ? F0 : Fe + (long long)lo * 256, nl, g);
         for (int b = lo; b < hi; ++b) {
             int at[4];
-            Reg::full_at(at, tab, entry);
+            Reg::full_at(at, tab, entry, lane);
             if (PF && b + 1 < hi) An.load_n(Fe + (long long)(b + 1) * 256, nl, g);
             if (b + 1 < a.nb) entry = tab[kLaneTab + LT_LANE + lane];
             // each exchange group reads and stores its own columns only
@@ -139,7 +142,7 @@ __global__ __launch_bounds__(256, 2) void k_fused_cost(FusedCostArgs a, const in
 #pragma unroll
             for (int k = 0; k < 4 * T; ++k) {
                 cpx<R> y;
-                ldsq.get(fc_slot<N>(row_q + k * (64 / W)) + wq * D, y.re, y.im);
+                ldsq.get(fc_slot<N>(row_q + k * (64 / W)) + wq * Reg::CS, y.re, y.im);
                 p[k * step] = y;
             }
         }
@@ -153,7 +156,7 @@ __global__ __launch_bounds__(256, 2) void k_fused_cost(FusedCostArgs a, const in
         const int* tab = tabs + (a.nb - 1) * kLaneTab;
         R xr[T][4], xi[T][4];
         int at[4];
-        Reg::full_at(at, tab, tab[LT_LANE + lane]);
+        Reg::full_at(at, tab, tab[LT_LANE + lane], lane);
         lds.load_full(at, tab, xr, xi);
         const int* mp = a.maps + (a.nb - 1) * kFusedMapStride;
         const int mask = mp[15];  // the block's four row bits (off of local index 15)
@@ -216,7 +219,7 @@ __global__ __launch_bounds__(256, 2) void k_fused_trace(FusedCostArgs a, const i
                                                         const int* __restrict__ tmaps) {
     typedef FcMfma<R> MF;
     typedef FcRegion<R, N, T> Reg;
-    constexpr int D = Reg::D, O = Reg::O, W = Reg::W;
+    constexpr int O = Reg::O, W = Reg::W;
     static_assert(W >= 1, "a wavefront holds whole columns");
     extern __shared__ __align__(16) unsigned char fc_smem[];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -373,12 +376,11 @@ bool fused_cost_cfg_valid(int N, bool f32, int nb, FusedCostCfg cfg) {
         return false;
     if (cfg.waves != 1 && cfg.waves != 2 && cfg.waves != 4) return false;
     if (16 * cfg.tiles < O || (16 * cfg.tiles / cfg.groups) % O != 0) return false;
-    return fused_cost_lds_bytes(f32, nb, cfg) <= device_max_lds();
+    return fused_cost_lds_bytes(f32, N, cfg) <= device_max_lds();
 }
 
-size_t fused_cost_lds_bytes(bool f32, int nb, FusedCostCfg cfg) {
-    (void)nb;
-    return (size_t)cfg.waves * cfg.tiles * 256 * (f32 ? 8 : 16);
+size_t fused_cost_lds_bytes(bool f32, int N, FusedCostCfg cfg) {
+    return (size_t)cfg.waves * 2 * fc_plane(N, cfg.tiles, true) * (f32 ? 4 : 8);
 }
 
 template <typename R, int N, int T, int H, bool PF>
@@ -420,7 +422,7 @@ hipError_t launch_fused_cost(bool f32, int N, FusedCostArgs a, FusedCostCfg cfg,
     const long long waves = (long long)a.B * a.groups;
     const long long wgs = (waves + cfg.waves - 1) / cfg.waves;
     const int grid = (int)((wgs + 7) / 8 * 8);
-    const size_t shm = fused_cost_lds_bytes(f32, a.nb, cfg);
+    const size_t shm = fused_cost_lds_bytes(f32, N, cfg);
     return f32 ? launch_fc<float>(N, a, cfg, grid, shm, s) : launch_fc<double>(N, a, cfg, grid, shm, s);
 }
 

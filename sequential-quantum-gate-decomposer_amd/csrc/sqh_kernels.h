@@ -235,7 +235,7 @@ struct FusedCostCfg {
     int tiles = 0, groups = 0, waves = 0, prefetch = 0;
 };
 bool fused_cost_cfg_valid(int N, bool f32, int nb, FusedCostCfg cfg);
-size_t fused_cost_lds_bytes(bool f32, int nb, FusedCostCfg cfg);
+size_t fused_cost_lds_bytes(bool f32, int N, FusedCostCfg cfg);
 hipError_t launch_fused_cost(bool f32, int N, FusedCostArgs a, FusedCostCfg cfg, hipStream_t s);
 // The cost pass as a transposed chain from unit vectors (k_fused_trace, nb >= 2): the
 // rows of the circuit matrix the trace needs, built block by block on the rows inside

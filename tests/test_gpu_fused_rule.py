@@ -83,3 +83,35 @@ def test_derivatives_and_apply_to_are_tuned_apart():
         times.append(tuned_ms())
     ctx.synchronize()
     assert times[0] < times[1] == times[2] < times[3] == times[4]
+
+
+@pytest.mark.parametrize("n", [4, 5, 6, 7, 8, 9, 10])
+@pytest.mark.parametrize("f32", [False, True])
+def test_store_pass_shapes_agree(oracle, n, f32):
+    """The store pass at every launch shape (the columns' padding in LDS differs): the same
+    bits, odd column counts, and the oracle's matrices."""
+    gates = W.mixed_gate_circuit(n, 4 * n, 90 + n)
+    P, d, B, cols = W.param_count(gates), 1 << n, 3, min(37, (1 << n) - 1)
+    rng = np.random.default_rng(n)
+    M = rng.standard_normal((B, d, cols)) + 1j * rng.standard_normal((B, d, cols))
+    M = M.astype(np.complex64 if f32 else np.complex128)
+    ps = W.random_params(P, 5, batch=B)
+    ctx = nat.Context(0)
+    ctx.set_circuit(n, gates)
+    ctx.set_fused_cost(True)
+    dp, first = torch.from_numpy(ps).cuda(), None
+    for shape in ((4, 1, 1, 0), (4, 1, 2, 1), (4, 1, 4, 0), (4, 2, 2, 1), (2, 1, 1, 0), (2, 1, 4, 1)):
+        if n == 10 and shape[0] == 2 or shape[1] == 2 and n > 8 or n == 9 and shape[1] == 2:
+            continue
+        ctx.set_fused_cost_config(*shape)
+        X = torch.from_numpy(M).cuda()
+        torch.cuda.synchronize()
+        ctx.check(ctx._L.sqh_apply_to_dev(ctx.h, dp.data_ptr(), P, X.data_ptr(), d, cols, cols, d * cols, B, int(f32)))
+        ctx.synchronize()
+        X = X.cpu().numpy()
+        if first is None:
+            first = X
+            for b in range(B):
+                want = oracle.apply_to(gates, ps[b], M[b].astype(np.complex128))
+                assert np.linalg.norm(X[b] - want) <= (1e-5 if f32 else 1e-12) * np.linalg.norm(want)
+        assert np.array_equal(X, first), shape
