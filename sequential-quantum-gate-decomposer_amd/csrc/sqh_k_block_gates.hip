@@ -210,7 +210,7 @@ __device__ __forceinline__ void partial_sum(const double* __restrict__ M, unsign
 // the pair correlations of y and x summed over the wavefront, y <- G^T y.
 // corr[e][slot][8] is the register-tile adjoint's layout.
 template <typename R, bool SPLIT>
-__global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const uint32_t* __restrict__ ops,
+__global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 2 : 3) void k_fused_block_corr(const uint32_t* __restrict__ ops,
                                                           const int* __restrict__ first, int nb,
                                                           const cpx<R>* __restrict__ kern, long long kern_bstride,
                                                           const double* __restrict__ params, int pstride,
@@ -219,8 +219,11 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
                                                           int B, double* __restrict__ corr, int ns,
                                                           const int* __restrict__ count) {
     constexpr int E = SPLIT ? 1 : 4;  // elements per workgroup
-    __shared__ double sums[E][512];  // 256 real, then 256 imaginary parts
+    // M_b (256 real, then 256 imaginary parts) waits where x and y change pairs once it is
+    // read: 48 KiB a workgroup, three per CU (two with a buffer of its own; 512 elements of
+    // 6 blocks: 36 us against 46)
     __shared__ cpx<double> states[E][512], tables[E][64 * 4];
+    double* const sums = reinterpret_cast<double*>(states[SPLIT ? 0 : threadIdx.x >> 6]);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int blk = blockIdx.x % nb, e = (blockIdx.x / nb) * E + (SPLIT ? 0 : wave);
     if (count) {
@@ -238,11 +241,11 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
         if constexpr (SPLIT) {
             double v[1];
             partial_sum(M + threadIdx.x, stride, n, up, 0, v);
-            sums[0][threadIdx.x] = v[0];
+            sums[threadIdx.x] = v[0];
             __syncthreads();
             if (wave != 0) return;
         } else {
-            double* s = sums[wave] + lane;
+            double* s = sums + lane;
             M += lane;
             if (n <= 4 && n <= 1 << up) {
                 double v[8];
@@ -275,8 +278,7 @@ __global__ __launch_bounds__(SPLIT ? 512 : 256) void k_fused_block_corr(const ui
     for (int k = 0; k < 4; ++k) {
         const int at = quad_row(q, k) * 16 + col;
         x[k] = widen(Fb[at]);
-        const double* sw = sums[SPLIT ? 0 : wave];
-        y[k] = mk(sw[at], sw[256 + at]);
+        y[k] = mk(sums[at], sums[256 + at]);
     }
     for (int pe = p1; pe > p0; pe -= 64) {
         const int p = max(p0, pe - 64), cnt = pe - p;
