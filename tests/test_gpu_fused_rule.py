@@ -115,3 +115,44 @@ def test_store_pass_shapes_agree(oracle, n, f32):
                 want = oracle.apply_to(gates, ps[b], M[b].astype(np.complex128))
                 assert np.linalg.norm(X[b] - want) <= (1e-5 if f32 else 1e-12) * np.linalg.norm(want)
         assert np.array_equal(X, first), shape
+
+
+@pytest.mark.parametrize("B", [4096, 4097])
+def test_four_qubits_across_the_batch_line(oracle, B):
+    """Around the batch beyond which 4-qubit complex64 batches and matrices run the tile
+    kernels: complex128 costs and gradients keep their bits, the rest agrees to rounding with a
+    small batch and the oracle."""
+    gates = W.ansatz_layers(4, W.alternating_pairs(4, 20))
+    P = W.param_count(gates)
+    U = W.haar_unitary(16, 3)
+    ps = W.random_params(P, 4, batch=B)
+    ctx = nat.Context(0)
+    ctx.set_circuit(4, gates)
+    ctx.set_target(U)
+
+    def both(p, prec):
+        b = p.shape[0]
+        c, f, g = np.empty(b), np.empty(b), np.empty((b, P))
+        p = np.ascontiguousarray(p)
+        ctx.check(ctx._L.sqh_optimization_problem_batch(ctx.h, p.ctypes.data, b, prec, c.ctypes.data))
+        ctx.check(ctx._L.sqh_optimization_problem_combined_batch(ctx.h, p.ctypes.data, b, prec, f.ctypes.data,
+                                                                 g.ctypes.data))
+        return c, f, g
+
+    few = [0, B // 2, B - 1]
+    for prec, tol in ((nat.PREC_F64, 0.0), (nat.PREC_F32, 2e-5)):
+        for x, y in zip(both(ps, prec), both(ps[few], prec)):
+            assert np.abs(x[few] - y).max() <= tol
+    f, g = oracle.optimization_problem_combined(gates, U, 4, ps[B - 1])
+    c = both(ps[few], nat.PREC_F64)
+    assert abs(c[0][2] - f) < 1e-12 and np.abs(c[2][2] - g).max() < 1e-12
+    for dt, tol in ((torch.complex128, 1e-12), (torch.complex64, 1e-5)):
+        M = torch.from_numpy(np.broadcast_to(U, (B, 16, 16)).copy()).cuda().to(dt)
+        dp = torch.from_numpy(ps).cuda()
+        torch.cuda.synchronize()
+        ctx.check(ctx._L.sqh_apply_to_dev(ctx.h, dp.data_ptr(), P, M.data_ptr(), 16, 16, 16, 256, B,
+                                          int(dt == torch.complex64)))
+        ctx.synchronize()
+        for b in few:
+            want = oracle.apply_to(gates, ps[b], U)
+            assert np.linalg.norm(M[b].cpu().numpy() - want) <= tol * np.linalg.norm(want)
