@@ -143,8 +143,9 @@ __device__ __forceinline__ void fc_mma(const FcA<R>& A, const R (&xr)[T][4], con
     }
 }
 
-// Entries between the columns of a region beyond 2^N, for passes whose lanes run along the
-// rows of the matrix: W columns then start 16 / W banks apart, four wavefronts' regions 16.
+// Entries between the columns of a region beyond 2^N where the lanes of an access are in
+// several columns (which else all start in the same bank): W columns then start 16 / W banks
+// apart, four wavefronts' regions 16.
 __host__ __device__ constexpr int fc_pad(int N, int T) {
     const int W = 16 * T / ((1 << N) >> 4);
     return W < 1 || W > 16 ? 1 : 16 / W;
@@ -174,7 +175,7 @@ struct FcRegion {
         if constexpr (O <= 16) return at[s] + t * (16 / O) * CS;
         return (at[s] ^ tab[LT_T + t]) + t / (O > 16 ? O / 16 : 1) * PAD;
     }
-    static __device__ __forceinline__ void full_at(int (&at)[4], const int* tab, int lane_entry, int lane = 0) {
+    static __device__ __forceinline__ void full_at(int (&at)[4], const int* tab, int lane_entry, int lane) {
 #pragma unroll
         for (int s = 0; s < 4; ++s) at[s] = (lane_entry ^ tab[LT_S + s]) + (PADDED && O < 16 ? (lane & 15) / O * PAD : 0);
     }
@@ -225,13 +226,12 @@ __device__ __forceinline__ void fc_column_sums(const double (&sr)[C], const doub
 // (rho = c0 + w + trace_off; columns past m take row trace_off).  On return xr / xi hold
 // block 0's B operand in the chain's grouping of block 0 and A block 0's operand F_0^T.
 // With PF, block b - 1's matrix is loaded while block b runs.
-template <typename R, int N, int T, bool PF>
+template <typename R, int N, int T, bool PF, typename Reg>
 __device__ __forceinline__ void fused_chain_to_block0(const int* __restrict__ tabs, const int* __restrict__ tmaps,
-                                                      int nb, FcRegion<R, N, T> lds, const cpx<R>* __restrict__ Fe,
+                                                      int nb, Reg lds, const cpx<R>* __restrict__ Fe,
                                                       int c0, int m, int trace_off, int lane, R (&xr)[T][4],
                                                       R (&xi)[T][4], FcA<R>& A) {
     typedef FcMfma<R> MF;
-    typedef FcRegion<R, N, T> Reg;
     constexpr int D = Reg::D, W = Reg::W;
     const int nl = lane & 15, g = lane >> 4;
     auto rho_of = [&](int w) { return (c0 + w < m ? c0 + w : 0) + trace_off; };
@@ -241,27 +241,30 @@ __device__ __forceinline__ void fused_chain_to_block0(const int* __restrict__ ta
     {
         typedef int zero4 __attribute__((ext_vector_type(4)));
         zero4* z = reinterpret_cast<zero4*>(lds.p);
+        constexpr int n = 2 * Reg::PL * (int)sizeof(R) / 16;
 #pragma unroll
-        for (int i = 0; i < (int)(512 * T * sizeof(R) / 1024); ++i) z[64 * i + lane] = zero4{0, 0, 0, 0};
+        for (int i = 0; i < (n + 63) / 64; ++i)
+            if (64 * i + 63 < n || 64 * i + lane < n) z[64 * i + lane] = zero4{0, 0, 0, 0};
     }
     // the support layout's entry of each tile of block b; vector columns past the
     // wavefront's columns read column 0 (their products are never stored)
-    auto support_at = [&](const int* tab, int entry, int ts, int (&at)[T]) {
+    auto support_at = [&](const int* tab, int entry, int ts, int (&at)[T], int (&pad)[T]) {
         const int lg = tab[LT_LG], nS = tab[LT_NS];
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             if (t < ts) {
                 const int w = (16 * t + nl) >> lg, wc = w < W ? w : 0;
                 at[t] = entry ^ tab[LT_ST + t] ^ fc_slot<N>(rho_of(wc) & nS) ^ (wc * D);
+                pad[t] = wc * Reg::PAD;
             }
         }
     };
-    auto load_support = [&](const int* tab, const int (&at)[T], int ts) {
+    auto load_support = [&](const int* tab, const int (&at)[T], const int (&pad)[T], int ts) {
 #pragma unroll
         for (int t = 0; t < T; ++t)
             if (t < ts) {
 #pragma unroll
-                for (int s = 0; s < 4; ++s) lds.get(at[t] ^ tab[LT_S + s], xr[t][s], xi[t][s]);
+                for (int s = 0; s < 4; ++s) lds.get((at[t] ^ tab[LT_S + s]) + pad[t], xr[t][s], xi[t][s]);
             }
         fc_wave_fence();
     };
@@ -280,7 +283,7 @@ __device__ __forceinline__ void fused_chain_to_block0(const int* __restrict__ ta
             const int w = p >> 4, i = p & 15;
             const int rho = rho_of(w);
             const cpx<R> f = Fq[ft_local(mq, rho) * 16 + i];
-            lds.put((tq[LT_S + (i >> 2)] ^ tq[LT_SLANE + 16 * (i & 3)] ^ fc_slot<N>(rho & mq[81])) + w * D, f.re, f.im);
+            lds.put((tq[LT_S + (i >> 2)] ^ tq[LT_SLANE + 16 * (i & 3)] ^ fc_slot<N>(rho & mq[81])) + w * Reg::CS, f.re, f.im);
         }
         fc_wave_fence();
     }
@@ -292,8 +295,8 @@ __device__ __forceinline__ void fused_chain_to_block0(const int* __restrict__ ta
     int ts = tiles(tab);
     for (; b > 0 && ts < T; --b) {
         const int* tn = tab - kLaneTab;
-        int at[T];
-        support_at(tab, entry, ts, at);
+        int at[T], pad[T];
+        support_at(tab, entry, ts, at, pad);
         if constexpr (PF) An.load_t(Fe + (long long)(b - 1) * 256, nl, g);
         entry = tn[LT_SLANE + lane];
         auto run = [&](auto tiles_run) __attribute__((always_inline)) {
@@ -303,14 +306,14 @@ __device__ __forceinline__ void fused_chain_to_block0(const int* __restrict__ ta
 #pragma unroll
             for (int t = 0; t < TS; ++t)
 #pragma unroll
-                for (int s = 0; s < 4; ++s) lds.get(at[t] ^ tab[LT_S + s], vr[t][s], vi[t][s]);
+                for (int s = 0; s < 4; ++s) lds.get((at[t] ^ tab[LT_S + s]) + pad[t], vr[t][s], vi[t][s]);
             fc_wave_fence();
             fc_mma<R, TS, TS>(A, vr, vi, yr, yi);
 #pragma unroll
             for (int t = 0; t < TS; ++t) {
                 if ((16 * t + nl) >> tab[LT_LG] < W) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) lds.put(at[t] ^ tab[LT_S + r], yr[t][r], yi[t][r]);
+                    for (int r = 0; r < 4; ++r) lds.put((at[t] ^ tab[LT_S + r]) + pad[t], yr[t][r], yi[t][r]);
                 }
             }
             fc_wave_fence();
@@ -327,9 +330,9 @@ __device__ __forceinline__ void fused_chain_to_block0(const int* __restrict__ ta
         for (int t = 0; t < T; ++t)
 #pragma unroll
             for (int s = 0; s < 4; ++s) xr[t][s] = xi[t][s] = 0;
-        int at[T];
-        support_at(tab, entry, ts, at);
-        load_support(tab, at, ts);
+        int at[T], pad[T];
+        support_at(tab, entry, ts, at, pad);
+        load_support(tab, at, pad, ts);
         return;
     }
     // Blocks of full support (no row outside it): vector column 16 t + nl is column
@@ -339,7 +342,7 @@ __device__ __forceinline__ void fused_chain_to_block0(const int* __restrict__ ta
     for (; b > 0; --b) {
         const int* tn = tab - kLaneTab;
         if constexpr (PF) An.load_t(Fe + (long long)(b - 1) * 256, nl, g);
-        Reg::full_at(af, tab, entry);
+        Reg::full_at(af, tab, entry, lane);
         entry = tn[LT_LANE + lane];
         typename MF::V yr[T], yi[T];
         R vr[T][4], vi[T][4];
@@ -350,7 +353,7 @@ __device__ __forceinline__ void fused_chain_to_block0(const int* __restrict__ ta
         if constexpr (PF) A = An;
         else A.load_t(Fe + (long long)(b - 1) * 256, nl, g);
     }
-    Reg::full_at(af, tab, entry);
+    Reg::full_at(af, tab, entry, lane);
     lds.load_full(af, tab, xr, xi);
 }
 

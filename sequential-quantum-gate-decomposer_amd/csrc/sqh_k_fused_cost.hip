@@ -214,11 +214,16 @@ __global__ __launch_bounds__(256, 2) void k_fused_cost(FusedCostArgs a, const in
 // support instead.  Every launch shape performs the same operations per column in the
 // same order: results are bit-identical across shapes.
 
+// The chain's regions are padded below 8 qubits, where a tile's 16 vector columns are of
+// several columns (5 blocks on 5 qubits, 4096 vectors: 45 us in complex128, 27 in complex64;
+// unpadded 61 and 33).
+constexpr bool ft_padded(int N) { return N < 8; }
+
 template <typename R, int N, int T, bool PF>
 __global__ __launch_bounds__(256, 2) void k_fused_trace(FusedCostArgs a, const int* __restrict__ tabs,
                                                         const int* __restrict__ tmaps) {
     typedef FcMfma<R> MF;
-    typedef FcRegion<R, N, T> Reg;
+    typedef FcRegion<R, N, T, ft_padded(N)> Reg;
     constexpr int O = Reg::O, W = Reg::W;
     static_assert(W >= 1, "a wavefront holds whole columns");
     extern __shared__ __align__(16) unsigned char fc_smem[];
@@ -229,13 +234,13 @@ __global__ __launch_bounds__(256, 2) void k_fused_trace(FusedCostArgs a, const i
     if (wave >= (long long)a.B * a.groups) return;
     const int e = (int)(wave / a.groups);
     const int c0 = (int)(wave % a.groups) * W;
-    const Reg lds{reinterpret_cast<R*>(fc_smem) + wv * 512 * T};
+    const Reg lds{reinterpret_cast<R*>(fc_smem) + wv * 2 * Reg::PL};
     const int nl = lane & 15, g = lane >> 4;
     const int m = a.m;
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.F_bstride;
     R xr[T][4], xi[T][4];
     FcA<R> A;
-    fused_chain_to_block0<R, N, T, PF>(tabs, tmaps, a.nb, lds, Fe, c0, m, a.trace_off, lane, xr, xi, A);
+    fused_chain_to_block0<R, N, T, PF, Reg>(tabs, tmaps, a.nb, lds, Fe, c0, m, a.trace_off, lane, xr, xi, A);
     // block 0, then row rho of V times column c of U: per lane its rows of the column,
     // then the lanes of the column
     typename MF::V yr[T], yi[T];
@@ -315,12 +320,11 @@ bool fused_trace_cfg_valid(int N, bool f32, int nb, FusedCostCfg cfg) {
     if ((cfg.tiles != 2 && cfg.tiles != 4) || cfg.groups != 1) return false;
     if (cfg.waves != 1 && cfg.waves != 2 && cfg.waves != 4) return false;
     if (16 * cfg.tiles < ((1 << N) >> 4)) return false;
-    return fused_trace_lds_bytes(f32, nb, cfg) <= device_max_lds();
+    return fused_trace_lds_bytes(f32, N, cfg) <= device_max_lds();
 }
 
-size_t fused_trace_lds_bytes(bool f32, int nb, FusedCostCfg cfg) {
-    (void)nb;
-    return (size_t)cfg.waves * cfg.tiles * 256 * (f32 ? 8 : 16);
+size_t fused_trace_lds_bytes(bool f32, int N, FusedCostCfg cfg) {
+    return (size_t)cfg.waves * 2 * fc_plane(N, cfg.tiles, ft_padded(N)) * (f32 ? 4 : 8);
 }
 
 template <typename R, int N>
@@ -364,7 +368,7 @@ hipError_t launch_fused_trace(bool f32, int N, FusedCostArgs a, FusedCostCfg cfg
     const long long waves = (long long)a.B * a.groups;
     const long long wgs = (waves + cfg.waves - 1) / cfg.waves;
     const int grid = (int)((wgs + 7) / 8 * 8);
-    const size_t shm = fused_trace_lds_bytes(f32, a.nb, cfg);
+    const size_t shm = fused_trace_lds_bytes(f32, N, cfg);
     return f32 ? launch_ft<float>(N, a, cfg, grid, shm, s) : launch_ft<double>(N, a, cfg, grid, shm, s);
 }
 

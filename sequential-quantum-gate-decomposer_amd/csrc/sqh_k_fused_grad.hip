@@ -35,6 +35,11 @@ namespace {
 // row-wise and a column-wise sweep of 16 lanes touch 16 different bank groups.
 __device__ __forceinline__ int fg_tile(int r, int c) { return r * 16 + (c ^ r); }
 
+// The regions are padded on 4 and 5 qubits, where a tile's 16 vector columns are of 8 and 16
+// columns (4096 gradients on 5 qubits: 255 us against 275); on 6 and 7 the addresses cost as
+// much as the conflicts.
+constexpr bool fg_padded(int N) { return N < 6; }
+
 // Y = A X (CONJ: with A's conjugate) on all tiles.
 template <typename R, int T, bool CONJ>
 __device__ __forceinline__ void fg_mma(const FcA<R>& A, const R (&xr)[T][4], const R (&xi)[T][4],
@@ -205,7 +210,7 @@ __device__ __forceinline__ void fg_correlate(R* lds, const Y& yr, const Y& yi, c
 template <typename R, int N, int T>
 __global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const int* __restrict__ tabs) {
     typedef FcMfma<R> MF;
-    typedef FcRegion<R, N, T> Reg;
+    typedef FcRegion<R, N, T, fg_padded(N)> Reg;
     constexpr int O = Reg::O, W = Reg::W;
     static_assert(W >= 1, "a wavefront holds whole columns");
     extern __shared__ __align__(16) unsigned char fg_smem[];
@@ -214,7 +219,7 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const in
     const FgTask task = fg_task<T>(a, wv);
     if (!task.live) return;
     const int e = task.e, m = a.m;
-    const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 512 * T};
+    const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 2 * Reg::PL};
     const cpx<R>* U = static_cast<const cpx<R>*>(a.U);
     if (a.count) U += (long long)a.run_target[a.elem_run[e]] * a.tgt_stride;
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.nb * 256;
@@ -232,10 +237,10 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const in
             fg_mma<R, T, false>(A, xr, xi, dr, di);
             if (b + 1 < a.nb) {
                 int at[4];
-                Reg::full_at(at, tab, tab[LT_LANE + lane]);
+                Reg::full_at(at, tab, tab[LT_LANE + lane], lane);
                 lds.template store_full<T>(at, tab, dr, di);
                 const int* tn = tab + kLaneTab;
-                Reg::full_at(at, tn, tn[LT_LANE + lane]);
+                Reg::full_at(at, tn, tn[LT_LANE + lane], lane);
                 lds.load_full(at, tn, xr, xi);
             }
         }
@@ -279,8 +284,8 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const in
             A.load_t(Fe + (long long)(b - 1) * 256, nl, g);
             const int* tn = tab - kLaneTab;
             int at[4], an[4];
-            Reg::full_at(at, tab, tab[LT_LANE + lane]);
-            Reg::full_at(an, tn, tn[LT_LANE + lane]);
+            Reg::full_at(at, tab, tab[LT_LANE + lane], lane);
+            Reg::full_at(an, tn, tn[LT_LANE + lane], lane);
             lds.template store_full<T>(at, tab, dr, di);
             lds.load_full(an, tn, yr, yi);
 #pragma unroll
@@ -309,7 +314,7 @@ template <typename R, int N, int T>
 __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, const int* __restrict__ tabs,
                                                              const int* __restrict__ tmaps) {
     typedef FcMfma<R> MF;
-    typedef FcRegion<R, N, T> Reg;
+    typedef FcRegion<R, N, T, fg_padded(N)> Reg;
     constexpr int O = Reg::O, W = Reg::W;
     static_assert(W >= 1, "a wavefront holds whole columns");
     extern __shared__ __align__(16) unsigned char fg_smem[];
@@ -318,7 +323,7 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
     const FgTask task = fg_task<T>(a, wv);
     if (!task.live) return;
     const int e = task.e, m = a.m;
-    const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 512 * T};
+    const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 2 * Reg::PL};
     const cpx<R>* U = static_cast<const cpx<R>*>(a.U);
     if (a.count) U += (long long)a.run_target[a.elem_run[e]] * a.tgt_stride;
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.nb * 256;
@@ -331,7 +336,7 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
         R zr[T][4], zi[T][4], xr[T][4], xi[T][4];
         typename MF::V er[T], ei[T];
         FcA<R> A;
-        fused_chain_to_block0<R, N, T, false>(tabs, tmaps, a.nb, lds, Fe, c0, m, a.trace_off, lane, zr, zi, A);
+        fused_chain_to_block0<R, N, T, false, Reg>(tabs, tmaps, a.nb, lds, Fe, c0, m, a.trace_off, lane, zr, zi, A);
         fg_mma<R, T, false>(A, zr, zi, er, ei);
         {
             constexpr int C = O > 16 ? W : T;  // sums: per column, or per tile of whole columns
@@ -369,8 +374,8 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
             const int* tab = tabs + b * kLaneTab;
             const int* tn = tab + kLaneTab;
             int at[4], an[4];
-            Reg::full_at(at, tab, tab[LT_LANE + lane]);
-            Reg::full_at(an, tn, tn[LT_LANE + lane]);
+            Reg::full_at(at, tab, tab[LT_LANE + lane], lane);
+            Reg::full_at(an, tn, tn[LT_LANE + lane], lane);
             {
                 typename MF::V dr[T], di[T];
                 if constexpr (!AHEAD) An.load_n(Fe + (long long)b * 256, nl, g);
@@ -413,9 +418,8 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
     }
 }
 
-size_t fused_grad_lds_bytes(bool f32, int nb, int T, int waves) {
-    (void)nb;
-    return (f32 ? 8 : 16) * (size_t)(256 * T) * waves;  // a region per wavefront
+size_t fused_grad_lds_bytes(bool f32, int N, int T, int waves) {
+    return (size_t)waves * 2 * fc_plane(N, T, fg_padded(N)) * (f32 ? 4 : 8);  // a region per wavefront
 }
 
 // The kernel of a shape, or null.
@@ -455,7 +459,7 @@ int fused_grad_groups(int N, int m, int T) {
 bool fused_grad_shape_valid(bool f32, int N, int m, int nb, int T, int waves) {
     if (N < 4 || N > kFusedCostMaxQubits || (T != 2 && T != 4) || m <= 0 || nb <= 0) return false;
     if (waves != 1 && waves != 2 && waves != 4 && waves != 8) return false;
-    return fused_grad_groups(N, m, T) > 0 && fused_grad_lds_bytes(f32, nb, T, waves) <= device_max_lds();
+    return fused_grad_groups(N, m, T) > 0 && fused_grad_lds_bytes(f32, N, T, waves) <= device_max_lds();
 }
 
 // Wavefronts of the kernel that are resident together on the current device.
@@ -489,7 +493,7 @@ FusedGradSplit fused_grad_split(bool f32, int N, int m, int nb, int T, int waves
     const long long total = (long long)B * s.groups;
     const int levels = fused_grad_levels(T);
     if (live || total > 1024)
-        s.resident = fg_resident(fg_kernel(f32, N, T, chain), fused_grad_lds_bytes(f32, nb, T, waves), waves);
+        s.resident = fg_resident(fg_kernel(f32, N, T, chain), fused_grad_lds_bytes(f32, N, T, waves), waves);
     const long long R = s.resident;
     if (live) {
         FusedGradSplit most = s;
@@ -544,7 +548,7 @@ hipError_t launch_fused_grad(bool f32, int N, FusedGradArgs a, int T, int waves,
     const int* tabs = a.tabs;
     const int* tmaps = a.tmaps;
     void* args[] = {&a, &tabs, &tmaps};  // k_fused_grad takes the first two
-    return hipLaunchKernel(kernel, dim3(grid), dim3(64 * waves), args, fused_grad_lds_bytes(f32, a.nb, T, waves), s);
+    return hipLaunchKernel(kernel, dim3(grid), dim3(64 * waves), args, fused_grad_lds_bytes(f32, N, T, waves), s);
 }
 
 }  // namespace sqh

@@ -208,7 +208,7 @@ int fused_grad_groups(int N, int m, int T);  // column groups per element
 // pending sums it needs.
 FusedGradSplit fused_grad_split(bool f32, int N, int m, int nb, int T, int waves, bool chain, int B, bool live,
                                 size_t* partials, size_t* pending);
-size_t fused_grad_lds_bytes(bool f32, int nb, int T, int waves);
+size_t fused_grad_lds_bytes(bool f32, int N, int T, int waves);
 hipError_t launch_fused_grad(bool f32, int N, FusedGradArgs a, int T, int waves, hipStream_t s);
 // Per (element, block): the partials summed (split as the kernel's), then the block's gates
 // run backwards on
@@ -245,7 +245,7 @@ hipError_t launch_fused_cost(bool f32, int N, FusedCostArgs a, FusedCostCfg cfg,
 // with one exchange group; every valid shape gives bit-identical results.
 constexpr int kTraceMapStride = 16 + 64 + 2;
 bool fused_trace_cfg_valid(int N, bool f32, int nb, FusedCostCfg cfg);
-size_t fused_trace_lds_bytes(bool f32, int nb, FusedCostCfg cfg);
+size_t fused_trace_lds_bytes(bool f32, int N, FusedCostCfg cfg);
 hipError_t launch_fused_trace(bool f32, int N, FusedCostArgs a, FusedCostCfg cfg, hipStream_t s);
 
 }  // namespace sqh
