@@ -182,8 +182,13 @@ __device__ __forceinline__ void partial_sum(const double* __restrict__ M, unsign
             double s[128 / C][E];
 #pragma unroll
             for (int j = 0; j < 128 / C; ++j) {
-                if (C * j < left) {
-                    partial_nodes<C>(P + C * j * stride, stride, left - C * j, step, s[j]);
+                const int l = left - C * j;  // a chunk's last partials in a block no wider than they need
+                if (l > (C > 16 ? 32 : 0)) {
+                    partial_nodes<C>(P + C * j * stride, stride, l, step, s[j]);
+                } else if (l > 16) {
+                    partial_nodes<32>(P + C * j * stride, stride, l, step, s[j]);
+                } else if (l > 0) {
+                    partial_nodes<16>(P + C * j * stride, stride, l, step, s[j]);
                 } else {
 #pragma unroll
                     for (int i = 0; i < E; ++i) s[j][i] = 0.0;
