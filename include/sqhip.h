@@ -84,6 +84,10 @@ typedef struct sqh_gate {
 
 /* ---- context -------------------------------------------------------------- */
 int sqh_create(int device, sqh_ctx** out);
+/* A context keeps its device memory from call to call, and only sqh_destroy gives it back:
+ * the scratch of the largest evaluation so far (batches of gradients through the fused
+ * blocks run in parts of about 4 GiB), and up to 512 MiB of buffers of the last
+ * sqh_decompose_batch or sqh_decompose_problems (a call that needed more frees them all). */
 void sqh_destroy(sqh_ctx* ctx);
 const char* sqh_last_error(const sqh_ctx* ctx);
 void* sqh_get_stream(sqh_ctx* ctx);            /* the context's hipStream_t */
@@ -110,12 +114,12 @@ int sqh_set_correction_weights(sqh_ctx* ctx, double prev_cost, double scale1, do
 int sqh_apply_to(sqh_ctx* ctx, const void* params, void* inout, int rows, int cols, int stride, int is_f32);
 /* Device variant: B matrices at inout + b*bstride elements, parameters shared
  * (pbstride = 0) or per matrix (pbstride = P).  Up to 10 qubits it runs the register-tile
- * kernels, or -- where sqh_set_fused_cost selects it (by default where the blocks
- * do little enough arithmetic beside the gates) -- the
- * tile-resident pass of the circuit's fused 4-qubit blocks on the matrix cores, which
- * writes each column back to where it read it; above 10 qubits the same pass with
- * whole columns in a workgroup's LDS (to 13 qubits, 14 in complex64) where that is the
- * faster way, else the fused streaming path. */
+ * kernels, or -- where sqh_set_fused_cost selects it (by default where the blocks do little
+ * enough arithmetic beside the gates; on 4 qubits up to 4096 matrices) -- the tile-resident
+ * pass of the circuit's fused 4-qubit blocks on the matrix cores, which writes each column
+ * back to where it read it.  Above 10 qubits the blocks run with whole columns in a
+ * workgroup's LDS where that is the faster way (to 13 qubits; on 14 in complex64 for deep
+ * circuits), else one after the other through memory.  The ways agree to rounding. */
 int sqh_apply_to_dev(sqh_ctx* ctx, const double* d_params, int pbstride, void* d_inout, int rows, int cols,
                      int stride, long long bstride, int B, int is_f32);
 /* The same result computed by one streaming HBM pass per gate (the unfused path). */
@@ -325,7 +329,9 @@ int sqh_get_jit_stats(sqh_ctx* ctx, double* compile_ms, int* compiles);
  * faster than the tile kernels, by the qubits and the blocks' arithmetic over the gates' --
  * against the run-time specialised kernels from 7 qubits when the blocks do no more;
  * against the generic ones from 4 qubits for deep circuits and from 6 for all but shallow
- * ones).  The same mode selects the fused blocks' adjoint for cost + gradient batches
+ * ones).  _AUTO looks at the batch only on 4 qubits, where complex64 batches beyond 4096
+ * vectors take the tile kernels.  The fused blocks give a vector the same bits in every
+ * batch.  The same mode selects the fused blocks' adjoint for cost + gradient batches
  * (sqh_optimization_problem_combined_batch[_dev]; _AUTO: from 6 qubits against the
  * specialised kernels): forward and backward block products on the matrix cores, each
  * block's correlations then resolved to its gates.  sqh_decompose_batch's lockstep

@@ -772,7 +772,7 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
         a.F = c->d_fused.p;
         a.F_bstride = Bk > 1 ? (long long)nb * 256 : 0;
         a.maps = c->d_fmaps.as<int>();
-    a.tabs = c->d_ftabs.as<int>();
+        a.tabs = c->d_ftabs.as<int>();
         a.out = d_inout;
         a.out_bstride = bstride;
         a.out_stride = stride;
@@ -803,8 +803,8 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
 // Gates_block::apply_derivate_to: a forward store pass over P elements, element k running
 // the circuit with parameter k's gate replaced by its derivative kernel (a controlled
 // gate's control-0 block zeroed) -- through the fused blocks where that path applies
-// (fused_pass_applies), else the register-tile store kernel on per-element kernel tables.  Output k is at d_out + k * rows * cols, row
-// stride cols.
+// (fused_pass_applies), else the register-tile store kernel on per-element kernel tables.
+// Output k is at d_out + k * rows * cols, row stride cols.
 int deriv_dev(sqh_ctx* c, const double* d_params, const void* d_in, int rows, int cols, int stride, void* d_out) {
     int rc = require_circuit(c);
     if (rc) return rc;

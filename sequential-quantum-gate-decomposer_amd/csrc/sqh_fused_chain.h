@@ -4,8 +4,9 @@
 //
 // What bounds these kernels: FP64 MFMA and the vector ALU do not overlap on gfx950.  With
 // four wavefronts per SIMD, a v_mfma_f64_16x16x4f64 takes 65 cycles alone (77 TFLOP/s on the
-// card) and about 3 more for every VALU instruction and 13 more for every 16-byte LDS access
-// that accompanies it.  So the code around the MFMAs is what can be saved: addresses come
+// card) and 2.5 to 3 more for every 32-bit VALU instruction, 6 for an FP64 FMA and 13 for
+// every 16-byte LDS access that accompanies it
+// (profiles/f64_mfma_beside_vector_and_lds.md).  So the code around the MFMAs is what can be saved: addresses come
 // from lane tables built by the host, one XOR with a uniform value each (LT_*,
 // sqh_kernels.h); real and imaginary parts are separate LDS planes, so a result register
 // pair is stored without packing; the negated imaginary part is the MFMA's own operand

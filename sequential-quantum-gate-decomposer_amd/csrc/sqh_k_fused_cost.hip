@@ -3,8 +3,8 @@
 // first load to its trace entry.
 //
 // The circuit is the product of nb dense 16 x 16 blocks on sorted 4-qubit sets (the
-// fusion plan; per batch element the block matrices F_b are built from its kernel
-// tables).  A wavefront owns 64 "vector columns": W = 64 / O columns of the target,
+// fusion plan; per batch element the block matrices F_b are built from its parameters,
+// k_fuse_blocks).  A wavefront owns 64 "vector columns": W = 64 / O columns of the target,
 // each split into O = 2^N / 16 outer groups of the 16 rows its block touches.  Per
 // block it computes Y = F_b X for its 64 vector columns as four 16 x 16 output tiles,
 // 16 MFMAs each (four real products, K = 16 in four steps):
@@ -14,7 +14,9 @@
 // cost needs only row c + trace_off of each column c: a 16-term dot product with that
 // row of F_nb per column replaces the block product.  The target
 // is read once per wavefront (it is shared by the batch and stays in L2); nothing
-// else touches HBM but the block matrices and the per-column trace entries.
+// else touches HBM but the block matrices and the per-column trace entries.  The columns
+// come in (and, in the store pass, go out) through the regions of all the workgroup's
+// wavefronts, so it is the workgroup that owns them in that pass.
 //
 // Row j of a column under block b: j = base_b[o] + off_b[i] for local index i (bit q of
 // i <-> the q-th smallest qubit of the block, as apply_large_kernel_to_input,
@@ -210,8 +212,8 @@ __global__ __launch_bounds__(256, 2) void k_fused_cost(FusedCostArgs a, const in
 // column n holds column w = n >> lg_b, support group k = n & (2^lg_b - 1), rows
 // kb_b[k] | (rho_w & nS_b) | off_b[i] (kTraceMapStride ints per block: off[16],
 // kb[64], lg, nS).  Only the first ceil(W 2^lg_b / 16) tiles carry work.  Rows outside
-// the support are never stored; loads test the row against the previous block's
-// support instead.  Every launch shape performs the same operations per column in the
+// the support are never stored: the region starts at zero, and since the supports only
+// grow they read as zero until a block reaches them.  Every launch shape performs the same operations per column in the
 // same order: results are bit-identical across shapes.
 
 // The chain's regions are padded below 8 qubits, where a tile's 16 vector columns are of

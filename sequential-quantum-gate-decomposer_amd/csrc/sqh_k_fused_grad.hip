@@ -10,8 +10,8 @@
 //                                                              (MFMA on transposed tiles)
 //   Y_{b-1} = F_b^T Y_b                                        (MFMA)
 // so that dTr/dtheta = sum_ik (dF_b/dtheta)_ik M_b[i][k] for a parameter of block b.
-// A wavefront sums its M_b over its column groups in registers and its own partials, so no
-// wavefront waits for another; k_fused_block_corr then sums the partials and runs the
+// A wavefront sums its M_b over its task's column groups (a node of FusedGradSplit's tree) in
+// registers and memory of its own, so no wavefront waits for another; k_fused_block_corr then sums the partials and runs the
 // block's gates backwards, producing each gate's 2x2 correlations in the layout of the
 // register-tile adjoint kernel, from which k_finish forms the gradient.
 //

@@ -310,9 +310,9 @@ class Context:
         self.check(self._L.sqh_set_jit(self.h, int(bool(enable))))
 
     def set_fused_cost(self, mode=True):
-        """Batched evaluations through the fused 4-qubit blocks on the matrix cores
-        (4-10 qubits, costs without correction channels): True / False, or "auto" (the
-        default: where it measured faster than the register-tile kernels in use)."""
+        """Evaluations, apply_to and derivatives through the fused 4-qubit blocks on the
+        matrix cores (4-10 qubits, costs without correction channels): True / False, or "auto"
+        (the default: where it measured faster than the register-tile kernels in use)."""
         m = FUSED_COST_AUTO if mode == "auto" else (FUSED_COST_ON if mode else FUSED_COST_OFF)
         self.check(self._L.sqh_set_fused_cost(self.h, m))
 
