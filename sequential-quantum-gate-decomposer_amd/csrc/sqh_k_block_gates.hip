@@ -167,7 +167,7 @@ __device__ __forceinline__ void partial_nodes(const double* __restrict__ M, unsi
 template <int E>
 __device__ __forceinline__ void partial_sum(const double* __restrict__ M, unsigned stride, int n, int up, int step,
                                             double (&out)[E]) {
-    constexpr int C = E == 1 ? 64 : 16;  // as many partials at a time as registers hold
+    constexpr int C = 16;  // partials at a time; 64 of one entry leave a CU one workgroup
 #pragma unroll
     for (int i = 0; i < E; ++i) out[i] = 0.0;
     for (int c = 0; c < n; c += 1 << up) {
@@ -182,13 +182,8 @@ __device__ __forceinline__ void partial_sum(const double* __restrict__ M, unsign
             double s[128 / C][E];
 #pragma unroll
             for (int j = 0; j < 128 / C; ++j) {
-                const int l = left - C * j;  // a chunk's last partials in a block no wider than they need
-                if (l > (C > 16 ? 32 : 0)) {
-                    partial_nodes<C>(P + C * j * stride, stride, l, step, s[j]);
-                } else if (l > 16) {
-                    partial_nodes<32>(P + C * j * stride, stride, l, step, s[j]);
-                } else if (l > 0) {
-                    partial_nodes<16>(P + C * j * stride, stride, l, step, s[j]);
+                if (C * j < left) {
+                    partial_nodes<C>(P + C * j * stride, stride, left - C * j, step, s[j]);
                 } else {
 #pragma unroll
                     for (int i = 0; i < E; ++i) s[j][i] = 0.0;
@@ -212,10 +207,11 @@ __device__ __forceinline__ void partial_sum(const double* __restrict__ M, unsign
 // element), an entry per thread, then only the first wavefront goes on; else a wavefront per
 // (block, element), four elements per workgroup), starts from x = the
 // columns of F_b and y = the columns of M_b and walks the gates backwards: x <- G^dagger x,
-// the pair correlations of y and x summed over the wavefront, y <- G^T y.
+// the pair correlations of y and x summed over the wavefront, y <- G^T y.  Two workgroups per
+// CU with SPLIT (564 workgroups on 5 qubits: 25.2 us against 26.6 with one), three else.
 // corr[e][slot][8] is the register-tile adjoint's layout.
 template <typename R, bool SPLIT>
-__global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 2 : 3) void k_fused_block_corr(const uint32_t* __restrict__ ops,
+__global__ __launch_bounds__(SPLIT ? 512 : 256, SPLIT ? 4 : 3) void k_fused_block_corr(const uint32_t* __restrict__ ops,
                                                           const int* __restrict__ first, int nb,
                                                           const cpx<R>* __restrict__ kern, long long kern_bstride,
                                                           const double* __restrict__ params, int pstride,
