@@ -377,11 +377,12 @@ bool fused_grad_uses_chain(const sqh_ctx* c) {
 // columns (live: at most B, counted on the device): the shape set by
 // sqh_set_fused_grad_config when it fits, else four 16-column tiles per wavefront from 9
 // qubits or from 64 elements (fewer partials), two below (more wavefronts for small
-// batches), and four wavefronts per workgroup, fewer where every wavefront can then have a
-// compute unit's LDS to itself (256 one-group tasks on 5 and 6 qubits: 62 and 83 us a call
-// instead of 71 and 90; from 1024 tasks on, small workgroups are packed on some of the
-// units: 117 instead of 91) -- the fastest shapes measured on MI355X -- with the scratch it
-// needs.  Returns false when no shape fits the device's LDS.
+// batches), and four wavefronts per workgroup, fewer where the units then share the work
+// more evenly: one up to 256 column groups (5 and 6 qubits: 62 and 83 us a call instead of 71
+// and 90), two up to 512, one up to 768 (560 groups on 6 qubits: 98, 132 and 103 us with one,
+// two and four); beyond, small workgroups are packed on some of the units (900 groups on 5
+// qubits: 138 us instead of 116).  These are the fastest shapes measured on MI355X.  Also the
+// scratch it needs.  Returns false when no shape fits the device's LDS.
 bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, bool live, FusedGradPlan& p) {
     const int N = c->prog.N, nb = (int)c->fplan.qubits.size(), ns = (int)c->prog.slots.size();
     p.T = 0;
@@ -391,7 +392,7 @@ bool fused_grad_plan(const sqh_ctx* c, bool f32, int B, int m, bool live, FusedG
     } else {
         for (int t : {N >= 9 || B >= 64 ? 4 : 2, 4}) {
             const long long groups = (long long)B * fused_grad_groups(N, m, t);
-            for (int w : {live || groups > 512 ? 4 : groups > 256 ? 2 : 1, 1})
+            for (int w : {live || groups > 768 ? 4 : groups > 256 && groups <= 512 ? 2 : 1, 1})
                 if (fused_grad_shape_valid(f32, N, m, nb, t, w)) {
                     p.T = t;
                     p.waves = w;
