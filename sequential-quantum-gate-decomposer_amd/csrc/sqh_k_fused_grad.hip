@@ -66,15 +66,25 @@ __device__ __forceinline__ void fg_mma(const FcA<R>& A, const R (&xr)[T][4], con
     }
 }
 
-// What a wavefront of the gradient kernels works on: the column groups first .. last - 1 of
-// element e, a node of the summation tree (FusedGradSplit), whose correlations go to part;
-// sums pending at level l > 0 of the tree wait in pend + (l - 1) nb 512, at level 0 in part.
+// What a wavefront of the gradient kernels works on: n column groups of element e, a node of
+// the summation tree (FusedGradSplit), whose correlations go to part; sums pending at level
+// l > 0 of the tree wait in pend + (l - 1) nb 512, at level 0 in part.
+//
+// The same node of all full chunks goes to wavefronts side by side, which read neighbouring
+// columns.  A column has 16 bytes of a cache line in each row; with chunks of consecutive
+// columns the lines were gone from the L2 before a task came to the next of them (calls of 23
+// vectors on 10 qubits in 3 blocks: 513 us, 803 so; 365 and 680 in complex64).
 struct FgTask {
-    int e, first, last;
+    int e, first, stride, chunk, n;
     bool live;
     double *part, *pend;
+    template <int T>
+    __device__ int group(int turn) const {  // its turn-th; with two tiles in the pairs that four would take
+        const int p = first + turn;
+        return T == 4 ? p * stride + chunk : ((p >> 1) * stride + chunk) * 2 + (p & 1);
+    }
 };
-template <int T>
+template <int T, int W>
 __device__ __forceinline__ FgTask fg_task(const FusedGradArgs& a, int wv) {
     FusedGradSplit sp = a.split;
     // The workgroups of either part of the split ordered for the XCDs, each XCD a contiguous
@@ -100,12 +110,25 @@ __device__ __forceinline__ FgTask fg_task(const FusedGradArgs& a, int wv) {
     t.live = id < (long long)n * per;
     const int k = (int)(id / per), c = (int)(id % per);
     t.e = (rest ? sp.n0 : 0) + k;
-    t.first = c << l;
-    t.last = min((c + 1) << l, sp.groups);
-    const long long before = rest ? (long long)sp.n0 * per0 : 0;
+    constexpr int levels = fused_grad_levels(T);
+    const int full = a.m / (W << levels), nodes = 1 << (levels - l);  // full chunks; a chunk's nodes
+    int node = c;  // the task's place in the tree's order
+    if (c < full * nodes) {
+        t.chunk = c % full;
+        t.stride = full;
+        t.first = c / full << l;
+        t.n = 1 << l;
+        node = t.chunk * nodes + c / full;
+    } else {
+        t.chunk = 0;
+        t.stride = 1;
+        t.first = c << l;
+        t.n = min(1 << l, sp.groups - t.first);
+    }
+    const long long before = rest ? (long long)sp.n0 * per0 : 0, at = (long long)k * per + node;
     const long long size = (long long)a.nb * 512;
-    t.part = a.mpart + (before + id) * size;
-    t.pend = a.pend + (before * max(sp.l0 - 1, 0) + id * max(l - 1, 0)) * size;
+    t.part = a.mpart + (before + at) * size;
+    t.pend = a.pend + (before * max(sp.l0 - 1, 0) + at * max(l - 1, 0)) * size;
     return t;
 }
 
@@ -136,12 +159,11 @@ __device__ __forceinline__ void fg_load_target(const cpx<R>* __restrict__ U, con
 // idled.  idx: the group's number in the task; the sums pending are those of idx's set bits.
 template <typename R, int T, typename Y>
 __device__ __forceinline__ void fg_correlate(R* lds, const Y& yr, const Y& yi, const R (&xr)[T][4],
-                                             const R (&xi)[T][4], const FgTask& task, int nb, int b, int cg,
+                                             const R (&xi)[T][4], const FgTask& task, int nb, int b, int idx,
                                              int lane) {
     typedef FcMfma<R> MF;
     const int nl = lane & 15, g = lane >> 4;
-    const unsigned idx = cg - task.first;
-    const bool last = cg + 1 == task.last;
+    const bool last = idx + 1 == task.n;
     const unsigned carry = idx & ~(idx + 1);  // the levels whose second half this group completes
     unsigned set = last ? idx : carry;
     auto at_level = [&](int l) { return (l ? task.pend + (long long)(l - 1) * nb * 512 : task.part) + b * 512; };
@@ -218,15 +240,15 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const in
     extern __shared__ __align__(16) unsigned char fg_smem[];
     int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const FgTask task = fg_task<T>(a, wv);
+    const FgTask task = fg_task<T, W>(a, wv);
     if (!task.live) return;
     const int e = task.e, m = a.m;
     const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 2 * Reg::PL};
     const cpx<R>* U = static_cast<const cpx<R>*>(a.U);
     if (a.count) U += (long long)a.run_target[a.elem_run[e]] * a.tgt_stride;
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.nb * 256;
-    for (int cg = task.first; cg < task.last; ++cg) {
-        const int c0 = cg * W;
+    for (int turn = 0; turn < task.n; ++turn) {
+        const int c0 = task.template group<T>(turn) * W;
         const int nl = lane & 15, g = lane >> 4;
         R xr[T][4], xi[T][4], yr[T][4], yi[T][4];
         FcA<R> A;
@@ -280,7 +302,7 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad(FusedGradArgs a, const in
                     xr[t][s] = dr[t][s];
                     xi[t][s] = di[t][s];
                 }
-            fg_correlate<R, T>(lds.p, yr, yi, xr, xi, task, a.nb, b, cg, lane);
+            fg_correlate<R, T>(lds.p, yr, yi, xr, xi, task, a.nb, b, turn, lane);
             if (b == 0) break;
             fg_mma<R, T, false>(A, yr, yi, dr, di);
             A.load_t(Fe + (long long)(b - 1) * 256, nl, g);
@@ -322,15 +344,15 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
     extern __shared__ __align__(16) unsigned char fg_smem[];
     int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const FgTask task = fg_task<T>(a, wv);
+    const FgTask task = fg_task<T, W>(a, wv);
     if (!task.live) return;
     const int e = task.e, m = a.m;
     const Reg lds{reinterpret_cast<R*>(fg_smem) + wv * 2 * Reg::PL};
     const cpx<R>* U = static_cast<const cpx<R>*>(a.U);
     if (a.count) U += (long long)a.run_target[a.elem_run[e]] * a.tgt_stride;
     const cpx<R>* Fe = static_cast<const cpx<R>*>(a.F) + (long long)e * a.nb * 256;
-    for (int cg = task.first; cg < task.last; ++cg) {
-        const int c0 = cg * W;
+    for (int turn = 0; turn < task.n; ++turn) {
+        const int c0 = task.template group<T>(turn) * W;
         asm volatile("" : "+v"(lane));  // no lane's addresses kept in registers from group to group
         const int nl = lane & 15, g = lane >> 4;
         // phase 1: Z_1 in block 0's grouping, X = the target's columns there, and the trace
@@ -366,7 +388,7 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
         constexpr bool AHEAD = T == 4;
         FcA<R> An;
         if constexpr (AHEAD) An.load_n(Fe, nl, g);
-        fg_correlate<R, T>(lds.p, zr, zi, xr, xi, task, a.nb, 0, cg, lane);
+        fg_correlate<R, T>(lds.p, zr, zi, xr, xi, task, a.nb, 0, turn, lane);
         // phase 2, one step up: X_b into block b + 1's grouping, Z_{b+2} (block b + 1's
         // grouping, as a result) from Z_{b+1} -- block 0's operand for the first step, the
         // last step's result after it -- then M_{b+1}.  The first step runs on its own, so
@@ -413,7 +435,7 @@ __global__ __launch_bounds__(512, 2) void k_fused_grad_chain(FusedGradArgs a, co
                     }
                 }
             }
-            fg_correlate<R, T>(lds.p, er, ei, xr, xi, task, a.nb, b + 1, cg, lane);
+            fg_correlate<R, T>(lds.p, er, ei, xr, xi, task, a.nb, b + 1, turn, lane);
         };
         step(0, std::true_type{});
         for (int b = 1; b + 1 < a.nb; ++b) step(b, std::false_type{});

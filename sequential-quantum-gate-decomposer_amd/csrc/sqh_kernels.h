@@ -157,7 +157,8 @@ hipError_t launch_fuse_deriv_blocks(const uint32_t* ops, const int* first, int n
 //
 // How the correlations of an element's column groups are summed, whoever computes them: the
 // groups of each chunk of 2^fused_grad_levels(T) as a binary tree over aligned pairs, then
-// the chunks in order.  A wavefront takes 2^l aligned groups, a node of the tree, as its
+// the chunks in order.  Full chunks are interleaved (of F, chunk k's groups of four tiles are k,
+// k + F, ...), so that tasks side by side stay at neighbouring columns as they proceed.  A wavefront takes 2^l aligned groups, a node of the tree, as its
 // task and leaves the node's sum in a partial; k_fused_block_corr does the rest of the tree.
 // So the result's bits depend neither on l nor on the batch (nor on T: a group of four tiles
 // is a node of two groups of two).
