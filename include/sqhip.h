@@ -115,7 +115,8 @@ int sqh_apply_to(sqh_ctx* ctx, const void* params, void* inout, int rows, int co
 /* Device variant: B matrices at inout + b*bstride elements, parameters shared
  * (pbstride = 0) or per matrix (pbstride = P).  Up to 10 qubits it runs the register-tile
  * kernels, or -- where sqh_set_fused_cost selects it (by default where the blocks do little
- * enough arithmetic beside the gates; on 4 qubits up to 4096 matrices) -- the tile-resident
+ * enough arithmetic beside the gates, and not for thousands of parameter vectors that each
+ * act on few columns) -- the tile-resident
  * pass of the circuit's fused 4-qubit blocks on the matrix cores, which writes each column
  * back to where it read it.  Above 10 qubits the blocks run with whole columns in a
  * workgroup's LDS where that is the faster way (to 13 qubits; on 14 in complex64 for deep
@@ -329,8 +330,9 @@ int sqh_get_jit_stats(sqh_ctx* ctx, double* compile_ms, int* compiles);
  * faster than the tile kernels, by the qubits and the blocks' arithmetic over the gates' --
  * against the run-time specialised kernels from 7 qubits when the blocks do no more;
  * against the generic ones from 4 qubits for deep circuits and from 6 for all but shallow
- * ones).  _AUTO looks at the batch only on 4 qubits, where complex64 batches beyond 4096
- * vectors take the tile kernels.  The fused blocks give a vector the same bits in every
+ * ones).  _AUTO looks at the batch where thousands of vectors meet few columns, which go to
+ * the tile kernels: on 4 qubits complex64 beyond 4096 vectors; on more, targets of up to 512
+ * entries (256 for complex128 gradients; complex128 costs never) beyond 2048.  The fused blocks give a vector the same bits in every
  * batch.  The same mode selects the fused blocks' adjoint for cost + gradient batches
  * (sqh_optimization_problem_combined_batch[_dev]; _AUTO: from 6 qubits against the
  * specialised kernels): forward and backward block products on the matrix cores, each

@@ -273,7 +273,7 @@ double fused_ratio(const sqh_ctx* c, bool grad) {
 // register-tile kernels.  Against the circuit-specialised ones: from 7 qubits (with a
 // gradient from 6), when the blocks do no more arithmetic than the gates.  Against the
 // generic ones the line is the arithmetic ratio up to which both precisions gain at
-// B = 1 to 4096 (time of the tile kernels over that of the fused ones).  With the one exception
+// B = 1 to 4096 (time of the tile kernels over that of the fused ones).  With the exceptions
 // below it does not look at B, and neither do the fused kernels' sums, so that a vector's
 // result does not depend on the batch it came in:
 //   gradients  8+ qubits: 2.5 (1.3 - 3.2 at 1.9 - 2.4, 2.0 - 6.1 below 1.2)
@@ -287,15 +287,24 @@ double fused_ratio(const sqh_ctx* c, bool grad) {
 // On 4 qubits a block is the whole circuit, its gates in FP64 are most of the work, and beyond
 // 4096 elements the card is full of them: larger complex64 batches and matrices go back to the
 // tile kernels (8192 and 20000: complex64 costs 0.7 - 0.8, gradients 0.7 - 0.8, store pass 0.6 -
-// 0.7, in complex128 0.8 - 0.9).  Complex128 costs and gradients (0.9 - 1.3) do not: runs in
+// 0.7, in complex128 0.8 - 0.9).  Complex128 costs and gradients (0.9 - 1.3) do not.
+// It is the same on more qubits with few columns, where the blocks' 256 entries are built for
+// each of B parameter vectors and then act on not many more.  Beyond 2048 vectors, up to 512
+// entries a matrix (256 for complex128 gradients) go to the tile kernels: at 4096 costs 0.7 -
+// 0.95, gradients 0.5 - 0.95, store pass 0.6 - 1, at 8192 and 16384 0.3 - 0.8; up to 2048, and
+// with twice the entries, 0.9 - 1.6.  Complex128 costs do not (0.7 - 1): runs in
 // lockstep (sqh_agents_batch) end at the bits of single ones whatever their batches.
-constexpr int kFused4Batch = 4096;
+constexpr int kFused4Batch = 4096, kFusedFewBatch = 2048, kFusedFewEntries = 512;
 enum FusedKind { FUSED_COST_PASS, FUSED_STORE_PASS, FUSED_GRAD_PASS };
-bool fused_auto(const sqh_ctx* c, FusedKind kind, bool f32, int B) {
+// B: parameter vectors; m: columns of a matrix.
+bool fused_auto(const sqh_ctx* c, FusedKind kind, bool f32, int B, int m) {
     const int N = c->prog.N;
     const double r = fused_ratio(c, kind == FUSED_GRAD_PASS);
     if (c->jit) return N >= (kind == FUSED_GRAD_PASS ? 6 : 7) && r <= 1.0;
     if (N == 4 && B > kFused4Batch && (kind == FUSED_STORE_PASS || f32)) return false;
+    if (N > 4 && B > kFusedFewBatch && (kind != FUSED_COST_PASS || f32) &&
+        ((long long)m << N) <= (kind == FUSED_GRAD_PASS && !f32 ? kFusedFewEntries / 2 : kFusedFewEntries))
+        return false;
     static const double line[3][5] = {{0.25, 1.0, 1.2, 1.2, 1.5}, {0.25, 1.0, 1.0, 1.2, 1.2}, {0.3, 1.0, 1.5, 1.5, 2.5}};
     return r <= line[kind][std::min(N, 8) - 4];
 }
@@ -304,15 +313,15 @@ bool fused_auto(const sqh_ctx* c, FusedKind kind, bool f32, int B) {
 // fused-block kernel: 4 <= N <= 10, the circuit has blocks, and the switch is on, or
 // automatic (the default) and the rule above holds.  Costs also need no correction channels
 // (fused_cost_applies).
-bool fused_pass_applies(const sqh_ctx* c, bool store, bool f32, int B) {
+bool fused_pass_applies(const sqh_ctx* c, bool store, bool f32, int B, int m) {
     if (!fused_plan_fits(c)) return false;
     if (c->fused_cost == SQH_FUSED_COST_AUTO)
-        return fused_auto(c, store ? FUSED_STORE_PASS : FUSED_COST_PASS, f32, B);
+        return fused_auto(c, store ? FUSED_STORE_PASS : FUSED_COST_PASS, f32, B, m);
     return c->fused_cost == SQH_FUSED_COST_ON;
 }
 
-bool fused_cost_applies(const sqh_ctx* c, bool grad, const TraceSpec& ts, bool f32, int B) {
-    return !grad && ts.nch == 0 && fused_pass_applies(c, false, f32, B);
+bool fused_cost_applies(const sqh_ctx* c, bool grad, const TraceSpec& ts, bool f32, int B, int m) {
+    return !grad && ts.nch == 0 && fused_pass_applies(c, false, f32, B, m);
 }
 
 // The 2x2 kernels of a batch computed from its parameters where they are used.
@@ -417,7 +426,7 @@ bool fused_grad_applies(const sqh_ctx* c, const TraceSpec& ts, bool f32, int B, 
                         FusedGradPlan* plan) {
     if (ts.nch != 0 || !fused_plan_fits(c)) return false;
     const bool automatic = c->fused_cost == SQH_FUSED_COST_AUTO;
-    if (c->fused_cost == SQH_FUSED_COST_OFF || (automatic && !fused_auto(c, FUSED_GRAD_PASS, f32, B))) return false;
+    if (c->fused_cost == SQH_FUSED_COST_OFF || (automatic && !fused_auto(c, FUSED_GRAD_PASS, f32, B, m))) return false;
     FusedGradPlan p;
     if (!fused_grad_plan(c, f32, B, m, live, p)) return false;
     if (plan) *plan = p;
@@ -570,7 +579,7 @@ int eval_batch(sqh_ctx* c, const double* d_params, int B, int precision, double*
     // the fused blocks' kernels compute their 2x2 kernels from the parameters: no table
     FusedGradPlan fgp;
     const bool fused_grad = d_grad && !fixed && fused_grad_applies(c, ts, f32, B, m, false, &fgp);
-    const bool fused_costs = !fixed && fused_cost_applies(c, d_grad != nullptr, ts, f32, B);
+    const bool fused_costs = !fixed && fused_cost_applies(c, d_grad != nullptr, ts, f32, B, m);
     if (fused_grad && fgp.bytes() > kFusedGradScratch && B > 1) {
         // part by part; an element's result does not depend on the others
         const int part = (int)std::max<size_t>(1, B / ((fgp.bytes() + kFusedGradScratch - 1) / kFusedGradScratch));
@@ -706,7 +715,7 @@ int eval_targets(sqh_ctx* c, const double* d_params, int B, const void* d_target
     if (rows != (1 << N) || cols <= 0 || cols + off > rows)
         return fail(c, SQH_ERR_ARG, "targets must be %d x m with m + trace offset <= %d", 1 << N, 1 << N);
     const TraceSpec ts = trace_spec(c, B, m);
-    const bool fused_costs = fused_cost_applies(c, false, ts, false, B);
+    const bool fused_costs = fused_cost_applies(c, false, ts, false, B, m);
     if (!fused_costs && (rc = build_kernels(c, d_params, B, false))) return rc;
     HIPTRY(c, c->d_diag.ensure((size_t)(ts.nch + 1) * B * m * 2 * sizeof(double)));
     TileLaunch t = base_launch(c, false);
@@ -753,7 +762,7 @@ int apply_dev(sqh_ctx* c, const double* d_params, int pbstride, void* d_inout, i
         return fused_big_apply(c, d_inout, stride, bstride, d_inout, stride, bstride, cols, B, f32, d_params, pbstride);
     if (path == 0 && N > kMaxTileQubits) path = 2;
     if (path == 2) return fused_apply(c, d_inout, rows, cols, stride, bstride, B, f32, d_params, pbstride);
-    const bool fused = path == 0 && fused_pass_applies(c, true, f32, B);
+    const bool fused = path == 0 && fused_pass_applies(c, true, f32, Bk, cols);
     if (!fused && (rc = build_kernels(c, d_params, Bk, f32))) return rc;
     if (fused) {
         // the circuit's fused 4-qubit blocks on the matrix cores, every column resident
@@ -816,7 +825,7 @@ int deriv_dev(sqh_ctx* c, const double* d_params, const void* d_in, int rows, in
         return fail(c, SQH_ERR_ARG, "apply_derivate_to supports up to %d qubits", kMaxTileQubits);
     if (c->prog.slots.empty()) return SQH_OK;
     const int ns = (int)c->prog.slots.size(), P = c->prog.P;
-    if (fused_pass_applies(c, true, false, P)) {
+    if (fused_pass_applies(c, true, false, 1, cols)) {
         // Through the fused blocks: a derivative shares the blocks before its gate's with
         // the others, so the products F_{b-1} ... F_0 in are formed once per block and
         // element k starts from its block's, with that block differentiated.  The 8-qubit

@@ -156,3 +156,49 @@ def test_four_qubits_across_the_batch_line(oracle, B):
         for b in few:
             want = oracle.apply_to(gates, ps[b], U)
             assert np.linalg.norm(M[b].cpu().numpy() - want) <= tol * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("B", [2048, 2049])
+@pytest.mark.parametrize("n,m", [(5, 8), (7, 4)])
+def test_few_columns_across_the_batch_line(oracle, n, m, B):
+    """Around the batch beyond which matrices of few entries run the tile kernels: complex128
+    costs keep their bits, the rest agrees to rounding with a small batch and the oracle; so do
+    matrices that share one parameter vector."""
+    gates = W.ansatz_layers(n, W.alternating_pairs(n, 3 * n))
+    d, P = 1 << n, W.param_count(gates)
+    U = np.ascontiguousarray(W.haar_unitary(d, 3)[:, :m])
+    ps = W.random_params(P, 4, batch=B)
+    ctx = nat.Context(0)
+    ctx.set_circuit(n, gates)
+    ctx.set_target(U)
+
+    def both(p, prec):
+        b = p.shape[0]
+        c, f, g = np.empty(b), np.empty(b), np.empty((b, P))
+        p = np.ascontiguousarray(p)
+        ctx.check(ctx._L.sqh_optimization_problem_batch(ctx.h, p.ctypes.data, b, prec, c.ctypes.data))
+        ctx.check(ctx._L.sqh_optimization_problem_combined_batch(ctx.h, p.ctypes.data, b, prec, f.ctypes.data,
+                                                                 g.ctypes.data))
+        return c, f, g
+
+    few = [0, B // 2, B - 1]
+    for prec, tol in ((nat.PREC_F64, 1e-12), (nat.PREC_F32, 2e-5)):
+        many, small = both(ps, prec), both(ps[few], prec)
+        for x, y in zip(many, small):
+            assert np.abs(x[few] - y).max() <= tol
+        if prec == nat.PREC_F64:
+            assert np.array_equal(many[0][few], small[0])
+            for i, b in enumerate(few):
+                f, g = oracle.optimization_problem_combined(gates, U, n, ps[b])
+                assert abs(many[0][b] - f) < 1e-12 and np.abs(many[2][b] - g).max() < 1e-12
+    for dt, tol in ((torch.complex128, 1e-12), (torch.complex64, 1e-5)):
+        for shared in (False, True):
+            M = torch.from_numpy(np.broadcast_to(U, (B, d, m)).copy()).cuda().to(dt)
+            dp = torch.from_numpy(ps).cuda()
+            torch.cuda.synchronize()
+            ctx.check(ctx._L.sqh_apply_to_dev(ctx.h, dp.data_ptr(), 0 if shared else P, M.data_ptr(), d, m, m, d * m, B,
+                                              int(dt == torch.complex64)))
+            ctx.synchronize()
+            for b in few:
+                want = oracle.apply_to(gates, ps[0 if shared else b], U)
+                assert np.linalg.norm(M[b].cpu().numpy() - want) <= tol * np.linalg.norm(want)
