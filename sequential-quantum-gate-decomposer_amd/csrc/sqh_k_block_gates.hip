@@ -13,7 +13,7 @@
 // code that a gate runs is kept short enough to stay in the instruction cache: the same
 // few operations for every pair, where a walk with every target and control of a 16-row
 // register column unrolled took 27 us a block build and 74 us a correlation walk with the
-// partials' sum (8 qubits, one element; 30 and 100 for 512).  Now 13 and 29 (16 and 36),
+// partials' sum (8 qubits, one element; 30 and 100 for 512).  Now 13 and 28 (16 and 36),
 // with the kernel table's launch gone: gradient of one 8-qubit vector 209 -> 95 us.
 // Both compute in FP64 in either precision: a complex64 block matrix is then rounded once,
 // not after each of its gates.
